@@ -3,11 +3,15 @@
 #include <stdlib.h>
 
 #include "gemm_kernel.h"
+#include "gemm_wide_kernel.h"
 #include "host_common.h"
 
 #include <atomic>
 
 namespace flute {
+
+flute_status gemm_wide_f16(int mb, int b1, int b2, int slices, const WideParams &p, hipStream_t stream);
+flute_status gemm_wide_bf16(int mb, int b1, int b2, int slices, const WideParams &p, hipStream_t stream);
 
 namespace {
 
@@ -27,7 +31,7 @@ struct GemmShape {
 // with eight k ways while that fits the device in one round, else 128 rows (two m groups,
 // four k ways); further rows go to gridDim.y.  The tables plus staging take most of a
 // CU's LDS, so one workgroup per CU is resident.  FLUTE_GEMM_ROWS = 16, 32, 64 or 128
-// forces the shape (a tuning and test knob, like FLUTE_GEMV_RW).
+// forces the shape (a tuning and test knob, like FLUTE_GEMV_RW), 256 or 512 the many-row kernel.
 GemmShape choose_gemm_shape(int M, int tiles, int64_t index_bytes) {
     {
         const int v = tuning().gemm_rows;
@@ -101,6 +105,21 @@ flute_status launch_gemm_shape(const GemmShape &s, const GemmParams &p, dim3 gri
 }
 
 
+// xb[m, r] = sum_k A[m, k] * resB[r, k] in fp32.
+flute_status launch_coeff(const void *A, int64_t lda, const void *resB, float *xb, int M, int K, int R, int is_bf16,
+                          hipStream_t stream) {
+    const dim3 grid((M + 15) / 16, (R + 15) / 16);
+    const int aligned = ((uintptr_t)A & 15) == 0 && lda % 8 == 0 && ((uintptr_t)resB & 15) == 0;
+    if (is_bf16)
+        hipLaunchKernelGGL(gemm_coeff_kernel<true>, grid, dim3(1024), 0, stream, (const uint16_t *)A, lda,
+                           (const uint16_t *)resB, xb, M, K, R, aligned);
+    else
+        hipLaunchKernelGGL(gemm_coeff_kernel<false>, grid, dim3(1024), 0, stream, (const uint16_t *)A, lda,
+                           (const uint16_t *)resB, xb, M, K, R, aligned);
+    FLUTE_HIP_CHECK(hipGetLastError());
+    return FLUTE_OK;
+}
+
 // LDS plan of one launch: pair tables (+ staging on the fast path), sized against the
 // reduction tree and the totals tile that reuse the same memory afterwards.
 // A single 4-bit stream with at most two LUT groups per 128-row tile gets 64-lane
@@ -149,6 +168,193 @@ int plan_lds(GemmParams &p, const GemmShape &shape) {
 
 }  // namespace flute
 
+namespace flute {
+namespace {
+
+// How the many-row kernel would serve a call; rows = 0: the other kernels do.
+struct WidePlan {
+    int rows;      // rows of A per workgroup: 512 or 256
+    int ksplit;
+};
+
+// The many-row kernel or the others, and its shape.  Each form's time is a line in what it has to
+// do, in microseconds, fitted to measurements (4-bit stream, bfloat16; `steps` = 64-k tiles of all
+// streams that a workgroup takes, `rounds` = workgroups / 256 CUs, rounded up):
+//   128-row workgroups of gemm_kernel.h   8 + 0.43 a tile (64-row ones 0.26) per round; two
+//                                         streams are two launches, other widths 15 % more
+//   512-row workgroups                    14 + 0.95 ... 1.35 a step (the clock falls as the chip
+//                                         fills); slices of K cost 5 each (256 KB written, read)
+//   256-row workgroups                    14 + 0.65 ... 0.90 a step; slices 2.5 each
+// e.g. M = 1024, 4096 -> 12288: 120 / 92 / 118 us (estimated 105 / 94 / 122); M = 512: 74 / 61
+// (two slices) / 61; M = 512, 12288 -> 4096: 59 / 77 (four) / 65 (four), the others stay; two
+// streams (4, 1) at M = 1024, 4096 -> 12288: 263 / 165 / 190, at M = 192: 76 / - / 60 (two).
+// Calls that the 16- and 32-row workgroups serve in one round stay with them (M = 128,
+// 4096 -> 12288: 27 us there, 41 us here).
+WidePlan choose_wide(int M, int tiles, int G, int streams, bool four_bit, const GemmShape &other) {
+    {
+        const int v = tuning().gemm_rows;
+        if (v == 512 || v == 256) {
+            const int k = tuning().gemm_ksplit;
+            return {v, k > 1 ? (k < G ? k : G) : 1};
+        }
+        if (v) return {0, 1};
+    }
+    if (other.mb < 4) return {0, 1};
+    const int rows_other = other.mb * other.mw * 16;
+    const int64_t units_other = (int64_t)tiles * ((M + rows_other - 1) / rows_other);
+    int ks_other = 1;
+    while (units_other * ks_other * 2 <= kNumCU && ks_other < 4 && G / (ks_other * 2) >= other.kw * 2) ks_other *= 2;
+    const double per_tile = (other.mw == 1 ? 0.26 : 0.43) * (four_bit && streams == 1 ? 1.0 : 1.15);
+    double best = streams * (double)((units_other * ks_other + kNumCU - 1) / kNumCU) *
+                  (8.0 + per_tile * G / ks_other) + (ks_other > 1 ? 5.0 : 0.0);
+    WidePlan plan = {0, 1};
+    for (int rows = 512; rows >= 256; rows /= 2) {
+        const int64_t units = (int64_t)tiles * ((M + rows - 1) / rows);
+        for (int ks = 1; ks <= 8 && G / ks >= 8; ks *= 2) {
+            const int64_t groups = units * ks, rounds = (groups + kNumCU - 1) / kNumCU;
+            const double fill = groups < kNumCU ? (double)groups / kNumCU : 1.0;
+            const double step = rows == 512 ? 0.95 + 0.40 * fill : 0.65 + 0.25 * fill;
+            const double us = 14.0 + rounds * (step * streams * ((G + ks - 1) / ks)) +
+                              (ks > 1 ? (rows == 512 ? 5.0 : 2.5) * ks : 0.0);
+            if (us < best) {
+                best = us;
+                plan = {rows, ks};
+            }
+        }
+    }
+    return plan;
+}
+
+// Up to four weights over the same rows of A: C[i] = A @ W[i]^T (+ residual, bias).  They share
+// their LUT's type and K; weights of one width pair go in one launch.
+flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *const *C, const int64_t *ldc, int M,
+                       int64_t lda, int act_dtype, WidePlan plan, hipStream_t stream) {
+    const int K = ws[0].K, G = K / 64, lut_dtype = ws[0].lut_dtype;
+    const int out_bf16 = act_dtype == FLUTE_BF16;
+    const bool scale_rows = act_dtype == FLUTE_BF16 && lut_dtype == FLUTE_F16;
+    const int mb = plan.rows / 128;
+    const int mtiles = (M + plan.rows - 1) / plan.rows, mblk = mtiles * plan.rows / 16;
+    const int gper = (G + plan.ksplit - 1) / plan.ksplit, slices = (G + gper - 1) / gper;
+    FLUTE_REQUIRE(slices <= 65535, FLUTE_ERR_UNSUPPORTED, "flute_gemm: %d slices of K exceed the grid", slices);
+
+    // what a weight needs of the activations: one image per distinct rotation
+    int image_of[kWideMaxSegs], owner[kWideMaxSegs], images = 0;
+    for (int i = 0; i < count; ++i) {
+        int k = 0;
+        while (k < images && !(ws[owner[k]].signs == ws[i].signs && ws[owner[k]].awq == ws[i].awq &&
+                               ws[owner[k]].rot_block == ws[i].rot_block))
+            ++k;
+        if (k == images) owner[images++] = i;
+        image_of[i] = k;
+    }
+    auto up4 = [](size_t n) { return (n + 3) & ~(size_t)3; };
+    const size_t image_floats = (size_t)K * mblk * 8, rot_floats = up4((size_t)M * K / 2);
+    const size_t shift_floats = scale_rows ? up4(M) : 0;
+    size_t xb_floats = 0;
+    int tiles = 0;
+    for (int i = 0; i < count; ++i) {
+        xb_floats += up4((size_t)M * ws[i].R);
+        tiles += ws[i].N / 128;
+    }
+    const size_t part_floats = slices > 1 ? (size_t)slices * mtiles * tiles * plan.rows * 128 : 0;
+    size_t total = part_floats + xb_floats + 64;
+    for (int k = 0; k < images; ++k) total += image_floats + shift_floats + (ws[owner[k]].signs ? rot_floats : 0);
+    float *base = nullptr;
+    int *tickets = nullptr;
+    flute_status st = get_workspace(total, (size_t)mtiles * tiles + 1, stream, &base, &tickets);
+    if (st != FLUTE_OK) return st;
+    float *next = base + part_floats;
+
+    const u4_t *image[kWideMaxSegs];
+    const int *shift[kWideMaxSegs];
+    const void *rows[kWideMaxSegs];
+    int64_t ldr[kWideMaxSegs];
+    for (int k = 0; k < images; ++k) {
+        const flute_linear &w = ws[owner[k]];
+        rows[k] = A;
+        ldr[k] = lda;
+        if (w.signs) {
+            st = fht_launch(A, lda, w.signs, w.awq, next, K, M, K, act_dtype, 0, w.rot_block, stream, nullptr);
+            if (st != FLUTE_OK) return st;
+            rows[k] = next;
+            ldr[k] = K;
+            next += rot_floats;
+        }
+        shift[k] = nullptr;
+        if (scale_rows) {
+            hipLaunchKernelGGL(gemm_rowshift_kernel, dim3(M), dim3(256), 0, stream, (const uint16_t *)rows[k], ldr[k], K,
+                               (int *)next);
+            FLUTE_HIP_CHECK(hipGetLastError());
+            shift[k] = (const int *)next;
+            next += shift_floats;
+        }
+        const int64_t blocks = (int64_t)(2 * G) * ((M + 15) / 16);
+        const int grid = (int)((blocks + 3) / 4 < 8192 ? (blocks + 3) / 4 : 8192);
+        hipLaunchKernelGGL(gemm_image_kernel, dim3(grid), dim3(256), 0, stream, (const uint16_t *)rows[k], (u4_t *)next, M,
+                           ldr[k], 2 * G, mblk, out_bf16, (int)(lut_dtype == FLUTE_BF16),
+                           (int)(((uintptr_t)rows[k] & 15) == 0 && ldr[k] % 8 == 0), shift[k]);
+        FLUTE_HIP_CHECK(hipGetLastError());
+        image[k] = (const u4_t *)next;
+        next += image_floats;
+    }
+    const float *xb[kWideMaxSegs];
+    for (int i = 0; i < count; ++i) {
+        xb[i] = nullptr;
+        if (ws[i].R == 0) continue;
+        xb[i] = next;
+        st = launch_coeff(rows[image_of[i]], ldr[image_of[i]], ws[i].resB, next, M, K, ws[i].R, out_bf16, stream);
+        if (st != FLUTE_OK) return st;
+        next += up4((size_t)M * ws[i].R);
+    }
+    bool done[kWideMaxSegs] = {};
+    for (int i = 0; i < count; ++i) {
+        if (done[i]) continue;
+        WideParams p = {};
+        p.M = M;
+        p.G = G;
+        p.mblk = mblk;
+        p.mtiles = mtiles;
+        p.gper = gper;
+        p.out_bf16 = out_bf16;
+        p.P = base;
+        p.tickets = tickets;
+        // the sum does not depend on the order of the streams beyond fp32 rounding: the wider first
+        const int b1 = ws[i].b1 > ws[i].b2 ? ws[i].b1 : ws[i].b2, b2 = ws[i].b1 + ws[i].b2 - b1;
+        for (int k = i; k < count; ++k) {
+            const flute_linear &w = ws[k];
+            const bool swap = w.b2 > w.b1;
+            if (done[k] || (swap ? w.b2 : w.b1) != b1 || (swap ? w.b1 : w.b2) != b2) continue;
+            done[k] = true;
+            WideSeg &g = p.seg[p.nsegs++];
+            g.q[0] = (const uint8_t *)(swap ? w.q2 : w.q1);
+            g.q[1] = (const uint8_t *)(swap ? w.q1 : w.q2);
+            g.lut[0] = (const uint16_t *)(swap ? w.lut2 : w.lut1);
+            g.lut[1] = (const uint16_t *)(swap ? w.lut1 : w.lut2);
+            g.Ap = image[image_of[k]];
+            g.rowshift = shift[image_of[k]];
+            g.xb = xb[k];
+            g.resA = (const uint16_t *)w.resA;
+            g.bias = (const uint16_t *)w.bias;
+            g.C = C[k];
+            g.ldc = ldc[k];
+            g.tile0 = p.ntiles;
+            g.gs = w.group_size;
+            g.lut_rows = w.lut_rows;
+            g.R = w.R;
+            g.vec_store = (ldc[k] % 8 == 0) && (((uintptr_t)C[k] & 15) == 0);
+            p.ntiles += w.N / 128;
+        }
+        st = lut_dtype == FLUTE_BF16 ? gemm_wide_bf16(mb, b1, b2, slices, p, stream)
+                                     : gemm_wide_f16(mb, b1, b2, slices, p, stream);
+        if (st != FLUTE_OK) return st;
+    }
+    workspace_done(stream);
+    return FLUTE_OK;
+}
+
+}  // namespace
+}  // namespace flute
+
 using namespace flute;
 
 extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C, int M,
@@ -166,13 +372,11 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
                   (long long)lda, w->K, (long long)ldc, w->N);
     FLUTE_REQUIRE(((uintptr_t)A & 1) == 0 && ((uintptr_t)C & 1) == 0, FLUTE_ERR_INVALID,
                   "flute_gemm: A and C must be 2-byte aligned");
-    FLUTE_REQUIRE(w->R == 0 || (int64_t)M * w->R <= 16384, FLUTE_ERR_UNSUPPORTED,
-                  "flute_gemm: the fused residual serves M*R <= 16384 (got M=%d, R=%d); add "
-                  "(A @ resB^T) @ resA^T outside for larger products",
-                  M, w->R);
     hipStream_t stream = (hipStream_t)stream_;
 
     GemmShape shape = choose_gemm_shape(M, w->N / 128, w->q1_bytes + (w->b2 > 0 ? w->q2_bytes : 0));
+    const WidePlan wide = choose_wide(M, w->N / 128, w->K / 64, w->b2 > 0 ? 2 : 1, w->b1 == 4, shape);
+    if (wide.rows) return gemm_wide(w, 1, A, &C, &ldc, M, lda, act_dtype, wide, stream);
     GemmParams p = {};
     p.nstreams = w->b2 > 0 ? 2 : 1;
     p.q[0] = (const uint8_t *)w->q1;
@@ -318,10 +522,8 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
         FLUTE_HIP_CHECK(hipGetLastError());
     }
     if (w->R > 0) {
-        hipLaunchKernelGGL(gemm_coeff_kernel, dim3(w->R, M), dim3(256), 0, stream,
-                           (const uint16_t *)A, lda, (const uint16_t *)w->resB, xb, w->K, w->R,
-                           p.out_bf16);
-        FLUTE_HIP_CHECK(hipGetLastError());
+        st = launch_coeff(A, lda, w->resB, xb, M, w->K, w->R, p.out_bf16, stream);
+        if (st != FLUTE_OK) return st;
         p.xb = xb;
     }
 

@@ -1,0 +1,74 @@
+// What the two LUT GEMM kernels share: operand types and the matrix instruction.
+#pragma once
+
+#include <type_traits>
+
+#include "common.h"
+
+namespace flute {
+
+typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
+
+// Activation image of the many-row kernel: operand (g, half j of the 64-k tile, 16-row block mb) is
+// 1 KB, lane kg*16 + row holding A[mb*16 + row][g*64 + j*32 + kg*8 ... + 7].  The 16-byte piece
+// that starts at column k (a multiple of 8) of row m:
+__host__ __device__ inline int64_t wide_piece(int m, int k, int mblk) {
+    return ((int64_t)(k >> 5) * mblk + (m >> 4)) * 64 + ((k >> 3) & 3) * 16 + (m & 15);
+}
+
+template <bool BF16>
+__device__ __forceinline__ f4_t mfma16(u4_t w, u4_t a, f4_t acc) {
+    if constexpr (BF16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8_t, w),
+                                                       __builtin_bit_cast(bf8_t, a), acc, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, w),
+                                                      __builtin_bit_cast(h8_t, a), acc, 0, 0, 0);
+}
+
+// Partial sums cross workgroups (and so the per-XCD L2s) inside one launch: they are
+// written through and read around the L2 with device-scope (sc1) accesses, the same
+// instructions a relaxed agent-scope atomic compiles to, but 16 bytes at a time.
+__device__ __forceinline__ void ws_store16(float *p, f4_t v) {
+    // s_nop: a store of more than 8 bytes reads its data registers after issue, and the
+    // compiler does not know what this statement is, so it would not keep the next write to
+    // those registers away from it
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+__device__ __forceinline__ void ws_stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// Four 16-byte device-scope loads in flight, complete on return.
+__device__ __forceinline__ void ws_load16x4(const float *p0, const float *p1, const float *p2,
+                                            const float *p3, f4_t &a, f4_t &b, f4_t &c, f4_t &d) {
+    asm volatile(
+        "global_load_dwordx4 %0, %4, off sc1\n"
+        "global_load_dwordx4 %1, %5, off sc1\n"
+        "global_load_dwordx4 %2, %6, off sc1\n"
+        "global_load_dwordx4 %3, %7, off sc1\n"
+        "s_waitcnt vmcnt(0)"
+        : "=&v"(a), "=&v"(b), "=&v"(c), "=&v"(d)
+        : "v"(p0), "v"(p1), "v"(p2), "v"(p3)
+        : "memory");
+}
+
+// Eight of them, `step` floats apart.
+__device__ __forceinline__ void ws_load16x8(const float *p, int64_t step, f4_t (&v)[8]) {
+    asm volatile(
+        "global_load_dwordx4 %0, %8, off sc1\n"
+        "global_load_dwordx4 %1, %9, off sc1\n"
+        "global_load_dwordx4 %2, %10, off sc1\n"
+        "global_load_dwordx4 %3, %11, off sc1\n"
+        "global_load_dwordx4 %4, %12, off sc1\n"
+        "global_load_dwordx4 %5, %13, off sc1\n"
+        "global_load_dwordx4 %6, %14, off sc1\n"
+        "global_load_dwordx4 %7, %15, off sc1\n"
+        "s_waitcnt vmcnt(0)"
+        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7])
+        : "v"(p), "v"(p + step), "v"(p + 2 * step), "v"(p + 3 * step), "v"(p + 4 * step), "v"(p + 5 * step),
+          "v"(p + 6 * step), "v"(p + 7 * step)
+        : "memory");
+}
+
+}  // namespace flute

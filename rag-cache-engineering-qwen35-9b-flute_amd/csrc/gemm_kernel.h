@@ -26,16 +26,10 @@
 // and a ticket; the last arrival folds them in a fixed order.
 #pragma once
 
-#include <type_traits>
 
-#include "common.h"
+#include "gemm_common.h"
 
 namespace flute {
-
-typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
-typedef float f4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
 
 #ifdef FLUTE_STAMPS
 // Instrumented builds only: per-wavefront phase times (s_memrealtime, 10 ns units) and the shader
@@ -200,6 +194,45 @@ __global__ void __launch_bounds__(256) gemm_prep_quad_kernel(const uint16_t *A, 
     }
 }
 
+// The activation image of the many-row kernel (wide_piece) from rows: a wavefront moves one 1 KB block,
+// sixteen rows by 64 bytes, so that every line of the image is written whole by one instruction.
+__global__ void __launch_bounds__(256) gemm_image_kernel(const uint16_t *A, u4_t *Ap, int M, int64_t lda, int segs,
+                                                         int mblk, int in_bf16, int out_bf16, int aligned,
+                                                         const int *rowshift) {
+    const int lane = threadIdx.x & 63;
+    const int64_t blocks = (int64_t)segs * ((M + 15) >> 4);          // (16-row block, 32-k segment)
+    for (int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); b < blocks; b += (int64_t)gridDim.x * 4) {
+        int mb, seg;
+        if (blocks <= 0x7fffffff) {                      // uniform; a 64-bit division costs some hundred instructions
+            mb = (int)((uint32_t)b / (uint32_t)segs);
+            seg = (int)((uint32_t)b - (uint32_t)mb * (uint32_t)segs);
+        } else {
+            mb = (int)(b / segs);
+            seg = (int)(b - (int64_t)mb * segs);
+        }
+        const int m = min(mb * 16 + (lane >> 2), M - 1); // rows past the end repeat the last: nobody stores their products
+        const uint16_t *src = A + (int64_t)m * lda + seg * 32 + (lane & 3) * 8;
+        u4_t v;
+        if (aligned) {
+            v = *(const u4_t *)src;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (uint32_t)src[2 * e] | ((uint32_t)src[2 * e + 1] << 16);
+        }
+        if (in_bf16 != out_bf16) {
+            const int shift = rowshift ? rowshift[m] : 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint16_t lo = (uint16_t)(v[e] & 0xffffu), hi = (uint16_t)(v[e] >> 16);
+                const float flo = ldexpf(in_bf16 ? bf2f(lo) : h2f(lo), -shift);
+                const float fhi = ldexpf(in_bf16 ? bf2f(hi) : h2f(hi), -shift);
+                v[e] = (uint32_t)round_act(flo, out_bf16) | ((uint32_t)round_act(fhi, out_bf16) << 16);
+            }
+        }
+        Ap[((int64_t)seg * mblk + mb) * 64 + (lane & 3) * 16 + (lane >> 2)] = v;
+    }
+}
+
 // bfloat16 rows in front of float16 operands: shift[m] = the power of two that brings the
 // largest magnitude of row m to [1, 2) (bf16_row_shift), one workgroup per row.
 __global__ void __launch_bounds__(256) gemm_rowshift_kernel(const uint16_t *A, int64_t lda, int K,
@@ -219,57 +252,35 @@ __global__ void __launch_bounds__(256) gemm_rowshift_kernel(const uint16_t *A, i
     if (threadIdx.x == 0) shift[blockIdx.x] = bf16_row_shift(e);
 }
 
-// xb[m, r] = sum_k A[m, k] * resB[r, k] in fp32 (one workgroup per (r, m)).
-__global__ void __launch_bounds__(256) gemm_coeff_kernel(const uint16_t *A, int64_t lda,
-                                                         const uint16_t *resB, float *xb, int K,
-                                                         int R, int is_bf16) {
-    const int r = blockIdx.x, m = blockIdx.y;
-    float s = 0.0f;
-    for (int k = threadIdx.x; k < K; k += 256)
-        s = fmaf(load_act(A, m * lda + k, is_bf16), load_act(resB, (int64_t)r * K + k, is_bf16), s);
-    __shared__ float red[256];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) xb[(int64_t)m * R + r] = red[0];
-}
-
-// Partial sums cross workgroups (and so the per-XCD L2s) inside one launch: they are
-// written through and read around the L2 with device-scope (sc1) accesses, the same
-// instructions a relaxed agent-scope atomic compiles to, but 16 bytes at a time.
-__device__ __forceinline__ void ws_store16(float *p, f4_t v) {
-    // s_nop: a store of more than 8 bytes reads its data registers after issue, and the
-    // compiler does not know what this statement is, so it would not keep the next write to
-    // those registers away from it
-    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
-}
-__device__ __forceinline__ void ws_stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// Four 16-byte device-scope loads in flight, complete on return.
-__device__ __forceinline__ void ws_load16x4(const float *p0, const float *p1, const float *p2,
-                                            const float *p3, f4_t &a, f4_t &b, f4_t &c, f4_t &d) {
-    asm volatile(
-        "global_load_dwordx4 %0, %4, off sc1\n"
-        "global_load_dwordx4 %1, %5, off sc1\n"
-        "global_load_dwordx4 %2, %6, off sc1\n"
-        "global_load_dwordx4 %3, %7, off sc1\n"
-        "s_waitcnt vmcnt(0)"
-        : "=&v"(a), "=&v"(b), "=&v"(c), "=&v"(d)
-        : "v"(p0), "v"(p1), "v"(p2), "v"(p3)
-        : "memory");
-}
-
-
+// xb[m, r] = sum_k A[m, k] * resB[r, k] in fp32: sixteen rows by sixteen ranks per workgroup on the
+// matrix cores, sixteen wavefronts taking the 32-k pieces of K in turn (a single workgroup serves
+// a small call, so K is what there is to spread), their sums added in wavefront order.
 template <bool BF16>
-__device__ __forceinline__ f4_t mfma16(u4_t w, u4_t a, f4_t acc) {
-    if constexpr (BF16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8_t, w),
-                                                       __builtin_bit_cast(bf8_t, a), acc, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, w),
-                                                      __builtin_bit_cast(h8_t, a), acc, 0, 0, 0);
+__global__ void __launch_bounds__(1024) gemm_coeff_kernel(const uint16_t *A, int64_t lda, const uint16_t *resB, float *xb,
+                                                          int M, int K, int R, int aligned) {
+    __shared__ f4_t red[16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m = min((int)blockIdx.x * 16 + (lane & 15), M - 1), rr = min((int)blockIdx.y * 16 + (lane & 15), R - 1);
+    const uint16_t *a = A + (int64_t)m * lda + (lane >> 4) * 8, *b = resB + (int64_t)rr * K + (lane >> 4) * 8;
+    auto load8 = [&](const uint16_t *p) {
+        u4_t v;
+        if (aligned) return *(const u4_t *)p;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = (uint32_t)p[2 * e] | ((uint32_t)p[2 * e + 1] << 16);
+        return v;
+    };
+    f4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int k = wave * 32; k < K; k += 512) acc = mfma16<BF16>(load8(b + k), load8(a + k), acc);
+    red[wave][lane] = acc;
+    __syncthreads();
+    if (wave == 0) {
+        for (int w = 1; w < 16; ++w) acc += red[w][lane];
+        const int mo = blockIdx.x * 16 + (lane & 15), r0 = blockIdx.y * 16 + (lane >> 4) * 4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (mo < M && r0 + e < R) xb[(int64_t)mo * R + r0 + e] = acc[e];
+    }
 }
 
 // The 2B-bit code of pair p of a chunk held as 4*B dwords (all indices constant

@@ -342,3 +342,52 @@ def test_scalar_twin_refusals_and_bf16():
         fx.qgemm_debug_simple(x, w["blob_d"], w["lut_d"][:, :8], 4, 128)      # wrong LUT width
     with pytest.raises(RuntimeError):
         fx.qgemm_debug_simple(x, w["blob_d"], w["lut_d"], 5, 128)
+
+
+# ---- many rows: every weight looked up once per workgroup (gemm_wide_kernel.h) ------------------
+WIDE = [
+    # M, N, K, bits, gs, bits2, rank, bias, lut, act
+    (1, 128, 64, 4, 128, 0, 0, False, torch.float16, torch.float16),       # one tile, one row
+    (33, 384, 192, 4, 64, 0, 0, True, torch.bfloat16, torch.bfloat16),     # odd number of tiles
+    (257, 256, 320, 4, 16, 0, 0, False, torch.float16, torch.float16),     # eight LUT groups a tile
+    (513, 256, 512, 3, 128, 0, 5, False, torch.float16, torch.float16),    # one row past a workgroup
+    (511, 256, 448, 2, 32, 0, 0, False, torch.bfloat16, torch.bfloat16),
+    (130, 128, 1088, 1, 256, 0, 0, True, torch.float16, torch.float16),
+    (300, 256, 512, 4, 128, 1, 16, True, torch.float16, torch.float16),
+    (300, 256, 512, 1, 128, 4, 0, False, torch.bfloat16, torch.bfloat16),  # the wider stream second
+    (100, 256, 576, 3, 64, 3, 40, False, torch.bfloat16, torch.bfloat16),  # ranks beyond one 32-wide step
+    (300, 256, 512, 2, 16, 4, 0, False, torch.float16, torch.float16),
+    (300, 256, 448, 2, 256, 3, 0, False, torch.float16, torch.bfloat16),   # rows scaled into float16
+    (70, 512, 512, 4, 64, 4, 8, True, torch.float16, torch.bfloat16),      # two 32 KB tables
+    (130, 256, 512, 1, 64, 1, 0, False, torch.float16, torch.float16),
+    (130, 256, 512, 3, 128, 1, 0, False, torch.float16, torch.bfloat16),
+]
+
+
+@pytest.mark.parametrize("rows,slices", [("512", None), ("256", None), ("512", "3"), ("256", "5")])
+@pytest.mark.parametrize("M,N,K,bits,gs,bits2,rank,bias,lut,act", WIDE)
+def test_gemm_many_row_workgroups(tuning_env, rows, slices, M, N, K, bits, gs, bits2, rank, bias, lut, act):
+    """The many-row kernel at the edges of its tiles, forced with FLUTE_GEMM_ROWS = 512 / 256, with
+    and without slices of K (FLUTE_GEMM_KSPLIT), against the closed form; repeats bit identical.
+    One rounding of an fp32 sum to the output type: 2^-12 of a value at most in float16, 2^-9 in
+    bfloat16, the tolerances of this file."""
+    tuning_env("FLUTE_GEMM_ROWS", rows)
+    if slices:
+        tuning_env("FLUTE_GEMM_KSPLIT", slices)
+    w = make_weight(N, K, bits, gs, seed=M + N + K + bits, bits2=bits2, rank=rank, bias=bias, lut_dtype=lut,
+                    act_dtype=act, device=DEV)
+    x = make_x(M, K, seed=43, dtype=act)
+    y = _dual(w, x)
+    assert rel_l2(y.cpu(), _exact(w, x).to(act)) <= (TOL if act == torch.float16 else TOL_BF16)
+    assert torch.equal(y, _dual(w, x))
+
+
+@pytest.mark.parametrize("M,N,K,bits2", [(1100, 12288, 1024, 0), (600, 4096, 4096, 1), (200, 12288, 512, 1)])
+def test_gemm_many_rows_by_the_rule_agree_with_the_other_kernels(tuning_env, M, N, K, bits2):
+    """Sizes the launcher gives to the many-row kernel by itself, rotated rows among them, against
+    the 128-row workgroups: the same fp32 sums in another order, one rounding."""
+    w = make_weight(N, K, 4, 128, seed=3, bits2=bits2, rank=16, bias=True, device=DEV)
+    x = make_x(M, K, seed=5)
+    y = _dual(w, x)
+    tuning_env("FLUTE_GEMM_ROWS", "128")
+    assert rel_l2(y.cpu(), _dual(w, x).cpu()) <= TOL
