@@ -136,36 +136,6 @@ __device__ __forceinline__ void store_cols8(const FhtParams &p, int64_t orow, in
     }
 }
 
-// Stages of length 1, 2, 4 between a thread's own eight columns.
-__device__ __forceinline__ void stages_in_thread(float (&f)[8]) {
-#pragma unroll
-    for (int len = 1; len < 8; len <<= 1) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            if ((q & len) == 0) {
-                const float a = f[q], c = f[q | len];
-                f[q] = a + c;
-                f[q | len] = a - c;
-            }
-        }
-    }
-}
-
-// One stage against the lane whose number differs in bit M (M = 1 ... 16: ds_swizzle,
-// the LDS crossbar without a memory access).  The lower lane of a pair keeps a + b and
-// the upper a - b, formed as fma(mine, +-1, other): the product is exact, so every value
-// sees the same single rounding per stage as in the buffered butterfly.
-template <int M>
-__device__ __forceinline__ void stage_across_lanes(float (&f)[8], int lane) {
-    const float sgn = (lane & M) ? -1.0f : 1.0f;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        const float other = __int_as_float(
-            __builtin_amdgcn_ds_swizzle(__float_as_int(f[q]), (M << 10) | 0x1f));
-        f[q] = fmaf(f[q], sgn, other);
-    }
-}
-
 // Equal blocks of at most 256 columns without the LDS buffer: three stages in a thread's
 // registers, the stages of length 8 ... block/2 across lanes, in the same ascending order
 // as the buffered butterfly and bit-identical to it.  One memory round trip, no barrier.
@@ -225,16 +195,8 @@ __device__ __forceinline__ void fht_segment_fast(const FhtParams &p, int64_t row
         for (int h = 0; h < S; ++h) stage_across_lanes<8>(f[h], lane);
 #pragma unroll
         for (int h = 0; h < S; ++h) stage_across_lanes<16>(f[h], lane);
-        const float sgn = (lane & 32) ? -1.0f : 1.0f;
-        const int partner = (lane ^ 32) << 2;
 #pragma unroll
-        for (int h = 0; h < S; ++h)
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const float other = __int_as_float(
-                    __builtin_amdgcn_ds_bpermute(partner, __float_as_int(f[h][q])));
-                f[h][q] = fmaf(f[h][q], sgn, other);
-            }
+        for (int h = 0; h < S; ++h) stage_across_lanes<32>(f[h], lane);
     }
     if (nst > 9) {                                     // uniform: stages of length 512 and up
         if (one) {

@@ -15,27 +15,178 @@ namespace flute {
 
 namespace {
 
-// Residual coefficients: xb[r] = sum_k x[k] * resB[r][k] in fp32, one workgroup
-// per residual row, x taken as given (already rotated).  A thread-strided sum
-// followed by a fixed-order tree: deterministic.
-__global__ void __launch_bounds__(256) residual_coeff_kernel(const uint16_t *x,
-                                                             const uint16_t *resB, float *xb,
-                                                             int K, int act_bf16) {
-    __shared__ float part[256];
-    const uint16_t *row = resB + (size_t)blockIdx.x * K;
-    float s = 0.0f;
-    for (int k = threadIdx.x; k < K; k += 256) {
-        const float a = act_bf16 ? bf2f(x[k]) : h2f(x[k]);
-        const float b = act_bf16 ? bf2f(row[k]) : h2f(row[k]);
-        s = fmaf(a, b, s);
+// What has to be known before a GEMV launch can finish a row: the rotated input of every weight
+// that carries a residual, and the residual coefficients xb[r] = sum_k x[k] * resB[r][k] (fp32, x
+// rotated and rounded to the activation type where the weight is rotated).  One launch for all
+// weights of a call: eight residual rows per workgroup, one per wavefront, and every workgroup
+// transforms the input itself (a few microseconds of one CU) instead of waiting for another launch
+// to do it.  The butterflies are fht_dev.h's in the same order, so the rotated row has the bits of
+// flute_fht; a lane's sum runs over its columns in ascending order, then a fixed tree.
+// What bounds it: latency.  The row, its multipliers and the first 4096 columns of a residual row
+// are requested together; what follows is LDS passes between barriers.  Rotated q/k/v of rank 16,
+// K = 4096: three rotations of 5.2 us and three coefficient launches of 8.9 us, six launches in a
+// row, against one of 7.4 us; the whole call 50.5 -> 22.1 us.
+constexpr int kPreThreads = 512, kPreRows = kPreThreads / 64;
+
+struct PreSeg {
+    const uint16_t *resB;
+    const float *signs, *awq;
+    float *xb;
+    uint16_t *xrot;         // where the first workgroup of this weight leaves the rotated row, or NULL
+    int R;
+    int block0;             // first workgroup of this weight
+    int vec_b, vec_m;       // resB / signs and awq allow 16-byte loads
+};
+
+struct PreParams {
+    PreSeg seg[kGemvMaxSegs];
+    const uint16_t *x;
+    int nsegs, K, act_bf16, rot_block;
+};
+
+__device__ __forceinline__ void pre_unpack8(const uint4 raw, int bf16, float (&f)[8]) {
+    const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const uint16_t h = (uint16_t)(w[q >> 1] >> (16 * (q & 1)));
+        f[q] = bf16 ? bf2f(h) : h2f(h);
     }
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int step = 128; step > 0; step >>= 1) {
-        if ((int)threadIdx.x < step) part[threadIdx.x] += part[threadIdx.x + step];
-        __syncthreads();
+}
+
+__device__ __forceinline__ uint4 pre_load8(const uint16_t *p, int vec) {
+    if (vec) return *(const uint4 *)p;
+    uint32_t w[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[q] = (uint32_t)p[2 * q] | ((uint32_t)p[2 * q + 1] << 16);
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+__device__ __forceinline__ void pre_mul8(const float *p, int vec, float (&f)[8]) {
+    if (vec) {
+        const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 4);
+        f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w;
+        f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
+    } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) f[q] = p[q];
     }
-    if (threadIdx.x == 0) xb[blockIdx.x] = part[0];
+}
+
+__global__ void __launch_bounds__(kPreThreads) gemv_pre_kernel(const PreParams p) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    float *const buf = (float *)lds;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int si = 0;
+    while (si + 1 < p.nsegs && (int)blockIdx.x >= p.seg[si + 1].block0) ++si;
+    const PreSeg &w = p.seg[si];
+    const int part = blockIdx.x - w.block0;
+    const int r = part * kPreRows + wave;               // this wavefront's residual row
+    const bool mine = r < w.R;
+    const uint16_t *const row = w.resB + (size_t)(mine ? r : 0) * p.K;
+    constexpr int AHEAD = 8;                            // steps of 512 columns requested up front
+    uint4 first[AHEAD];
+    if (mine) {
+#pragma unroll
+        for (int h = 0; h < AHEAD; ++h) {
+            const int k = h * 512 + lane * 8;
+            first[h] = pre_load8(row + (k < p.K ? k : 0), w.vec_b);
+        }
+    }
+    float acc = 0.0f;
+    // products of the columns [off, off + count), x from `get`
+    auto dot = [&](int off, int count, auto get) {
+        if (!mine) return;
+        auto step = [&](int j, const uint4 raw) {
+            float b[8], x[8];
+            pre_unpack8(raw, p.act_bf16, b);
+            get(j, x);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) acc = fmaf(x[q], b[q], acc);
+        };
+        int j = lane * 8;
+        if (off == 0) {
+#pragma unroll
+            for (int h = 0; h < AHEAD; ++h)
+                if (h * 512 + lane * 8 < count) step(h * 512 + lane * 8, first[h]);
+            j += AHEAD * 512;
+        }
+        for (; j < count; j += 512) step(j, pre_load8(row + off + j, w.vec_b));
+    };
+    if (w.signs == nullptr) {
+        dot(0, p.K, [&](int j, float (&x)[8]) { pre_unpack8(*(const uint4 *)(p.x + j), p.act_bf16, x); });
+    } else {
+        for (int off = 0; off < p.K;) {
+            int count, nst;
+            if (p.rot_block > 0) {
+                nst = 31 - __builtin_clz((unsigned)p.rot_block);
+                count = min((16384 / p.rot_block) * p.rot_block, p.K - off);
+            } else {
+                nst = 31 - __builtin_clz((unsigned)(p.K - off));
+                count = 1 << nst;
+            }
+            const float inv = inv_sqrt_pow2(nst);
+            // eight consecutive columns a thread and step: their first stages in registers
+            // (multipliers of the first step travel with the row)
+            float sg[8], sc[8];
+            const int j0 = tid * 8 < count ? tid * 8 : 0;
+            pre_mul8(w.signs + off + j0, w.vec_m, sg);
+            if (w.awq) pre_mul8(w.awq + off + j0, w.vec_m, sc);
+            for (int j = tid * 8; j < count; j += kPreThreads * 8) {
+                float f[8];
+                pre_unpack8(*(const uint4 *)(p.x + off + j), p.act_bf16, f);
+                if (w.awq) {
+                    float s[8];
+                    pre_mul8(w.awq + off + j, w.vec_m, s);
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) f[q] *= s[q];
+                }
+                fht_head(f, lane, nst);
+                const int s0 = fht_slot(j);             // a multiple of 8: slot(j + q) = s0 ^ q
+#pragma unroll
+                for (int q = 0; q < 8; ++q) buf[s0 ^ q] = f[q];
+            }
+            __syncthreads();
+            fht_tail(buf, count, nst, 9, tid, kPreThreads);
+            for (int j = tid * 8; j < count; j += kPreThreads * 8) {
+                if (j != tid * 8) {
+                    pre_mul8(w.signs + off + j, w.vec_m, sg);
+                    if (w.awq) pre_mul8(w.awq + off + j, w.vec_m, sc);
+                }
+                const int s0 = fht_slot(j);
+                float t[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) t[q] = buf[s0 ^ q] * sg[q] * inv;
+                if (w.awq) {
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) t[q] = t[q] / sc[q];
+                }
+                uint16_t o[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    o[q] = round_act(t[q], p.act_bf16);
+                    buf[s0 ^ q] = p.act_bf16 ? bf2f(o[q]) : h2f(o[q]);
+                }
+                if (w.xrot && part == 0)
+                    *(uint4 *)(w.xrot + off + j) =
+                        make_uint4((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16),
+                                   (uint32_t)o[4] | ((uint32_t)o[5] << 16), (uint32_t)o[6] | ((uint32_t)o[7] << 16));
+            }
+            __syncthreads();
+            dot(off, count, [&](int j, float (&x)[8]) {
+                const int s0 = fht_slot(j);
+#pragma unroll
+                for (int q = 0; q < 8; ++q) x[q] = buf[s0 ^ q];
+            });
+            off += count;
+            if (off < p.K) __syncthreads();             // the next segment reuses the buffer
+        }
+    }
+    if (mine) {
+#pragma unroll
+        for (int m = 32; m > 0; m >>= 1) acc += __shfl_xor(acc, m);
+        if (lane == 0) w.xb[r] = acc;
+    }
 }
 
 int entries_log2(int bits) { return bits == 3 ? 6 : 8; }
@@ -597,26 +748,44 @@ flute_status launch(Plan &plan, int act_dtype, hipStream_t stream, float *fixed_
         plan.p.tickets = tickets;
         float *xb_base = base + plan.p_floats;
         uint16_t *xrot_base = (uint16_t *)(xb_base + xb_pad);
+        PreParams pp = {};
+        pp.x = plan.p.x;
+        pp.K = plan.p.K;
+        pp.act_bf16 = plan.p.act_bf16;
+        pp.rot_block = plan.rot_block;
+        int blocks = 0;
+        size_t lds = 0;
         for (int i = 0; i < plan.npre; ++i) {
             const Plan::Pre &pre = plan.pre[i];
-            const uint16_t *xin = plan.p.x;
+            uint16_t *const xr = xrot_base + pre.xrot_off;
+            float *const xb = xb_base + pre.xb_off;
             if (pre.signs) {
-                uint16_t *xr = xrot_base + pre.xrot_off;
-                if (pre.share < 0) {
-                    st = flute_fht(plan.p.x, pre.signs, pre.awq, xr, 1, plan.p.K, act_dtype, 0,
-                                   plan.rot_block, stream);
-                    if (st != FLUTE_OK) return st;
-                }
-                xin = xr;
+                const size_t cols = plan.rot_block > 0
+                                        ? (size_t)(plan.p.K <= 16384 ? plan.p.K : (16384 / plan.rot_block) * plan.rot_block)
+                                        : (size_t)make_segments(plan.p.K, 0).len[0];
+                FLUTE_REQUIRE(cols <= 16384 && plan.p.K <= 65504, FLUTE_ERR_UNSUPPORTED,
+                              "flute_gemv: the rotation of K=%d columns is not served", plan.p.K);
+                lds = cols * 4;
                 plan.p.seg[pre.seg].xsrc = xr;
             }
-            if (pre.R > 0) {
-                float *xb = xb_base + pre.xb_off;
-                hipLaunchKernelGGL(residual_coeff_kernel, dim3(pre.R), dim3(256), 0, stream, xin,
-                                   pre.resB, xb, plan.p.K, plan.p.act_bf16);
-                FLUTE_HIP_CHECK(hipGetLastError());
-                plan.p.seg[pre.seg].xb = xb;
-            }
+            if (pre.R > 0) plan.p.seg[pre.seg].xb = xb;
+            const int rowblocks = (pre.R + kPreRows - 1) / kPreRows;
+            if (rowblocks == 0 && pre.share >= 0) continue;      // another weight's rotation is all it needs
+            PreSeg &g = pp.seg[pp.nsegs++];
+            g.resB = pre.resB;
+            g.signs = pre.signs;
+            g.awq = pre.awq;
+            g.xb = xb;
+            g.xrot = pre.signs && pre.share < 0 ? xr : nullptr;
+            g.R = pre.R;
+            g.block0 = blocks;
+            g.vec_b = ((uintptr_t)pre.resB & 15) == 0;
+            g.vec_m = ((uintptr_t)pre.signs & 15) == 0 && ((uintptr_t)pre.awq & 15) == 0;
+            blocks += rowblocks ? rowblocks : 1;
+        }
+        if (blocks) {
+            hipLaunchKernelGGL(gemv_pre_kernel, dim3(blocks), dim3(kPreThreads), lds, stream, pp);
+            FLUTE_HIP_CHECK(hipGetLastError());
         }
     }
     const flute_status st = plan.lut_bf16 ? launch_width<true>(plan, stream) : launch_width<false>(plan, stream);

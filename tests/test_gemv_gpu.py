@@ -606,3 +606,30 @@ def test_merged_gate_up_with_two_stream_members():
         y1 = y.clone()
         fx.qgemm_gemv_mlp(x.to(DEV), table, out)
         assert torch.equal(out.cpu(), y1)
+
+
+@pytest.mark.parametrize("rank", [1, 8, 9, 17])
+@pytest.mark.parametrize("K,form", [(64, "plain"), (576, "plain"), (12288, "plain"),
+                                    (64, "full"), (1088, "full"), (4608, "full"), (12288, "full"),
+                                    (4096, "awq"), (1024, "block32"), (1024, "block512")])
+def test_residual_coefficients_of_every_form(rank, K, form):
+    """The launch in front of a GEMV with a residual: workgroups of eight residual rows, rows of one
+    and several loads, segments inside and beyond the stages held in registers, blocks, scales.
+    The coefficients are fp32 sums of the rotated and rounded row, so the output differs from the
+    64-bit one by its own rounding (2^-11) and by fp32 sums: the tolerance of the other forms."""
+    N = 256
+    w = make_weight(N, K, 4, 128, seed=K + rank, rank=rank, device=DEV)
+    x = make_x(1, K, seed=K)
+    signs = None if form == "plain" else O.rotation_signs(K, 3)
+    awq, extra, xr = None, {}, x
+    if form == "full":
+        xr = O.fht_reference(x, signs)
+    elif form == "awq":
+        awq = torch.rand(K, generator=torch.Generator().manual_seed(4)) + 0.5
+        xr = O.fht_awq_reference(x, signs, awq)
+    elif form.startswith("block"):
+        extra = dict(rot_block=int(form[5:]))
+        xr = O.block_fht_reference(x, extra["rot_block"], signs)
+    y = _run(w, x, signs=signs, awq=awq, **extra)
+    assert rel_l2(y.cpu(), _exact(w, xr)) <= TOL
+    assert torch.equal(y, _run(w, x, signs=signs, awq=awq, **extra))
