@@ -238,6 +238,14 @@ flute_status flute_embedding(const flute_linear *w, const int64_t *ids, int64_t 
                              void *out, void *stream);
 
 /*
+ * flute_embedding for ids that nobody has looked over yet: the launch checks them itself and
+ * the call returns once it knows (the rows may still be on their way then): *in_range = 1 when
+ * every id lies in [0, N), else 0.  Refused while the stream is capturing.
+ */
+flute_status flute_embedding_checked(const flute_linear *w, const int64_t *ids, int64_t count,
+                                     void *out, void *stream, int *in_range);
+
+/*
  * The K-split the library would choose for an (N, K) GEMV without a fused rotation on this
  * device (the MI355X counterpart of gemv_pick_split, src/gemv_host.cpp:29-38; the numbers
  * are this device's, not the A10G's).  Up to K = 24576 the unsplit launch measured fastest

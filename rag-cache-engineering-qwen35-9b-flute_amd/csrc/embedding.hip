@@ -10,6 +10,9 @@
 #include "host_common.h"
 
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
+#include <mutex>
 
 namespace flute {
 
@@ -29,38 +32,51 @@ struct EmbParams {
     int N, K, gs, lut_rows, R;
     int bf16;        // LUT / output / residual dtype
     int block;       // rotation block (0: descending power-of-two segments)
+    int vec_out;     // rows of out allow 16-byte stores
 };
 
-// The two values of logical pair (n, k), k even, of one stream.
-__device__ __forceinline__ void pair_values(const uint8_t *q, const uint16_t *lut, int b, int G,
-                                            int n, int k, int grp, uint32_t &e0, uint32_t &e1) {
-    const int t = n >> 7, r = n & 127;
-    const int wx = r >> 6, v = (r >> 4) & 3, d = (r >> 3) & 1, r8 = r & 7;
-    const int g = k >> 6, kk = k & 63;
-    const int kt = kk >> 4, s2 = (kk >> 3) & 1, c4 = (kk >> 1) & 3;
-    const int th = wx * 32 + r8 * 4 + c4;
-    const int p = kt * 16 + v * 4 + d * 2 + s2;
-    const uint8_t *chunk = q + (((size_t)t * G + g) * 64 + th) * (16 * b);
-    const int bit = 2 * b * p, byte = bit >> 3;
-    uint32_t w = chunk[byte];
-    if (byte + 1 < 16 * b) w |= (uint32_t)chunk[byte + 1] << 8;
-    const uint32_t code = (w >> (bit & 7)) & ((1u << (2 * b)) - 1u);
-    const uint16_t *row = lut + ((size_t)grp << b);
-    e0 = row[code & ((1u << b) - 1u)];
-    e1 = row[code >> b];
+// A thread's share of a row is quarter kt of tile g: sixteen consecutive columns, whose codes lie
+// in the four chunks c4 = 0 ... 3 of the row's chunk group (columns c4*2 + 8*s2 (+1) of the quarter
+// are the pairs s2 = 0, 1 of chunk c4), 4*B consecutive bits each: byte B*v + (4*B*d)/8 of the
+// quarter's 4*B bytes.  Sixteen neighbouring threads' bytes are the 256*B ones of four chunk groups.
+__device__ __forceinline__ uint32_t chunk_codes(const uint8_t *p, int b, int d) {
+    if (b == 4) return *(const uint16_t *)(p + 2 * d);
+    if (b == 3) return (((uint32_t)p[d] | ((uint32_t)p[d + 1] << 8)) >> (4 * d)) & 0xfffu;
+    if (b == 2) return p[d];
+    return (uint32_t)*p >> (4 * d);
 }
 
 __device__ __forceinline__ float to_f(uint32_t h, int bf16) {
     return bf16 ? bf2f((uint16_t)h) : h2f((uint16_t)h);
 }
 
-// One workgroup per requested row.
-__global__ void __launch_bounds__(kEmbThreads) embedding_kernel(const EmbParams p) {
+// One workgroup per requested row, sixteen consecutive columns a thread.  What bounds it: the chain
+// id -> codes -> values -> butterfly -> store, so everything a phase needs is requested together
+// (the LUT row goes to LDS beside the codes and signs, a value costs one LDS read) and the first ten
+// stages of the butterfly stay in registers.  (One pair at a time, byte loads of the codes and trips
+// to memory for the LUT, all stages in LDS: 15.2 us for 1000 rotated rows of 4096 columns, 4 bits,
+// against 13.6; the check of the ids as five launches and a copy before it: 71 us a call against 27.)
+// check != NULL: the first workgroup of the grid looks all ids over instead and leaves its verdict
+// in host memory, 1 = every id lies in the table, 2 = some do not.
+__global__ void __launch_bounds__(kEmbThreads) embedding_kernel(const EmbParams p, int64_t count, int *check) {
     extern __shared__ __align__(16) uint8_t lds[];
     float *buf = (float *)lds;
+    __shared__ uint16_t luts[2][16];
     const int tid = threadIdx.x;
-    const int64_t n64 = p.ids[blockIdx.x];
-    uint16_t *out = p.out + (size_t)blockIdx.x * p.K;
+    if (check && blockIdx.x == 0) {
+        __shared__ int bad;
+        if (tid == 0) bad = 0;
+        __syncthreads();
+        int mine = 0;
+        for (int64_t i = tid; i < count; i += kEmbThreads) mine |= p.ids[i] < 0 || p.ids[i] >= p.N;
+        if (mine) bad = 1;
+        __syncthreads();
+        if (tid == 0) __hip_atomic_store(check, bad ? 2 : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        return;
+    }
+    const int64_t at = (int64_t)blockIdx.x - (check ? 1 : 0);
+    const int64_t n64 = p.ids[at];
+    uint16_t *out = p.out + (size_t)at * p.K;
     if (n64 < 0 || n64 >= p.N) {                  // refused on the host; never read out of range
         for (int k = tid; k < p.K; k += kEmbThreads) out[k] = 0;
         return;
@@ -68,66 +84,170 @@ __global__ void __launch_bounds__(kEmbThreads) embedding_kernel(const EmbParams 
     const int n = (int)n64;
     const int G = p.K >> 6;
     const int grp = min(n / p.gs, p.lut_rows - 1);
-
-    auto pair_row = [&](int k, float &f0, float &f1) {
-        uint32_t a0, a1;
-        pair_values(p.q[0], p.lut[0], p.bits[0], G, n, k, grp, a0, a1);
-        f0 = to_f(a0, p.bf16);
-        f1 = to_f(a1, p.bf16);
+    const int wx = (n >> 6) & 1, v = (n >> 4) & 3, d = (n >> 3) & 1, r8 = n & 7;
+    const uint8_t *q[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) q[s] = p.q[s] + (size_t)(n >> 7) * G * (1024 * p.bits[s]);
+    if (tid < 32) {
+        const int s = tid >> 4, e = tid & 15;
+        if (s < p.nstreams && e < (1 << p.bits[s])) luts[s][e] = p.lut[s][((size_t)grp << p.bits[s]) + e];
+    }
+    const uint8_t *src[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) src[s] = q[s] + (wx * 32 + r8 * 4) * (16 * p.bits[s]) + p.bits[s] * v;
+    // codes of the columns k ... k + 15 (k a multiple of 16), as chunk c4 of stream s
+    auto codes = [&](int s, int k, uint32_t (&c)[4]) {
+        const int b = p.bits[s];
+        const uint8_t *at_k = src[s] + (size_t)(k >> 6) * (1024 * b) + ((k >> 4) & 3) * (4 * b);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[i] = chunk_codes(at_k + i * 16 * b, b, d);
+    };
+    auto values = [&](int k, const uint32_t (&c)[2][4], float (&f)[16]) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int i = (j >> 1) & 3, shift = 2 * (j >> 3) + (j & 1);    // in codes
+            const int b = p.bits[0];
+            f[j] = to_f(luts[0][(c[0][i] >> (b * shift)) & ((1 << b) - 1)], p.bf16);
+        }
         if (p.nstreams == 2) {
-            uint32_t b0, b1;
-            pair_values(p.q[1], p.lut[1], p.bits[1], G, n, k, grp, b0, b1);
-            // the 16-bit add of the module: exact sum, one rounding to the LUT's type
-            f0 = to_f(round_act(f0 + to_f(b0, p.bf16), p.bf16), p.bf16);
-            f1 = to_f(round_act(f1 + to_f(b1, p.bf16), p.bf16), p.bf16);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const int i = (j >> 1) & 3, shift = 2 * (j >> 3) + (j & 1);
+                const int b = p.bits[1];
+                // the 16-bit add of the module: exact sum, one rounding to the LUT's type
+                f[j] = to_f(round_act(f[j] + to_f(luts[1][(c[1][i] >> (b * shift)) & ((1 << b) - 1)], p.bf16), p.bf16), p.bf16);
+            }
         }
         if (p.R > 0) {
-            float r0 = 0.0f, r1 = 0.0f;
+            float sum[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) sum[j] = 0.0f;
             for (int r = 0; r < p.R; ++r) {
                 const float a = to_f(p.resA[(size_t)n * p.R + r], p.bf16);
-                r0 = fmaf(a, to_f(p.resB[(size_t)r * p.K + k], p.bf16), r0);
-                r1 = fmaf(a, to_f(p.resB[(size_t)r * p.K + k + 1], p.bf16), r1);
+                const uint16_t *row = p.resB + (size_t)r * p.K + k;
+#pragma unroll
+                for (int j = 0; j < 16; ++j) sum[j] = fmaf(a, to_f(row[j], p.bf16), sum[j]);
             }
-            f0 += r0;
-            f1 += r1;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) f[j] += sum[j];
         }
     };
+    auto store = [&](int k, const float (&f)[16]) {
+        uint32_t o[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            o[e] = (uint32_t)round_act(f[2 * e], p.bf16) | ((uint32_t)round_act(f[2 * e + 1], p.bf16) << 16);
+        if (p.vec_out) {
+            *(uint4 *)(out + k) = make_uint4(o[0], o[1], o[2], o[3]);
+            *(uint4 *)(out + k + 8) = make_uint4(o[4], o[5], o[6], o[7]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) *(uint32_t *)(out + k + 2 * e) = o[e];
+        }
+    };
+    constexpr int STEP = kEmbThreads * 16;
+    const int lane = tid & 63;
+    uint32_t c[2][4];
+    {
+        // codes of this thread's first columns, beside the LUT row
+        const int k = min(tid * 16, p.K - 16);
+        codes(0, k, c[0]);
+        if (p.nstreams == 2) codes(1, k, c[1]);
+    }
+    __syncthreads();                                      // the LUT rows are in
 
     if (p.signs == nullptr) {
-        for (int k = tid * 2; k < p.K; k += kEmbThreads * 2) {
-            float f0, f1;
-            pair_row(k, f0, f1);
-            *(uint32_t *)(out + k) =
-                (uint32_t)round_act(f0, p.bf16) | ((uint32_t)round_act(f1, p.bf16) << 16);
+        for (int k = tid * 16; k < p.K; k += STEP) {
+            if (k >= STEP) {
+                codes(0, k, c[0]);
+                if (p.nstreams == 2) codes(1, k, c[1]);
+            }
+            float f[16];
+            values(k, c, f);
+            store(k, f);
         }
         return;
     }
     // rotated table: the adjoint transform of the row, segment by segment
     for (int off = 0; off < p.K;) {
-        int count, nst;
+        int cols, nst;
         if (p.block > 0) {
             nst = 31 - __builtin_clz((unsigned)p.block);
-            count = min((16384 / p.block) * p.block, p.K - off);
+            cols = min((16384 / p.block) * p.block, p.K - off);
         } else {
             nst = 31 - __builtin_clz((unsigned)(p.K - off));
-            count = 1 << nst;
+            cols = 1 << nst;
         }
-        for (int j = tid * 2; j < count; j += kEmbThreads * 2) {
-            float f0, f1;
-            pair_row(off + j, f0, f1);
-            buf[fht_slot(j)] = f0 * p.signs[off + j];
-            buf[fht_slot(j + 1)] = f1 * p.signs[off + j + 1];
-        }
-        __syncthreads();
-        fht_lds(buf, count, nst, tid, kEmbThreads);
         const float inv = inv_sqrt_pow2(nst);
-        for (int j = tid * 2; j < count; j += kEmbThreads * 2)
-            *(uint32_t *)(out + off + j) =
-                (uint32_t)round_act(buf[fht_slot(j)] * inv, p.bf16) |
-                ((uint32_t)round_act(buf[fht_slot(j + 1)] * inv, p.bf16) << 16);
-        __syncthreads();
-        off += count;
+        for (int j = tid * 16; j < cols; j += STEP) {
+            const int k = off + j;
+            float sg[16], f[16];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sg[e] = p.signs[k + e];
+            if (k >= STEP || off > 0) {
+                codes(0, k, c[0]);
+                if (p.nstreams == 2) codes(1, k, c[1]);
+            }
+            values(k, c, f);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) f[e] *= sg[e];
+            fht_head(f, lane, nst);
+            if (nst <= 10) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) f[e] *= inv;
+                store(k, f);
+            } else {
+                const int s0 = fht_slot(j);               // a multiple of 16: slot(j + q) = s0 ^ q
+#pragma unroll
+                for (int e = 0; e < 16; ++e) buf[s0 ^ e] = f[e];
+            }
+        }
+        if (nst > 10) {
+            __syncthreads();
+            fht_tail(buf, cols, nst, 10, tid, kEmbThreads);
+            for (int j = tid * 16; j < cols; j += STEP) {
+                const int s0 = fht_slot(j);
+                float f[16];
+#pragma unroll
+                for (int e = 0; e < 16; ++e) f[e] = buf[s0 ^ e] * inv;
+                store(off + j, f);
+            }
+            __syncthreads();                              // the next segment reuses the buffer
+        }
+        off += cols;
     }
+}
+
+// ---- verdicts ----------------------------------------------------------------------------
+// Pinned words the kernel leaves its verdict on a call's ids in, one per call that waits for it:
+// taken and given back under a lock, at most kVerdicts at a time (a further call waits for one).
+constexpr int kVerdicts = 64, kVerdictStride = 16;        // one per 64-byte line
+std::mutex g_verdict_mu;
+std::condition_variable g_verdict_cv;
+int *g_verdict_mem = nullptr;
+uint64_t g_verdict_free = ~(uint64_t)0;
+
+flute_status take_verdict(int *slot, int **word) {
+    std::unique_lock<std::mutex> lock(g_verdict_mu);
+    if (!g_verdict_mem) {
+        void *mem = nullptr;
+        FLUTE_HIP_CHECK(hipHostMalloc(&mem, kVerdicts * kVerdictStride * sizeof(int),
+                                      hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
+        g_verdict_mem = (int *)mem;
+    }
+    g_verdict_cv.wait(lock, [] { return g_verdict_free != 0; });
+    *slot = __builtin_ctzll(g_verdict_free);
+    g_verdict_free &= ~((uint64_t)1 << *slot);
+    *word = g_verdict_mem + *slot * kVerdictStride;
+    __atomic_store_n(*word, 0, __ATOMIC_RELAXED);
+    return FLUTE_OK;
+}
+void give_verdict(int slot) {
+    {
+        std::lock_guard<std::mutex> lock(g_verdict_mu);
+        g_verdict_free |= (uint64_t)1 << slot;
+    }
+    g_verdict_cv.notify_one();
 }
 
 }  // namespace
@@ -136,8 +256,10 @@ __global__ void __launch_bounds__(kEmbThreads) embedding_kernel(const EmbParams 
 
 using namespace flute;
 
-extern "C" flute_status flute_embedding(const flute_linear *w, const int64_t *ids, int64_t count,
-                                        void *out, void *stream) {
+namespace {
+
+flute_status embedding(const flute_linear *w, const int64_t *ids, int64_t count, void *out, hipStream_t stream,
+                       int *check) {
     flute_status st = validate_linear(w, 1, "flute_embedding");
     if (st != FLUTE_OK) return st;
     FLUTE_REQUIRE(count >= 0 && count <= 0x7fffffffLL, FLUTE_ERR_INVALID,
@@ -172,6 +294,7 @@ extern "C" flute_status flute_embedding(const flute_linear *w, const int64_t *id
     p.lut_rows = w->lut_rows;
     p.bf16 = w->lut_dtype == FLUTE_BF16;
     p.block = w->rot_block;
+    p.vec_out = ((uintptr_t)out & 15) == 0;             // (rows are K * 2 bytes, K a multiple of 64)
     size_t lds = 0;
     if (w->signs) {
         if (w->rot_block > 0) {
@@ -187,12 +310,54 @@ extern "C" flute_status flute_embedding(const flute_linear *w, const int64_t *id
         static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
         if (!attr_done) {
             FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)embedding_kernel,
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, 98304));
             attr_done = true;
         }
     }
-    hipLaunchKernelGGL(embedding_kernel, dim3((unsigned)count), dim3(kEmbThreads), lds,
-                       (hipStream_t)stream, p);
+    hipLaunchKernelGGL(embedding_kernel, dim3((unsigned)(count + (check ? 1 : 0))), dim3(kEmbThreads), lds, stream, p,
+                       count, check);
     FLUTE_HIP_CHECK(hipGetLastError());
+    return FLUTE_OK;
+}
+
+}  // namespace
+
+extern "C" flute_status flute_embedding(const flute_linear *w, const int64_t *ids, int64_t count,
+                                        void *out, void *stream) {
+    return embedding(w, ids, count, out, (hipStream_t)stream, nullptr);
+}
+
+extern "C" flute_status flute_embedding_checked(const flute_linear *w, const int64_t *ids, int64_t count,
+                                                void *out, void *stream_, int *in_range) {
+    FLUTE_REQUIRE(in_range != nullptr, FLUTE_ERR_INVALID, "flute_embedding_checked: in_range must not be NULL");
+    hipStream_t stream = (hipStream_t)stream_;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    FLUTE_HIP_CHECK(hipStreamIsCapturing(stream, &cap));
+    FLUTE_REQUIRE(cap == hipStreamCaptureStatusNone, FLUTE_ERR_INVALID,
+                  "flute_embedding_checked: no value can reach the host while the stream is capturing; "
+                  "flute_embedding writes zeros for an id outside the table");
+    *in_range = 1;
+    if (count == 0) return flute_embedding(w, ids, count, out, stream_);
+    int slot = 0, *word = nullptr;
+    flute_status st = take_verdict(&slot, &word);
+    if (st != FLUTE_OK) return st;
+    st = embedding(w, ids, count, out, stream, word);
+    if (st != FLUTE_OK) {
+        give_verdict(slot);                             // nothing was launched
+        return st;
+    }
+    // The verdict comes from the grid's first workgroup, usually while the rows are still being
+    // gathered; a stream that has much to do before it is waited for without spinning.
+    int verdict = 0;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    while (!(verdict = __atomic_load_n(word, __ATOMIC_ACQUIRE)) && std::chrono::steady_clock::now() < until)
+        __builtin_ia32_pause();
+    if (!verdict) {
+        FLUTE_HIP_CHECK(hipStreamSynchronize(stream));
+        verdict = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+        FLUTE_REQUIRE(verdict != 0, FLUTE_ERR_HIP, "flute_embedding_checked: the launch left no verdict");
+    }
+    give_verdict(slot);
+    *in_range = verdict == 1;
     return FLUTE_OK;
 }

@@ -46,7 +46,7 @@ from ._C import qgemm_gemv_splitk_fht_stream as _qgemm_gemv_splitk_fht_stream
 from ._C import qgemm_gemv_multi as _qgemm_gemv_multi
 from ._C import qgemm_gemv_mlp as _qgemm_gemv_mlp
 from ._C import dequant_idxn
-from ._C import embedding_gather
+from ._C import embedding_gather, IdRangeError
 from ._C import qgemm_gemv_kgroup, dequant_kgroup
 
 Backend = Literal["debug_simple", "cutlass_dense", "cutlass_streaming", "auto"]

@@ -709,6 +709,14 @@ class PalettizedEmbedding(nn.Module):
             self._logical[key] = torch.from_numpy(idx).to(blob.device)
         return self._logical[key]
 
+    def _signs_on(self, device):
+        """The rotation's signs on `device`, copied there once."""
+        if self.rot_signs is None or self.rot_signs.device == device:
+            return self.rot_signs
+        if ("signs", device) not in self._logical:
+            self._logical["signs", device] = self.rot_signs.to(device)
+        return self._logical["signs", device]
+
     def _gather_stream(self, ids, lut, which):
         rows = lut[torch.clamp(ids // self.group_size, max=lut.shape[0] - 1)]
         return rows.gather(-1, self._logical_indices(which)[ids].long())
@@ -721,18 +729,24 @@ class PalettizedEmbedding(nn.Module):
                              f"dtype {ids.dtype}")
         ids = ids.long()
         capturing = ids.is_cuda and torch.cuda.is_current_stream_capturing()
-        # one reduction and one host read; skipped under graph capture, where no value can
-        # reach the host (the kernel writes a row of zeros for an id outside the table)
-        if ids.numel() and not capturing and bool(((ids < 0) | (ids >= self.N)).any()):
-            raise ValueError(f"PalettizedEmbedding.forward: ids must lie in [0, {self.N})")
+        outside = f"PalettizedEmbedding.forward: ids must lie in [0, {self.N})"
         if not self.reference and ids.is_cuda:
             _count("embedding_gather")
-            signs = None if self.rot_signs is None else self.rot_signs.to(ids.device)
-            return _flute().embedding_gather(
-                ids, self.indices, self.lut, self.N, self.K, self.bitwidth, self.group_size,
-                indices2=self.indices2, lut2=self.lut2,
-                bitwidth2=self.bitwidth2 if self.has_stream2 else 0,
-                resB=self.resB, resA=self.resA, signs=signs, check_ids=False)
+            fx = _flute()
+            try:
+                # the gather looks the ids over itself; skipped under graph capture, where no value
+                # can reach the host (the kernel writes a row of zeros for an id outside the table)
+                return fx.embedding_gather(
+                    ids, self.indices, self.lut, self.N, self.K, self.bitwidth, self.group_size,
+                    indices2=self.indices2, lut2=self.lut2,
+                    bitwidth2=self.bitwidth2 if self.has_stream2 else 0,
+                    resB=self.resB, resA=self.resA, signs=self._signs_on(ids.device),
+                    check_ids=not capturing)
+            except fx.IdRangeError:
+                raise ValueError(outside) from None
+        # one reduction and one host read
+        if ids.numel() and not capturing and bool(((ids < 0) | (ids >= self.N)).any()):
+            raise ValueError(outside)
         w = self._gather_stream(ids, self.lut, 1)
         if self.has_stream2:
             w = w + self._gather_stream(ids, self.lut2, 2)

@@ -114,3 +114,60 @@ def test_hip_gather_bf16_table_and_refusals():
     with pytest.raises(RuntimeError, match="integer"):
         fx.embedding_gather(torch.zeros(2, device=DEV), w["blob"].to(DEV), w["lut"].to(DEV), N, K,
                             4, 128)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [64, 192, 1088, 2048, 4160, 12288])
+@pytest.mark.parametrize("bits,bits2", [(1, 0), (3, 2), (4, 1), (2, 3)])
+@pytest.mark.parametrize("block", [None, 0, 32])
+def test_hip_gather_column_edges(K, bits, bits2, block):
+    """Rows shorter and longer than a workgroup's sixteen columns a thread, every width's place in
+    a chunk (all eight rows of a chunk group, both halves of a tile), segments within and beyond the
+    stages held in registers.  Unrotated rows are a gather: bit exact."""
+    import flute_extended as fx
+    if block and K % block:
+        pytest.skip("blocks divide K")
+    N = 256
+    w = make_weight(N, K, bits, 64, seed=K + bits, bits2=bits2)
+    ids = torch.arange(0, N, 5)
+    signs = None if block is None else O.rotation_signs(K, 3)
+    kw = {} if not bits2 else dict(indices2=w["blob2"].to(DEV), lut2=w["lut2"].to(DEV), bitwidth2=bits2)
+    y = fx.embedding_gather(ids.to(DEV), w["blob"].to(DEV), w["lut"].to(DEV), N, K, bits, 64,
+                            signs=None if signs is None else signs.to(DEV), rot_block=block or 0, **kw)
+    row = O.embedding_reference(ids, w["blob"].numpy(), w["lut"], N, K, 64, bits,
+                                w["blob2"].numpy() if bits2 else None, w["lut2"], bits2)
+    if signs is None:
+        assert torch.equal(y.cpu(), row)
+        return
+    # the adjoint in blocks is the block transform of the signed row without signs behind it
+    one = torch.ones(K)
+    want = O.fht_adjoint_reference(row.float(), signs) if not block else \
+        O.block_fht_reference(row.float() * signs, block, one)
+    assert rel_l2(y.cpu(), want) <= 1e-3
+
+
+@pytest.mark.gpu
+def test_ids_are_checked_by_the_launch():
+    """One id outside the table anywhere, the first and the last one included, is refused, from
+    several threads at a time; the next good call is served."""
+    from concurrent.futures import ThreadPoolExecutor
+    N, K = 256, 128
+    m = _module(make_weight(N, K, seed=2), True, False).to(DEV)
+    good = torch.arange(N, device=DEV).repeat(5)
+    want = m(good)
+    for at in (0, 700, len(good) - 1):
+        for value in (-1, N, 1 << 40):
+            ids = good.clone()
+            ids[at] = value
+            with pytest.raises(ValueError, match=r"\[0, 256\)"):
+                m(ids)
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            torch.cuda.current_stream().wait_stream(torch.cuda.default_stream())
+            y = m(good)
+            torch.cuda.current_stream().synchronize()
+            return torch.equal(y.cpu(), want_cpu)
+    want_cpu = want.cpu()
+    with ThreadPoolExecutor(4) as pool:
+        assert all(pool.map(work, range(16)))
