@@ -12,7 +12,7 @@ namespace flute {
 
 namespace {
 
-constexpr int kFhtThreads = 256;
+constexpr int kFhtThreads = 512;
 
 struct FhtParams {
     const void *x;
@@ -25,6 +25,7 @@ struct FhtParams {
     int adjoint;
     int block;      // > 0: equal blocks
     int chunk;      // columns transformed per pass in block mode
+    int *shift;     // bfloat16 rows: bf16_row_shift of each result row's largest exponent, or NULL
     // Operand-order output for the LUT GEMM instead of rows (ap != NULL): the rotated row
     // m is rounded to `dtype`, converted to the LUT's 16-bit type and written where the
     // GEMM's activation pre-pass would put it, Ap[g][j][m / 16][lane][8]; rows from M up
@@ -101,7 +102,7 @@ __device__ __forceinline__ void load_cols8(const FhtParams &p, int64_t row, int 
 // to the I/O type, as rows or in the GEMM's operand order.
 __device__ __forceinline__ void store_cols8(const FhtParams &p, int64_t orow, int k, float inv,
                                             const float (&f)[8], const float (&sg)[8],
-                                            const float (&sc)[8]) {
+                                            const float (&sc)[8], uint32_t &top) {
     const int bf16 = p.dtype == FLUTE_BF16;
     uint16_t op[8];
     float t[8];
@@ -118,6 +119,10 @@ __device__ __forceinline__ void store_cols8(const FhtParams &p, int64_t orow, in
             if (p.ap && bf16 != p.ap_bf16) a = round_act(bf16 ? bf2f(a) : h2f(a), p.ap_bf16);
             op[q] = a;
         }
+    }
+    if (p.shift) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) top = max(top, (uint32_t)(op[q] >> 7) & 0xffu);
     }
     if (p.ap) {
         store_operand_order(p, blockIdx.x, k, op);
@@ -136,217 +141,73 @@ __device__ __forceinline__ void store_cols8(const FhtParams &p, int64_t orow, in
     }
 }
 
-// Equal blocks of at most 256 columns without the LDS buffer: three stages in a thread's
-// registers, the stages of length 8 ... block/2 across lanes, in the same ascending order
-// as the buffered butterfly and bit-identical to it.  One memory round trip, no barrier.
-// The lanes of a block are always in the same step of the loop (a step covers 2048
-// columns, a multiple of every block), so a lane's partners are active.
-__device__ __forceinline__ void fht_blocks_inwave(const FhtParams &p, int64_t row, int64_t orow,
-                                                  int tid) {
-    const int nst = 31 - __builtin_clz((unsigned)p.block);
-    const float inv = inv_sqrt_pow2(nst);
-    const int lane = tid & 63;
-    const int pair_lanes = p.block >> 3;               // lanes of one block: 4 ... 32
-    // one step at a time: holding several steps of loads in registers measured slower
-    // (K = 4096: 5.4 us against 3.8 us per launch)
-    for (int j = tid * 8; j < p.K; j += kFhtThreads * 8) {
-        float f[8], sg[8], sc[8];
-        load_cols8(p, row, j, f, sg, sc);
-        stages_in_thread(f);
-        if (pair_lanes > 1) stage_across_lanes<1>(f, lane);
-        if (pair_lanes > 2) stage_across_lanes<2>(f, lane);
-        if (pair_lanes > 4) stage_across_lanes<4>(f, lane);
-        if (pair_lanes > 8) stage_across_lanes<8>(f, lane);
-        if (pair_lanes > 16) stage_across_lanes<16>(f, lane);
-        store_cols8(p, orow, j, inv, f, sg, sc);
-    }
-}
-
-// One power-of-two segment of 512 ... 8192 columns starting at column `off`.  The first
-// nine stages (lengths 1 ... 256) run as in fht_blocks_inwave, the last of them against
-// the lane 32 away (ds_bpermute); the remaining stages (lengths 512 ... b/2, at most
-// four) are one pass over the fp32 buffer in LDS.  Same butterflies in the same ascending
-// order as fht_lds alone, so bit-identical; one memory round trip instead of two, two
-// barriers instead of five, a third of the LDS traffic.  A thread holds up to S steps of
-// eight columns; b/8 is a multiple of 64, so wavefronts are active as a whole, and a
-// step a thread does not have repeats its first one (loads stay unconditional).
-template <int S>
-__device__ __forceinline__ void fht_segment_fast(const FhtParams &p, int64_t row, int64_t orow,
-                                                 int off, int b, int nst, float *buf, int tid) {
-    const float inv = inv_sqrt_pow2(nst);
-    const int lane = tid & 63;
-    const int j0 = tid * 8;
-    constexpr int STEP = kFhtThreads * 8;
-    const bool one = j0 < b;
-    float f[S][8], sg[S][8], sc[S][8];
-    if (one) {
-#pragma unroll
-        for (int h = 0; h < S; ++h)
-            load_cols8(p, row, off + (j0 + h * STEP < b ? j0 + h * STEP : j0), f[h], sg[h], sc[h]);
-#pragma unroll
-        for (int h = 0; h < S; ++h) stages_in_thread(f[h]);
-#pragma unroll
-        for (int h = 0; h < S; ++h) stage_across_lanes<1>(f[h], lane);
-#pragma unroll
-        for (int h = 0; h < S; ++h) stage_across_lanes<2>(f[h], lane);
-#pragma unroll
-        for (int h = 0; h < S; ++h) stage_across_lanes<4>(f[h], lane);
-#pragma unroll
-        for (int h = 0; h < S; ++h) stage_across_lanes<8>(f[h], lane);
-#pragma unroll
-        for (int h = 0; h < S; ++h) stage_across_lanes<16>(f[h], lane);
-#pragma unroll
-        for (int h = 0; h < S; ++h) stage_across_lanes<32>(f[h], lane);
-    }
-    if (nst > 9) {                                     // uniform: stages of length 512 and up
-        if (one) {
-#pragma unroll
-            for (int h = 0; h < S; ++h) {
-                if (j0 + h * STEP < b) {
-                    const int s0 = fht_slot(j0 + h * STEP);   // multiple of 8: slot(j + q) = s0 ^ q
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) buf[s0 ^ q] = f[h][q];
-                }
-            }
-        }
-        __syncthreads();
-        switch (nst - 9) {
-            case 1: fht_pass<1>(buf, b, 9, tid, kFhtThreads); break;
-            case 2: fht_pass<2>(buf, b, 9, tid, kFhtThreads); break;
-            case 3: fht_pass<3>(buf, b, 9, tid, kFhtThreads); break;
-            default: fht_pass<4>(buf, b, 9, tid, kFhtThreads); break;
-        }
-        __syncthreads();
-        if (one) {
-#pragma unroll
-            for (int h = 0; h < S; ++h) {
-                if (j0 + h * STEP < b) {
-                    const int s0 = fht_slot(j0 + h * STEP);
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) f[h][q] = buf[s0 ^ q];
-                }
-            }
-        }
-        __syncthreads();                               // the next segment reuses the buffer
-    }
-    if (one) {
-#pragma unroll
-        for (int h = 0; h < S; ++h)
-            if (j0 + h * STEP < b) store_cols8(p, orow, off + j0 + h * STEP, inv, f[h], sg[h], sc[h]);
-    }
-}
-
-// MAXS: steps of eight columns a thread may hold in the register-resident segment path
-// (0: every segment through the LDS buffer; 2: segments up to 4096 columns in registers;
-// 4: up to 8192, at twice the registers).
-template <int MAXS>
+// One workgroup per row, eight consecutive columns a thread and step.  The first nine stages stay in
+// registers (fht_head: between a thread's columns, then between lanes), the rest are one or two
+// passes over an fp32 buffer in LDS; blocks and segments of up to 512 columns never touch it.  What
+// bounds it: for few rows the chain load -> stages -> barriers -> store, so a row's values and
+// multipliers are one memory round trip; for many rows the loads and stores.  Eight wavefronts of
+// one step each keep 4096 columns in few registers, so a CU holds several rows: the earlier form,
+// four wavefronts of two steps, took 204 registers, its form for 8192 columns 270.  Before and now:
+// 1 x 4096 5.3 -> 3.9 us, 1 x 12288 12.1 -> 8.1, 1000 x 4096 12.1 -> 8.9, 1024 x 12288 38.4 -> 22.1.
 __global__ void __launch_bounds__(kFhtThreads) fht_kernel(const FhtParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
     float *buf = (float *)lds;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
     const int64_t row = (int64_t)blockIdx.x * p.ldx;
     const int64_t orow = (int64_t)blockIdx.x * p.ldo;
+    constexpr int STEP = kFhtThreads * 8;
     if (p.ap && (int)blockIdx.x >= p.ap_M) {           // padding row of the operand image
         const uint16_t zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (int j = tid * 8; j < p.K; j += kFhtThreads * 8)
+        for (int j = tid * 8; j < p.K; j += STEP)
             store_operand_order(p, blockIdx.x, j, zero);
         return;
     }
-    if (p.block > 0 && p.block <= 256) {
-        fht_blocks_inwave(p, row, orow, tid);
-        return;
-    }
+    uint32_t top = 0;
     // block mode: chunks of whole blocks; otherwise the descending power-of-two
     // segments of K (fht.py:118-134 upstream)
     for (int off = 0; off < p.K;) {
-        int count, nstages;
+        int count, nst;
         if (p.block > 0) {
             count = min(p.chunk, p.K - off);
-            nstages = 31 - __builtin_clz((unsigned)p.block);
+            nst = 31 - __builtin_clz((unsigned)p.block);
         } else {
-            nstages = 31 - __builtin_clz((unsigned)(p.K - off));
-            count = 1 << nstages;
+            nst = 31 - __builtin_clz((unsigned)(p.K - off));
+            count = 1 << nst;
         }
-        if constexpr (MAXS > 0) {
-            if (p.block == 0 && count >= 512 && count <= kFhtThreads * 8 * MAXS) {
-                if (MAXS == 2 || count <= kFhtThreads * 16)
-                    fht_segment_fast<2>(p, row, orow, off, count, nstages, buf, tid);
-                else
-                    fht_segment_fast<MAXS>(p, row, orow, off, count, nstages, buf, tid);
-                off += count;
-                continue;
+        const float inv = inv_sqrt_pow2(nst);
+        float f[8], sg[8], sc[8];
+        for (int j = tid * 8; j < count; j += STEP) {
+            load_cols8(p, row, off + j, f, sg, sc);
+            fht_head(f, lane, nst);
+            if (nst <= 9) {
+                store_cols8(p, orow, off + j, inv, f, sg, sc, top);
+            } else {
+                const int s0 = fht_slot(j);            // a multiple of 8: slot(j + q) = s0 ^ q
+#pragma unroll
+                for (int q = 0; q < 8; ++q) buf[s0 ^ q] = f[q];
             }
         }
-        const float inv = inv_sqrt_pow2(nstages);
-        // The output multipliers of a thread's first two steps are requested together
-        // with the row, so the output phase does not start with a memory round trip.
-        const int j0 = tid * 8, j1 = j0 + kFhtThreads * 8;
-        float sg0[8], sg1[8], sc0[8], sc1[8];
-        auto load_mul = [&](int j, float (&sg)[8], float (&sc)[8]) {
-            if (p.adjoint) return;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) sg[q] = p.signs[off + j + q];
-            if (p.awq) {
-#pragma unroll
-                for (int q = 0; q < 8; ++q) sc[q] = p.awq[off + j + q];
-            }
-        };
-        if (j0 < count) load_mul(j0, sg0, sc0);
-        if (j1 < count) load_mul(j1, sg1, sc1);
-        // Eight columns per thread and step; the loads of a step (row, signs, scale) are
-        // independent and issued together, so each phase is one memory round trip.
-#pragma unroll 2
-        for (int j = tid * 8; j < count; j += kFhtThreads * 8) {
-            float f[8], m[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) f[q] = load_any(p.x, row + off + j + q, p.dtype);
-            if (p.adjoint || p.awq) {
-                const float *mul = p.adjoint ? p.signs : p.awq;
-#pragma unroll
-                for (int q = 0; q < 8; ++q) m[q] = mul[off + j + q];
-#pragma unroll
-                for (int q = 0; q < 8; ++q) f[q] *= m[q];
-            }
-#pragma unroll
-            for (int q = 0; q < 8; ++q) buf[fht_slot(j + q)] = f[q];
-        }
-        __syncthreads();
-        fht_lds(buf, count, nstages, tid, kFhtThreads);
-        auto emit = [&](int j, const float (&sg)[8], const float (&sc)[8]) {
-            uint16_t op[8];
-            float tt[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const float b = buf[fht_slot(j + q)];
-                tt[q] = p.adjoint ? b * inv : b * sg[q] * inv;
-            }
-            if (!p.adjoint && p.awq) {
-#pragma unroll
-                for (int q = 0; q < 8; ++q) tt[q] = tt[q] / sc[q];
-            }
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const float t = tt[q];
-                if (p.ap) {
-                    const int in_bf16 = p.dtype == FLUTE_BF16;
-                    uint16_t a = round_act(t, in_bf16);
-                    if (in_bf16 != p.ap_bf16) a = round_act(in_bf16 ? bf2f(a) : h2f(a), p.ap_bf16);
-                    op[q] = a;
-                } else {
-                    store_any(p.out, orow + off + j + q, p.dtype, t);
+        if (nst > 9) {
+            __syncthreads();
+            fht_tail(buf, count, nst, 9, tid, kFhtThreads);
+            for (int j = tid * 8; j < count; j += STEP) {
+                if (count > STEP) {                    // (one step: the multipliers are still here)
+                    load_mul8(p.signs, off + j, p.vec_mul, sg);
+                    if (p.awq) load_mul8(p.awq, off + j, p.vec_mul, sc);
                 }
+                const int s0 = fht_slot(j);
+#pragma unroll
+                for (int q = 0; q < 8; ++q) f[q] = buf[s0 ^ q];
+                store_cols8(p, orow, off + j, inv, f, sg, sc, top);
             }
-            if (p.ap) store_operand_order(p, blockIdx.x, off + j, op);
-        };
-        if (j0 < count) emit(j0, sg0, sc0);
-        if (j1 < count) emit(j1, sg1, sc1);
-        for (int j = j1 + kFhtThreads * 8; j < count; j += kFhtThreads * 8) {
-            float sg[8], sc[8];
-            load_mul(j, sg, sc);
-            emit(j, sg, sc);
+            __syncthreads();                           // the next segment reuses the buffer
         }
-        __syncthreads();
         off += count;
+    }
+    if (p.shift) {
+        __shared__ uint32_t slots[kFhtThreads / 64];
+        top = workgroup_max(top, slots, tid, kFhtThreads);
+        if (tid == 0) p.shift[blockIdx.x] = bf16_row_shift(top);
     }
 }
 
@@ -358,7 +219,7 @@ namespace flute {
 
 flute_status fht_launch(const void *x, int64_t ldx, const float *signs, const float *awq, void *out,
                         int64_t ldo, int M, int K, int dtype, int adjoint, int block,
-                        hipStream_t stream, const FhtOperandOut *operand) {
+                        hipStream_t stream, const FhtOperandOut *operand, int *shift) {
     FhtParams p;
     p.x = x;
     p.out = out;
@@ -371,6 +232,7 @@ flute_status fht_launch(const void *x, int64_t ldx, const float *signs, const fl
     p.adjoint = adjoint ? 1 : 0;
     p.block = block;
     p.chunk = 0;
+    p.shift = shift;
     p.ap = operand ? operand->ap : nullptr;
     p.ap_M = M;
     p.ap_mblk_pad = operand ? operand->mblk_pad : 0;
@@ -381,50 +243,28 @@ flute_status fht_launch(const void *x, int64_t ldx, const float *signs, const fl
                (operand || (((uintptr_t)out & 15) == 0 && ldo % 8 == 0));
     p.vec_mul = ((uintptr_t)signs & 15) == 0 && (!awq || ((uintptr_t)awq & 15) == 0);
     size_t lds_bytes;
-    bool wide = false;
     if (block > 0) {
         FLUTE_REQUIRE(is_pow2(block) && block >= 32 && block <= 16384 && K % block == 0,
                       FLUTE_ERR_INVALID,
                       "flute_fht: block must be a power of two in [32, 16384] dividing K (got %d)",
                       block);
         p.chunk = K <= 16384 ? K : (16384 / block) * block;
-        lds_bytes = (size_t)p.chunk * 4;
+        lds_bytes = block > 512 ? (size_t)p.chunk * 4 : 0;
     } else {
         const Segs segs = make_segments(K, 0);
         FLUTE_REQUIRE(segs.len[0] <= 16384, FLUTE_ERR_UNSUPPORTED,
                       "flute_fht: segment of %d columns exceeds the 16384-column LDS tile",
                       segs.len[0]);
-        lds_bytes = (size_t)segs.len[0] * 4;
-        wide = segs.len[0] > kFhtThreads * 16 && segs.len[0] <= kFhtThreads * 32;
+        lds_bytes = segs.len[0] > 512 ? (size_t)segs.len[0] * 4 : 0;
     }
     const int rows = operand ? operand->mblk_pad * 16 : M;
     if (rows == 0) return FLUTE_OK;
     static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
     if (!attr_done) {
-        FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)fht_kernel<2>,
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
-        FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)fht_kernel<0>,
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
-        FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)fht_kernel<4>,
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
+        FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)fht_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 98304));
         attr_done = true;
     }
-    // Which variant: the register-resident segment path wins wherever it applies, except
-    // that its wide form (segments of 8192 columns, 270 registers, one workgroup per CU)
-    // loses to the buffered kernel once there are many rows (K = 12288: 12.4 us against
-    // 21.0 us for one row, 52.6 us against 40.3 us for 1024 rows).  FLUTE_FHT_STEPS = 0, 2
-    // or 4 forces a variant (tuning and test knob).
-    int steps = wide ? (rows <= 512 ? 4 : 0) : 2;
-    {
-        const int v = tuning().fht_steps;
-        if (v == 0 || v == 2 || v == 4) steps = v;
-    }
-    if (steps == 0)
-        hipLaunchKernelGGL(fht_kernel<0>, dim3(rows), dim3(kFhtThreads), lds_bytes, stream, p);
-    else if (steps == 4)
-        hipLaunchKernelGGL(fht_kernel<4>, dim3(rows), dim3(kFhtThreads), lds_bytes, stream, p);
-    else
-        hipLaunchKernelGGL(fht_kernel<2>, dim3(rows), dim3(kFhtThreads), lds_bytes, stream, p);
+    hipLaunchKernelGGL(fht_kernel, dim3(rows), dim3(kFhtThreads), lds_bytes, stream, p);
     FLUTE_HIP_CHECK(hipGetLastError());
     return FLUTE_OK;
 }

@@ -6,6 +6,7 @@
 #include "gemm_wide_kernel.h"
 #include "host_common.h"
 
+#include <algorithm>
 #include <atomic>
 
 namespace flute {
@@ -105,17 +106,34 @@ flute_status launch_gemm_shape(const GemmShape &s, const GemmParams &p, dim3 gri
 }
 
 
+// Slices of K a coefficient launch takes: as many blocks as the chip has CUs, 512 columns (one
+// step of a workgroup) or more each.
+int coeff_slices(int M, int K, int R) {
+    const int64_t blocks = (int64_t)((M + 15) / 16) * ((R + 15) / 16);
+    int s = 1;
+    while (s < 16 && blocks * s * 2 <= kNumCU && K / (s * 2) >= 512) s *= 2;
+    return s >= 4 ? s : 1;
+}
+// What that takes of the workspace: floats of partial sums, tickets.
+size_t coeff_floats(int M, int K, int R) {
+    const int s = R > 0 ? coeff_slices(M, K, R) : 1;
+    return s > 1 ? (size_t)s * ((M + 15) / 16) * ((R + 15) / 16) * 256 : 0;
+}
+size_t coeff_tickets(int M, int R) { return (size_t)((M + 15) / 16) * ((R + 15) / 16); }
+
 // xb[m, r] = sum_k A[m, k] * resB[r, k] in fp32.
 flute_status launch_coeff(const void *A, int64_t lda, const void *resB, float *xb, int M, int K, int R, int is_bf16,
-                          hipStream_t stream) {
-    const dim3 grid((M + 15) / 16, (R + 15) / 16);
+                          float *part, int *tickets, hipStream_t stream) {
+    const int slices = coeff_slices(M, K, R);
+    const int kper = (K / 32 + slices - 1) / slices * 32;
+    const dim3 grid((M + 15) / 16, (R + 15) / 16, slices);
     const int aligned = ((uintptr_t)A & 15) == 0 && lda % 8 == 0 && ((uintptr_t)resB & 15) == 0;
     if (is_bf16)
         hipLaunchKernelGGL(gemm_coeff_kernel<true>, grid, dim3(1024), 0, stream, (const uint16_t *)A, lda,
-                           (const uint16_t *)resB, xb, M, K, R, aligned);
+                           (const uint16_t *)resB, xb, M, K, R, aligned, kper, part, tickets);
     else
         hipLaunchKernelGGL(gemm_coeff_kernel<false>, grid, dim3(1024), 0, stream, (const uint16_t *)A, lda,
-                           (const uint16_t *)resB, xb, M, K, R, aligned);
+                           (const uint16_t *)resB, xb, M, K, R, aligned, kper, part, tickets);
     FLUTE_HIP_CHECK(hipGetLastError());
     return FLUTE_OK;
 }
@@ -182,9 +200,9 @@ struct WidePlan {
 // streams that a workgroup takes, `rounds` = workgroups / 256 CUs, rounded up):
 //   128-row workgroups of gemm_kernel.h   8 + 0.43 a tile (64-row ones 0.26) per round; two
 //                                         streams are two launches, other widths 15 % more
-//   512-row workgroups                    14 + 0.95 ... 1.35 a step (the clock falls as the chip
+//   512-row workgroups                    14 a round + 0.95 ... 1.35 a step (the clock falls as the chip
 //                                         fills); slices of K cost 5 each (256 KB written, read)
-//   256-row workgroups                    14 + 0.65 ... 0.90 a step; slices 2.5 each
+//   256-row workgroups                    14 a round + 0.65 ... 0.90 a step; slices 2.5 each
 // e.g. M = 1024, 4096 -> 12288: 120 / 92 / 118 us (estimated 105 / 94 / 122); M = 512: 74 / 61
 // (two slices) / 61; M = 512, 12288 -> 4096: 59 / 77 (four) / 65 (four), the others stay; two
 // streams (4, 1) at M = 1024, 4096 -> 12288: 263 / 165 / 190, at M = 192: 76 / - / 60 (two).
@@ -214,7 +232,7 @@ WidePlan choose_wide(int M, int tiles, int G, int streams, bool four_bit, const 
             const int64_t groups = units * ks, rounds = (groups + kNumCU - 1) / kNumCU;
             const double fill = groups < kNumCU ? (double)groups / kNumCU : 1.0;
             const double step = rows == 512 ? 0.95 + 0.40 * fill : 0.65 + 0.25 * fill;
-            const double us = 14.0 + rounds * (step * streams * ((G + ks - 1) / ks)) +
+            const double us = rounds * (14.0 + step * streams * ((G + ks - 1) / ks)) +
                               (ks > 1 ? (rows == 512 ? 5.0 : 2.5) * ks : 0.0);
             if (us < best) {
                 best = us;
@@ -250,20 +268,24 @@ flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *c
     auto up4 = [](size_t n) { return (n + 3) & ~(size_t)3; };
     const size_t image_floats = (size_t)K * mblk * 8, rot_floats = up4((size_t)M * K / 2);
     const size_t shift_floats = scale_rows ? up4(M) : 0;
-    size_t xb_floats = 0;
+    size_t xb_floats = 0, part_xb = 0, want_tickets = 0;
     int tiles = 0;
     for (int i = 0; i < count; ++i) {
         xb_floats += up4((size_t)M * ws[i].R);
+        part_xb = std::max(part_xb, coeff_floats(M, K, ws[i].R));
+        want_tickets = std::max(want_tickets, coeff_tickets(M, ws[i].R));
         tiles += ws[i].N / 128;
     }
     const size_t part_floats = slices > 1 ? (size_t)slices * mtiles * tiles * plan.rows * 128 : 0;
-    size_t total = part_floats + xb_floats + 64;
+    size_t total = part_floats + xb_floats + part_xb + 64;
     for (int k = 0; k < images; ++k) total += image_floats + shift_floats + (ws[owner[k]].signs ? rot_floats : 0);
     float *base = nullptr;
     int *tickets = nullptr;
-    flute_status st = get_workspace(total, (size_t)mtiles * tiles + 1, stream, &base, &tickets);
+    want_tickets = std::max(want_tickets, (size_t)mtiles * tiles) + 1;
+    flute_status st = get_workspace(total, want_tickets, stream, &base, &tickets);
     if (st != FLUTE_OK) return st;
-    float *next = base + part_floats;
+    float *const xb_part = base + part_floats;
+    float *next = xb_part + part_xb;
 
     const u4_t *image[kWideMaxSegs];
     const int *shift[kWideMaxSegs];
@@ -274,14 +296,19 @@ flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *c
         rows[k] = A;
         ldr[k] = lda;
         if (w.signs) {
-            st = fht_launch(A, lda, w.signs, w.awq, next, K, M, K, act_dtype, 0, w.rot_block, stream, nullptr);
+            // (the rotation knows its rows' largest exponents)
+            int *const row_shift = scale_rows ? (int *)(next + rot_floats) : nullptr;
+            st = fht_launch(A, lda, w.signs, w.awq, next, K, M, K, act_dtype, 0, w.rot_block, stream, nullptr, row_shift);
             if (st != FLUTE_OK) return st;
             rows[k] = next;
             ldr[k] = K;
             next += rot_floats;
         }
         shift[k] = nullptr;
-        if (scale_rows) {
+        if (scale_rows && w.signs) {
+            shift[k] = (const int *)next;
+            next += shift_floats;
+        } else if (scale_rows) {
             hipLaunchKernelGGL(gemm_rowshift_kernel, dim3(M), dim3(256), 0, stream, (const uint16_t *)rows[k], ldr[k], K,
                                (int *)next);
             FLUTE_HIP_CHECK(hipGetLastError());
@@ -302,7 +329,8 @@ flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *c
         xb[i] = nullptr;
         if (ws[i].R == 0) continue;
         xb[i] = next;
-        st = launch_coeff(rows[image_of[i]], ldr[image_of[i]], ws[i].resB, next, M, K, ws[i].R, out_bf16, stream);
+        st = launch_coeff(rows[image_of[i]], ldr[image_of[i]], ws[i].resB, next, M, K, ws[i].R, out_bf16, xb_part, tickets,
+                          stream);
         if (st != FLUTE_OK) return st;
         next += up4((size_t)M * ws[i].R);
     }
@@ -437,7 +465,7 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
     const size_t image = (size_t)shape.mw * shape.mb * 8 * 64 * 4;
     const int zparts = ksplit * ((p.nstreams == 2 && shape.mb > 1) ? 2 : 1);
     const size_t p_floats = zparts > 1 ? (size_t)zparts * units * image : 0;
-    const size_t xb_floats = ((size_t)M * w->R + 3) & ~(size_t)3;
+    const size_t xb_floats = (((size_t)M * w->R + 3) & ~(size_t)3) + coeff_floats(M, w->K, w->R);
     const size_t ap_floats = (size_t)p.G * 2 * p.mblk_pad * 64 * 4;
     const size_t rot_floats = w->signs ? ((size_t)M * w->K / 2 + 4) & ~(size_t)3 : 0;
     // bfloat16 activations presented as float16 operands: one power-of-two scale per row
@@ -445,7 +473,8 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
     const size_t shift_floats = scale_rows ? ((size_t)M + 3) & ~(size_t)3 : 0;
     float *base = nullptr;
     int *tickets = nullptr;
-    st = get_workspace(p_floats + xb_floats + ap_floats + rot_floats + shift_floats + 64, (size_t)units + 1, stream, &base,
+    const size_t want_tickets = std::max((size_t)units, coeff_tickets(M, w->R)) + 1;
+    st = get_workspace(p_floats + xb_floats + ap_floats + rot_floats + shift_floats + 64, want_tickets, stream, &base,
                        &tickets);
     if (st != FLUTE_OK) return st;
     p.P = base;
@@ -453,20 +482,6 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
     float *xb = base + p_floats;
     u4_t *Ap = (u4_t *)(xb + xb_floats);
     p.Ap = Ap;
-    // One block of rows per wavefront on the single-stream 4-bit fast path: the kernel reads
-    // A itself (16-byte pieces of a row, put into operand order in registers), so the
-    // pre-pass launch is dropped.  Needs 16-byte aligned rows.
-    {
-        const int ngrp = w->group_size >= 128 ? 1 : 128 / w->group_size;
-        const bool fast = p.nstreams == 1 && w->b1 == 4 && ngrp <= 2 &&
-                          !tuning().gemm_no_perm;
-        if (shape.mb == 1 && fast && !w->signs && ((uintptr_t)A & 15) == 0 && lda % 8 == 0 &&
-            !tuning().gemm_no_direct) {
-            p.A8 = (const u4_t *)A;
-            p.lda8 = lda / 8;
-            p.a_bf16 = act_dtype == FLUTE_BF16;
-        }
-    }
     int *rowshift = scale_rows
         ? (int *)(base + p_floats + xb_floats + ap_floats + rot_floats) : nullptr;
     auto launch_rowshift = [&](const void *rows, int64_t ld) -> flute_status {
@@ -476,13 +491,16 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
         p.rowshift = rowshift;
         return FLUTE_OK;
     };
-    if (p.A8) {
-        // nothing to prepare but the row scales
-        if (scale_rows) {
-            st = launch_rowshift(A, lda);
-            if (st != FLUTE_OK) return st;
-        }
-    } else if (w->signs && w->R == 0 && !scale_rows) {
+    // One block of rows per wavefront on the single-stream 4-bit fast path: the kernel reads
+    // A itself (16-byte pieces of a row, put into operand order in registers), so the
+    // pre-pass launch is dropped.  Needs 16-byte aligned rows; rotated rows are read the same way
+    // (the rotation can write the image itself, but only without a residual and row scales).
+    const bool direct = [&] {
+        const int ngrp = w->group_size >= 128 ? 1 : 128 / w->group_size;
+        return shape.mb == 1 && p.nstreams == 1 && w->b1 == 4 && ngrp <= 2 && !tuning().gemm_no_perm &&
+               !tuning().gemm_no_direct;
+    }();
+    if (w->signs && w->R == 0 && !scale_rows) {
         // the rotation writes the operand image itself: one launch instead of two
         FhtOperandOut image_out = {(uint32_t *)Ap, p.mblk_pad, (int)(w->lut_dtype == FLUTE_BF16), block_xor};
         st = fht_launch(A, lda, w->signs, w->awq, nullptr, 0, M, w->K, act_dtype, 0, w->rot_block,
@@ -494,18 +512,23 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
             // rotated copy first, then the ordinary pre-pass on it
             void *Arot = (void *)(Ap + (size_t)p.G * 2 * p.mblk_pad * 64);
             st = fht_launch(A, lda, w->signs, w->awq, Arot, w->K, M, w->K, act_dtype, 0,
-                            w->rot_block, stream, nullptr);
+                            w->rot_block, stream, nullptr, rowshift);
             if (st != FLUTE_OK) return st;
             A = Arot;
             lda = w->K;
-        }
-        if (scale_rows) {
+            p.rowshift = rowshift;                      // (the rotation knows its rows' largest exponents)
+        } else if (scale_rows) {
             st = launch_rowshift(A, lda);
             if (st != FLUTE_OK) return st;
         }
         const int64_t total = (int64_t)p.G * 2 * p.mblk_pad * 64;
         const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
-        if (((uintptr_t)A & 15) == 0 && lda % 8 == 0) {
+        const bool rows16 = ((uintptr_t)A & 15) == 0 && lda % 8 == 0;
+        if (direct && rows16) {
+            p.A8 = (const u4_t *)A;
+            p.lda8 = lda / 8;
+            p.a_bf16 = act_dtype == FLUTE_BF16;
+        } else if (rows16) {
             // 16-byte aligned rows: one coalesced 16-byte load per thread and a transpose
             // inside each quad (M = 256, K = 4096: 2.2 us against 5.2 us for the gathers)
             hipLaunchKernelGGL(gemm_prep_quad_kernel, dim3(blocks), dim3(256), 0, stream,
@@ -522,9 +545,11 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
         FLUTE_HIP_CHECK(hipGetLastError());
     }
     if (w->R > 0) {
-        st = launch_coeff(A, lda, w->resB, xb, M, w->K, w->R, p.out_bf16, stream);
+        st = launch_coeff(A, lda, w->resB, xb, M, w->K, w->R, p.out_bf16, xb + (((size_t)M * w->R + 3) & ~(size_t)3),
+                          tickets, stream);
         if (st != FLUTE_OK) return st;
         p.xb = xb;
+        p.vec_res = w->R % 8 == 0 && ((uintptr_t)w->resA & 15) == 0 && ((uintptr_t)xb & 15) == 0;
     }
 
     // Two streams with four blocks per wavefront: one launch per stream through the

@@ -35,20 +35,21 @@ int workspace_decision(size_t have_floats, size_t need_floats, size_t have_ints,
 // (flute_reload_tuning re-reads them): FLUTE_GEMV_RW, FLUTE_GEMV_WAVES,
 // FLUTE_GEMV_TABLE_LOG2, FLUTE_GEMV_PREROTATE, FLUTE_GEMV4_PF, FLUTE_GEMV_NO_FAST,
 // FLUTE_GEMV4_WALK, FLUTE_GEMV_XCD, FLUTE_GEMM_ROWS, FLUTE_GEMM_NO_PERM, FLUTE_GEMM_KSPLIT,
-// FLUTE_GEMM_NO_DIRECT, FLUTE_GEMM_NO_LEAN, FLUTE_GEMM_NO_BALANCE, FLUTE_GEMM_NO_HANDOVER,
-// FLUTE_FHT_STEPS.  Unset or empty = 0, except fht_steps and
+// FLUTE_GEMM_NO_DIRECT, FLUTE_GEMM_NO_LEAN, FLUTE_GEMM_NO_BALANCE, FLUTE_GEMM_NO_HANDOVER;
+// unset or empty = 0, except
 // gemv4_walk = -1 (the launcher's own choice) and gemv_xcd = 1 (0: workgroup b of the lean GEMV takes
 // row slice b instead of a contiguous run of slices per XCD).
 struct Tuning {
     int gemv_rw, gemv_waves, gemv_table_log2, gemv_prerotate, gemv4_pf, gemv_no_fast, gemv4_walk, gemv_xcd;
     int gemm_rows, gemm_no_perm, gemm_ksplit, gemm_no_direct, gemm_no_lean, gemm_no_balance, gemm_no_handover;
-    int fht_steps;
 };
 const Tuning &tuning();
 
 // The Walsh-Hadamard rotation of flute_fht with row strides, and optionally with its
 // output written in the operand order of the LUT GEMM (the image the GEMM's activation
 // pre-pass would produce from the rotated rows, padding rows zeroed) instead of as rows.
+// shift: [M] or NULL; bfloat16 rows: the power of two that brings a result row's largest
+// magnitude to [1, 2) (bf16_row_shift).
 struct FhtOperandOut {
     uint32_t *ap;       // Ap[g][j][m / 16][lane][4 dwords]
     int mblk_pad;       // 16-row blocks the image holds per half tile
@@ -57,7 +58,7 @@ struct FhtOperandOut {
 };
 flute_status fht_launch(const void *x, int64_t ldx, const float *signs, const float *awq, void *out,
                         int64_t ldo, int M, int K, int dtype, int adjoint, int block,
-                        hipStream_t stream, const FhtOperandOut *operand);
+                        hipStream_t stream, const FhtOperandOut *operand, int *shift = nullptr);
 
 inline bool is_pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
 inline int ilog2(int v) { return 31 - __builtin_clz((unsigned)v); }
