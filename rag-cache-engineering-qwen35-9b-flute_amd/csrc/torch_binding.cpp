@@ -7,6 +7,7 @@
 //   qgemm_gemv_splitk_fht_stream            (src/bindings.cpp:277-354)
 //   qgemm_gemv_multi, qgemm_gemv_mlp        (src/bindings.cpp:368-384)
 //   qgemm_cutlass_streaming, qgemm_dual_stream   (src/bindings.cpp:245-270)
+//   qgemm_linear, embedding_rows            (what a module's forward calls; no upstream counterpart)
 //
 // Same positional signatures, same conventions (empty tensor = absent operand, N from the
 // blob's byte count, RuntimeError on every contract violation, fresh outputs, launches on the
@@ -184,7 +185,9 @@ Tensor gemv(const char *who, const Tensor &A_in, const Tensor &indices, const Te
 
 Tensor gemm(const char *who, const Tensor &A_in, const Tensor &indices, const Tensor &lut,
             int64_t b1, const Tensor &indices2, const Tensor &lut2, int64_t b2, const Tensor &resB,
-            const Tensor &resA, const Tensor &bias, int64_t gs) {
+            const Tensor &resA, const Tensor &bias, int64_t gs,
+            const c10::optional<Tensor> &signs = c10::nullopt,
+            const c10::optional<Tensor> &awq = c10::nullopt) {
     const Shape2 s = check_2d_input(who, A_in, false);
     if (s.K == 0 || s.M == 0 || indices.numel() == 0) {
         const int64_t rb = (s.K * b1) / 8;
@@ -192,7 +195,7 @@ Tensor gemm(const char *who, const Tensor &A_in, const Tensor &indices, const Te
         return torch::zeros({s.M, N}, A_in.options());
     }
     Described d = describe(who, A_in, s.K, indices, lut, b1, indices2, lut2, b2, resB, resA, bias,
-                           gs, c10::nullopt, c10::nullopt, 0, kGsAll, 256);
+                           gs, signs, awq, 0, kGsAll, 256);
     const Tensor A = aligned16(A_in);
     c10::DeviceGuard guard(A.device());
     Tensor C = torch::empty({s.M, d.N}, A.options());
@@ -358,6 +361,51 @@ Tensor qgemm_dual_stream(const Tensor &A, const Tensor &indices, const Tensor &l
     return gemm("qgemm_dual_stream", A, indices, lut, b1, indices2, lut2, b2, resB, resA, bias, gs);
 }
 
+// ---- one call per module forward ----------------------------------------------------------
+
+Tensor qgemm_linear(const Tensor &A, const Tensor &indices, const Tensor &lut, int64_t b1,
+                    const c10::optional<Tensor> &indices2, const c10::optional<Tensor> &lut2, int64_t b2,
+                    const c10::optional<Tensor> &resB, const c10::optional<Tensor> &resA,
+                    const c10::optional<Tensor> &bias, int64_t gs, const c10::optional<Tensor> &signs,
+                    const c10::optional<Tensor> &awq) {
+    const auto held = [](const c10::optional<Tensor> &t) { return t.has_value() ? *t : Tensor(); };
+    if (A.dim() == 2 && A.size(0) == 1)
+        return gemv("qgemm_linear", A, indices, lut, b1, held(indices2), held(lut2), b2, held(resB), held(resA),
+                    held(bias), gs, signs, awq, 0, 0, kGsAll, 256);
+    return gemm("qgemm_linear", A, indices, lut, b1, held(indices2), held(lut2), b2, held(resB), held(resA),
+                held(bias), gs, signs, awq);
+}
+
+// Rows `ids` (int64, contiguous, flat) of a table, and whether every id lay in it (true where
+// nobody asked).
+std::pair<Tensor, bool> embedding_rows(const Tensor &ids, const Tensor &indices, const Tensor &lut, int64_t N,
+                                       int64_t K, int64_t b1, int64_t gs, const c10::optional<Tensor> &indices2,
+                                       const c10::optional<Tensor> &lut2, int64_t b2,
+                                       const c10::optional<Tensor> &resB, const c10::optional<Tensor> &resA,
+                                       const c10::optional<Tensor> &signs, int64_t rot_block, bool check_ids) {
+    const char *who = "embedding_gather";
+    const auto held = [](const c10::optional<Tensor> &t) { return t.has_value() ? *t : Tensor(); };
+    c10::DeviceGuard guard(lut.device());
+    const Tensor out = torch::empty({ids.numel(), K}, lut.options());
+    // (the row whose type and device the checks compare the operands with)
+    const Tensor like = ids.numel() ? out.narrow(0, 0, 1) : torch::empty({1, K}, lut.options());
+    Described d = describe(who, like, K, indices, lut, b1, held(indices2), held(lut2), b2, held(resB), held(resA),
+                           Tensor(), gs, signs, c10::nullopt, rot_block, kGsAll, 256);
+    TORCH_CHECK(d.N == N, who, ": blob holds N=", d.N, ", not ", N);
+    TORCH_CHECK(ids.scalar_type() == at::kLong && ids.is_contiguous() && ids.device() == lut.device(), who,
+                ": ids must be contiguous int64 on the table's device");
+    int in_range = 1;
+    flute_status st;
+    {
+        pybind11::gil_scoped_release unlocked;            // the checked form waits for the launch's verdict
+        st = check_ids ? flute_embedding_checked(&d.w, ids.data_ptr<int64_t>(), ids.numel(), out.data_ptr(),
+                                                 stream_of(lut), &in_range)
+                       : flute_embedding(&d.w, ids.data_ptr<int64_t>(), ids.numel(), out.data_ptr(), stream_of(lut));
+    }
+    check_status(st);
+    return {out, in_range != 0};
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -375,6 +423,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("lut2"), py::arg("bitwidth2"), py::arg("resB"), py::arg("resA"), py::arg("bias"),
           py::arg("group_size"), py::arg("signs"), py::arg("s"), py::arg("split") = 0,
           py::arg("rot_block") = 0);
+    m.def("qgemm_linear", &qgemm_linear);
+    m.def("embedding_rows", &embedding_rows);
     m.def("qgemm_gemv_multi", &qgemm_gemv_multi, py::arg("A"), py::arg("seg_table"),
           py::arg("lut_dtype") = py::none(), py::arg("split") = 0);
     m.def("qgemm_gemv_mlp", &qgemm_gemv_mlp, py::arg("A"), py::arg("seg_table"), py::arg("C"),

@@ -334,13 +334,13 @@ def qgemm_gemv_mlp(A, seg_table, C, lut_dtype: Optional[torch.dtype] = None, spl
 # ---------------------------------------------------------------------------
 
 def _gemm(who, A, indices, lut, bitwidth, indices2, lut2, bitwidth2, resB, resA, bias,
-          group_size, gs_allowed=_GS_ALL, max_rank=256):
+          group_size, gs_allowed=_GS_ALL, max_rank=256, signs=None, s=None):
     M, K = _check_2d_input(who, A, need_m1=False)
     if K == 0 or M == 0 or indices.numel() == 0:
         N = 0 if K == 0 else indices.numel() // max(1, (K * int(bitwidth)) // 8)
         return torch.zeros((M, N), dtype=A.dtype, device=A.device)
     w, N, keep = _describe(who, A, K, indices, lut, bitwidth, indices2, lut2, bitwidth2,
-                           resB, resA, bias, group_size, None, None, 0, gs_allowed, max_rank)
+                           resB, resA, bias, group_size, signs, s, 0, gs_allowed, max_rank)
     A = _aligned16(A)
     with _on_device_of(A):
         C = torch.empty((M, N), dtype=A.dtype, device=A.device)
@@ -382,6 +382,15 @@ def qgemm_dual_stream(A, indices, lut, bitwidth, indices2, lut2, bitwidth2, resB
     (src/kernel_streaming.cu:2113-2294 upstream)."""
     return _gemm("qgemm_dual_stream", A, indices, lut, bitwidth, indices2, lut2, bitwidth2,
                  resB, resA, bias, group_size)
+
+
+def qgemm_linear(A, indices, lut, bitwidth, indices2, lut2, bitwidth2, resB, resA, bias, group_size,
+                 signs=None, s=None):
+    """A whole palettized layer on M rows, absent operands None: the GEMV for one row, the GEMM
+    for more; signs (and s) rotate A first."""
+    run = _gemv if A.dim() == 2 and A.shape[0] == 1 else _gemm
+    return run("qgemm_linear", A, indices, lut, bitwidth, indices2, lut2, bitwidth2, resB, resA,
+               bias, group_size, signs=signs, s=s)
 
 
 def qgemm_debug_simple(A, indices, lut, bitwidth, group_size, q_layout: int = 0):
@@ -610,6 +619,22 @@ def embedding_gather(ids, indices, lut, N: int, K: int, bitwidth: int, group_siz
         _fail(f"{who}: ids must be an integer tensor, got dtype {ids.dtype}")
     if ids.device != lut.device:
         _fail(f"{who}: ids are on {ids.device}, the table on {lut.device}")
+    flat = ids.reshape(-1).long().contiguous()
+    if native is not None:
+        out, ok = native.embedding_rows(flat, indices, lut, int(N), int(K), int(bitwidth),
+                                        int(group_size), indices2, lut2, int(bitwidth2), resB, resA,
+                                        signs, int(rot_block), bool(check_ids))
+    else:
+        out, ok = _embedding_rows(flat, indices, lut, N, K, bitwidth, group_size, indices2, lut2,
+                                  bitwidth2, resB, resA, signs, rot_block, check_ids)
+    if not ok:
+        raise IdRangeError(f"{who}: ids must lie in [0, {int(N)})")
+    return out.reshape(*ids.shape, int(K))
+
+
+def _embedding_rows(flat, indices, lut, N, K, bitwidth, group_size, indices2, lut2, bitwidth2, resB,
+                    resA, signs, rot_block, check_ids):
+    who = "embedding_gather"
     A = torch.empty((1, int(K)), dtype=lut.dtype, device=lut.device)
     e8 = _empty_like_u8(A)
     e16 = torch.empty(0, dtype=A.dtype, device=A.device)
@@ -620,17 +645,14 @@ def embedding_gather(ids, indices, lut, N: int, K: int, bitwidth: int, group_siz
                             e16, group_size, signs, None, rot_block)
     if N2 != int(N):
         _fail(f"{who}: blob holds N={N2}, not {N}")
-    flat = ids.reshape(-1).long().contiguous()
     ok = ctypes.c_int(1)
     with _on_device_of(A):
         out = torch.empty((flat.numel(), int(K)), dtype=lut.dtype, device=lut.device)
         args = (ctypes.byref(w), flat.data_ptr(), flat.numel(), out.data_ptr(), _stream_of(A))
         check(lib.flute_embedding_checked(*args, ctypes.byref(ok)) if check_ids
               else lib.flute_embedding(*args))
-    if not ok.value:
-        raise IdRangeError(f"{who}: ids must lie in [0, {N2})")
     del keep
-    return out.reshape(*ids.shape, int(K))
+    return out, bool(ok.value)
 
 
 # ---------------------------------------------------------------------------
@@ -646,7 +668,7 @@ def embedding_gather(ids, indices, lut, N: int, K: int, bitwidth: int, group_siz
 
 NATIVE_NAMES = ("qgemm_gemv_stream", "qgemm_gemv_fht_stream", "qgemm_gemv_splitk_stream",
                 "qgemm_gemv_splitk_fht_stream", "qgemm_gemv_multi", "qgemm_gemv_mlp",
-                "qgemm_cutlass_streaming", "qgemm_dual_stream")
+                "qgemm_cutlass_streaming", "qgemm_dual_stream", "qgemm_linear")
 PYTHON_BINDING = {name: globals()[name] for name in NATIVE_NAMES}
 native = None
 

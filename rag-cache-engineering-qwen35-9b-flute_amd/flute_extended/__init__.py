@@ -47,6 +47,7 @@ from ._C import qgemm_gemv_multi as _qgemm_gemv_multi
 from ._C import qgemm_gemv_mlp as _qgemm_gemv_mlp
 from ._C import dequant_idxn
 from ._C import embedding_gather, IdRangeError
+from ._C import qgemm_linear
 from ._C import qgemm_gemv_kgroup, dequant_kgroup
 
 Backend = Literal["debug_simple", "cutlass_dense", "cutlass_streaming", "auto"]
@@ -274,6 +275,7 @@ def gemv_splitk_fht_available() -> bool:
     return True
 
 
+@functools.lru_cache(maxsize=4096)
 def _splitk_gate(bitwidth, bitwidth2, group_size, N, K, M, residual_rank, fht) -> bool:
     b1, b2 = int(bitwidth), int(bitwidth2) if bitwidth2 else 0
     if int(M) != 1 or (b1, b2) not in GEMV_SPLITK_PAIRS:

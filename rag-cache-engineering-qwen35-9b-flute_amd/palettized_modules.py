@@ -73,6 +73,9 @@ def _get_fht():
 
 def _flute():
     """The kernel package; importing it loads libflute_hip.so or raises."""
+    fx = sys.modules.get("flute_extended")
+    if fx is not None:
+        return fx
     if _HERE not in sys.path:
         sys.path.insert(0, _HERE)
     import flute_extended
@@ -198,7 +201,7 @@ class PalettizedLinear(nn.Module):
         return self.resA is not None and self.resB is not None
 
     def _on(self, key: str, t: torch.Tensor, device) -> torch.Tensor:
-        k = (key, str(device))
+        k = (key, device)
         if k not in self._dev_cache:
             self._dev_cache[k] = t.to(device)
         return self._dev_cache[k]
@@ -268,7 +271,7 @@ class PalettizedLinear(nn.Module):
     def _cast_on(self, key: str, t: torch.Tensor, device, dtype) -> torch.Tensor:
         """t on `device` in `dtype`, contiguous; converted once and kept (artifact readers
         hand over float16 residual factors whatever the activation dtype is)."""
-        k = (key, str(device), str(dtype), t.data_ptr())
+        k = (key, device, dtype, t.data_ptr())
         if k not in self._dev_cache:
             self._dev_cache[k] = t.detach().to(device=device, dtype=dtype).contiguous()
         return self._dev_cache[k]
@@ -301,33 +304,68 @@ class PalettizedLinear(nn.Module):
             return None
         if self.lut.dtype == torch.bfloat16 and x.dtype != torch.bfloat16:
             return None                     # the kernels refuse this pair: a routing decision here
-        kw, b2 = self._stream_kwargs()
-        rot = {}
-        if rotated_in_kernel:
-            if _env_on("FLUTE_NO_FHT_FUSE") or self._rotation_backend() != "auto":
-                return None
-            rot = dict(rot_signs=self._signs_on(x.device),
-                       awq_scale=self._awq_scale_on(x.device) if self._compensated() else None)
-        wide = self.N // 128 >= 160 and not _env_on("FLUTE_NO_WIDE_PREF") and \
-            fx.gemv_stream_supported(self.bitwidth, b2, self.group_size, self.N, self.K, 1)
+        b1, b2, gs, N, K = self.bitwidth, self._bits2(), self.group_size, self.N, self.K
+        if rotated_in_kernel and not self._rotates_in_kernel():
+            return None
+        rank = int(self.resB.shape[0]) if self.resB is not None else 0
+        wide = N // 128 >= 160 and not _env_on("FLUTE_NO_WIDE_PREF") and \
+            fx.gemv_stream_supported(b1, b2, gs, N, K, 1)
         gate = fx.gemv_splitk_fht_supported if rotated_in_kernel else fx.gemv_splitk_supported
-        if not wide and not _env_on("FLUTE_NO_SPLITK"):
+        if not wide and not _env_on("FLUTE_NO_SPLITK") and gate(b1, b2, gs, N, K, 1, rank):
             fused = self._fusable(x, fx.GEMV_SPLITK_MAX_RESIDUAL_RANK)
-            rank = int(self.resB.shape[0]) if self.has_residual() else 0
-            if fused is not None and gate(self.bitwidth, b2, self.group_size, self.N, self.K, 1,
-                                          rank):
+            if fused is not None:
                 _count("gemv_splitk_fht" if rotated_in_kernel else "gemv_splitk")
-                return fx.qgemm_gemv_splitk_stream(x, self.indices, self.lut, self.bitwidth,
-                                                   self.group_size, resB=fused[0], resA=fused[1],
-                                                   bias=fused[2], **kw, **rot)
+                return self._launch(fx, x, fused, b2, rotated_in_kernel)
         gate = fx.gemv_fht_stream_supported if rotated_in_kernel else fx.gemv_stream_supported
         fused = self._fusable(x, 16)
-        if fused is not None and gate(self.bitwidth, b2, self.group_size, self.N, self.K, 1):
+        if fused is not None and gate(b1, b2, gs, N, K, 1):
             _count("gemv_fht" if rotated_in_kernel else "gemv")
-            return fx.qgemm_gemv_stream(x, self.indices, self.lut, self.bitwidth,
-                                        self.group_size, resB=fused[0], resA=fused[1],
-                                        bias=fused[2], **kw, **rot)
+            return self._launch(fx, x, fused, b2, rotated_in_kernel)
         return None
+
+    def _bits2(self) -> int:
+        return self.bitwidth2 if self.has_stream2 else 0
+
+    def _rotates_in_kernel(self) -> bool:
+        return not _env_on("FLUTE_NO_FHT_FUSE") and self._rotation_backend() == "auto"
+
+    def _launch(self, fx, x, fused, b2: int, rotate: bool):
+        """The whole layer in one call of the library."""
+        def held(name):                       # (attribute lookup on a module is ten times a dictionary's)
+            t = self._buffers.get(name)
+            return getattr(self, name) if t is None else t
+        signs = self._signs_on(x.device) if rotate else None
+        awq = self._awq_scale_on(x.device) if rotate and self._compensated() else None
+        return fx.qgemm_linear(x, held("indices"), held("lut"), self.bitwidth,
+                               held("indices2") if b2 else None, held("lut2") if b2 else None, b2,
+                               fused[0], fused[1], fused[2], self.group_size, signs, awq)
+
+    def _gemm_route(self, x, rotated_in_kernel: bool):
+        """Several rows in one library call: rotation, both streams, residual and bias with one
+        rounding at the end (the chain below it rounds per stream and per added term; at
+        M = 48, 12288 -> 4096, (4, 1) bits, rank 16: 91.6 us for the chain).  None where
+        something else has to see the terms: autograd, other dtypes, ranks beyond the kernels'."""
+        fx = _flute()
+        if x.dtype not in (torch.float16, torch.bfloat16) or not x.is_contiguous():
+            return None
+        if self.lut.dtype == torch.bfloat16 and x.dtype != torch.bfloat16:
+            return None
+        bias = self.bias
+        if torch.is_grad_enabled() and (x.requires_grad or (bias is not None and bias.requires_grad)):
+            return None
+        if bias is not None and bias.dtype != x.dtype:
+            return None
+        if rotated_in_kernel and not (self._rotates_in_kernel() and fx._fht_k_ok(self.K)):
+            return None
+        b2 = self._bits2()
+        if not fx.dual_stream_supported(self.bitwidth, b2, self.group_size, self.N, self.K):
+            return None
+        fused = self._fusable(x, fx.GEMV_SPLITK_MAX_RESIDUAL_RANK)
+        if fused is None:
+            return None
+        small = x.shape[0] <= fx.DUAL_STREAM_MAX_M and (fused[0] is None or fused[0].shape[0] <= 16)
+        _count("dual_stream" if small else "per_group_lut")
+        return self._launch(fx, x, fused, b2, rotated_in_kernel)
 
     def _forward_kernel(self, x: torch.Tensor) -> torch.Tensor:
         fx = _flute()
@@ -340,6 +378,8 @@ class PalettizedLinear(nn.Module):
         out_dtype = x.dtype
         if self.rot_signs is not None:
             y = self._gemv_route(x, rotated_in_kernel=True)
+            if y is None and x.shape[0] > 1:
+                y = self._gemm_route(x, rotated_in_kernel=True)
             if y is not None:
                 return y
             x = self._rotate_input(x)
@@ -348,8 +388,10 @@ class PalettizedLinear(nn.Module):
             xk = xk.to(torch.bfloat16)
         xk = xk.contiguous()
         y = self._gemv_route(xk, rotated_in_kernel=False)
+        if y is None and xk.shape[0] > 1 and xk.dtype == out_dtype:
+            y = self._gemm_route(xk, rotated_in_kernel=False)
         if y is not None:
-            return y.to(out_dtype)
+            return y if y.dtype == out_dtype else y.to(out_dtype)
         kw, b2 = self._stream_kwargs()
         if xk.shape[0] <= fx.DUAL_STREAM_MAX_M and \
                 fx.dual_stream_supported(self.bitwidth, b2, self.group_size, self.N, self.K):
@@ -389,7 +431,7 @@ class PalettizedLinear(nn.Module):
                 y = y + self.bias
         else:
             y = self._forward_kernel(x)
-        return y.reshape(*shape[:-1], self.N)
+        return y if len(shape) == 2 else y.reshape(*shape[:-1], self.N)
 
 
 def _operand_problem(m, device) -> Optional[str]:
@@ -416,8 +458,12 @@ def _operand_ptrs(members) -> tuple:
     changes (a module moved to another device and back, a buffer replaced)."""
     out = []
     for m in members:
+        buffers, plain = (m._buffers, m.__dict__) if isinstance(m, nn.Module) else ({}, {})
         for name in ("indices", "lut", "indices2", "lut2", "resA", "resB", "bias"):
-            t = getattr(m, name, None)
+            # (a buffer's own dictionary first: attribute lookup on a module is ten times that)
+            t = buffers.get(name) if name not in plain else plain[name]
+            if t is None:
+                t = getattr(m, name, None)
             out.append(t.data_ptr() if torch.is_tensor(t) else 0)
     return tuple(out)
 

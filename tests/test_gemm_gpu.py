@@ -391,3 +391,23 @@ def test_gemm_many_rows_by_the_rule_agree_with_the_other_kernels(tuning_env, M, 
     y = _dual(w, x)
     tuning_env("FLUTE_GEMM_ROWS", "128")
     assert rel_l2(y.cpu(), _dual(w, x).cpu()) <= TOL
+
+
+@pytest.mark.parametrize("rank", [5, 8, 24])
+@pytest.mark.parametrize("M,K", [(2, 64), (17, 2048), (40, 8192), (33, 12288), (300, 4096)])
+@pytest.mark.parametrize("form", ["f16", "bf16 over f16", "bf16 over f16, rotated"])
+def test_gemm_residual_slices_and_row_scales(M, K, rank, form):
+    """Residual coefficients in one, four and sixteen slices of K; ranks the epilogue reads eight at
+    a time and others; row scales found by the rotation and by their own launch, rows over a wide
+    range of magnitudes."""
+    N, act = 256, torch.float16 if form == "f16" else torch.bfloat16
+    w = make_weight(N, K, 4, 128, seed=M + K + rank, bits2=1, rank=rank, act_dtype=act, device=DEV)
+    x = make_x(M, K, seed=M, dtype=act)
+    if act is torch.bfloat16:
+        x = x * torch.logspace(-6, 6, M).unsqueeze(1).to(act)
+    signs = O.rotation_signs(K, 3) if "rotated" in form else None
+    y = fx.qgemm_linear(x.to(DEV), w["blob_d"], w["lut_d"], 4, w["blob2_d"], w["lut2_d"], 1, w["resB_d"],
+                        w["resA_d"], None, 128, None if signs is None else signs.to(DEV), None).cpu()
+    ref = _exact(w, x if signs is None else O.fht_reference(x, signs))
+    scale = ref.abs().amax(dim=1, keepdim=True)
+    assert rel_l2(y.double() / scale, ref / scale) <= (TOL if act is torch.float16 else TOL_BF16)

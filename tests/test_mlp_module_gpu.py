@@ -328,3 +328,26 @@ def test_split_qkv_module(rot):
     assert torch.equal(y2.cpu(), y.cpu().reshape(1, -1))
     xs = make_x(5, K, seed=6)
     assert rel_l2(ker(xs.to(DEV)).cpu(), ref(xs)) <= 2e-3
+
+
+@pytest.mark.parametrize("rot", [False, True])
+def test_many_rows_in_one_call_and_autograd_beside_it(rot):
+    """More than sixteen rows of a two-stream layer with residual and bias are one library call whose
+    only rounding is the last (2^-11 relative at most, so TOL); where autograd wants the bias, or the
+    bias has another type, the terms are added one by one as before."""
+    N, K, M = 256, 512, 40
+    w = make_weight(N, K, seed=5, bits2=1, rank=8, bias=True)
+    kw = dict(rotation_seed=9, rotation_k=K) if rot else {}
+    ref, ker = _modules(w, **kw)
+    x = make_x(M, K, seed=6)
+    with torch.no_grad():
+        want = ref(x)
+        y = ker(x.to(DEV))
+    assert not y.requires_grad and rel_l2(y.cpu(), want) <= TOL
+    z = ker(x.to(DEV))                                  # gradients on: the bias is a parameter
+    assert z.requires_grad and rel_l2(z.detach().cpu(), want) <= 2e-3
+    z.float().sum().backward()
+    assert torch.equal(ker.bias.grad.cpu().float(), torch.full((N,), float(M)))
+    with torch.no_grad():
+        ker.bias = torch.nn.Parameter(ker.bias.detach().float())
+        assert ker(x.to(DEV)).dtype == torch.float32    # as torch adds a float32 bias
