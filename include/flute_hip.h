@@ -183,6 +183,19 @@ flute_status flute_gemm(const flute_linear *w, const void *A, void *C, int M,
                         int64_t lda, int64_t ldc, int act_dtype, void *stream);
 
 /*
+ * Several weights over the same rows: C[i] = A @ W[i]^T (+ residual, bias), 1...4 weights that
+ * share K and the LUT's type; ldc[i] elements between the rows of C[i].  What SplitQKV and the
+ * gate/up pair of FusedPalettizedMLP need for more than one token (upstream runs the modules one
+ * by one there, scripts/palettized_modules.py:1643-1908): one launch where that is faster.
+ */
+flute_status flute_gemm_multi(const flute_linear *ws, int count, const void *A, void *const *C,
+                              const int64_t *ldc, int M, int64_t lda, int act_dtype, void *stream);
+
+/* h = silu(g) * u over `count` 16-bit values (a multiple of 8), all 16-byte aligned; h may be g or u. */
+flute_status flute_silu_mul(const void *g, const void *u, void *h, int64_t count, int act_dtype,
+                            void *stream);
+
+/*
  * Scalar differential twin of the LUT GEMM:  C[M, N] = A[M, K] @ W^T for one stream, one
  * thread per output, every weight decoded from its bit position and looked up in the LUT
  * in global memory, fp32 sum in ascending k, one rounding.  Shares no code with

@@ -193,6 +193,7 @@ namespace {
 struct WidePlan {
     int rows;      // rows of A per workgroup: 512 or 256
     int ksplit;
+    double us;     // estimate of the chosen form
 };
 
 // The many-row kernel or the others, and its shape.  Each form's time is a line in what it has to
@@ -208,24 +209,29 @@ struct WidePlan {
 // streams (4, 1) at M = 1024, 4096 -> 12288: 263 / 165 / 190, at M = 192: 76 / - / 60 (two).
 // Calls that the 16- and 32-row workgroups serve in one round stay with them (M = 128,
 // 4096 -> 12288: 27 us there, 41 us here).
-WidePlan choose_wide(int M, int tiles, int G, int streams, bool four_bit, const GemmShape &other) {
-    {
-        const int v = tuning().gemm_rows;
-        if (v == 512 || v == 256) {
-            const int k = tuning().gemm_ksplit;
-            return {v, k > 1 ? (k < G ? k : G) : 1};
-        }
-        if (v) return {0, 1};
-    }
-    if (other.mb < 4) return {0, 1};
+// (several weights in one launch: `tiles` counts theirs, `other_us` is the sum of their other_forms)
+double other_forms(int M, int tiles, int G, int streams, bool four_bit, const GemmShape &other) {
     const int rows_other = other.mb * other.mw * 16;
     const int64_t units_other = (int64_t)tiles * ((M + rows_other - 1) / rows_other);
     int ks_other = 1;
     while (units_other * ks_other * 2 <= kNumCU && ks_other < 4 && G / (ks_other * 2) >= other.kw * 2) ks_other *= 2;
     const double per_tile = (other.mw == 1 ? 0.26 : 0.43) * (four_bit && streams == 1 ? 1.0 : 1.15);
-    double best = streams * (double)((units_other * ks_other + kNumCU - 1) / kNumCU) *
-                  (8.0 + per_tile * G / ks_other) + (ks_other > 1 ? 5.0 : 0.0);
-    WidePlan plan = {0, 1};
+    return streams * (double)((units_other * ks_other + kNumCU - 1) / kNumCU) * (8.0 + per_tile * G / ks_other) +
+           (ks_other > 1 ? 5.0 : 0.0);
+}
+
+WidePlan choose_wide(int M, int tiles, int G, int streams, double other_us, const GemmShape &other) {
+    {
+        const int v = tuning().gemm_rows;
+        if (v == 512 || v == 256) {
+            const int k = tuning().gemm_ksplit;
+            return {v, k > 1 ? (k < G ? k : G) : 1, 0.0};
+        }
+        if (v) return {0, 1, other_us};
+    }
+    if (other.mb < 4) return {0, 1, other_us};
+    double best = other_us;
+    WidePlan plan = {0, 1, other_us};
     for (int rows = 512; rows >= 256; rows /= 2) {
         const int64_t units = (int64_t)tiles * ((M + rows - 1) / rows);
         for (int ks = 1; ks <= 8 && G / ks >= 8; ks *= 2) {
@@ -236,7 +242,7 @@ WidePlan choose_wide(int M, int tiles, int G, int streams, bool four_bit, const 
                               (ks > 1 ? (rows == 512 ? 5.0 : 2.5) * ks : 0.0);
             if (us < best) {
                 best = us;
-                plan = {rows, ks};
+                plan = {rows, ks, us};
             }
         }
     }
@@ -403,7 +409,9 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
     hipStream_t stream = (hipStream_t)stream_;
 
     GemmShape shape = choose_gemm_shape(M, w->N / 128, w->q1_bytes + (w->b2 > 0 ? w->q2_bytes : 0));
-    const WidePlan wide = choose_wide(M, w->N / 128, w->K / 64, w->b2 > 0 ? 2 : 1, w->b1 == 4, shape);
+    const int streams = w->b2 > 0 ? 2 : 1;
+    const WidePlan wide = choose_wide(M, w->N / 128, w->K / 64, streams,
+                                      other_forms(M, w->N / 128, w->K / 64, streams, w->b1 == 4, shape), shape);
     if (wide.rows) return gemm_wide(w, 1, A, &C, &ldc, M, lda, act_dtype, wide, stream);
     GemmParams p = {};
     p.nstreams = w->b2 > 0 ? 2 : 1;
@@ -577,6 +585,95 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
         if (st != FLUTE_OK) return st;
     }
     workspace_done(stream);
+    return FLUTE_OK;
+}
+
+extern "C" flute_status flute_gemm_multi(const flute_linear *ws, int count, const void *A, void *const *C,
+                                         const int64_t *ldc, int M, int64_t lda, int act_dtype, void *stream) {
+    FLUTE_REQUIRE(ws && C && ldc && count >= 1 && count <= kWideMaxSegs, FLUTE_ERR_INVALID,
+                  "flute_gemm_multi: 1..%d weights", kWideMaxSegs);
+    for (int i = 0; i < count; ++i) {
+        flute_status st = validate_linear(&ws[i], 1, "flute_gemm_multi");
+        if (st != FLUTE_OK) return st;
+        FLUTE_REQUIRE(ws[i].K == ws[0].K && ws[i].lut_dtype == ws[0].lut_dtype, FLUTE_ERR_INVALID,
+                      "flute_gemm_multi: the weights must share K and the LUT's type");
+        FLUTE_REQUIRE(M <= 0 || (C[i] && ((uintptr_t)C[i] & 1) == 0 && ldc[i] >= ws[i].N), FLUTE_ERR_INVALID,
+                      "flute_gemm_multi: output %d must be 2-byte aligned rows of N or more", i);
+    }
+    FLUTE_REQUIRE(act_dtype == FLUTE_F16 || act_dtype == FLUTE_BF16, FLUTE_ERR_INVALID,
+                  "flute_gemm_multi: activations must be float16 or bfloat16");
+    FLUTE_REQUIRE(M >= 0 && (M == 0 || (A && ((uintptr_t)A & 1) == 0 && lda >= ws[0].K)), FLUTE_ERR_INVALID,
+                  "flute_gemm_multi: A must be 2-byte aligned rows of K or more");
+    if (M == 0) return FLUTE_OK;
+    // One launch of the many-row kernel where the weights together are better off there than each
+    // in its own best form: they share the activations' image, and a chip that one weight's tiles
+    // leave partly idle (or cut into slices of K) is filled.  Gate and up, 2 x 4096 -> 12288, M = 509:
+    // 2 x 65.8 us in two slices each, 98.7 together.
+    const int streams = ws[0].b2 > 0 ? 2 : 1;
+    bool alike = count > 1, big = true;
+    int tiles = 0;
+    double other_us = 0.0;
+    GemmShape shape = {4, 4, 2, 1};
+    for (int i = 0; i < count; ++i) {
+        const flute_linear &w = ws[i];
+        alike &= w.b1 == ws[0].b1 && w.b2 == ws[0].b2;
+        tiles += w.N / 128;
+        shape = choose_gemm_shape(M, w.N / 128, w.q1_bytes + (w.b2 > 0 ? w.q2_bytes : 0));
+        big &= shape.mb == 4;
+        const WidePlan own = choose_wide(M, w.N / 128, w.K / 64, streams,
+                                         other_forms(M, w.N / 128, w.K / 64, streams, w.b1 == 4, shape), shape);
+        other_us += own.us;
+    }
+    if (alike && big) {
+        const WidePlan plan = choose_wide(M, tiles, ws[0].K / 64, streams, other_us, shape);
+        if (plan.rows) return gemm_wide(ws, count, A, C, ldc, M, lda, act_dtype, plan, (hipStream_t)stream);
+    }
+    for (int i = 0; i < count; ++i) {
+        flute_status st = flute_gemm(&ws[i], A, C[i], M, lda, ldc[i], act_dtype, stream);
+        if (st != FLUTE_OK) return st;
+    }
+    return FLUTE_OK;
+}
+
+namespace flute {
+namespace {
+
+// h = silu(g) * u, eight values a thread, fp32 inside, one rounding.  Bound by its three streams.
+__global__ void __launch_bounds__(256) silu_mul_kernel(const uint16_t *g, const uint16_t *u, uint16_t *h, int64_t pieces,
+                                                       int bf16) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < pieces; i += (int64_t)gridDim.x * 256) {
+        const u4_t a = *(const u4_t *)(g + i * 8), b = *(const u4_t *)(u + i * 8);
+        u4_t o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint32_t r = 0;
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const uint16_t x = (uint16_t)(a[e] >> (16 * s)), y = (uint16_t)(b[e] >> (16 * s));
+                const float f = bf16 ? bf2f(x) : h2f(x);
+                const float t = f / (1.0f + expf(-f)) * (bf16 ? bf2f(y) : h2f(y));
+                r |= (uint32_t)round_act(t, bf16) << (16 * s);
+            }
+            o[e] = r;
+        }
+        *(u4_t *)(h + i * 8) = o;
+    }
+}
+
+}  // namespace
+}  // namespace flute
+
+extern "C" flute_status flute_silu_mul(const void *g, const void *u, void *h, int64_t count, int act_dtype, void *stream) {
+    FLUTE_REQUIRE(act_dtype == FLUTE_F16 || act_dtype == FLUTE_BF16, FLUTE_ERR_INVALID,
+                  "flute_silu_mul: float16 or bfloat16");
+    FLUTE_REQUIRE(count >= 0 && count % 8 == 0, FLUTE_ERR_INVALID, "flute_silu_mul: count must be a multiple of 8");
+    if (count == 0) return FLUTE_OK;
+    FLUTE_REQUIRE(g && u && h && (((uintptr_t)g | (uintptr_t)u | (uintptr_t)h) & 15) == 0, FLUTE_ERR_INVALID,
+                  "flute_silu_mul: g, u and h must be 16-byte aligned");
+    const int64_t blocks = (count / 8 + 255) / 256;
+    hipLaunchKernelGGL(silu_mul_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, (hipStream_t)stream,
+                       (const uint16_t *)g, (const uint16_t *)u, (uint16_t *)h, count / 8, (int)(act_dtype == FLUTE_BF16));
+    FLUTE_HIP_CHECK(hipGetLastError());
     return FLUTE_OK;
 }
 

@@ -7,7 +7,7 @@
 //   qgemm_gemv_splitk_fht_stream            (src/bindings.cpp:277-354)
 //   qgemm_gemv_multi, qgemm_gemv_mlp        (src/bindings.cpp:368-384)
 //   qgemm_cutlass_streaming, qgemm_dual_stream   (src/bindings.cpp:245-270)
-//   qgemm_linear, embedding_rows            (what a module's forward calls; no upstream counterpart)
+//   qgemm_linear, qgemm_linear_multi, embedding_rows   (what a module's forward calls; no upstream counterpart)
 //
 // Same positional signatures, same conventions (empty tensor = absent operand, N from the
 // blob's byte count, RuntimeError on every contract violation, fresh outputs, launches on the
@@ -376,6 +376,58 @@ Tensor qgemm_linear(const Tensor &A, const Tensor &indices, const Tensor &lut, i
                 held(bias), gs, signs, awq);
 }
 
+// Several layers on the same rows, each (indices, lut, b1, indices2, lut2, b2, resB, resA, bias, gs,
+// signs, s) with None for what it has not: their outputs side by side, or silu(first) * second.
+// Layers of one rotation (the same signs and s) share the rotated rows.
+Tensor qgemm_linear_multi(const Tensor &A_in, const std::vector<pybind11::tuple> &layers, bool silu_mul) {
+    const char *who = "qgemm_linear_multi";
+    const Shape2 s = check_2d_input(who, A_in, false);
+    TORCH_CHECK(!layers.empty() && layers.size() <= 4 && (!silu_mul || layers.size() == 2), who,
+                ": 1..4 layers, two for silu_mul");
+    const auto opt = [](const pybind11::handle &h) {
+        return h.is_none() ? c10::optional<Tensor>() : c10::optional<Tensor>(h.cast<Tensor>());
+    };
+    const auto held = [&](const pybind11::handle &h) { return h.is_none() ? Tensor() : h.cast<Tensor>(); };
+    Tensor A = aligned16(A_in);
+    c10::DeviceGuard guard(A.device());
+    std::vector<Described> d;
+    std::vector<flute_linear> ws;
+    int64_t total = 0;
+    for (const pybind11::tuple &l : layers) {
+        TORCH_CHECK(l.size() == 12, who, ": a layer has 12 operands");
+        d.push_back(describe(who, A, s.K, l[0].cast<Tensor>(), l[1].cast<Tensor>(), l[2].cast<int64_t>(), held(l[3]),
+                             held(l[4]), l[5].cast<int64_t>(), held(l[6]), held(l[7]), held(l[8]), l[9].cast<int64_t>(),
+                             opt(l[10]), opt(l[11]), 0, kGsAll, 256));
+        ws.push_back(d.back().w);
+        total += d.back().N;
+    }
+    bool shared = ws[0].signs != nullptr;
+    for (const flute_linear &w : ws) shared &= w.signs == ws[0].signs && w.awq == ws[0].awq;
+    if (shared) {
+        Tensor rotated = torch::empty_like(A);
+        check_status(flute_fht(A.data_ptr(), ws[0].signs, ws[0].awq, rotated.data_ptr(), (int)s.M, (int)s.K, act_code(A), 0,
+                               0, stream_of(A)));
+        A = rotated;
+        for (flute_linear &w : ws) w.signs = w.awq = nullptr;
+    }
+    TORCH_CHECK(!silu_mul || d[0].N == d[1].N, who, ": gate and up must agree in N");
+    const Tensor out = silu_mul ? torch::empty({2, s.M, d[0].N}, A.options()) : torch::empty({s.M, total}, A.options());
+    std::vector<void *> C;
+    std::vector<int64_t> ldc;
+    char *at = (char *)out.data_ptr();
+    for (const Described &one : d) {
+        C.push_back(at);
+        at += 2 * one.N * (silu_mul ? s.M : 1);
+        ldc.push_back(silu_mul ? one.N : total);
+    }
+    check_status(flute_gemm_multi(ws.data(), (int)ws.size(), A.data_ptr(), C.data(), ldc.data(), (int)s.M, s.K, act_code(A),
+                                  stream_of(A)));
+    if (!silu_mul) return out;
+    const Tensor h = torch::empty({s.M, d[0].N}, A.options());
+    check_status(flute_silu_mul(C[0], C[1], h.data_ptr(), s.M * d[0].N, act_code(A), stream_of(A)));
+    return h;
+}
+
 // Rows `ids` (int64, contiguous, flat) of a table, and whether every id lay in it (true where
 // nobody asked).
 std::pair<Tensor, bool> embedding_rows(const Tensor &ids, const Tensor &indices, const Tensor &lut, int64_t N,
@@ -425,6 +477,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("rot_block") = 0);
     m.def("qgemm_linear", &qgemm_linear);
     m.def("embedding_rows", &embedding_rows);
+    m.def("qgemm_linear_multi", &qgemm_linear_multi);
     m.def("qgemm_gemv_multi", &qgemm_gemv_multi, py::arg("A"), py::arg("seg_table"),
           py::arg("lut_dtype") = py::none(), py::arg("split") = 0);
     m.def("qgemm_gemv_mlp", &qgemm_gemv_mlp, py::arg("A"), py::arg("seg_table"), py::arg("C"),

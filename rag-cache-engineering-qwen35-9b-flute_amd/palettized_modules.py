@@ -331,14 +331,18 @@ class PalettizedLinear(nn.Module):
 
     def _launch(self, fx, x, fused, b2: int, rotate: bool):
         """The whole layer in one call of the library."""
+        return fx.qgemm_linear(x, *self._layer(x, fused, b2, rotate))
+
+    def _layer(self, x, fused, b2: int, rotate: bool):
+        """The operands of qgemm_linear behind x."""
         def held(name):                       # (attribute lookup on a module is ten times a dictionary's)
             t = self._buffers.get(name)
             return getattr(self, name) if t is None else t
         signs = self._signs_on(x.device) if rotate else None
         awq = self._awq_scale_on(x.device) if rotate and self._compensated() else None
-        return fx.qgemm_linear(x, held("indices"), held("lut"), self.bitwidth,
-                               held("indices2") if b2 else None, held("lut2") if b2 else None, b2,
-                               fused[0], fused[1], fused[2], self.group_size, signs, awq)
+        return (held("indices"), held("lut"), self.bitwidth, held("indices2") if b2 else None,
+                held("lut2") if b2 else None, b2, fused[0], fused[1], fused[2], self.group_size,
+                signs, awq)
 
     def _gemm_route(self, x, rotated_in_kernel: bool):
         """Several rows in one library call: rotation, both streams, residual and bias with one
@@ -346,6 +350,14 @@ class PalettizedLinear(nn.Module):
         M = 48, 12288 -> 4096, (4, 1) bits, rank 16: 91.6 us for the chain).  None where
         something else has to see the terms: autograd, other dtypes, ranks beyond the kernels'."""
         fx = _flute()
+        fused = self._gemm_operands(fx, x, rotated_in_kernel)
+        if fused is None:
+            return None
+        small = x.shape[0] <= fx.DUAL_STREAM_MAX_M and (fused[0] is None or fused[0].shape[0] <= 16)
+        _count("dual_stream" if small else "per_group_lut")
+        return self._launch(fx, x, fused, self._bits2(), rotated_in_kernel)
+
+    def _gemm_operands(self, fx, x, rotated_in_kernel: bool):
         if x.dtype not in (torch.float16, torch.bfloat16) or not x.is_contiguous():
             return None
         if self.lut.dtype == torch.bfloat16 and x.dtype != torch.bfloat16:
@@ -360,12 +372,7 @@ class PalettizedLinear(nn.Module):
         b2 = self._bits2()
         if not fx.dual_stream_supported(self.bitwidth, b2, self.group_size, self.N, self.K):
             return None
-        fused = self._fusable(x, fx.GEMV_SPLITK_MAX_RESIDUAL_RANK)
-        if fused is None:
-            return None
-        small = x.shape[0] <= fx.DUAL_STREAM_MAX_M and (fused[0] is None or fused[0].shape[0] <= 16)
-        _count("dual_stream" if small else "per_group_lut")
-        return self._launch(fx, x, fused, b2, rotated_in_kernel)
+        return self._fusable(x, fx.GEMV_SPLITK_MAX_RESIDUAL_RANK)
 
     def _forward_kernel(self, x: torch.Tensor) -> torch.Tensor:
         fx = _flute()
@@ -468,6 +475,55 @@ def _operand_ptrs(members) -> tuple:
     return tuple(out)
 
 
+def _same_rotation(a, b) -> bool:
+    """Whether two members rotate their input alike (the same signs, no scale)."""
+    if a.rot_signs is None or b.rot_signs is None:
+        return a.rot_signs is b.rot_signs
+    if a._compensated() or b._compensated():
+        return False
+    return a.rot_signs is b.rot_signs or (
+        not a.rot_signs.is_cuda and not b.rot_signs.is_cuda and torch.equal(a.rot_signs, b.rot_signs))
+
+
+def _observed(m) -> bool:
+    """Whether somebody watches this module's call: it has to be made then."""
+    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+
+
+def _rows_together(members, x, silu_mul: bool):
+    """Several layers on the same rows in one call of the library, or None where they have to run
+    one by one (subclasses, hooks, other types, autograd, the reference path).  Gate and up of
+    4096 -> 12288 at M = 509: 2 x 65.8 us of GEMM, their activations prepared twice, and two
+    elementwise passes without it."""
+    if _env_on("FLUTE_NO_MERGE") or not x.is_cuda or nn.modules.module._has_any_global_hook():
+        return None
+    if any(type(m) is not PalettizedLinear or m.reference or _observed(m) for m in members):
+        return None
+    if silu_mul and members[0].N != members[1].N:
+        return None
+    fx = _flute()
+    first = members[0]
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
+    if fx._C.native is None or x2.shape[0] < 2 or x2.shape[1] != first.K or \
+            any(m.K != first.K or m.lut.dtype != first.lut.dtype or
+                (isinstance(m.lut, nn.Parameter) and m.lut.requires_grad) for m in members) or \
+            first.lut.dtype not in (torch.float16, torch.bfloat16):
+        return None
+    layers, signs = [], None
+    for m in members:
+        rotate = m.rot_signs is not None
+        fused = m._gemm_operands(fx, x2, rotate)
+        if fused is None:
+            return None
+        layer = m._layer(x2, fused, m._bits2(), rotate)
+        if m is not first and rotate and _same_rotation(first, m):
+            layer = (*layer[:10], layers[0][10], layers[0][11])
+        layers.append(layer)
+    y = fx._C.native.qgemm_linear_multi(x2, layers, silu_mul)
+    _count("gemm_multi")
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], y.shape[-1])
+
+
 class FusedPalettizedMLP(nn.Module):
     """down(act(gate(x)) * up(x)) with the decode shape (one token) collapsed
     into one merged gate+up+SiLU*mul launch followed by the down GEMV
@@ -484,6 +540,10 @@ class FusedPalettizedMLP(nn.Module):
         if h is not None:
             out = self.down_proj(h)
             return out.view(*x.shape[:-1], out.shape[-1]) if x.dim() == 3 else out
+        if act_name(self.act_fn) in ("silu", "swish") and not (isinstance(self.act_fn, nn.Module) and _observed(self.act_fn)):
+            h = _rows_together((self.gate_proj, self.up_proj), x, True)
+            if h is not None:
+                return self.down_proj(h)
         return self.down_proj(self.act_fn(self.gate_proj(x)) * self.up_proj(x))
 
     def _fused_gate_up(self, x):
@@ -549,7 +609,8 @@ class FusedPalettizedMLP(nn.Module):
             if m.rot_signs is not None:
                 if m._rotation_backend() != "auto":
                     return refuse("pinned rotation backend")
-                signs = m._signs_on(device).contiguous()
+                # one rotation, one address: the launch stages the input once for both
+                signs = (g if _same_rotation(g, m) else m)._signs_on(device).contiguous()
                 awq = m._awq_scale_on(device) if m._compensated() else None
             b2 = m.bitwidth2 if m.has_stream2 else 0
             ptr = lambda t: 0 if t is None else t.data_ptr()
@@ -584,6 +645,9 @@ class SplitQKV(nn.Module):
 
     def forward(self, x):
         y = self._gemv_multi_decode(x)
+        if y is not None:
+            return y
+        y = _rows_together((self.q_proj, self.k_proj, self.v_proj), x, False)
         if y is not None:
             return y
         return torch.cat([self.q_proj(x), self.k_proj(x), self.v_proj(x)], dim=-1)
@@ -652,7 +716,8 @@ class SplitQKV(nn.Module):
             if m.rot_signs is not None:
                 if m._rotation_backend() != "auto":
                     return refuse("pinned rotation backend")
-                signs = m._signs_on(device).contiguous()
+                # one rotation, one address: its members share the rotated input
+                signs = (members[0] if _same_rotation(members[0], m) else m)._signs_on(device).contiguous()
                 awq = m._awq_scale_on(device) if m._compensated() else None
             b2 = m.bitwidth2 if m.has_stream2 else 0
             ptr = lambda t: 0 if t is None else t.data_ptr()

@@ -351,3 +351,38 @@ def test_many_rows_in_one_call_and_autograd_beside_it(rot):
     with torch.no_grad():
         ker.bias = torch.nn.Parameter(ker.bias.detach().float())
         assert ker(x.to(DEV)).dtype == torch.float32    # as torch adds a float32 bias
+
+
+@pytest.mark.parametrize("M", [2, 17, 200, 600])
+@pytest.mark.parametrize("spec,act,rot", [
+    (dict(), torch.float16, False), (dict(bits2=1, rank=8), torch.bfloat16, True),
+    (dict(bits=3, gs=64, rank=5, bias=True), torch.float16, True), (dict(lut_dtype=torch.bfloat16), torch.bfloat16, False)])
+def test_layers_on_the_same_rows_in_one_call(monkeypatch, M, spec, act, rot):
+    """q/k/v side by side and silu(gate) * up for more than one token: launches of one weight and of
+    several, whole and ragged row blocks, shared rotated rows, against the members one by one, which
+    round once per output (and the product three times): two roundings of the type apart."""
+    K, rounding = 1024, 2 ** -11 if act is torch.float16 else 2 ** -8
+    kw = dict(rotation_seed=9, rotation_k=K) if rot else {}
+    layers = [_modules(make_weight(n, K, seed=i, act_dtype=act, **spec), **kw)[1] for i, n in
+              enumerate((1024, 256, 256, 1024))]
+    x = make_x(M, K, seed=6, dtype=act).to(DEV)
+    qkv = pm.SplitQKV(*layers[:3])
+    mlp = pm.FusedPalettizedMLP(layers[0], layers[3], torch.nn.Identity(), torch.nn.SiLU())
+    with torch.no_grad():
+        for block, n in ((qkv, 1536), (mlp, 1024)):
+            pm.ROUTE_CENSUS.clear()
+            y = block(x.view(1, M, K))
+            assert y.shape == (1, M, n) and y.dtype == act and list(pm.ROUTE_CENSUS) == ["gemm_multi"]
+            monkeypatch.setenv("FLUTE_NO_MERGE", "1")
+            want = block(x)
+            monkeypatch.delenv("FLUTE_NO_MERGE")
+            assert rel_l2(y.cpu().view(M, n), want.cpu()) <= 2 * rounding
+        # somebody who watches a member's call sees it
+        seen = []
+        handle = layers[0].register_forward_hook(lambda *a: seen.append(1))
+        pm.ROUTE_CENSUS.clear()
+        qkv(x), mlp(x)
+        handle.remove()
+        assert len(seen) == 2 and "gemm_multi" not in pm.ROUTE_CENSUS
+    if spec.get("bias") and M > 16:                     # (the small-M entry never tracked the bias)
+        assert qkv(x).requires_grad and mlp(x).requires_grad
