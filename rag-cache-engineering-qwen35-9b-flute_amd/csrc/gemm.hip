@@ -1,8 +1,9 @@
 // Host side of the small-M / prefill LUT GEMM: shape policy, workspace layout,
 // pre-passes (activation permutation, residual coefficients) and the launch.
+#include <limits.h>
 #include <stdlib.h>
 
-#include "gemm_kernel.h"
+#include "gemm_launch.h"
 #include "gemm_wide_kernel.h"
 #include "host_common.h"
 
@@ -11,6 +12,7 @@
 
 namespace flute {
 
+flute_status gemm_launch_segs(int bf16, int mb, int mw, const GemmParams &p, dim3 grid, int lds, hipStream_t stream);
 flute_status gemm_wide_f16(int mb, int b1, int b2, int slices, const WideParams &p, hipStream_t stream);
 flute_status gemm_wide_bf16(int mb, int b1, int b2, int slices, const WideParams &p, hipStream_t stream);
 
@@ -52,88 +54,48 @@ GemmShape choose_gemm_shape(int M, int tiles, int64_t index_bytes) {
     return {4, 4, 2, 1};
 }
 
-template <int MB, int KW, int MW, bool BF16, int B1, bool PERM = false, bool DIRECT = false,
-          bool LEAN = false>
-flute_status launch_gemm(const GemmParams &p, dim3 grid, int lds, hipStream_t stream) {
-    static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
-    if (!attr_done) {
-        FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)gemm_kernel<MB, KW, MW, BF16, B1, PERM, DIRECT, LEAN>,
-                                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                                            (int)kLdsPerCU));
-        attr_done = true;
+// The residual coefficients of a call's weights, xb[i][m, r] = sum_k A[m, k] * resB[i][r, k] in fp32:
+// 16-row by 16-rank blocks in as many slices of K as the chip has CUs for, 512 columns (one step of a
+// workgroup) or more each.
+struct CoeffPlan {
+    int rows, ranks, slices;                            // blocks
+    size_t floats() const { return slices > 1 ? (size_t)slices * rows * ranks * 256 : 0; }
+    size_t tickets() const { return (size_t)rows * ranks; }
+};
+CoeffPlan plan_coeff(const flute_linear *ws, int count, int M) {
+    CoeffPlan c = {(M + 15) / 16, 0, 1};
+    for (int i = 0; i < count; ++i) c.ranks += (ws[i].R + 15) / 16;
+    while (c.slices < 16 && (int64_t)c.rows * c.ranks * c.slices * 2 <= kNumCU && ws[0].K / (c.slices * 2) >= 512)
+        c.slices *= 2;
+    if (c.slices < 4) c.slices = 1;                     // (partial sums are read in fours)
+    return c;
+}
+
+flute_status launch_coeff(const CoeffPlan &plan, const flute_linear *ws, int count, const void *A, int64_t lda,
+                          float *const *xb, int M, int is_bf16, float *part, int *tickets, hipStream_t stream) {
+    CoeffParams p = {};
+    p.A = (const uint16_t *)A;
+    p.lda = lda;
+    p.M = M;
+    p.K = ws[0].K;
+    p.aligned = ((uintptr_t)A & 15) == 0 && lda % 8 == 0;
+    p.kper = (p.K / 32 + plan.slices - 1) / plan.slices * 32;
+    p.part = part;
+    p.tickets = tickets;
+    int n = 0, ranks = 0;
+    for (int i = 0; i < count; ++i) {
+        if (ws[i].R == 0) continue;
+        p.resB[n] = (const uint16_t *)ws[i].resB;
+        p.xb[n] = xb[i];
+        p.R[n] = ws[i].R;
+        p.rank0[n++] = ranks;
+        p.aligned &= ((uintptr_t)ws[i].resB & 15) == 0;
+        ranks += (ws[i].R + 15) / 16;
     }
-    hipLaunchKernelGGL((gemm_kernel<MB, KW, MW, BF16, B1, PERM, DIRECT, LEAN>), grid, dim3(64 * KW * MW), lds,
-                       stream, p);
-    FLUTE_HIP_CHECK(hipGetLastError());
-    return FLUTE_OK;
-}
-
-template <int MB, int KW, int MW, bool BF16>
-flute_status launch_gemm_bits(const GemmParams &p, dim3 grid, int lds, hipStream_t stream) {
-    if (p.nstreams == 1) {
-        switch (p.bits[0]) {
-            case 4:
-                if constexpr (MB == 1) {
-                    if (p.rep_log2[0] == 6 && p.A8)
-                        return launch_gemm<MB, KW, MW, BF16, 4, true, true>(p, grid, lds, stream);
-                }
-                if constexpr (MB == 4) {
-                    if (p.rep_log2[0] == 6 && p.lean)
-                        return launch_gemm<MB, KW, MW, BF16, 4, true, false, true>(p, grid, lds, stream);
-                }
-                if (p.rep_log2[0] == 6) return launch_gemm<MB, KW, MW, BF16, 4, true>(p, grid, lds, stream);
-                return launch_gemm<MB, KW, MW, BF16, 4>(p, grid, lds, stream);
-            case 3: return launch_gemm<MB, KW, MW, BF16, 3>(p, grid, lds, stream);
-            case 2: return launch_gemm<MB, KW, MW, BF16, 2>(p, grid, lds, stream);
-            default: return launch_gemm<MB, KW, MW, BF16, 1>(p, grid, lds, stream);
-        }
-    }
-    if constexpr (MB == 1) {
-        return launch_gemm<MB, KW, MW, BF16, 0>(p, grid, lds, stream);
-    } else {
-        set_error("flute_gemm: two streams at this size run as one launch per stream");
-        return FLUTE_ERR_UNSUPPORTED;
-    }
-}
-
-template <bool BF16>
-flute_status launch_gemm_shape(const GemmShape &s, const GemmParams &p, dim3 grid, int lds,
-                               hipStream_t stream) {
-    if (s.mb == 1) return launch_gemm_bits<1, 8, 1, BF16>(p, grid, lds, stream);
-    if (s.mb == 2) return launch_gemm_bits<2, 8, 1, BF16>(p, grid, lds, stream);
-    if (s.mw == 1) return launch_gemm_bits<4, 8, 1, BF16>(p, grid, lds, stream);
-    return launch_gemm_bits<4, 4, 2, BF16>(p, grid, lds, stream);
-}
-
-
-// Slices of K a coefficient launch takes: as many blocks as the chip has CUs, 512 columns (one
-// step of a workgroup) or more each.
-int coeff_slices(int M, int K, int R) {
-    const int64_t blocks = (int64_t)((M + 15) / 16) * ((R + 15) / 16);
-    int s = 1;
-    while (s < 16 && blocks * s * 2 <= kNumCU && K / (s * 2) >= 512) s *= 2;
-    return s >= 4 ? s : 1;
-}
-// What that takes of the workspace: floats of partial sums, tickets.
-size_t coeff_floats(int M, int K, int R) {
-    const int s = R > 0 ? coeff_slices(M, K, R) : 1;
-    return s > 1 ? (size_t)s * ((M + 15) / 16) * ((R + 15) / 16) * 256 : 0;
-}
-size_t coeff_tickets(int M, int R) { return (size_t)((M + 15) / 16) * ((R + 15) / 16); }
-
-// xb[m, r] = sum_k A[m, k] * resB[r, k] in fp32.
-flute_status launch_coeff(const void *A, int64_t lda, const void *resB, float *xb, int M, int K, int R, int is_bf16,
-                          float *part, int *tickets, hipStream_t stream) {
-    const int slices = coeff_slices(M, K, R);
-    const int kper = (K / 32 + slices - 1) / slices * 32;
-    const dim3 grid((M + 15) / 16, (R + 15) / 16, slices);
-    const int aligned = ((uintptr_t)A & 15) == 0 && lda % 8 == 0 && ((uintptr_t)resB & 15) == 0;
-    if (is_bf16)
-        hipLaunchKernelGGL(gemm_coeff_kernel<true>, grid, dim3(1024), 0, stream, (const uint16_t *)A, lda,
-                           (const uint16_t *)resB, xb, M, K, R, aligned, kper, part, tickets);
-    else
-        hipLaunchKernelGGL(gemm_coeff_kernel<false>, grid, dim3(1024), 0, stream, (const uint16_t *)A, lda,
-                           (const uint16_t *)resB, xb, M, K, R, aligned, kper, part, tickets);
+    for (; n < kGemmMaxSegs; ++n) p.rank0[n] = INT_MAX;
+    const dim3 grid(plan.rows, plan.ranks, plan.slices);
+    if (is_bf16) hipLaunchKernelGGL(gemm_coeff_kernel<true>, grid, dim3(1024), 0, stream, p);
+    else hipLaunchKernelGGL(gemm_coeff_kernel<false>, grid, dim3(1024), 0, stream, p);
     FLUTE_HIP_CHECK(hipGetLastError());
     return FLUTE_OK;
 }
@@ -145,7 +107,7 @@ flute_status launch_coeff(const void *A, int64_t lda, const void *resB, float *x
 // layout the one-instruction address needs).  Everything else: as much replication as
 // the budget allows, 32 lanes at most.
 int plan_lds(GemmParams &p, const GemmShape &shape) {
-    const int ngrp = p.gs >= 128 ? 1 : 128 / p.gs;
+    const int ngrp = p.seg[0].gs >= 128 ? 1 : 128 / p.seg[0].gs;
     const bool perm = p.nstreams == 1 && p.bits[0] == 4 && ngrp <= 2 &&
                       !tuning().gemm_no_perm;
     const int table_budget = (shape.mb == 1 ? 64 : 96) * 1024 / p.nstreams;
@@ -193,7 +155,6 @@ namespace {
 struct WidePlan {
     int rows;      // rows of A per workgroup: 512 or 256
     int ksplit;
-    double us;     // estimate of the chosen form
 };
 
 // The many-row kernel or the others, and its shape.  Each form's time is a line in what it has to
@@ -209,7 +170,7 @@ struct WidePlan {
 // streams (4, 1) at M = 1024, 4096 -> 12288: 263 / 165 / 190, at M = 192: 76 / - / 60 (two).
 // Calls that the 16- and 32-row workgroups serve in one round stay with them (M = 128,
 // 4096 -> 12288: 27 us there, 41 us here).
-// (several weights in one launch: `tiles` counts theirs, `other_us` is the sum of their other_forms)
+// (several weights in one launch: `tiles` counts theirs; `other_us` is other_forms' estimate)
 double other_forms(int M, int tiles, int G, int streams, bool four_bit, const GemmShape &other) {
     const int rows_other = other.mb * other.mw * 16;
     const int64_t units_other = (int64_t)tiles * ((M + rows_other - 1) / rows_other);
@@ -225,13 +186,13 @@ WidePlan choose_wide(int M, int tiles, int G, int streams, double other_us, cons
         const int v = tuning().gemm_rows;
         if (v == 512 || v == 256) {
             const int k = tuning().gemm_ksplit;
-            return {v, k > 1 ? (k < G ? k : G) : 1, 0.0};
+            return {v, k > 1 ? (k < G ? k : G) : 1};
         }
-        if (v) return {0, 1, other_us};
+        if (v) return {0, 1};
     }
-    if (other.mb < 4) return {0, 1, other_us};
+    if (other.mb < 4) return {0, 1};
     double best = other_us;
-    WidePlan plan = {0, 1, other_us};
+    WidePlan plan = {0, 1};
     for (int rows = 512; rows >= 256; rows /= 2) {
         const int64_t units = (int64_t)tiles * ((M + rows - 1) / rows);
         for (int ks = 1; ks <= 8 && G / ks >= 8; ks *= 2) {
@@ -242,7 +203,7 @@ WidePlan choose_wide(int M, int tiles, int G, int streams, double other_us, cons
                               (ks > 1 ? (rows == 512 ? 5.0 : 2.5) * ks : 0.0);
             if (us < best) {
                 best = us;
-                plan = {rows, ks, us};
+                plan = {rows, ks};
             }
         }
     }
@@ -278,8 +239,9 @@ flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *c
     int tiles = 0;
     for (int i = 0; i < count; ++i) {
         xb_floats += up4((size_t)M * ws[i].R);
-        part_xb = std::max(part_xb, coeff_floats(M, K, ws[i].R));
-        want_tickets = std::max(want_tickets, coeff_tickets(M, ws[i].R));
+        const CoeffPlan c = plan_coeff(ws + i, 1, M);
+        part_xb = std::max(part_xb, c.floats());
+        want_tickets = std::max(want_tickets, c.tickets());
         tiles += ws[i].N / 128;
     }
     const size_t part_floats = slices > 1 ? (size_t)slices * mtiles * tiles * plan.rows * 128 : 0;
@@ -330,15 +292,15 @@ flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *c
         image[k] = (const u4_t *)next;
         next += image_floats;
     }
-    const float *xb[kWideMaxSegs];
+    float *xb[kWideMaxSegs] = {};
     for (int i = 0; i < count; ++i) {
-        xb[i] = nullptr;
         if (ws[i].R == 0) continue;
         xb[i] = next;
-        st = launch_coeff(rows[image_of[i]], ldr[image_of[i]], ws[i].resB, next, M, K, ws[i].R, out_bf16, xb_part, tickets,
-                          stream);
-        if (st != FLUTE_OK) return st;
         next += up4((size_t)M * ws[i].R);
+        // (weights of different rotations have different rows: one launch each)
+        st = launch_coeff(plan_coeff(ws + i, 1, M), ws + i, 1, rows[image_of[i]], ldr[image_of[i]], xb + i, M, out_bf16,
+                          xb_part, tickets, stream);
+        if (st != FLUTE_OK) return st;
     }
     bool done[kWideMaxSegs] = {};
     for (int i = 0; i < count; ++i) {
@@ -386,58 +348,43 @@ flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *c
     return FLUTE_OK;
 }
 
-}  // namespace
-}  // namespace flute
-
-using namespace flute;
-
-extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C, int M,
-                                   int64_t lda, int64_t ldc, int act_dtype, void *stream_) {
-    flute_status st = validate_linear(w, 1, "flute_gemm");
-    if (st != FLUTE_OK) return st;
-    FLUTE_REQUIRE(act_dtype == FLUTE_F16 || act_dtype == FLUTE_BF16, FLUTE_ERR_INVALID,
-                  "flute_gemm: activations must be float16 or bfloat16");
-    FLUTE_REQUIRE(M >= 0, FLUTE_ERR_INVALID, "flute_gemm: M must be >= 0 (got %d)", M);
-    if (M == 0) return FLUTE_OK;
-    FLUTE_REQUIRE(A != nullptr && C != nullptr, FLUTE_ERR_INVALID,
-                  "flute_gemm: A and C must not be NULL");
-    FLUTE_REQUIRE(lda >= w->K && ldc >= w->N, FLUTE_ERR_INVALID,
-                  "flute_gemm: row strides must cover a row (lda=%lld < K=%d or ldc=%lld < N=%d)",
-                  (long long)lda, w->K, (long long)ldc, w->N);
-    FLUTE_REQUIRE(((uintptr_t)A & 1) == 0 && ((uintptr_t)C & 1) == 0, FLUTE_ERR_INVALID,
-                  "flute_gemm: A and C must be 2-byte aligned");
-    hipStream_t stream = (hipStream_t)stream_;
-
-    GemmShape shape = choose_gemm_shape(M, w->N / 128, w->q1_bytes + (w->b2 > 0 ? w->q2_bytes : 0));
-    const int streams = w->b2 > 0 ? 2 : 1;
-    const WidePlan wide = choose_wide(M, w->N / 128, w->K / 64, streams,
-                                      other_forms(M, w->N / 128, w->K / 64, streams, w->b1 == 4, shape), shape);
-    if (wide.rows) return gemm_wide(w, 1, A, &C, &ldc, M, lda, act_dtype, wide, stream);
+// Up to four weights of one width pair, group size and rotation over the same rows of A through the
+// small-M kernel, in the given shape: one launch of each pre-pass and one (per stream) of the kernel.
+flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *const *C, const int64_t *ldc, int M,
+                       int64_t lda, int act_dtype, const GemmShape &shape, hipStream_t stream) {
+    const flute_linear *w = ws;                         // what they share
+    flute_status st;
     GemmParams p = {};
     p.nstreams = w->b2 > 0 ? 2 : 1;
-    p.q[0] = (const uint8_t *)w->q1;
-    p.q[1] = (const uint8_t *)w->q2;
-    p.lut[0] = (const uint16_t *)w->lut1;
-    p.lut[1] = (const uint16_t *)w->lut2;
     p.bits[0] = w->b1;
     p.bits[1] = w->b2;
     p.M = M;
-    p.N = w->N;
-    p.K = w->K;
     p.G = w->K / 64;
-    p.gs = w->group_size;
-    p.lut_rows = w->lut_rows;
-    p.R = w->R;
-    p.resA = (const uint16_t *)w->resA;
-    p.bias = (const uint16_t *)w->bias;
-    p.C = C;
-    p.ldc = ldc;
     p.out_bf16 = act_dtype == FLUTE_BF16;
-    p.vec_store = (ldc % 8 == 0) && (((uintptr_t)C & 15) == 0);
+    int tiles = 0;
+    bool any_res = false;
+    for (int i = 0; i < kGemmMaxSegs; ++i) {
+        p.tile0[i] = i < count ? tiles : INT_MAX;
+        if (i >= count) continue;
+        GemmSeg &g = p.seg[i];
+        g.q[0] = (const uint8_t *)ws[i].q1;
+        g.q[1] = (const uint8_t *)ws[i].q2;
+        g.lut[0] = (const uint16_t *)ws[i].lut1;
+        g.lut[1] = (const uint16_t *)ws[i].lut2;
+        g.gs = ws[i].group_size;
+        g.lut_rows = ws[i].lut_rows;
+        g.R = ws[i].R;
+        g.resA = (const uint16_t *)ws[i].resA;
+        g.bias = (const uint16_t *)ws[i].bias;
+        g.C = C[i];
+        g.ldc = ldc[i];
+        g.vec_store = (ldc[i] % 8 == 0) && (((uintptr_t)C[i] & 15) == 0);
+        any_res |= ws[i].R > 0;
+        tiles += ws[i].N / 128;
+    }
     p.mblk_total = (M + 15) / 16;
 
     // ---- grid and K split --------------------------------------------------------
-    const int tiles = w->N / 128;
     const int mchunks = (p.mblk_total + shape.mb * shape.mw - 1) / (shape.mb * shape.mw);
     const int64_t units = (int64_t)tiles * mchunks;
     p.mblk_pad = mchunks * shape.mb * shape.mw;
@@ -473,7 +420,9 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
     const size_t image = (size_t)shape.mw * shape.mb * 8 * 64 * 4;
     const int zparts = ksplit * ((p.nstreams == 2 && shape.mb > 1) ? 2 : 1);
     const size_t p_floats = zparts > 1 ? (size_t)zparts * units * image : 0;
-    const size_t xb_floats = (((size_t)M * w->R + 3) & ~(size_t)3) + coeff_floats(M, w->K, w->R);
+    const CoeffPlan coeff = plan_coeff(ws, count, M);
+    size_t xb_floats = any_res ? coeff.floats() : 0;
+    for (int i = 0; i < count; ++i) xb_floats += ((size_t)M * ws[i].R + 3) & ~(size_t)3;
     const size_t ap_floats = (size_t)p.G * 2 * p.mblk_pad * 64 * 4;
     const size_t rot_floats = w->signs ? ((size_t)M * w->K / 2 + 4) & ~(size_t)3 : 0;
     // bfloat16 activations presented as float16 operands: one power-of-two scale per row
@@ -481,7 +430,7 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
     const size_t shift_floats = scale_rows ? ((size_t)M + 3) & ~(size_t)3 : 0;
     float *base = nullptr;
     int *tickets = nullptr;
-    const size_t want_tickets = std::max((size_t)units, coeff_tickets(M, w->R)) + 1;
+    const size_t want_tickets = std::max((size_t)units, any_res ? coeff.tickets() : 0) + 1;
     st = get_workspace(p_floats + xb_floats + ap_floats + rot_floats + shift_floats + 64, want_tickets, stream, &base,
                        &tickets);
     if (st != FLUTE_OK) return st;
@@ -508,7 +457,7 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
         return shape.mb == 1 && p.nstreams == 1 && w->b1 == 4 && ngrp <= 2 && !tuning().gemm_no_perm &&
                !tuning().gemm_no_direct;
     }();
-    if (w->signs && w->R == 0 && !scale_rows) {
+    if (w->signs && !any_res && !scale_rows) {
         // the rotation writes the operand image itself: one launch instead of two
         FhtOperandOut image_out = {(uint32_t *)Ap, p.mblk_pad, (int)(w->lut_dtype == FLUTE_BF16), block_xor};
         st = fht_launch(A, lda, w->signs, w->awq, nullptr, 0, M, w->K, act_dtype, 0, w->rot_block,
@@ -552,12 +501,17 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
         }
         FLUTE_HIP_CHECK(hipGetLastError());
     }
-    if (w->R > 0) {
-        st = launch_coeff(A, lda, w->resB, xb, M, w->K, w->R, p.out_bf16, xb + (((size_t)M * w->R + 3) & ~(size_t)3),
-                          tickets, stream);
+    if (any_res) {
+        float *next = xb + coeff.floats(), *to[kGemmMaxSegs] = {};
+        for (int i = 0; i < count; ++i) {
+            if (ws[i].R == 0) continue;
+            to[i] = next;
+            p.seg[i].xb = next;
+            p.seg[i].vec_res = ws[i].R % 8 == 0 && ((uintptr_t)ws[i].resA & 15) == 0 && ((uintptr_t)next & 15) == 0;
+            next += ((size_t)M * ws[i].R + 3) & ~(size_t)3;
+        }
+        st = launch_coeff(coeff, ws, count, A, lda, to, M, p.out_bf16, xb, tickets, stream);
         if (st != FLUTE_OK) return st;
-        p.xb = xb;
-        p.vec_res = w->R % 8 == 0 && ((uintptr_t)w->resA & 15) == 0 && ((uintptr_t)xb & 15) == 0;
     }
 
     // Two streams with four blocks per wavefront: one launch per stream through the
@@ -571,8 +525,10 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
         GemmParams q = p;
         if (per_stream) {
             q.nstreams = 1;
-            q.q[0] = p.q[pass];
-            q.lut[0] = p.lut[pass];
+            for (int i = 0; i < count; ++i) {
+                q.seg[i].q[0] = p.seg[i].q[pass];
+                q.seg[i].lut[0] = p.seg[i].lut[pass];
+            }
             q.bits[0] = p.bits[pass];
         }
         q.z_base = pass * ksplit;
@@ -580,12 +536,44 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
         const int lds = plan_lds(q, shape);
         FLUTE_REQUIRE(lds <= kLdsPerCU, FLUTE_ERR_UNSUPPORTED,
                       "flute_gemm: %d bytes of LDS exceed the %d of one CU", lds, kLdsPerCU);
-        st = w->lut_dtype == FLUTE_BF16 ? launch_gemm_shape<true>(shape, q, grid, lds, stream)
-                                        : launch_gemm_shape<false>(shape, q, grid, lds, stream);
+        const int bf16 = w->lut_dtype == FLUTE_BF16;
+        st = count > 1 ? gemm_launch_segs(bf16, shape.mb, shape.mw, q, grid, lds, stream)
+             : bf16    ? launch_gemm_shape<true, false>(shape.mb, shape.mw, q, grid, lds, stream)
+                       : launch_gemm_shape<false, false>(shape.mb, shape.mw, q, grid, lds, stream);
         if (st != FLUTE_OK) return st;
     }
     workspace_done(stream);
     return FLUTE_OK;
+}
+
+}  // namespace
+}  // namespace flute
+
+using namespace flute;
+
+extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C, int M,
+                                   int64_t lda, int64_t ldc, int act_dtype, void *stream_) {
+    flute_status st = validate_linear(w, 1, "flute_gemm");
+    if (st != FLUTE_OK) return st;
+    FLUTE_REQUIRE(act_dtype == FLUTE_F16 || act_dtype == FLUTE_BF16, FLUTE_ERR_INVALID,
+                  "flute_gemm: activations must be float16 or bfloat16");
+    FLUTE_REQUIRE(M >= 0, FLUTE_ERR_INVALID, "flute_gemm: M must be >= 0 (got %d)", M);
+    if (M == 0) return FLUTE_OK;
+    FLUTE_REQUIRE(A != nullptr && C != nullptr, FLUTE_ERR_INVALID,
+                  "flute_gemm: A and C must not be NULL");
+    FLUTE_REQUIRE(lda >= w->K && ldc >= w->N, FLUTE_ERR_INVALID,
+                  "flute_gemm: row strides must cover a row (lda=%lld < K=%d or ldc=%lld < N=%d)",
+                  (long long)lda, w->K, (long long)ldc, w->N);
+    FLUTE_REQUIRE(((uintptr_t)A & 1) == 0 && ((uintptr_t)C & 1) == 0, FLUTE_ERR_INVALID,
+                  "flute_gemm: A and C must be 2-byte aligned");
+    hipStream_t stream = (hipStream_t)stream_;
+
+    const GemmShape shape = choose_gemm_shape(M, w->N / 128, w->q1_bytes + (w->b2 > 0 ? w->q2_bytes : 0));
+    const int streams = w->b2 > 0 ? 2 : 1;
+    const WidePlan wide = choose_wide(M, w->N / 128, w->K / 64, streams,
+                                      other_forms(M, w->N / 128, w->K / 64, streams, w->b1 == 4, shape), shape);
+    if (wide.rows) return gemm_wide(w, 1, A, &C, &ldc, M, lda, act_dtype, wide, stream);
+    return gemm_rows(w, 1, A, &C, &ldc, M, lda, act_dtype, shape, stream);
 }
 
 extern "C" flute_status flute_gemm_multi(const flute_linear *ws, int count, const void *A, void *const *C,
@@ -609,24 +597,25 @@ extern "C" flute_status flute_gemm_multi(const flute_linear *ws, int count, cons
     // in its own best form: they share the activations' image, and a chip that one weight's tiles
     // leave partly idle (or cut into slices of K) is filled.  Gate and up, 2 x 4096 -> 12288, M = 509:
     // 2 x 65.8 us in two slices each, 98.7 together.
-    const int streams = ws[0].b2 > 0 ? 2 : 1;
-    bool alike = count > 1, big = true;
+    // Small calls share everything in front of the kernel, and its launch.
+    const int streams = ws[0].b2 > 0 ? 2 : 1, G = ws[0].K / 64;
+    bool widths = true, all = true;
     int tiles = 0;
-    double other_us = 0.0;
-    GemmShape shape = {4, 4, 2, 1};
+    int64_t bytes = 0;
     for (int i = 0; i < count; ++i) {
         const flute_linear &w = ws[i];
-        alike &= w.b1 == ws[0].b1 && w.b2 == ws[0].b2;
+        widths &= w.b1 == ws[0].b1 && w.b2 == ws[0].b2;
+        all &= w.group_size == ws[0].group_size && w.signs == ws[0].signs && w.awq == ws[0].awq &&
+               w.rot_block == ws[0].rot_block;
         tiles += w.N / 128;
-        shape = choose_gemm_shape(M, w.N / 128, w.q1_bytes + (w.b2 > 0 ? w.q2_bytes : 0));
-        big &= shape.mb == 4;
-        const WidePlan own = choose_wide(M, w.N / 128, w.K / 64, streams,
-                                         other_forms(M, w.N / 128, w.K / 64, streams, w.b1 == 4, shape), shape);
-        other_us += own.us;
+        bytes += w.q1_bytes + (w.b2 > 0 ? w.q2_bytes : 0);
     }
-    if (alike && big) {
-        const WidePlan plan = choose_wide(M, tiles, ws[0].K / 64, streams, other_us, shape);
+    if (widths) {
+        const GemmShape shape = choose_gemm_shape(M, tiles, bytes);
+        const WidePlan plan = choose_wide(M, tiles, G, streams, other_forms(M, tiles, G, streams, ws[0].b1 == 4, shape),
+                                          shape);
         if (plan.rows) return gemm_wide(ws, count, A, C, ldc, M, lda, act_dtype, plan, (hipStream_t)stream);
+        if (all) return gemm_rows(ws, count, A, C, ldc, M, lda, act_dtype, shape, (hipStream_t)stream);
     }
     for (int i = 0; i < count; ++i) {
         flute_status st = flute_gemm(&ws[i], A, C[i], M, lda, ldc[i], act_dtype, stream);

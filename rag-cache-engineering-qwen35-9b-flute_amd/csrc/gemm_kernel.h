@@ -34,7 +34,7 @@ namespace flute {
 #ifdef FLUTE_STAMPS
 // Instrumented builds only: per-wavefront phase times (s_memrealtime, 10 ns units) and the shader
 // clock count across the K loop, written to the buffer flute_debug_stamps() was given.
-__device__ long long *g_gemm_stamps = nullptr;
+static __device__ long long *g_gemm_stamps = nullptr;
 #define FLUTE_STAMP(slot)                                                                       \
     do {                                                                                        \
         if (g_gemm_stamps && (threadIdx.x & 63) == 0)                                           \
@@ -46,18 +46,30 @@ __device__ long long *g_gemm_stamps = nullptr;
 #else
 #define FLUTE_STAMP(slot) do { } while (0)
 #endif
-struct GemmParams {
+constexpr int kGemmMaxSegs = 4;
+
+// One weight of a launch.
+struct GemmSeg {
     const uint8_t *q[2];
     const uint16_t *lut[2];
-    const u4_t *Ap;        // permuted activations, LUT dtype, rows padded to 16
     void *C;
     const float *xb;       // [M, R] fp32 residual coefficients (A @ resB^T) or NULL
     const uint16_t *resA;  // [N, R] activation dtype
-    int vec_res;           // R % 8 == 0 and rows of resA and xb allow 16-byte loads
     const uint16_t *bias;  // [N] activation dtype
+    int64_t ldc;
+    int gs, lut_rows, R;
+    int vec_res;           // R % 8 == 0 and rows of resA and xb allow 16-byte loads
+    int vec_store;         // C rows allow 16-byte stores
+};
+
+// Up to four weights of one width pair and group size over the same rows: gridDim.x counts the
+// 128-row tiles of all of them.
+struct GemmParams {
+    int tile0[kGemmMaxSegs];   // first tile of each weight; past the last one INT_MAX
+    GemmSeg seg[kGemmMaxSegs];
+    const u4_t *Ap;        // permuted activations, LUT dtype, rows padded to 16
     float *P;              // split-K partial images
     int *tickets;
-    int64_t ldc;
     int bits[2];
     int tab_off[2];        // byte offset of each stream's pair tables in LDS
     int rep_log2[2];       // log2 of the table replication (lanes per entry)
@@ -68,14 +80,13 @@ struct GemmParams {
     int scatter;           // four blocks per wavefront: the mode of image_block_xor the image was written with;
                            // not 0: the k ways hand blocks to each other instead of reducing through the tree
     int nstreams;
-    int M, N, K, G, gs, lut_rows, R;
+    int M, G;
     int mblk_total;        // ceil(M / 16)
     int mblk_pad;          // blocks Ap holds per half tile: gridDim.y * MW * MB
     int ksplit, gper;      // gridDim.z and k-tiles per z slice
     int z_base, ztotal;    // partial tiles: this launch writes [z_base, z_base + gridDim.z) of
                            // ztotal (several launches, one per stream, may share a fold)
     int out_bf16;          // dtype of C, resA, bias
-    int vec_store;         // C rows allow 16-byte stores
     const u4_t *A8;        // direct mode: A itself, rows of lda8 16-byte pieces, no pre-pass
     int64_t lda8;
     int a_bf16;            // dtype of A in direct mode
@@ -84,7 +95,7 @@ struct GemmParams {
 
 // Activation pre-pass: Ap[g][j][mb][lane][slot] in the LUT's 16-bit type.
 // block_xor: the mode of image_block_xor (common.h).
-__global__ void __launch_bounds__(256) gemm_prep_kernel(const uint16_t *A, u4_t *Ap, int M,
+static __global__ void __launch_bounds__(256) gemm_prep_kernel(const uint16_t *A, u4_t *Ap, int M,
                                                         int64_t lda, int G, int mblk,
                                                         int in_bf16, int out_bf16, int pairs,
                                                         const int *rowshift, int block_xor) {
@@ -134,7 +145,7 @@ template <int J>
 __device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, J * 0x55, 0xf, 0xf, true);
 }
-__global__ void __launch_bounds__(256) gemm_prep_quad_kernel(const uint16_t *A, u4_t *Ap, int M,
+static __global__ void __launch_bounds__(256) gemm_prep_quad_kernel(const uint16_t *A, u4_t *Ap, int M,
                                                              int64_t lda, int G, int mblk,
                                                              int in_bf16, int out_bf16,
                                                              const int *rowshift,
@@ -197,7 +208,7 @@ __global__ void __launch_bounds__(256) gemm_prep_quad_kernel(const uint16_t *A, 
 
 // The activation image of the many-row kernel (wide_piece) from rows: a wavefront moves one 1 KB block,
 // sixteen rows by 64 bytes, so that every line of the image is written whole by one instruction.
-__global__ void __launch_bounds__(256) gemm_image_kernel(const uint16_t *A, u4_t *Ap, int M, int64_t lda, int segs,
+static __global__ void __launch_bounds__(256) gemm_image_kernel(const uint16_t *A, u4_t *Ap, int M, int64_t lda, int segs,
                                                          int mblk, int in_bf16, int out_bf16, int aligned,
                                                          const int *rowshift) {
     const int lane = threadIdx.x & 63;
@@ -236,7 +247,7 @@ __global__ void __launch_bounds__(256) gemm_image_kernel(const uint16_t *A, u4_t
 
 // bfloat16 rows in front of float16 operands: shift[m] = the power of two that brings the
 // largest magnitude of row m to [1, 2) (bf16_row_shift), one workgroup per row.
-__global__ void __launch_bounds__(256) gemm_rowshift_kernel(const uint16_t *A, int64_t lda, int K,
+static __global__ void __launch_bounds__(256) gemm_rowshift_kernel(const uint16_t *A, int64_t lda, int K,
                                                             int *shift) {
     __shared__ uint32_t slots[4];
     const uint16_t *row = A + (int64_t)blockIdx.x * lda;
@@ -259,14 +270,26 @@ __global__ void __launch_bounds__(256) gemm_rowshift_kernel(const uint16_t *A, i
 // loads (sixteen rows each) are a chain of trips to memory; gridDim.z slices of K leave their sums in
 // `part`, and the last arrival of a block adds them in slice order.  M = 48, K = 12288, R = 16: 22.8
 // us in one slice, 6.3 in sixteen.
+struct CoeffParams {
+    const uint16_t *A;
+    const uint16_t *resB[kGemmMaxSegs];
+    float *xb[kGemmMaxSegs];
+    int R[kGemmMaxSegs];
+    int rank0[kGemmMaxSegs];   // first block of ranks (blockIdx.y) of each weight; past the last one INT_MAX
+    int64_t lda;
+    int M, K, aligned, kper;
+    float *part;
+    int *tickets;
+};
 template <bool BF16>
-__global__ void __launch_bounds__(1024) gemm_coeff_kernel(const uint16_t *A, int64_t lda, const uint16_t *resB, float *xb,
-                                                          int M, int K, int R, int aligned, int kper, float *part,
-                                                          int *tickets) {
+__global__ void __launch_bounds__(1024) gemm_coeff_kernel(const CoeffParams p) {
     __shared__ f4_t red[16][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int m = min((int)blockIdx.x * 16 + (lane & 15), M - 1), rr = min((int)blockIdx.y * 16 + (lane & 15), R - 1);
-    const uint16_t *a = A + (int64_t)m * lda + (lane >> 4) * 8, *b = resB + (int64_t)rr * K + (lane >> 4) * 8;
+    const int si = ((int)blockIdx.y >= p.rank0[1]) + ((int)blockIdx.y >= p.rank0[2]) + ((int)blockIdx.y >= p.rank0[3]);
+    const int M = p.M, K = p.K, R = p.R[si], rb = blockIdx.y - p.rank0[si], aligned = p.aligned;
+    float *const xb = p.xb[si];
+    const int m = min((int)blockIdx.x * 16 + (lane & 15), M - 1), rr = min(rb * 16 + (lane & 15), R - 1);
+    const uint16_t *a = p.A + (int64_t)m * p.lda + (lane >> 4) * 8, *b = p.resB[si] + (int64_t)rr * K + (lane >> 4) * 8;
     auto load8 = [&](const uint16_t *p) {
         u4_t v;
         if (aligned) return *(const u4_t *)p;
@@ -275,7 +298,7 @@ __global__ void __launch_bounds__(1024) gemm_coeff_kernel(const uint16_t *A, int
         return v;
     };
     f4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const int k0 = blockIdx.z * kper, k1 = min(k0 + kper, K);
+    const int k0 = blockIdx.z * p.kper, k1 = min(k0 + p.kper, K);
 #pragma unroll 4
     for (int k = k0 + wave * 32; k < k1; k += 512) acc = mfma16<BF16>(load8(b + k), load8(a + k), acc);
     red[wave][lane] = acc;
@@ -285,23 +308,23 @@ __global__ void __launch_bounds__(1024) gemm_coeff_kernel(const uint16_t *A, int
         if (gridDim.z > 1) {
             const int block = blockIdx.y * gridDim.x + blockIdx.x, Z = gridDim.z;
             const int64_t step = (int64_t)gridDim.x * gridDim.y * 256;       // floats of one slice
-            float *const mine = part + (int64_t)block * 256 + lane * 4;
+            float *const mine = p.part + (int64_t)block * 256 + lane * 4;
             ws_store16(mine + blockIdx.z * step, acc);
             ws_stores_done();
             int old = 0;
-            if (lane == 0) old = __hip_atomic_fetch_add(tickets + block, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (lane == 0) old = __hip_atomic_fetch_add(p.tickets + block, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (__builtin_amdgcn_readfirstlane(old) != Z - 1) return;
-            if (lane == 0) __hip_atomic_store(tickets + block, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (lane == 0) __hip_atomic_store(p.tickets + block, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             acc = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
             for (int z = 0; z < Z; z += 4) {                                 // (slices come in fours)
                 f4_t v[4];
-                const float *p = mine + z * step;
-                ws_load16x4(p, p + step, p + 2 * step, p + 3 * step, v[0], v[1], v[2], v[3]);
+                const float *s = mine + z * step;
+                ws_load16x4(s, s + step, s + 2 * step, s + 3 * step, v[0], v[1], v[2], v[3]);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc += v[i];
             }
         }
-        const int mo = blockIdx.x * 16 + (lane & 15), r0 = blockIdx.y * 16 + (lane >> 4) * 4;
+        const int mo = blockIdx.x * 16 + (lane & 15), r0 = rb * 16 + (lane >> 4) * 4;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (mo < M && r0 + e < R) xb[(int64_t)mo * R + r0 + e] = acc[e];
@@ -435,7 +458,7 @@ __device__ __forceinline__ void lean_load16(u4_t &dst, const u4_t *src, int mb) 
 // hold; the compiler cannot count such loads next to its own (it answers one in flight with
 // vmcnt(0) in front of the next use of any loaded register), hence all or nothing.
 template <int MB, int KW, int MW, bool BF16, int B1, bool PERM = false, bool DIRECT = false,
-          bool LEAN = false>
+          bool LEAN = false, bool SEGS = false>
 __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) {
     static_assert(!DIRECT || (PERM && MB == 1), "direct activations: one block, fast path");
     static_assert(!LEAN || (PERM && !DIRECT && MB >= 2 && B1 == 4), "lean loop: fast path, operand image");
@@ -443,7 +466,13 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
     constexpr int NT = 64 * KW * MW;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int kw = wave % KW, mw = wave / KW;
-    const int t = blockIdx.x;
+    // (instantiations of their own for several weights: the tile numbers have to be read before the
+    // weight's arguments can be, and M = 256, 4096 -> 12288 went from 36.6 to 37.6 us with it)
+    int si = 0;
+    if constexpr (SEGS)
+        si = ((int)blockIdx.x >= p.tile0[1]) + ((int)blockIdx.x >= p.tile0[2]) + ((int)blockIdx.x >= p.tile0[3]);
+    const GemmSeg &w = p.seg[SEGS ? si : 0];
+    const int t = SEGS ? blockIdx.x - p.tile0[si] : blockIdx.x;
     FLUTE_STAMP(0);
     const int mb0 = (blockIdx.y * MW + mw) * MB;       // first 16-row block of this wavefront
     const int z = blockIdx.z;
@@ -490,20 +519,20 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
     // fast path: first tile and first activation operands are requested before the
     // tables are built, so their latency hides behind the build
     u4_t R[4], A0[MB], A1[MB];
-    const uint8_t *tp = p.q[0] + ((int64_t)t * p.G + g_first) * 4096 + lane * 16;
+    const uint8_t *tp = w.q[0] + ((int64_t)t * p.G + g_first) * 4096 + lane * 16;
     auto load_tile = [&]() {
 #pragma unroll
         for (int i = 0; i < 4; ++i) R[i] = __builtin_nontemporal_load((const u4_t *)(tp + i * 1024));
     };
-    const int ngrp = p.gs >= 128 ? 1 : 128 / p.gs;
+    const int ngrp = w.gs >= 128 ? 1 : 128 / w.gs;
     uint32_t lutv[2] = {0u, 0u};                       // fast path: LUT row(s), one value per lane
     if constexpr (PERM) {
 #pragma unroll
         for (int gl = 0; gl < 2; ++gl) {
             if (LEAN || gl >= ngrp) break;
-            int row = p.gs >= 128 ? (t * 128) / p.gs : t * ngrp + gl;
-            row = min(row, p.lut_rows - 1);
-            lutv[gl] = p.lut[0][((size_t)row << 4) + (lane & 15)];
+            int row = w.gs >= 128 ? (t * 128) / w.gs : t * ngrp + gl;
+            row = min(row, w.lut_rows - 1);
+            lutv[gl] = w.lut[0][((size_t)row << 4) + (lane & 15)];
         }
         // Unconditional, after the LUT row: the table build below then waits for the LUT
         // values only, not for the first tile (a conditional load here made that wait a
@@ -527,7 +556,7 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
     const int lean_kt = ((lane & 3) - (lane >> 4)) & 3;
     const uint32_t lean_even = (uint32_t)((lane >> 2) * 64 + lean_kt * 16);
     const uint32_t lean_odd = (uint32_t)(((lane >> 2) ^ 1) * 64 + lean_kt * 16);
-    const uint8_t *lean_tq = p.q[0] + ((int64_t)t * p.G + g_first) * 4096;   // wavefront-uniform
+    const uint8_t *lean_tq = w.q[0] + ((int64_t)t * p.G + g_first) * 4096;   // wavefront-uniform
     auto lean_tile = [&](int buf) {                    // four loads, straight into LDS
         const uint32_t m0v = lean_stage + (uint32_t)buf * 4096u;
         // (the pointer is the same in every lane; the compiler cannot see that through the
@@ -544,9 +573,9 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
                      :: "s"(m0v), "v"(lean_even), "v"(lean_odd), "s"(tq_s) : "memory", "m0");
     };
     if constexpr (LEAN) {
-        int row = (t * 128) / p.gs;
-        row = min(row, p.lut_rows - 1);
-        const uint16_t *lp = p.lut[0] + ((size_t)row << 4) + (lane & 15);
+        int row = (t * 128) / w.gs;
+        row = min(row, w.lut_rows - 1);
+        const uint16_t *lp = w.lut[0] + ((size_t)row << 4) + (lane & 15);
         uint32_t lv;
         asm volatile("global_load_ushort %0, %1, off" : "=&v"(lv) : "v"(lp) : "memory");
         lean_tile(0);                                  // tile 0
@@ -582,12 +611,12 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
             const int rl = p.rep_log2[s];
             const int total = ngrp << (2 * b + rl);
             uint32_t *tab = (uint32_t *)(smem + p.tab_off[s]);
-            const uint16_t *lut = p.lut[s];
+            const uint16_t *lut = w.lut[s];
             for (int i = tid; i < total; i += NT) {
                 const int code = (i >> rl) & ((1 << (2 * b)) - 1);
                 const int gl = i >> (rl + 2 * b);
-                int row = p.gs >= 128 ? (t * 128) / p.gs : t * ngrp + gl;
-                row = min(row, p.lut_rows - 1);
+                int row = w.gs >= 128 ? (t * 128) / w.gs : t * ngrp + gl;
+                row = min(row, w.lut_rows - 1);
                 const uint16_t *lr = lut + ((size_t)row << b);
                 tab[i] = (uint32_t)lr[code & ((1 << b) - 1)] | ((uint32_t)lr[code >> b] << 16);
             }
@@ -614,7 +643,7 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int row = wx * 64 + v * 16;
-            const int gl = p.gs >= 128 ? 0 : row / p.gs;
+            const int gl = w.gs >= 128 ? 0 : row / w.gs;
             lb[v] = lds_base + p.tab_off[s] +
                     (((gl << (2 * b + rl)) + (lane & ((1 << rl) - 1))) << 2);
         }
@@ -829,7 +858,7 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
             table_bases(lb, 0, B1);
             const int cs = p.rep_log2[0] + 2;
             uint32_t Qa[4 * B1], Qb[4 * B1];
-            const uint8_t *qp = p.q[0] + (((int64_t)t * p.G + g0) * 64 + th) * (16 * B1);
+            const uint8_t *qp = w.q[0] + (((int64_t)t * p.G + g0) * 64 + th) * (16 * B1);
             constexpr int64_t qstep = (int64_t)KW * 64 * 16 * B1;
             const int64_t astep = (int64_t)KW * 2 * p.mblk_pad * 64;
             if (left > 0) {
@@ -873,28 +902,28 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
                         case 1: {
                             uint32_t Q[4];
                             table_bases(lb, s, 1);
-                            load_chunk<1>(Q, p.q[s] + (tile * 64 + th) * (16 * 1));
+                            load_chunk<1>(Q, w.q[s] + (tile * 64 + th) * (16 * 1));
                             half_mma<1, MB, BF16>(Q, 0, A0, acc, lb, cs);
                             half_mma<1, MB, BF16>(Q, 1, A1, acc, lb, cs);
                         } break;
                         case 2: {
                             uint32_t Q[8];
                             table_bases(lb, s, 2);
-                            load_chunk<2>(Q, p.q[s] + (tile * 64 + th) * (16 * 2));
+                            load_chunk<2>(Q, w.q[s] + (tile * 64 + th) * (16 * 2));
                             half_mma<2, MB, BF16>(Q, 0, A0, acc, lb, cs);
                             half_mma<2, MB, BF16>(Q, 1, A1, acc, lb, cs);
                         } break;
                         case 3: {
                             uint32_t Q[12];
                             table_bases(lb, s, 3);
-                            load_chunk<3>(Q, p.q[s] + (tile * 64 + th) * (16 * 3));
+                            load_chunk<3>(Q, w.q[s] + (tile * 64 + th) * (16 * 3));
                             half_mma<3, MB, BF16>(Q, 0, A0, acc, lb, cs);
                             half_mma<3, MB, BF16>(Q, 1, A1, acc, lb, cs);
                         } break;
                         default: {
                             uint32_t Q[16];
                             table_bases(lb, s, 4);
-                            load_chunk<4>(Q, p.q[s] + (tile * 64 + th) * (16 * 4));
+                            load_chunk<4>(Q, w.q[s] + (tile * 64 + th) * (16 * 4));
                             half_mma<4, MB, BF16>(Q, 0, A0, acc, lb, cs);
                             half_mma<4, MB, BF16>(Q, 1, A1, acc, lb, cs);
                         } break;
@@ -1087,14 +1116,14 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
 #pragma unroll
             for (int e = 0; e < 8; ++e) y[e] = ldexpf(y[e], sh);
         }
-        if (p.R > 0 && p.vec_res) {
+        if (w.R > 0 && w.vec_res) {
             // eight ranks a step, ten 16-byte loads at once instead of a chain of 2-byte ones
             // (M = 48, rank 16, 12288 -> 4096: the launch that folds the partial tiles 46.1 -> 22.6 us)
-            const float *xr = p.xb + (size_t)m * p.R;
-            for (int r0 = 0; r0 < p.R; r0 += 8) {
+            const float *xr = w.xb + (size_t)m * w.R;
+            for (int r0 = 0; r0 < w.R; r0 += 8) {
                 u4_t a[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) a[e] = *(const u4_t *)(p.resA + (int64_t)(n0 + e) * p.R + r0);
+                for (int e = 0; e < 8; ++e) a[e] = *(const u4_t *)(w.resA + (int64_t)(n0 + e) * w.R + r0);
                 const f4_t c0 = *(const f4_t *)(xr + r0), c1 = *(const f4_t *)(xr + r0 + 4);
 #pragma unroll
                 for (int r = 0; r < 8; ++r) {
@@ -1106,26 +1135,26 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
                     }
                 }
             }
-        } else if (p.R > 0) {
-            const float *xr = p.xb + (size_t)m * p.R;
-            for (int r = 0; r < p.R; ++r) {
+        } else if (w.R > 0) {
+            const float *xr = w.xb + (size_t)m * w.R;
+            for (int r = 0; r < w.R; ++r) {
                 const float c = xr[r];
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
-                    y[e] = fmaf(c, load_act(p.resA, (int64_t)(n0 + e) * p.R + r, p.out_bf16), y[e]);
+                    y[e] = fmaf(c, load_act(w.resA, (int64_t)(n0 + e) * w.R + r, p.out_bf16), y[e]);
             }
         }
-        if (p.bias) {
+        if (w.bias) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) y[e] += load_act(p.bias, n0 + e, p.out_bf16);
+            for (int e = 0; e < 8; ++e) y[e] += load_act(w.bias, n0 + e, p.out_bf16);
         }
         uint32_t o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             o[e] = (uint32_t)round_act(y[2 * e], p.out_bf16) |
                    ((uint32_t)round_act(y[2 * e + 1], p.out_bf16) << 16);
-        uint16_t *dst = (uint16_t *)p.C + (size_t)m * p.ldc + n0;
-        if (p.vec_store) {
+        uint16_t *dst = (uint16_t *)w.C + (size_t)m * w.ldc + n0;
+        if (w.vec_store) {
             *(u4_t *)dst = u4_t{o[0], o[1], o[2], o[3]};
         } else {
 #pragma unroll

@@ -378,7 +378,7 @@ Tensor qgemm_linear(const Tensor &A, const Tensor &indices, const Tensor &lut, i
 
 // Several layers on the same rows, each (indices, lut, b1, indices2, lut2, b2, resB, resA, bias, gs,
 // signs, s) with None for what it has not: their outputs side by side, or silu(first) * second.
-// Layers of one rotation (the same signs and s) share the rotated rows.
+// Layers of one rotation (the same signs and s at the same address) share the rotated rows.
 Tensor qgemm_linear_multi(const Tensor &A_in, const std::vector<pybind11::tuple> &layers, bool silu_mul) {
     const char *who = "qgemm_linear_multi";
     const Shape2 s = check_2d_input(who, A_in, false);
@@ -388,7 +388,7 @@ Tensor qgemm_linear_multi(const Tensor &A_in, const std::vector<pybind11::tuple>
         return h.is_none() ? c10::optional<Tensor>() : c10::optional<Tensor>(h.cast<Tensor>());
     };
     const auto held = [&](const pybind11::handle &h) { return h.is_none() ? Tensor() : h.cast<Tensor>(); };
-    Tensor A = aligned16(A_in);
+    const Tensor A = aligned16(A_in);
     c10::DeviceGuard guard(A.device());
     std::vector<Described> d;
     std::vector<flute_linear> ws;
@@ -400,15 +400,6 @@ Tensor qgemm_linear_multi(const Tensor &A_in, const std::vector<pybind11::tuple>
                              opt(l[10]), opt(l[11]), 0, kGsAll, 256));
         ws.push_back(d.back().w);
         total += d.back().N;
-    }
-    bool shared = ws[0].signs != nullptr;
-    for (const flute_linear &w : ws) shared &= w.signs == ws[0].signs && w.awq == ws[0].awq;
-    if (shared) {
-        Tensor rotated = torch::empty_like(A);
-        check_status(flute_fht(A.data_ptr(), ws[0].signs, ws[0].awq, rotated.data_ptr(), (int)s.M, (int)s.K, act_code(A), 0,
-                               0, stream_of(A)));
-        A = rotated;
-        for (flute_linear &w : ws) w.signs = w.awq = nullptr;
     }
     TORCH_CHECK(!silu_mul || d[0].N == d[1].N, who, ": gate and up must agree in N");
     const Tensor out = silu_mul ? torch::empty({2, s.M, d[0].N}, A.options()) : torch::empty({s.M, total}, A.options());
