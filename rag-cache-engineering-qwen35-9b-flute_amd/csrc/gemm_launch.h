@@ -14,7 +14,7 @@ template <int MB, int KW, int MW, bool BF16, int B1, bool PERM = false, bool DIR
 flute_status launch_gemm(const GemmParams &p, dim3 grid, int lds, hipStream_t stream) {
     static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
     if (!attr_done) {
-        FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)gemm_kernel<MB, KW, MW, BF16, B1, PERM, DIRECT, LEAN>,
+        FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)gemm_kernel<MB, KW, MW, BF16, B1, PERM, DIRECT, LEAN, SEGS>,
                                             hipFuncAttributeMaxDynamicSharedMemorySize,
                                             (int)kLdsPerCU));
         attr_done = true;
