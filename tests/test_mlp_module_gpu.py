@@ -386,3 +386,28 @@ def test_layers_on_the_same_rows_in_one_call(monkeypatch, M, spec, act, rot):
         assert len(seen) == 2 and "gemm_multi" not in pm.ROUTE_CENSUS
     if spec.get("bias") and M > 16:                     # (the small-M entry never tracked the bias)
         assert qkv(x).requires_grad and mlp(x).requires_grad
+
+
+@pytest.mark.parametrize("rows", [16, 32, 64, 128])
+@pytest.mark.parametrize("M", [2, 33, 130])
+@pytest.mark.parametrize("spec,act,rot", [
+    (dict(), torch.bfloat16, False), (dict(gs=64), torch.float16, True), (dict(gs=32), torch.float16, False),
+    (dict(bits=3, rank=5, bias=True), torch.bfloat16, True), (dict(bits=2, bits2=4, rank=16), torch.float16, False),
+    (dict(lut_dtype=torch.bfloat16, rank=8), torch.bfloat16, False)])
+def test_several_weights_in_every_workgroup_shape(tuning_env, rows, M, spec, act, rot):
+    """The launch of several weights in every shape of the small-M kernel: its loops, ragged row
+    blocks, slices of K, weights that begin inside the grid.  fp32 sums (K terms: far below the type's
+    rounding), so it and the members one by one, which sum in slices of their own, differ by one
+    rounding each; the reference mode rounds the rotated rows, each stream, residual and bias (four)."""
+    K, rounding = 1024, 2 ** -11 if act is torch.float16 else 2 ** -8
+    kw = dict(rotation_seed=9, rotation_k=K) if rot else {}
+    tuning_env("FLUTE_GEMM_ROWS", str(rows))
+    pairs = [_modules(make_weight(n, K, seed=i, act_dtype=act, **spec), **kw) for i, n in enumerate((384, 128, 256))]
+    x = make_x(M, K, seed=6, dtype=act)
+    pm.ROUTE_CENSUS.clear()
+    with torch.no_grad():
+        y = pm.SplitQKV(*[p[1] for p in pairs])(x.to(DEV))
+        want = torch.cat([p[1](x.to(DEV)) for p in pairs], dim=-1)
+    assert pm.ROUTE_CENSUS["gemm_multi"] == 1
+    assert rel_l2(y.cpu(), want.cpu()) <= rounding
+    assert rel_l2(y.cpu(), torch.cat([p[0](x) for p in pairs], dim=-1)) <= 2 * rounding    # half a unit each
