@@ -486,8 +486,9 @@ def _same_rotation(a, b) -> bool:
 
 
 def _observed(m) -> bool:
-    """Whether somebody watches this module's call: it has to be made then."""
-    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+    """Whether somebody watches this module's call (a hook, or a forward of this one object, which
+    is how placement libraries wrap a module): it has to be made then."""
+    return bool("forward" in m.__dict__ or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
 
 
 def _rows_together(members, x, silu_mul: bool):

@@ -388,6 +388,18 @@ def test_layers_on_the_same_rows_in_one_call(monkeypatch, M, spec, act, rot):
         assert qkv(x).requires_grad and mlp(x).requires_grad
 
 
+def test_layers_wrapped_on_the_object_are_called_one_by_one():
+    """A forward set on one object (placement libraries wrap modules so) is called, as torch would."""
+    K = 1024
+    layers = [_modules(make_weight(n, K, seed=i))[1] for i, n in enumerate((256, 128, 128))]
+    seen, inner = [], layers[1].forward
+    layers[1].forward = lambda x: (seen.append(1), inner(x))[1]
+    qkv, x = pm.SplitQKV(*layers), make_x(5, K, seed=6).to(DEV)
+    with torch.no_grad():
+        y = qkv(x)
+        assert seen == [1] and torch.equal(y[:, 256:384], inner(x))
+
+
 @pytest.mark.parametrize("rows", [16, 32, 64, 128])
 @pytest.mark.parametrize("M", [2, 33, 130])
 @pytest.mark.parametrize("spec,act,rot", [
