@@ -35,7 +35,14 @@ struct GemmShape {
 // four k ways); further rows go to gridDim.y.  The tables plus staging take most of a
 // CU's LDS, so one workgroup per CU is resident.  FLUTE_GEMM_ROWS = 16, 32, 64 or 128
 // forces the shape (a tuning and test knob, like FLUTE_GEMV_RW), 256 or 512 the many-row kernel.
-GemmShape choose_gemm_shape(int M, int tiles, int64_t index_bytes) {
+// Two streams are one launch in 16-row workgroups and two in all others, so for two chunks of rows
+// (M = 17 ... 32) the next shape wins from 80 MB on only: (3, 3) bits, 12288 -> 4096 30.8 us with 16 rows,
+// 41.2 with 32; (2, 4) 32.7 and 35.6; (3, 3), 4096 -> 12288 32.5 and 34.4.  A 4-bit stream, though, has
+// its one-instruction lookups in a launch of its own only (`fast_stream`), which is worth the second
+// launch where a 16-row workgroup would have a K range of 4096 or more: (4, 1) bits, M = 32 with 16
+// rows and 32, 4096 -> 12288 34.2 and 30.2 us (rank 16: 42.2, 39.5), 8192 -> 6144 in two slices 35.9 and
+// 32.1, 12288 -> 4096 in four 31.7 and 35.2, 2048 -> 12288 22.4 and 25.4; M = 96, 4096 -> 4096 33.1 and 30.2.
+GemmShape choose_gemm_shape(int M, int tiles, int64_t index_bytes, int G, bool two_streams, bool fast_stream) {
     {
         const int v = tuning().gemm_rows;
         if (v == 16) return {1, 8, 1, 1};
@@ -45,7 +52,11 @@ GemmShape choose_gemm_shape(int M, int tiles, int64_t index_bytes) {
     }
     if (M <= 16) return {1, 8, 1, 1};
     const int chunks16 = (M + 15) / 16, chunks32 = (M + 31) / 32;
-    if ((int64_t)tiles * chunks16 <= kNumCU && chunks16 * index_bytes <= (int64_t)64 << 20)
+    const int64_t units16 = (int64_t)tiles * chunks16, limit16 = (int64_t)(two_streams && chunks16 == 2 ? 80 : 64) << 20;
+    int slices = 1;                                     // of K, as gemm_rows would cut it
+    while (units16 * slices * 2 <= kNumCU && G / (slices * 2) >= 16) slices *= 2;
+    const bool fast_wins = two_streams && fast_stream && G / slices >= 64;
+    if (units16 <= kNumCU && chunks16 * index_bytes <= limit16 && !fast_wins)
         return {1, 8, 1, 1};
     if ((int64_t)tiles * chunks32 <= kNumCU && chunks32 * index_bytes <= (int64_t)100 << 20)
         return {2, 8, 1, 1};
@@ -53,6 +64,8 @@ GemmShape choose_gemm_shape(int M, int tiles, int64_t index_bytes) {
     if ((int64_t)tiles * chunks64 <= kNumCU) return {4, 8, 1, 1};
     return {4, 4, 2, 1};
 }
+
+bool fast_stream(const flute_linear &w) { return (w.b1 == 4 || w.b2 == 4) && w.group_size >= 64; }
 
 // The residual coefficients of a call's weights, xb[i][m, r] = sum_k A[m, k] * resB[i][r, k] in fp32:
 // 16-row by 16-rank blocks in as many slices of K as the chip has CUs for, 512 columns (one step of a
@@ -568,7 +581,8 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
                   "flute_gemm: A and C must be 2-byte aligned");
     hipStream_t stream = (hipStream_t)stream_;
 
-    const GemmShape shape = choose_gemm_shape(M, w->N / 128, w->q1_bytes + (w->b2 > 0 ? w->q2_bytes : 0));
+    const GemmShape shape = choose_gemm_shape(M, w->N / 128, w->q1_bytes + (w->b2 > 0 ? w->q2_bytes : 0), w->K / 64,
+                                              w->b2 > 0, fast_stream(*w));
     const int streams = w->b2 > 0 ? 2 : 1;
     const WidePlan wide = choose_wide(M, w->N / 128, w->K / 64, streams,
                                       other_forms(M, w->N / 128, w->K / 64, streams, w->b1 == 4, shape), shape);
@@ -611,7 +625,7 @@ extern "C" flute_status flute_gemm_multi(const flute_linear *ws, int count, cons
         bytes += w.q1_bytes + (w.b2 > 0 ? w.q2_bytes : 0);
     }
     if (widths) {
-        const GemmShape shape = choose_gemm_shape(M, tiles, bytes);
+        const GemmShape shape = choose_gemm_shape(M, tiles, bytes, G, streams == 2, fast_stream(ws[0]));
         const WidePlan plan = choose_wide(M, tiles, G, streams, other_forms(M, tiles, G, streams, ws[0].b1 == 4, shape),
                                           shape);
         if (plan.rows) return gemm_wide(ws, count, A, C, ldc, M, lda, act_dtype, plan, (hipStream_t)stream);
