@@ -13,6 +13,10 @@
 namespace flute {
 
 flute_status gemm_launch_segs(int bf16, int mb, int mw, const GemmParams &p, dim3 grid, int lds, hipStream_t stream);
+flute_status gemm_few_f16(int mb, const GemmParams &p, dim3 grid, hipStream_t stream);
+flute_status gemm_few_bf16(int mb, const GemmParams &p, dim3 grid, hipStream_t stream);
+flute_status gemm_few_f16_segs(int mb, const GemmParams &p, dim3 grid, hipStream_t stream);
+flute_status gemm_few_bf16_segs(int mb, const GemmParams &p, dim3 grid, hipStream_t stream);
 flute_status gemm_wide_f16(int mb, int b1, int b2, int slices, const WideParams &p, hipStream_t stream);
 flute_status gemm_wide_bf16(int mb, int b1, int b2, int slices, const WideParams &p, hipStream_t stream);
 
@@ -23,49 +27,77 @@ struct GemmShape {
     int wg_per_cu;        // workgroups the policy expects to be resident per CU
 };
 
-// Rows of A per workgroup.  One or two 16-row blocks per wavefront with eight k ways (the
-// launch is then a weight stream, like the GEMV) as long as one workgroup per 16 (32) rows
-// and tile fits the device in one round and the indices are not re-read too often: every
-// chunk of rows streams its tile again, and beyond about 64 MB (100 MB) of index traffic
-// the next shape wins.  Measured: M = 32, 4096 -> 12288: 18.0 us with 16 rows, 24.6 us
-// with 64; M = 64: 21.5 us with 32 rows, 26.0 us with 64; M = 256, 4096 -> 4096: 23.8 us
-// with 32 rows, 29.0 us with 64; M = 96, 12288 -> 4096: 31.6 us with 32 rows, 37.8 us
-// with 16, 34.7 us with 64.  Otherwise four blocks per wavefront: 64 rows per workgroup
-// with eight k ways while that fits the device in one round, else 128 rows (two m groups,
-// four k ways); further rows go to gridDim.y.  The tables plus staging take most of a
-// CU's LDS, so one workgroup per CU is resident.  FLUTE_GEMM_ROWS = 16, 32, 64 or 128
-// forces the shape (a tuning and test knob, like FLUTE_GEMV_RW), 256 or 512 the many-row kernel.
-// Two streams are one launch in 16-row workgroups and two in all others, so for two chunks of rows
-// (M = 17 ... 32) the next shape wins from 80 MB on only: (3, 3) bits, 12288 -> 4096 30.8 us with 16 rows,
-// 41.2 with 32; (2, 4) 32.7 and 35.6; (3, 3), 4096 -> 12288 32.5 and 34.4.  A 4-bit stream, though, has
-// its one-instruction lookups in a launch of its own only (`fast_stream`), which is worth the second
-// launch where a 16-row workgroup would have a K range of 4096 or more: (4, 1) bits, M = 32 with 16
-// rows and 32, 4096 -> 12288 34.2 and 30.2 us (rank 16: 42.2, 39.5), 8192 -> 6144 in two slices 35.9 and
-// 32.1, 12288 -> 4096 in four 31.7 and 35.2, 2048 -> 12288 22.4 and 25.4; M = 96, 4096 -> 4096 33.1 and 30.2.
-GemmShape choose_gemm_shape(int M, int tiles, int64_t index_bytes, int G, bool two_streams, bool fast_stream) {
-    {
-        const int v = tuning().gemm_rows;
-        if (v == 16) return {1, 8, 1, 1};
-        if (v == 32) return {2, 8, 1, 1};
-        if (v == 64) return {4, 8, 1, 1};
-        if (v == 128) return {4, 4, 2, 1};
-    }
-    if (M <= 16) return {1, 8, 1, 1};
-    const int chunks16 = (M + 15) / 16, chunks32 = (M + 31) / 32;
-    const int64_t units16 = (int64_t)tiles * chunks16, limit16 = (int64_t)(two_streams && chunks16 == 2 ? 80 : 64) << 20;
-    int slices = 1;                                     // of K, as gemm_rows would cut it
-    while (units16 * slices * 2 <= kNumCU && G / (slices * 2) >= 16) slices *= 2;
-    const bool fast_wins = two_streams && fast_stream && G / slices >= 64;
-    if (units16 <= kNumCU && chunks16 * index_bytes <= limit16 && !fast_wins)
-        return {1, 8, 1, 1};
-    if ((int64_t)tiles * chunks32 <= kNumCU && chunks32 * index_bytes <= (int64_t)100 << 20)
-        return {2, 8, 1, 1};
-    const int chunks64 = (M + 63) / 64;
-    if ((int64_t)tiles * chunks64 <= kNumCU) return {4, 8, 1, 1};
-    return {4, 4, 2, 1};
+// Slices of K: split until the grid reaches one workgroup per CU, while every wavefront keeps two
+// tiles or more; with more than 16 rows a workgroup at most four, because the workgroup that arrives
+// last reads every partial tile of its unit back (64 rows, M = 64: 12288 -> 4096 29.7 us four ways,
+// 36.4 eight ways; 4096 -> 4096 21.8 four ways, 23.0 two ways, 24.6 eight ways).
+int slices_of_k(int64_t units, int G, const GemmShape &shape) {
+    const int most = shape.mb == 1 ? 64 : 4;
+    int ks = 1;
+    while (units * ks * 2 <= (int64_t)kNumCU * shape.wg_per_cu && ks * 2 <= most && G / (ks * 2) >= shape.kw * 2) ks *= 2;
+    return ks;
 }
 
-bool fast_stream(const flute_linear &w) { return (w.b1 == 4 || w.b2 == 4) && w.group_size >= 64; }
+// Width pairs (the wider first) that the few-row kernel takes in one launch: those of deployed weights.
+bool few_takes(int b1, int b2) { return b1 == 3 ? b2 >= 2 : b1 == 4 ? b2 <= 2 : false; }
+
+// Microseconds of a call (one round = a workgroup per CU; `turns` = K tiles of a wavefront), fitted to
+// measurements on tiles of 16 and 32 rows: a fixed part, the pre-pass for 32 rows (16-row workgroups
+// read A themselves) and, per round, prologue, sums and epilogue, then what a wavefront's tile costs.
+// M = 32, 4096 -> 12288, 16 and 32 rows: 4 bits 14.6 / 16.0, (4, 1) bits 19.6 / 18.5, (3, 3) 24.7 / 21.1;
+// M = 64: 27.5 / 17.1, 36.4 / 23.5, 46.6 / 28.3; M = 64, 12288 -> 4096: 22.2 / 19.6, 29.6 / 24.5,
+// 37.9 / 28.4; M = 128, 4096 -> 4096: 15.5 / 16.1, 20.6 / 19.5, 25.7 / 22.0.
+double few_us(int mb, int M, int tiles, int G, int b1, int b2) {
+    static const double tile_us[5] = {0.0, 0.6, 0.75, 1.2, 1.15};
+    const GemmShape shape = {mb, 8, 1, 1};
+    const int64_t units = (int64_t)tiles * ((M + 16 * mb - 1) / (16 * mb));
+    const int ks = slices_of_k(units, G, shape), turns = ((G + ks - 1) / ks + 7) / 8;
+    const int64_t rounds = (units * ks + kNumCU - 1) / kNumCU;
+    const double tile = (tile_us[b1] + tile_us[b2]) * (mb == 1 ? 1.0 : 1.09);
+    const double launches = b2 && !few_takes(std::max(b1, b2), std::min(b1, b2)) ? 2.0 : 1.0;
+    return (mb == 1 ? 1.5 : 5.0) + rounds * ((mb == 1 ? 4.0 : 5.0) * launches + tile * turns) +
+           (ks > 1 ? (mb == 1 ? 0.5 : 0.75) * ks * launches : 0.0);
+}
+
+// The same for 64-row (in one round) and 128-row workgroups of gemm_kernel.h: 8 us + 0.26 (0.43) a tile
+// per round, two streams are two launches, other widths 15 % more.
+GemmShape other_shape(int M, int tiles) {
+    return (int64_t)tiles * ((M + 63) / 64) <= kNumCU ? GemmShape{4, 8, 1, 1} : GemmShape{4, 4, 2, 1};
+}
+double other_us(int M, int tiles, int G, int streams, bool four_bit) {
+    const GemmShape other = other_shape(M, tiles);
+    const int rows = other.mb * other.mw * 16;
+    const int64_t units = (int64_t)tiles * ((M + rows - 1) / rows);
+    const int ks = slices_of_k(units, G, other);
+    const double per_tile = (other.mw == 1 ? 0.26 : 0.43) * (four_bit && streams == 1 ? 1.0 : 1.15);
+    return streams * (double)((units * ks + kNumCU - 1) / kNumCU) * (8.0 + per_tile * G / ks) + (ks > 1 ? 2.5 * ks : 0.0);
+}
+
+// Rows of A per workgroup and what the call then takes.  One or two 16-row blocks per wavefront with
+// eight k ways (gemm_few_kernel.h) while there are few rows, else four blocks: 64 rows per workgroup
+// with eight k ways while that fits the device in one round, else 128 rows (two m groups, four k ways);
+// further rows go to gridDim.y.  The tables plus staging take most of a CU's LDS, so one workgroup per
+// CU is resident.  FLUTE_GEMM_ROWS = 16, 32, 64 or 128 forces the shape (a tuning and test knob, like
+// FLUTE_GEMV_RW), 256 or 512 the many-row kernel.
+GemmShape choose_gemm_shape(int M, int tiles, int G, int b1, int b2, double &us) {
+    const int v = tuning().gemm_rows;
+    const double other = other_us(M, tiles, G, b2 ? 2 : 1, b1 == 4);
+    us = other;
+    if (v == 16) return {1, 8, 1, 1};
+    if (v == 32) return {2, 8, 1, 1};
+    if (v == 64) return {4, 8, 1, 1};
+    if (v == 128) return {4, 4, 2, 1};
+    const double few1 = few_us(1, M, tiles, G, b1, b2), few2 = few_us(2, M, tiles, G, b1, b2);
+    if (M <= 16 || (few1 <= few2 && few1 < other)) {
+        us = few1;
+        return {1, 8, 1, 1};
+    }
+    if (few2 < other) {
+        us = few2;
+        return {2, 8, 1, 1};
+    }
+    return other_shape(M, tiles);
+}
 
 // The residual coefficients of a call's weights, xb[i][m, r] = sum_k A[m, k] * resB[i][r, k] in fp32:
 // 16-row by 16-rank blocks in as many slices of K as the chip has CUs for, 512 columns (one step of a
@@ -123,7 +155,7 @@ int plan_lds(GemmParams &p, const GemmShape &shape) {
     const int ngrp = p.seg[0].gs >= 128 ? 1 : 128 / p.seg[0].gs;
     const bool perm = p.nstreams == 1 && p.bits[0] == 4 && ngrp <= 2 &&
                       !tuning().gemm_no_perm;
-    const int table_budget = (shape.mb == 1 ? 64 : 96) * 1024 / p.nstreams;
+    const int table_budget = 96 * 1024 / p.nstreams;
     int lds_tables = 0;
     for (int s = 0; s < p.nstreams; ++s) {
         const int entries = ngrp << (2 * p.bits[s]);
@@ -170,31 +202,18 @@ struct WidePlan {
     int ksplit;
 };
 
-// The many-row kernel or the others, and its shape.  Each form's time is a line in what it has to
+// The many-row kernel or the others (`us`), and its shape.  Each form's time is a line in what it has to
 // do, in microseconds, fitted to measurements (4-bit stream, bfloat16; `steps` = 64-k tiles of all
-// streams that a workgroup takes, `rounds` = workgroups / 256 CUs, rounded up):
-//   128-row workgroups of gemm_kernel.h   8 + 0.43 a tile (64-row ones 0.26) per round; two
-//                                         streams are two launches, other widths 15 % more
+// streams that a workgroup takes, `rounds` = workgroups / 256 CUs, rounded up; several weights in one
+// launch: `tiles` counts theirs):
 //   512-row workgroups                    14 a round + 0.95 ... 1.35 a step (the clock falls as the chip
 //                                         fills); slices of K cost 5 each (256 KB written, read)
-//   256-row workgroups                    14 a round + 0.65 ... 0.90 a step; slices 2.5 each
-// e.g. M = 1024, 4096 -> 12288: 120 / 92 / 118 us (estimated 107 / 94 / 133); M = 512: 74 / 61
-// (two slices) / 61; M = 512, 12288 -> 4096: 59 / 77 (four) / 65 (four), the others stay; two
-// streams (4, 1) at M = 1024, 4096 -> 12288: 263 / 165 / 190, at M = 192: 76 / - / 60 (two).
-// Calls that the 16- and 32-row workgroups serve in one round stay with them (M = 128,
-// 4096 -> 12288: 27 us there, 41 us here).
-// (several weights in one launch: `tiles` counts theirs; `other_us` is other_forms' estimate)
-double other_forms(int M, int tiles, int G, int streams, bool four_bit, const GemmShape &other) {
-    const int rows_other = other.mb * other.mw * 16;
-    const int64_t units_other = (int64_t)tiles * ((M + rows_other - 1) / rows_other);
-    int ks_other = 1;
-    while (units_other * ks_other * 2 <= kNumCU && ks_other < 4 && G / (ks_other * 2) >= other.kw * 2) ks_other *= 2;
-    const double per_tile = (other.mw == 1 ? 0.26 : 0.43) * (four_bit && streams == 1 ? 1.0 : 1.15);
-    return streams * (double)((units_other * ks_other + kNumCU - 1) / kNumCU) * (8.0 + per_tile * G / ks_other) +
-           (ks_other > 1 ? 5.0 : 0.0);
-}
-
-WidePlan choose_wide(int M, int tiles, int G, int streams, double other_us, const GemmShape &other) {
+//   256-row workgroups                    11 a round + 0.60 ... 0.80 a step; slices 2.5 each
+// e.g. 128-row, 512-row and 256-row workgroups at M = 1024, 4096 -> 12288: 120 / 92 / 118 us (estimated
+// 107 / 94 / 124); M = 512: 74 / 61 (two slices) / 61; M = 512, 12288 -> 4096: 59 / 77 (four) / 65
+// (four), the others stay; two streams (4, 1) at M = 1024, 4096 -> 12288: 263 / 165 / 190; (3, 3) at
+// M = 600, 4096 -> 4096: 32-row workgroups 80, 256-row ones in two slices 61 (estimated 64).
+WidePlan choose_wide(int M, int tiles, int G, int streams, double us_others) {
     {
         const int v = tuning().gemm_rows;
         if (v == 512 || v == 256) {
@@ -203,16 +222,16 @@ WidePlan choose_wide(int M, int tiles, int G, int streams, double other_us, cons
         }
         if (v) return {0, 1};
     }
-    if (other.mb < 4) return {0, 1};
-    double best = other_us;
+    if (M <= 16) return {0, 1};
+    double best = us_others;
     WidePlan plan = {0, 1};
     for (int rows = 512; rows >= 256; rows /= 2) {
         const int64_t units = (int64_t)tiles * ((M + rows - 1) / rows);
         for (int ks = 1; ks <= 8 && G / ks >= 8; ks *= 2) {
             const int64_t groups = units * ks, rounds = (groups + kNumCU - 1) / kNumCU;
             const double fill = groups < kNumCU ? (double)groups / kNumCU : 1.0;
-            const double step = rows == 512 ? 0.95 + 0.40 * fill : 0.65 + 0.25 * fill;
-            const double us = rounds * (14.0 + step * streams * ((G + ks - 1) / ks)) +
+            const double step = rows == 512 ? 0.95 + 0.40 * fill : 0.60 + 0.20 * fill;
+            const double us = rounds * ((rows == 512 ? 14.0 : 11.0) + step * streams * ((G + ks - 1) / ks)) +
                               (ks > 1 ? (rows == 512 ? 5.0 : 2.5) * ks : 0.0);
             if (us < best) {
                 best = us;
@@ -364,8 +383,10 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
     flute_status st;
     GemmParams p = {};
     p.nstreams = w->b2 > 0 ? 2 : 1;
-    p.bits[0] = w->b1;
-    p.bits[1] = w->b2;
+    // (the sum does not depend on the order of the streams beyond fp32 rounding: the wider first)
+    const bool few = shape.mb <= 2, swap = few && w->b2 > w->b1;
+    p.bits[0] = swap ? w->b2 : w->b1;
+    p.bits[1] = swap ? w->b1 : w->b2;
     p.M = M;
     p.G = w->K / 64;
     p.out_bf16 = act_dtype == FLUTE_BF16;
@@ -375,10 +396,10 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
         p.tile0[i] = i < count ? tiles : INT_MAX;
         if (i >= count) continue;
         GemmSeg &g = p.seg[i];
-        g.q[0] = (const uint8_t *)ws[i].q1;
-        g.q[1] = (const uint8_t *)ws[i].q2;
-        g.lut[0] = (const uint16_t *)ws[i].lut1;
-        g.lut[1] = (const uint16_t *)ws[i].lut2;
+        g.q[swap] = (const uint8_t *)ws[i].q1;
+        g.q[!swap] = (const uint8_t *)ws[i].q2;
+        g.lut[swap] = (const uint16_t *)ws[i].lut1;
+        g.lut[!swap] = (const uint16_t *)ws[i].lut2;
         g.gs = ws[i].group_size;
         g.lut_rows = ws[i].lut_rows;
         g.R = ws[i].R;
@@ -396,17 +417,7 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
     const int mchunks = (p.mblk_total + shape.mb * shape.mw - 1) / (shape.mb * shape.mw);
     const int64_t units = (int64_t)tiles * mchunks;
     p.mblk_pad = mchunks * shape.mb * shape.mw;
-    const int64_t cap = (int64_t)kNumCU * shape.wg_per_cu;
-    // K is split until the grid reaches one workgroup per CU, while every wavefront keeps
-    // two tiles or more; with four blocks of rows per wavefront at most four ways, because
-    // the workgroup that arrives last reads every 32 KB partial tile of its unit back
-    // (measured at M = 64: 12288 -> 4096 29.7 us four ways, 36.4 us eight ways; 4096 -> 4096
-    // 21.8 us four ways, 23.0 us two ways, 24.6 us eight ways).
-    const int max_split = shape.mb == 1 ? 64 : 4;
-    int ksplit = 1;
-    while (units * ksplit * 2 <= cap && ksplit * 2 <= max_split &&
-           p.G / (ksplit * 2) >= shape.kw * 2)
-        ksplit *= 2;
+    int ksplit = slices_of_k(units, p.G, shape);
     {
         const int v = tuning().gemm_ksplit;
         if (v >= 1 && v <= p.G) ksplit = v;
@@ -426,7 +437,11 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
 
     // ---- workspace: [partial images][xb][Ap] -----------------------------------------
     const size_t image = (size_t)shape.mw * shape.mb * 8 * 64 * 4;
-    const int zparts = ksplit * ((p.nstreams == 2 && shape.mb > 1) ? 2 : 1);
+    // Two streams where no kernel takes both (four blocks of rows per wavefront: they do not fit the
+    // register file; widths that no deployed weight has): one launch per stream, both write partial
+    // tiles and the last workgroup of the second launch folds everything, exactly as a K split does.
+    const bool per_stream = p.nstreams == 2 && !(few && few_takes(p.bits[0], p.bits[1]));
+    const int zparts = ksplit * (per_stream ? 2 : 1);
     const size_t p_floats = zparts > 1 ? (size_t)zparts * units * image : 0;
     const CoeffPlan coeff = plan_coeff(ws, count, M);
     size_t xb_floats = any_res ? coeff.floats() : 0;
@@ -456,15 +471,11 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
         p.rowshift = rowshift;
         return FLUTE_OK;
     };
-    // One block of rows per wavefront on the single-stream 4-bit fast path: the kernel reads
-    // A itself (16-byte pieces of a row, put into operand order in registers), so the
-    // pre-pass launch is dropped.  Needs 16-byte aligned rows; rotated rows are read the same way
-    // (the rotation can write the image itself, but only without a residual and row scales).
-    const bool direct = [&] {
-        const int ngrp = w->group_size >= 128 ? 1 : 128 / w->group_size;
-        return shape.mb == 1 && p.nstreams == 1 && w->b1 == 4 && ngrp <= 2 && !tuning().gemm_no_perm &&
-               !tuning().gemm_no_direct;
-    }();
+    // One block of rows per wavefront: the kernel reads A itself (16-byte pieces of a row, put into
+    // operand order in registers), so the pre-pass launch is dropped.  Needs 16-byte aligned rows;
+    // rotated rows are read the same way (the rotation can write the image itself, but only without a
+    // residual and row scales).
+    const bool direct = shape.mb == 1 && !tuning().gemm_no_direct;
     if (w->signs && !any_res && !scale_rows) {
         // the rotation writes the operand image itself: one launch instead of two
         FhtOperandOut image_out = {(uint32_t *)Ap, p.mblk_pad, (int)(w->lut_dtype == FLUTE_BF16), block_xor};
@@ -522,11 +533,6 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
         if (st != FLUTE_OK) return st;
     }
 
-    // Two streams with four blocks per wavefront: one launch per stream through the
-    // single-stream kernels (the two-stream kernel does not fit the register file at
-    // that size); both write partial tiles and the last workgroup of the second launch
-    // folds everything, exactly as a K split does.
-    const bool per_stream = p.nstreams == 2 && shape.mb > 1;
     const int passes = per_stream ? 2 : 1;
     const dim3 grid(tiles, mchunks, ksplit);
     for (int pass = 0; pass < passes; ++pass) {
@@ -541,13 +547,18 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
         }
         q.z_base = pass * ksplit;
         q.ztotal = passes * ksplit;
-        const int lds = plan_lds(q, shape);
-        FLUTE_REQUIRE(lds <= kLdsPerCU, FLUTE_ERR_UNSUPPORTED,
-                      "flute_gemm: %d bytes of LDS exceed the %d of one CU", lds, kLdsPerCU);
         const int bf16 = w->lut_dtype == FLUTE_BF16;
-        st = count > 1 ? gemm_launch_segs(bf16, shape.mb, shape.mw, q, grid, lds, stream)
-             : bf16    ? launch_gemm_shape<true, false>(shape.mb, shape.mw, q, grid, lds, stream)
-                       : launch_gemm_shape<false, false>(shape.mb, shape.mw, q, grid, lds, stream);
+        if (few) {
+            st = count > 1 ? (bf16 ? gemm_few_bf16_segs : gemm_few_f16_segs)(shape.mb, q, grid, stream)
+                           : (bf16 ? gemm_few_bf16 : gemm_few_f16)(shape.mb, q, grid, stream);
+        } else {
+            const int lds = plan_lds(q, shape);
+            FLUTE_REQUIRE(lds <= kLdsPerCU, FLUTE_ERR_UNSUPPORTED,
+                          "flute_gemm: %d bytes of LDS exceed the %d of one CU", lds, kLdsPerCU);
+            st = count > 1 ? gemm_launch_segs(bf16, shape.mb, shape.mw, q, grid, lds, stream)
+                 : bf16    ? launch_gemm_shape<true, false>(shape.mb, shape.mw, q, grid, lds, stream)
+                           : launch_gemm_shape<false, false>(shape.mb, shape.mw, q, grid, lds, stream);
+        }
         if (st != FLUTE_OK) return st;
     }
     workspace_done(stream);
@@ -570,19 +581,18 @@ GemmPlan plan_gemm(const flute_linear *ws, int count, int M) {
     const int streams = ws[0].b2 > 0 ? 2 : 1, G = ws[0].K / 64;
     bool widths = true, all = true;
     int tiles = 0;
-    int64_t bytes = 0;
     for (int i = 0; i < count; ++i) {
         const flute_linear &w = ws[i];
         widths &= w.b1 == ws[0].b1 && w.b2 == ws[0].b2;
         all &= w.group_size == ws[0].group_size && w.signs == ws[0].signs && w.awq == ws[0].awq &&
                w.rot_block == ws[0].rot_block;
         tiles += w.N / 128;
-        bytes += w.q1_bytes + (w.b2 > 0 ? w.q2_bytes : 0);
     }
     GemmPlan plan = {};
     if (!widths) return plan;
-    plan.shape = choose_gemm_shape(M, tiles, bytes, G, streams == 2, fast_stream(ws[0]));
-    plan.wide = choose_wide(M, tiles, G, streams, other_forms(M, tiles, G, streams, ws[0].b1 == 4, plan.shape), plan.shape);
+    double us = 0.0;
+    plan.shape = choose_gemm_shape(M, tiles, G, ws[0].b1, ws[0].b2, us);
+    plan.wide = choose_wide(M, tiles, G, streams, us);
     plan.together = plan.wide.rows || all;
     return plan;
 }

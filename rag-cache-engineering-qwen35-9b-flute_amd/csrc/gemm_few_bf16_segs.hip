@@ -1,0 +1,8 @@
+// The few-row LUT GEMM over bfloat16 LUTs, several weights in a launch.
+#include "gemm_few_launch.h"
+
+namespace flute {
+flute_status gemm_few_bf16_segs(int mb, const GemmParams &p, dim3 grid, hipStream_t stream) {
+    return launch_few_shape<true, true>(mb, p, grid, stream);
+}
+}  // namespace flute

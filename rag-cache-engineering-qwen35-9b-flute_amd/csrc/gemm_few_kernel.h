@@ -1,0 +1,446 @@
+// LUT GEMM for few rows (workgroups of 16 or 32 rows of A):  C[M, N] = A[M, K] @ (W1 (+ W2))^T, fp32
+// accumulate, one rounding.  The operands' layout is that of gemm_kernel.h: a lane's chunk of codes
+// is what it needs of the matrix instruction's row side, the weights never exist as a dense tile.
+//
+// Workgroup = eight wavefronts on one 128-row tile of the weight; wavefront w takes the K tiles w,
+// w + 8, ... of the workgroup's slice of K, for MB blocks of 16 rows of A, both streams of a tile one
+// after the other on the same activations.  What bounds it: such a launch is a few trips to memory and
+// through LDS around a loop of a few microseconds (M = 48, 12288 -> 4096, four slices of K: 5 us of
+// loop in a launch of 18), so a second stream costs its loop here and not a launch of its own, and the
+// eight wavefronts' sums cross LDS once, every thread adding the eight terms of the outputs it then
+// stores, instead of a tree of three steps with two barriers each and a totals tile behind it.
+#pragma once
+
+#include "gemm_kernel.h"
+
+namespace flute {
+
+// Lookup tables of a stream in LDS.  An entry holds `slots` copies, split evenly over the LUT groups
+// of the 128-row tile, so that the lanes of an instruction lie on different banks.  4 and 3 bits: an
+// entry is a pair of weights (a dword).  2 and 1 bits: the four weights of a byte (a nibble) of
+// codes, half an operand, which halves the lookups and their addresses.  4 bits: 256 bytes an entry,
+// table at LDS offset 0, so that one v_perm_b32 drops a code byte into the address.
+template <int B>
+struct FewTable {
+    static constexpr int entries = B == 4 ? 256 : B == 3 ? 64 : B == 2 ? 256 : B == 1 ? 16 : 0;
+    static constexpr int stride_log2 = B == 4 ? 8 : 7;
+    static constexpr int unit = B >= 3 ? 4 : 8;
+    static constexpr int slots = (1 << stride_log2) / unit;
+    static constexpr int bytes = entries << stride_log2;
+    static constexpr int stage = B * 1024;                       // one tile of codes
+};
+
+template <int B1, int B2, int MB>
+constexpr int few_lds_bytes() {
+    constexpr int loop = FewTable<B1>::bytes + FewTable<B2>::bytes + 8 * (FewTable<B1>::stage + FewTable<B2>::stage);
+    constexpr int sums = 8 * MB * 8 * 64 * 16 + 16;              // every wavefront's accumulators, a flag
+    return loop > sums ? loop : sums;
+}
+
+// What a thread contributes to a table: the LUT values its entries are made of, requested with the
+// kernel's first loads; `build` waits for them only.
+template <int B>
+struct FewLut {
+    uint32_t v[B == 4 ? 6 : B == 3 ? 2 : B == 2 ? 4 : 2];
+
+    // lanes per entry, and the LUT group of this lane's 16 bytes of an entry
+    static constexpr int lanes = B == 4 ? 16 : 8;
+    __device__ __forceinline__ void load(const GemmSeg &w, int s, int t, int lane, int wave) {
+        const int lg = __builtin_ctz((unsigned)w.gs);            // a power of two, 16 or more
+        const int ngrp = lg >= 7 ? 1 : 128 >> lg;
+        const int gl = ((lane & (lanes - 1)) * ngrp) / lanes;
+        const int row = min(lg >= 7 ? (t * 128) >> lg : t * ngrp + gl, w.lut_rows - 1);
+        const uint16_t *lr = w.lut[s] + ((size_t)row << B);
+        if constexpr (B == 4) {                                  // codes 32 * wave + 4 * it + lane / 16
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = lr[4 * i + (lane >> 4)];
+            v[4] = lr[2 * wave];
+            v[5] = lr[2 * wave + 1];
+        } else if constexpr (B == 3) {                           // code 8 * wave + lane / 8
+            v[0] = lr[lane >> 3];
+            v[1] = lr[wave];
+        } else {
+#pragma unroll
+            for (int i = 0; i < (1 << B); ++i) v[i] = lr[i];
+        }
+    }
+    __device__ __forceinline__ uint32_t of4(int i) const {       // B == 2
+        return (i & 2) ? ((i & 1) ? v[3] : v[2]) : ((i & 1) ? v[1] : v[0]);
+    }
+    __device__ __forceinline__ void build(unsigned char *table, int lane, int wave) const {
+        u4_t *const to = (u4_t *)table + lane;                   // an instruction writes 64 / lanes entries
+        if constexpr (B == 4) {
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                const uint32_t d = v[it & 3] | (v[4 + (it >> 2)] << 16);
+                to[(wave * 8 + it) * 64] = u4_t{d, d, d, d};
+            }
+        } else if constexpr (B == 3) {
+            const uint32_t d = v[0] | (v[1] << 16);
+            to[wave * 64] = u4_t{d, d, d, d};
+        } else if constexpr (B == 2) {
+#pragma unroll
+            for (int it = 0; it < 4; ++it) {
+                const int code = wave * 32 + it * 8 + (lane >> 3);
+                const uint32_t lo = of4(code & 3) | (of4((code >> 2) & 3) << 16);
+                const uint32_t hi = of4((code >> 4) & 3) | (of4(code >> 6) << 16);
+                to[(wave * 4 + it) * 64] = u4_t{lo, hi, lo, hi};
+            }
+        } else if (wave < 2) {
+            const int code = wave * 8 + (lane >> 3);
+            const uint32_t lo = ((code & 1) ? v[1] : v[0]) | (((code & 2) ? v[1] : v[0]) << 16);
+            const uint32_t hi = ((code & 4) ? v[1] : v[0]) | (((code & 8) ? v[1] : v[0]) << 16);
+            to[wave * 64] = u4_t{lo, hi, lo, hi};
+        }
+    }
+};
+
+// One stream of a workgroup's tile: its codes on their way from memory to the matrix operands.
+template <int B>
+struct FewStream {
+    u4_t raw[B];               // a tile on its way from memory, contiguous 1 KB rows
+    uint32_t Q[4 * B];         // this lane's chunk of the tile in work
+    uint32_t lb[4];            // table column of this lane for the rows (wx, v)
+    uint32_t wr[B], rd[B];     // staging: where a lane puts its piece of a row, where its chunk's pieces are
+    const uint8_t *p;
+
+    // A tile passes through LDS on its way (contiguous loads cost the address path a quarter of what
+    // loads of whole chunks do).  Piece i of chunk c = 4 * a + kg is q = B * c + i = 4 * B * a + m; it
+    // lies at m * 16 + (a ^ (m & 7)): lanes that write neighbouring pieces and lanes that read the
+    // chunks of neighbouring rows both meet different banks.
+    __device__ __forceinline__ void init(const GemmSeg &w, int s, int64_t tile, uint32_t table, uint32_t stage, int lane) {
+        typedef FewTable<B> T;
+        p = w.q[s] + tile * (1024 * B) + lane * 16;
+        const int rho = lane & 15, kg = lane >> 4, wx = rho >> 3;
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+            const uint32_t q = i * 64 + lane, m = q % (4 * B), a = q / (4 * B);
+            wr[i] = stage + (m * 16 + (a ^ (m & 7))) * 16;
+            const uint32_t mr = B * kg + i;
+            rd[i] = stage + (mr * 16 + ((uint32_t)rho ^ (mr & 7))) * 16;
+        }
+        const int lg = __builtin_ctz((unsigned)w.gs);
+        const int ngrp = lg >= 7 ? 1 : 128 >> lg;
+        const int reps = lg >= 7 ? T::slots : T::slots >> (7 - lg);
+        const int r = ngrp == 1 ? lane & (T::slots - 1) : ((kg * 8 + (rho & 7)) ^ (wx * 16)) & (reps - 1);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int gl = ngrp == 1 ? 0 : (wx * 64 + v * 16) >> lg;
+            lb[v] = table + (gl * reps + r) * T::unit;
+        }
+    }
+    __device__ __forceinline__ void load() {
+#pragma unroll
+        for (int i = 0; i < B; ++i) raw[i] = __builtin_nontemporal_load((const u4_t *)(p + i * 1024));
+    }
+    typedef __attribute__((address_space(3))) u4_t *LdsQuad;
+    __device__ __forceinline__ void put() const {
+#pragma unroll
+        for (int i = 0; i < B; ++i) *(LdsQuad)(uintptr_t)wr[i] = raw[i];
+    }
+    __device__ __forceinline__ void get() {
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+            const u4_t v = *(LdsQuad)(uintptr_t)rd[i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) Q[4 * i + e] = v[e];
+        }
+    }
+    // operand (rows v, d; half j of the tile)
+    __device__ __forceinline__ u4_t operand(int j, int v, int d) const {
+        if constexpr (B >= 3) {
+            return fetch_operand<B, B == 4>(Q, j, v, d, lb[v], FewTable<B>::stride_log2);
+        } else {
+            typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
+            typedef const __attribute__((address_space(3))) u2_t *LdsPair;
+            u4_t w;
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+                const int bit = 2 * B * ((2 * j + kt) * 16 + v * 4 + d * 2);       // four codes: 4 * B bits
+                const uint32_t code = __builtin_amdgcn_ubfe(Q[bit >> 5], bit & 31, 4 * B);
+                const u2_t two = *(LdsPair)(uintptr_t)((code << FewTable<B>::stride_log2) + lb[v]);
+                w[2 * kt] = two[0];
+                w[2 * kt + 1] = two[1];
+            }
+            return w;
+        }
+    }
+    // Half a tile: eight operands, MB products each.  The lookups run two pairs of operands ahead of
+    // the products that consume them, so that LDS latency hides behind matrix work.
+    template <int MB, bool BF16>
+    __device__ __forceinline__ void half(int j, const u4_t (&Aj)[MB], f4_t (&acc)[MB][8]) const {
+        constexpr int AHEAD = 2;
+        u4_t W[AHEAD + 1][2];
+#pragma unroll
+        for (int v = 0; v < AHEAD; ++v)
+#pragma unroll
+            for (int d = 0; d < 2; ++d) W[v][d] = operand(j, v, d);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if (v + AHEAD < 4)
+#pragma unroll
+                for (int d = 0; d < 2; ++d) W[(v + AHEAD) % (AHEAD + 1)][d] = operand(j, v + AHEAD, d);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+                    acc[mb][v * 2 + d] = mfma16<BF16>(W[v % (AHEAD + 1)][d], Aj[mb], acc[mb][v * 2 + d]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+};
+template <>
+struct FewStream<0> {};
+
+// B2 == 0: one stream (launches of one stream each may share a fold, p.z_base and p.ztotal).
+// SEGS: several weights in the launch.
+template <int MB, bool BF16, int B1, int B2, bool SEGS>
+__global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
+    static_assert(MB == 1 || MB == 2, "16 or 32 rows");
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int KW = 8, NT = 512;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int si = 0;
+    if constexpr (SEGS)
+        si = ((int)blockIdx.x >= p.tile0[1]) + ((int)blockIdx.x >= p.tile0[2]) + ((int)blockIdx.x >= p.tile0[3]);
+    const GemmSeg &w = p.seg[SEGS ? si : 0];
+    const int t = SEGS ? blockIdx.x - p.tile0[si] : blockIdx.x;
+    const int mb0 = blockIdx.y * MB;                   // first 16-row block
+    const int z = blockIdx.z;
+    const int rho = lane & 15, kg = lane >> 4;
+
+    const int gbeg = z * p.gper, gend = min(p.G, gbeg + p.gper);
+    const int g0 = gbeg + wave;
+    int left = g0 < gend ? (gend - g0 + KW - 1) / KW : 0;   // tiles of this wavefront
+    // A wavefront without tiles addresses the first one of the slice instead: the loads below are then
+    // unconditional like everyone's, and the compiler can count them.
+    const int g_first = left > 0 ? g0 : gbeg;
+
+    // ---- activations: the image (its blocks are padded to whole workgroups), or A itself (MB == 1 and
+    // rows of whole 16-byte pieces), whose pieces are put into operand order in registers ----------
+    const bool direct = MB == 1 && p.A8 != nullptr;
+    const int a_row = mb0 * 16 + rho;
+    const bool a_row_valid = a_row < p.M;
+    const int a_shift = direct && p.rowshift && a_row_valid ? p.rowshift[a_row] : 0;
+    const int64_t jstep = direct ? 4 : (int64_t)p.mblk_pad * 64, gstep = direct ? 8 : 2 * jstep;
+    const u4_t *ap = (direct ? p.A8 + (int64_t)(a_row_valid ? a_row : 0) * p.lda8 + kg : p.Ap + (int64_t)mb0 * 64 + lane) +
+                     (int64_t)g_first * gstep;
+    auto load_a = [&](u4_t (&Aj)[MB], const u4_t *src) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) Aj[mb] = src[mb * 64];
+    };
+    // (rows beyond M are zero; the activations are presented in the LUT's 16-bit type)
+    auto to_operand = [&](u4_t (&T)[MB]) {
+        if (!direct) return;
+        if constexpr (MB == 1) {
+            u4_t raw = T[0];
+            if (!a_row_valid) raw = u4_t{0u, 0u, 0u, 0u};
+            if (p.a_bf16 != (int)BF16) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint16_t lo16 = (uint16_t)(raw[q] & 0xffffu), hi16 = (uint16_t)(raw[q] >> 16);
+                    const float flo = ldexpf(p.a_bf16 ? bf2f(lo16) : h2f(lo16), -a_shift);
+                    const float fhi = ldexpf(p.a_bf16 ? bf2f(hi16) : h2f(hi16), -a_shift);
+                    raw[q] = (uint32_t)round_act(flo, BF16) | ((uint32_t)round_act(fhi, BF16) << 16);
+                }
+            }
+            T[0] = quad_transpose(raw, lane);
+        }
+    };
+
+    // ---- first loads, in the order they are waited for: LUT values, codes, activations ------------
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+    constexpr int tab2 = FewTable<B1>::bytes, stage0 = tab2 + FewTable<B2>::bytes;
+    constexpr int stage_wave = FewTable<B1>::stage + FewTable<B2>::stage;
+    const uint32_t stage = lds0 + stage0 + (uint32_t)wave * stage_wave;
+    FewLut<B1> lut1;
+    FewLut<B2 ? B2 : 1> lut2;
+    FewStream<B1> s1;
+    FewStream<B2> s2;
+    u4_t A0[MB], A1[MB];
+    lut1.load(w, 0, t, lane, wave);
+    if constexpr (B2 > 0) lut2.load(w, 1, t, lane, wave);
+    const int64_t tile = (int64_t)t * p.G + g_first;
+    s1.init(w, 0, tile, lds0, stage, lane);
+    if constexpr (B2 > 0) s2.init(w, 1, tile, lds0 + tab2, stage + FewTable<B1>::stage, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    s1.load();
+    if constexpr (B2 > 0) s2.load();
+    load_a(A0, ap);
+    load_a(A1, ap + jstep);
+    __builtin_amdgcn_sched_barrier(0);
+    lut1.build(smem, lane, wave);
+    if constexpr (B2 > 0) lut2.build(smem + tab2, lane, wave);
+    __syncthreads();
+
+    f4_t acc[MB][8];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[mb][i] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // ---- the K loop: codes a tile and a half ahead (through LDS), activations half a tile or more -------
+    auto next_codes = [&](bool more) {
+        s1.put();
+        if constexpr (B2 > 0) s2.put();
+        if (more) {                                     // else: a harmless reload
+            s1.p += KW * 1024 * B1;
+            if constexpr (B2 > 0) s2.p += KW * 1024 * B2;
+        }
+        s1.load();
+        if constexpr (B2 > 0) s2.load();
+    };
+    if (left > 0) next_codes(left > 1);
+    while (left > 0) {
+        // the two wavefronts of a SIMD (w and w + 4) take turns at the higher priority
+        if ((left + (wave >> 2)) & 1) __builtin_amdgcn_s_setprio(1);
+        else __builtin_amdgcn_s_setprio(0);
+        s1.get();
+        if constexpr (B2 > 0) s2.get();
+        __builtin_amdgcn_sched_barrier(0);
+        to_operand(A0);
+        s1.template half<MB, BF16>(0, A0, acc);
+        if constexpr (B2 > 0) s2.template half<MB, BF16>(0, A0, acc);
+        if (left > 1) ap += KW * gstep;
+        load_a(A0, ap);
+        // issue order activations -> codes: the wait for these activations at the top of the next
+        // round then does not include the codes'
+        __builtin_amdgcn_sched_barrier(0);
+        next_codes(left > 2);
+        __builtin_amdgcn_sched_barrier(0);
+        to_operand(A1);
+        s1.template half<MB, BF16>(1, A1, acc);
+        if constexpr (B2 > 0) s2.template half<MB, BF16>(1, A1, acc);
+        load_a(A1, ap + jstep);
+        __builtin_amdgcn_sched_barrier(0);
+        --left;
+    }
+    __builtin_amdgcn_s_setprio(0);
+
+    // ---- sums of the eight wavefronts ---------------------------------------------------------
+    // Four outputs of one row = one f4: accumulator i of lane (kg, rho) holds row rho, outputs
+    // (kg >> 1) * 64 + i * 8 + (kg & 1) * 4 ... + 3.  A wavefront's area is in that order, the lane's
+    // low bits XORed with the outputs' so that the sixteen (eight) threads that serve a row of C side
+    // by side read different banks.
+    __syncthreads();                                    // tables and staging are dead
+    f4_t *const red = (f4_t *)smem;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            red[(wave * MB + mb) * 512 + i * 64 + (lane ^ i ^ ((kg & 1) << 2))] = acc[mb][i];
+    __syncthreads();
+    constexpr int PW = 4 * MB;                          // outputs per thread: 16 * MB rows, 128 columns in all
+    const int ml = tid / (128 / PW), n_in = (tid % (128 / PW)) * PW;
+    float y[PW];
+#pragma unroll
+    for (int e = 0; e < MB; ++e) {
+        const int n = n_in + 4 * e, i = (n >> 3) & 7, lo = (n >> 2) & 1;
+        const f4_t *from = red + (ml >> 4) * 512 + i * 64 + ((((n >> 6) * 2 + lo) * 16 + (ml & 15)) ^ i ^ (lo << 2));
+        f4_t sum = from[0];
+#pragma unroll
+        for (int u = 1; u < 8; ++u) sum += from[u * MB * 512];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) y[4 * e + q] = sum[q];
+    }
+
+    // ---- across workgroups: partial sums and a ticket, the last arrival adds them in z order ---------
+    if (p.ztotal > 1) {
+        const int unit = blockIdx.y * gridDim.x + blockIdx.x, zmine = p.z_base + z;
+        constexpr int image = NT * PW;
+        const int64_t zstride = (int64_t)gridDim.x * gridDim.y * image;
+        float *const mine = p.P + (int64_t)unit * image + tid * 4;
+#pragma unroll
+        for (int e = 0; e < MB; ++e)
+            ws_store16(mine + zmine * zstride + e * (NT * 4), f4_t{y[4 * e], y[4 * e + 1], y[4 * e + 2], y[4 * e + 3]});
+        ws_stores_done();
+        __syncthreads();
+        int *const flag = (int *)(smem + 8 * MB * 8 * 64 * 16);
+        if (tid == 0) {
+            const int old = __hip_atomic_fetch_add(p.tickets + unit, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *flag = old == p.ztotal - 1;
+            if (old == p.ztotal - 1)
+                __hip_atomic_store(p.tickets + unit, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        if (!*flag) return;
+        f4_t sum[MB];
+#pragma unroll
+        for (int e = 0; e < MB; ++e) sum[e] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int z0 = 0; z0 < p.ztotal; z0 += 4) {      // past the last slice: that one again, not added
+#pragma unroll
+            for (int e = 0; e < MB; ++e) {
+                const float *s[4];
+                f4_t v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s[i] = mine + min(z0 + i, p.ztotal - 1) * zstride + e * (NT * 4);
+                ws_load16x4(s[0], s[1], s[2], s[3], v[0], v[1], v[2], v[3]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (z0 + i < p.ztotal) sum[e] += v[i];
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < MB; ++e)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) y[4 * e + q] = sum[e][q];
+    }
+
+    // ---- epilogue: scale back, residual, bias, one rounding, store --------------------------------
+    const int m = blockIdx.y * (16 * MB) + ml;
+    if (m >= p.M) return;
+    const int n0 = t * 128 + n_in;
+    if (p.rowshift) {                                   // exact
+        const int sh = p.rowshift[m];
+#pragma unroll
+        for (int e = 0; e < PW; ++e) y[e] = ldexpf(y[e], sh);
+    }
+    if (w.R > 0 && w.vec_res) {                         // eight ranks a step, all its loads at once
+        const float *xr = w.xb + (size_t)m * w.R;
+        for (int r0 = 0; r0 < w.R; r0 += 8) {
+            u4_t a[PW];
+#pragma unroll
+            for (int e = 0; e < PW; ++e) a[e] = *(const u4_t *)(w.resA + (int64_t)(n0 + e) * w.R + r0);
+            const f4_t c0 = *(const f4_t *)(xr + r0), c1 = *(const f4_t *)(xr + r0 + 4);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const float c = r < 4 ? c0[r & 3] : c1[r & 3];
+#pragma unroll
+                for (int e = 0; e < PW; ++e) {
+                    const uint16_t h = (uint16_t)(a[e][r >> 1] >> (16 * (r & 1)));
+                    y[e] = fmaf(c, p.out_bf16 ? bf2f(h) : h2f(h), y[e]);
+                }
+            }
+        }
+    } else if (w.R > 0) {
+        const float *xr = w.xb + (size_t)m * w.R;
+        for (int r = 0; r < w.R; ++r) {
+            const float c = xr[r];
+#pragma unroll
+            for (int e = 0; e < PW; ++e)
+                y[e] = fmaf(c, load_act(w.resA, (int64_t)(n0 + e) * w.R + r, p.out_bf16), y[e]);
+        }
+    }
+    if (w.bias) {
+#pragma unroll
+        for (int e = 0; e < PW; ++e) y[e] += load_act(w.bias, n0 + e, p.out_bf16);
+    }
+    uint32_t o[PW / 2];
+#pragma unroll
+    for (int e = 0; e < PW / 2; ++e)
+        o[e] = (uint32_t)round_act(y[2 * e], p.out_bf16) | ((uint32_t)round_act(y[2 * e + 1], p.out_bf16) << 16);
+    uint16_t *const dst = (uint16_t *)w.C + (size_t)m * w.ldc + n0;
+    if (w.vec_store) {
+        if constexpr (MB == 2) *(u4_t *)dst = u4_t{o[0], o[1], o[2], o[3]};
+        else *(uint2 *)dst = make_uint2(o[0], o[1]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < PW / 2; ++e) {
+            dst[2 * e] = (uint16_t)o[e];
+            dst[2 * e + 1] = (uint16_t)(o[e] >> 16);
+        }
+    }
+}
+
+}  // namespace flute

@@ -87,9 +87,9 @@ struct GemmParams {
     int z_base, ztotal;    // partial tiles: this launch writes [z_base, z_base + gridDim.z) of
                            // ztotal (several launches, one per stream, may share a fold)
     int out_bf16;          // dtype of C, resA, bias
-    const u4_t *A8;        // direct mode: A itself, rows of lda8 16-byte pieces, no pre-pass
+    const u4_t *A8;        // 16-row workgroups: A itself, rows of lda8 16-byte pieces, no pre-pass (or NULL)
     int64_t lda8;
-    int a_bf16;            // dtype of A in direct mode
+    int a_bf16;            // dtype of A there
     const int *rowshift;   // [M] or NULL: row m of the operands holds A[m] * 2^-rowshift[m]
 };
 
@@ -413,7 +413,7 @@ __device__ __forceinline__ void half_mma(const uint32_t (&Q)[4 * B], int j, cons
     }
 }
 
-// Direct mode of the one-block fast path: a lane has loaded eight consecutive k of its row
+// A itself instead of the image (16-row workgroups, gemm_few_kernel.h): a lane has loaded eight consecutive k of its row
 // (piece c = lane >> 4 of the 32-k half tile), the matrix cores want the pairs
 // (2*kg, 2*kg + 1) of all four pieces.  With the four lanes that share a row (16 apart)
 // this is a 4 x 4 transpose of dwords: in round r every lane offers dword (kg + r) & 3 and
@@ -437,10 +437,7 @@ __device__ __forceinline__ u4_t quad_transpose(u4_t v, int lane) {
     return out;
 }
 
-// B1 > 0: single stream of that width.  B1 == 0: widths read from the
-// parameters, one or two streams.
-// DIRECT (one block per wavefront on the fast path only): the activations are read from A
-// itself and put into operand order in registers; no pre-pass launch.
+// One stream of B1-bit codes.
 // Block mb of an activation half: 16 bytes per lane at src + mb KB, as a statement the compiler
 // does not take for a load (no wait of its own follows).
 __device__ __forceinline__ void lean_load16(u4_t &dst, const u4_t *src, int mb) {
@@ -457,11 +454,9 @@ __device__ __forceinline__ void lean_load16(u4_t &dst, const u4_t *src, int mb) 
 // into LDS (global_load_lds_dwordx4), which frees the sixteen registers a tile in flight would
 // hold; the compiler cannot count such loads next to its own (it answers one in flight with
 // vmcnt(0) in front of the next use of any loaded register), hence all or nothing.
-template <int MB, int KW, int MW, bool BF16, int B1, bool PERM = false, bool DIRECT = false,
-          bool LEAN = false, bool SEGS = false>
+template <int MB, int KW, int MW, bool BF16, int B1, bool PERM = false, bool LEAN = false, bool SEGS = false>
 __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) {
-    static_assert(!DIRECT || (PERM && MB == 1), "direct activations: one block, fast path");
-    static_assert(!LEAN || (PERM && !DIRECT && MB >= 2 && B1 == 4), "lean loop: fast path, operand image");
+    static_assert(!LEAN || (PERM && MB >= 2 && B1 == 4), "lean loop: fast path, operand image");
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int NT = 64 * KW * MW;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -484,34 +479,13 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
     const bool active = mb0 < p.mblk_total;            // whole wavefront
     const int g0 = gbeg + kw;
     int left = (active && g0 < gend) ? (gend - g0 + KW - 1) / KW : 0;   // tiles of this wavefront
-    // u4 units between the halves of a tile (direct mode: 32 k of a row are four pieces)
-    const int64_t jstep = DIRECT ? 4 : (int64_t)p.mblk_pad * 64;
+    const int64_t jstep = (int64_t)p.mblk_pad * 64;    // u4 units between the halves of a tile
     // Ap is padded to whole workgroups of blocks (zeros), so every block index below
     // gridDim.y * MW * MB is loadable.
     // A wavefront without tiles addresses the first tile of the K range instead: its
     // loads below are then unconditional like everyone's, and the compiler can count them.
     const int g_first = left > 0 ? g0 : gbeg;
-    const int a_row = mb0 * 16 + rho;                  // direct mode: this lane's row of A
-    const bool a_row_valid = a_row < p.M;
-    const int a_shift = (DIRECT && p.rowshift && a_row_valid) ? p.rowshift[a_row] : 0;
-    const u4_t *ap = DIRECT
-        ? p.A8 + (int64_t)(a_row_valid ? a_row : 0) * p.lda8 + (int64_t)g_first * 8 + kg
-        : p.Ap + ((int64_t)g_first * 2 * p.mblk_pad + mb0) * 64 + lane;
-    // direct mode: raw piece -> operand (rows beyond M are zero; the activations are
-    // presented in the LUT's 16-bit type)
-    auto operand_of = [&](u4_t raw) -> u4_t {
-        if (!a_row_valid) raw = u4_t{0u, 0u, 0u, 0u};
-        if (p.a_bf16 != (int)BF16) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint16_t lo16 = (uint16_t)(raw[q] & 0xffffu), hi16 = (uint16_t)(raw[q] >> 16);
-                const float flo = ldexpf(p.a_bf16 ? bf2f(lo16) : h2f(lo16), -a_shift);
-                const float fhi = ldexpf(p.a_bf16 ? bf2f(hi16) : h2f(hi16), -a_shift);
-                raw[q] = (uint32_t)round_act(flo, BF16) | ((uint32_t)round_act(fhi, BF16) << 16);
-            }
-        }
-        return quad_transpose(raw, lane);
-    };
+    const u4_t *ap = p.Ap + ((int64_t)g_first * 2 * p.mblk_pad + mb0) * 64 + lane;
     auto load_a = [&](u4_t (&Aj)[MB], const u4_t *src) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) Aj[mb] = src[mb * 64];
@@ -606,20 +580,16 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
             }
         }
     } else {
-        for (int s = 0; s < p.nstreams; ++s) {
-            const int b = B1 > 0 ? B1 : p.bits[s];
-            const int rl = p.rep_log2[s];
-            const int total = ngrp << (2 * b + rl);
-            uint32_t *tab = (uint32_t *)(smem + p.tab_off[s]);
-            const uint16_t *lut = w.lut[s];
-            for (int i = tid; i < total; i += NT) {
-                const int code = (i >> rl) & ((1 << (2 * b)) - 1);
-                const int gl = i >> (rl + 2 * b);
-                int row = w.gs >= 128 ? (t * 128) / w.gs : t * ngrp + gl;
-                row = min(row, w.lut_rows - 1);
-                const uint16_t *lr = lut + ((size_t)row << b);
-                tab[i] = (uint32_t)lr[code & ((1 << b) - 1)] | ((uint32_t)lr[code >> b] << 16);
-            }
+        const int rl = p.rep_log2[0];
+        const int total = ngrp << (2 * B1 + rl);
+        uint32_t *tab = (uint32_t *)(smem + p.tab_off[0]);
+        for (int i = tid; i < total; i += NT) {
+            const int code = (i >> rl) & ((1 << (2 * B1)) - 1);
+            const int gl = i >> (rl + 2 * B1);
+            int row = w.gs >= 128 ? (t * 128) / w.gs : t * ngrp + gl;
+            row = min(row, w.lut_rows - 1);
+            const uint16_t *lr = w.lut[0] + ((size_t)row << B1);
+            tab[i] = (uint32_t)lr[code & ((1 << B1) - 1)] | ((uint32_t)lr[code >> B1] << 16);
         }
     }
     if constexpr (LEAN) {
@@ -672,7 +642,7 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
 
             uint32_t Q[16];
             constexpr int64_t qstep = (int64_t)KW * 4096;
-            const int64_t astep = DIRECT ? (int64_t)KW * 8 : (int64_t)KW * 2 * p.mblk_pad * 64;
+            const int64_t astep = (int64_t)KW * 2 * p.mblk_pad * 64;
             auto stage_write = [&]() {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -826,12 +796,7 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
                 else __builtin_amdgcn_s_setprio(0);
                 stage_read();                             // this tile's chunk
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (DIRECT) {
-                    const u4_t T0[1] = {operand_of(A0[0])};
-                    half_mma<4, MB, BF16, true>(Q, 0, T0, acc, lb, 8);
-                } else {
-                    half_mma<4, MB, BF16, true>(Q, 0, A0, acc, lb, 8);
-                }
+                half_mma<4, MB, BF16, true>(Q, 0, A0, acc, lb, 8);
                 if (left > 1) ap += astep;
                 load_a(A0, ap);                           // half a tile ahead of its use
                 // issue order activations -> tile: the wait for these activations at the
@@ -841,19 +806,14 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
                 if (left > 2) tp += qstep;
                 load_tile();                              // the tile after it
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (DIRECT) {
-                    const u4_t T1[1] = {operand_of(A1[0])};
-                    half_mma<4, MB, BF16, true>(Q, 1, T1, acc, lb, 8);
-                } else {
-                    half_mma<4, MB, BF16, true>(Q, 1, A1, acc, lb, 8);
-                }
+                half_mma<4, MB, BF16, true>(Q, 1, A1, acc, lb, 8);
                 load_a(A1, ap + jstep);
                 __builtin_amdgcn_sched_barrier(0);
                 --left;
             }
             }
             __builtin_amdgcn_s_setprio(0);
-        } else if constexpr (B1 > 0) {
+        } else {
             uint32_t lb[4];
             table_bases(lb, 0, B1);
             const int cs = p.rep_log2[0] + 2;
@@ -887,48 +847,6 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
                 if (--left == 0) break;
                 step(Qb, Qa, left > 1);
                 --left;
-            }
-        } else {
-            for (int g = gbeg + kw; g < gend; g += KW) {
-                u4_t A0[MB], A1[MB];
-                const u4_t *ap = p.Ap + ((int64_t)g * 2 * p.mblk_pad + mb0) * 64 + lane;
-                load_a(A0, ap);
-                load_a(A1, ap + jstep);
-                for (int s = 0; s < p.nstreams; ++s) {
-                    uint32_t lb[4];
-                    const int cs = p.rep_log2[s] + 2;
-                    const int64_t tile = (int64_t)t * p.G + g;
-                    switch (p.bits[s]) {
-                        case 1: {
-                            uint32_t Q[4];
-                            table_bases(lb, s, 1);
-                            load_chunk<1>(Q, w.q[s] + (tile * 64 + th) * (16 * 1));
-                            half_mma<1, MB, BF16>(Q, 0, A0, acc, lb, cs);
-                            half_mma<1, MB, BF16>(Q, 1, A1, acc, lb, cs);
-                        } break;
-                        case 2: {
-                            uint32_t Q[8];
-                            table_bases(lb, s, 2);
-                            load_chunk<2>(Q, w.q[s] + (tile * 64 + th) * (16 * 2));
-                            half_mma<2, MB, BF16>(Q, 0, A0, acc, lb, cs);
-                            half_mma<2, MB, BF16>(Q, 1, A1, acc, lb, cs);
-                        } break;
-                        case 3: {
-                            uint32_t Q[12];
-                            table_bases(lb, s, 3);
-                            load_chunk<3>(Q, w.q[s] + (tile * 64 + th) * (16 * 3));
-                            half_mma<3, MB, BF16>(Q, 0, A0, acc, lb, cs);
-                            half_mma<3, MB, BF16>(Q, 1, A1, acc, lb, cs);
-                        } break;
-                        default: {
-                            uint32_t Q[16];
-                            table_bases(lb, s, 4);
-                            load_chunk<4>(Q, w.q[s] + (tile * 64 + th) * (16 * 4));
-                            half_mma<4, MB, BF16>(Q, 0, A0, acc, lb, cs);
-                            half_mma<4, MB, BF16>(Q, 1, A1, acc, lb, cs);
-                        } break;
-                    }
-                }
             }
         }
     }

@@ -141,6 +141,28 @@ def test_gemm_dual_stream_fp16(M, N, K, bits, gs, bits2, rank, bias):
     assert torch.equal(y, _dual(w, x).cpu())
 
 
+@pytest.mark.parametrize("bits,bits2", [(4, 0), (3, 0), (2, 0), (1, 0), (4, 1), (1, 4), (3, 3), (2, 4), (3, 2), (4, 4), (1, 2)])
+@pytest.mark.parametrize("M,N,K,gs,rows,slices", [
+    (1, 128, 64, 128, "16", None),      # one tile of K: seven wavefronts without one
+    (16, 256, 576, 16, "16", "2"),      # nine tiles in slices of five and four
+    (17, 128, 1088, 64, "16", "3"),     # the second block holds one row
+    (31, 256, 704, 32, "32", None),     # eleven tiles over eight wavefronts
+    (33, 384, 1024, 256, "32", "4"),    # two tiles share a LUT row, the last has its own
+])
+def test_gemm_few_row_workgroups(tuning_env, M, N, K, gs, rows, slices, bits, bits2):
+    """16- and 32-row workgroups, every width alone and the pairs of one launch and of two, at the
+    edges of their tiles.  The sums are fp32 over exact 16-bit weights, so what is left is the one
+    rounding of the output (2^-11 of a value at most): TOL."""
+    tuning_env("FLUTE_GEMM_ROWS", rows)
+    if slices:
+        tuning_env("FLUTE_GEMM_KSPLIT", slices)
+    w = make_weight(N, K, bits, gs, seed=M + bits, bits2=bits2, rank=8, bias=True, device=DEV)
+    x = make_x(M, K, seed=5)
+    y = _dual(w, x).cpu()
+    assert rel_l2(y, _exact(w, x).half()) <= TOL
+    assert torch.equal(y, _dual(w, x).cpu())
+
+
 @pytest.mark.parametrize("lut_dtype,act_dtype", [(torch.bfloat16, torch.bfloat16),
                                                  (torch.float16, torch.bfloat16)])
 def test_gemm_dtype_mixes(lut_dtype, act_dtype):
