@@ -583,25 +583,29 @@ flute_status launch_fast4_grid(const Plan &plan, int gx, hipStream_t stream) {
     return FLUTE_OK;
 }
 
+// A grid of several rounds of (four-wavefront) workgroups: as many workgroups as are resident at
+// once walk over the row slices instead, which stages the activations once per workgroup and lets a
+// slice's first loads travel under the previous slice's last products.  Their number, or 0.
+int walking_grid(Plan &plan) {
+    // three workgroups per CU is what the kernel's registers allow (3 wavefronts per SIMD)
+    const int per_cu = tuning().gemv4_walk >= 0 ? (tuning().gemv4_walk < 3 ? tuning().gemv4_walk : 3) : 3;
+    const int resident = per_cu * kNumCU;
+    if (per_cu == 0 || plan.p.split != 1 || !(plan.p.nsegs == 1 || plan.p.silu_mul) ||
+        plan.lds_bytes * per_cu > (size_t)kLdsPerCU || plan.grid_x <= resident)
+        return 0;
+    plan.p.slices = plan.grid_x;
+    plan.p.xcd_runs = tuning().gemv_xcd && resident % 8 == 0;
+    return resident;
+}
+
 template <int LPGL, int NW, int PF, bool BF16>
 flute_status launch_fast4(Plan &plan, hipStream_t stream) {
-    // A grid of several rounds of workgroups: as many workgroups as are resident at once walk
-    // over the row slices instead, which stages the activations once per workgroup and lets a
-    // slice's first loads travel under the previous slice's last products.
-    int gx = plan.grid_x;
     plan.p.slices = 0;
     if constexpr (NW == 4) {                     // (eight-wavefront workgroups serve short grids only)
-        // three workgroups per CU is what the kernel's registers allow (3 wavefronts per SIMD)
-        const int per_cu = tuning().gemv4_walk >= 0 ? (tuning().gemv4_walk < 3 ? tuning().gemv4_walk : 3) : 3;
-        const int resident = per_cu * kNumCU;
-        if (per_cu > 0 && plan.p.split == 1 && (plan.p.nsegs == 1 || plan.p.silu_mul) &&
-            plan.lds_bytes * per_cu <= (size_t)kLdsPerCU && gx > resident) {
-            plan.p.slices = gx;
-            plan.p.xcd_runs = tuning().gemv_xcd && resident % 8 == 0;
+        if (const int resident = walking_grid(plan))
             return launch_fast4_grid<LPGL, NW, PF, BF16, true>(plan, resident, stream);
-        }
     }
-    return launch_fast4_grid<LPGL, NW, PF, BF16, false>(plan, gx, stream);
+    return launch_fast4_grid<LPGL, NW, PF, BF16, false>(plan, plan.grid_x, stream);
 }
 
 // Loads a lane keeps in flight in the lean kernel: 4 when that divides the loads of a
@@ -617,6 +621,12 @@ int pick_prefetch(const Plan &plan, int nw) {
     const int pf = tuning().gemv4_pf;
     if ((pf == 2 || pf == 4) && u % pf == 0) return pf;
     return u % 4 == 0 ? 4 : 2;
+}
+
+// What the lean kernel takes besides: any whole number of loads, one or more per wavefront.
+bool ragged_fits(const Plan &plan, int nw) {
+    const int gpi = 64 >> plan.p.lpg_log2;
+    return (nw == 4 || nw == 8) && plan.p.gs_tiles % gpi == 0 && plan.p.gs_tiles / gpi >= nw;
 }
 
 template <int LPGL, int NW, bool BF16>
@@ -678,6 +688,24 @@ flute_status launch_width(Plan &plan, hipStream_t stream) {
             case 5: return launch_fast4_shape<5, BF16>(plan, nw, stream);
             default: return launch_fast4_shape<6, BF16>(plan, nw, stream);
         }
+    }
+    const bool lean = one_group && one_input && es == 7 && luts_aligned && tuning().gemv_no_fast == 0;
+    // K ranges that do not divide into equal, even numbers of loads: the lean kernel's ragged form, which
+    // is the faster one wherever it fits.  One token, the general kernel and this one, the launch alone:
+    //   3968 -> 2 x 11520, (1, 4) bits   30.0 -> 22.8 us      11520 -> 3968             25.7 -> 16.2
+    //   2944 -> 2 x 11904, rotated       23.5 -> 19.0         11904 -> 2944, rotated    20.6 -> 17.4
+    //   1152 -> 2 x 4480, (2, 4) bits    19.2 -> 14.8         4480 -> 1152              12.8 -> 9.1
+    //   2432 -> 2 x 2304, (3, 3), rotated 20.8 -> 16.1        4032 -> 2048, 512, 512    9.5 -> 6.4
+    //   2112 -> 144000: the call 57.9 -> 33.1 (a walking grid), (3, 3) bits 81.3 -> 64.2
+    if (lean && (bits == 4 || plan.pair) && pick_prefetch(plan, nw) == 0 && ragged_fits(plan, nw)) {
+        plan.p.slices = 0;
+        int gx = plan.grid_x;
+        if (bits == 4 && nw == 4)
+            if (const int resident = walking_grid(plan)) gx = resident;
+        const int pair = bits == 4 ? 0 : plan.pair;
+        return (pair == 0 || pair == 14 || pair == 41)
+                   ? launch_gemv_ragged_a(plan.p, pair, gx, nw, plan.lds_bytes, BF16, stream)
+                   : launch_gemv_ragged_b(plan.p, pair, gx, nw, plan.lds_bytes, BF16, stream);
     }
     if (plan.pair && one_group && one_input && es == 7 && luts_aligned &&
         (nw == 4 || (nw == 8 && plan.p.lpg_log2 <= 5)) && pick_prefetch(plan, nw) != 0 &&

@@ -245,8 +245,14 @@ constexpr int kKGroupPieces = 8;
 // refill can be back; the deeper ring costs four registers.  The host picks it when a wavefront's
 // loads are a multiple of eight ((1, 4) at 4096 -> 12288: 10.5 -> 9.7 us; with the 1-bit stream
 // second it measured no gain, so the host puts it first).
+// RAGGED: the wavefronts' loads may differ in number and need not come in PFs (any K range of whole
+// loads, a load or more per wavefront).  A refill past a wavefront's last load reads that one again,
+// what is left behind the last full ring is taken in pairs, a load without a partner against zeros
+// (in both operands: nothing else can come out of it), and the first loads of the next pass go out
+// behind the loop instead of under its last products.  What it measures against the general kernel
+// stands at the rule that picks it (launch_width, gemv.hip).
 template <int LPGL, int NW, int PF, bool BF16, bool WALK = false, int BA = 4, int BB = 4, bool KG = false,
-          bool DEEP = false>
+          bool DEEP = false, bool RAGGED = false>
 __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr int ES = 7;
@@ -269,6 +275,7 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
     static_assert(!TWO || !WALK, "walking grids: the (4, 4) kernel");
     static_assert(!KG || (!TWO && !WALK), "K-grouped LUTs: one 4-bit stream, one slice per workgroup");
     static_assert(!DEEP || (TWO && PF == 4 && BA == 1), "the deep ring is for a 1-bit first stream");
+    static_assert(!RAGGED || (!KG && !DEEP), "ragged K ranges: tables along N, rings of PF loads");
     constexpr int DA = (DEEP && BA == 1) ? 2 * PF : PF;  // loads in flight, first / second stream
     constexpr int DB = (DEEP && BB == 1) ? 2 * PF : PF;
     constexpr int KG_GROUP = RW * 64 + (RW / 8) * 64;   // LDS bytes of one K group's rows
@@ -335,7 +342,10 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
     const int s = blockIdx.y;
     const int g_lo = s * p.gs_tiles;
     const int units = p.gs_tiles / GPI;
-    const int my_units = units / NW;                // the host makes this exact, even, >= PF
+    // (not RAGGED: the host makes this exact, even, >= PF; RAGGED: one or more)
+    const int my_units = RAGGED ? (units - w + NW - 1) / NW : units / NW;
+    const int most_units = RAGGED ? (units + NW - 1) / NW : my_units;
+    auto unit_at = [&](int n) -> int { return RAGGED ? min(n, my_units - 1) : n; };
     const int k0 = g_lo * 64, kc = p.gs_tiles * 64;
     const int G = p.K >> 6;
 
@@ -387,7 +397,7 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
 #pragma unroll
         for (int n = 0; n < DA; ++n) {
             if (n >= from) {
-                qq[n] = load_idx<BA>(qr + (size_t)n * step + lane0);
+                qq[n] = load_idx<BA>(qr + (size_t)unit_at(n) * step + lane0);
                 __builtin_amdgcn_sched_barrier(0);  // issue order = consumption order
             }
         }
@@ -567,7 +577,7 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
         const int m = i * UPL + xu;
         return m < my_units ? (w + m * NW) * (64 * GPI) + xp * 8 : -1;
     };
-    const int x_loads = (my_units + UPL - 1) / UPL;
+    const int x_loads = (most_units + UPL - 1) / UPL;
     const bool x_short = x_loads <= XV;             // uniform
     // Equal rotation blocks that fit a unit of K (the block-128 form) are transformed by the
     // wavefront that consumes the unit, in the registers its pieces arrive in: sixteen lanes
@@ -609,7 +619,7 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int n = 0; n < PF0; ++n) {
-            q[n] = load_idx<BA>(qrow + (size_t)n * step + lane0);
+            q[n] = load_idx<BA>(qrow + (size_t)unit_at(n) * step + lane0);
             __builtin_amdgcn_sched_barrier(0);
         }
         FLUTE_GEMV_STAMP(1);                        // (waits for the scalar loads: the LUT row is in)
@@ -686,7 +696,7 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
         // index loads travel while it runs.
 #pragma unroll
         for (int n = 0; n < PF0; ++n) {
-            q[n] = load_idx<BA>(qrow + (size_t)n * step + lane0);
+            q[n] = load_idx<BA>(qrow + (size_t)unit_at(n) * step + lane0);
             __builtin_amdgcn_sched_barrier(0);
         }
         xshift = stage_x<BF16>(p, staged_x, staged_signs, staged_awq, lds, k0, kc, tid, NT);
@@ -756,12 +766,18 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
         const int a0 = u0 * (32 * GPI) + xnat, a1 = u1 * (32 * GPI) + xnat;
         return (gv_u4_t){xs32[a0], xs32[a0 + 4], xs32[a1], xs32[a1 + 4]};
     };
+    // (RAGGED: the load without a partner)
+    auto operand_b_alone = [&](int m0) -> gv_u4_t {
+        const gv_u4_t both = operand_b(m0, m0);
+        return (gv_u4_t){both[0], both[1], 0u, 0u};
+    };
     // per row group v, eight lookups feed two matrix products; pair pp = v * 4 + d * 2 + s2 of a
     // quarter, an operand is (s2 = 0, 1) of both units
     // (K-grouped LUT: ga, gb = LDS byte offsets of the two units' K groups plus this lane's rows)
-    auto unit_pair = [&](const auto &qa, const auto &qb, gv_u4_t Bop, uint32_t tslot, auto width,
-                         uint32_t ga = 0, uint32_t gb = 0) {
+    auto unit_products = [&](const auto &qa, const auto &qb, gv_u4_t Bop, uint32_t tslot, auto width, uint32_t ga,
+                             uint32_t gb, auto alone) {
         constexpr int B = decltype(width)::value;
+        constexpr bool ALONE = decltype(alone)::value;          // the second unit is not there
         if constexpr (KG) {
             // Row group v needs sixteen 16-bit reads (dword v of both units: four bytes of two
             // codes).  Their addresses are formed while the reads of group v - 1 are in flight, and
@@ -823,8 +839,11 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
                 // byte v of the quarter: low nibble = the four weights of row 2 v, high nibble = row 2 v + 1
                 const pair_t a0 = *(LdsPair)((__builtin_amdgcn_ubfe(wa, 8 * v, 4) << 8) + tslot);
                 const pair_t a1 = *(LdsPair)((__builtin_amdgcn_ubfe(wa, 8 * v + 4, 4) << 8) + tslot);
-                const pair_t b0 = *(LdsPair)((__builtin_amdgcn_ubfe(wb, 8 * v, 4) << 8) + tslot);
-                const pair_t b1 = *(LdsPair)((__builtin_amdgcn_ubfe(wb, 8 * v + 4, 4) << 8) + tslot);
+                pair_t b0 = {0u, 0u}, b1 = {0u, 0u};
+                if constexpr (!ALONE) {
+                    b0 = *(LdsPair)((__builtin_amdgcn_ubfe(wb, 8 * v, 4) << 8) + tslot);
+                    b1 = *(LdsPair)((__builtin_amdgcn_ubfe(wb, 8 * v + 4, 4) << 8) + tslot);
+                }
                 const gv_u4_t A0 = {a0.x, a0.y, b0.x, b0.y};
                 const gv_u4_t A1 = {a1.x, a1.y, b1.x, b1.y};
                 acc[v * 2] = gv_mfma<BF16>(A0, Bop, acc[v * 2]);
@@ -845,12 +864,22 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
                     return *(LdsWord)((quarter_code<B>(qq, v * 4 + j) << ES) + tslot);
                 }
             };
-            const gv_u4_t A0 = {look(qa, 0), look(qa, 1), look(qb, 0), look(qb, 1)};
-            const gv_u4_t A1 = {look(qa, 2), look(qa, 3), look(qb, 2), look(qb, 3)};
+            gv_u4_t A0 = {look(qa, 0), look(qa, 1), 0u, 0u};
+            if constexpr (!ALONE) {
+                A0[2] = look(qb, 0);
+                A0[3] = look(qb, 1);
+            }
+            gv_u4_t A1 = {look(qa, 2), look(qa, 3), 0u, 0u};
+            if constexpr (!ALONE) {
+                A1[2] = look(qb, 2);
+                A1[3] = look(qb, 3);
+            }
             acc[v * 2] = gv_mfma<BF16>(A0, Bop, acc[v * 2]);
             acc[v * 2 + 1] = gv_mfma<BF16>(A1, Bop, acc[v * 2 + 1]);
         }
     };
+    auto unit_pair = [&](const auto &qa, const auto &qb, gv_u4_t Bop, uint32_t tslot, auto width, uint32_t ga = 0,
+                         uint32_t gb = 0) { unit_products(qa, qb, Bop, tslot, width, ga, gb, std::false_type()); };
     // K-grouped LUT: LDS offset of unit m's K group (tile (w + m NW) GPI + gsub of the range, two
     // tiles per group) plus this lane's first row (chunk group cgl: eight rows and one pad).
     auto kg_off = [&](int m) -> uint32_t {
@@ -868,6 +897,32 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
         constexpr int D = (int)(sizeof(qc) / sizeof(qc[0])), DN = (int)(sizeof(qn) / sizeof(qn[0]));
         int nb = 0;
         __builtin_amdgcn_s_setprio(2);
+        if constexpr (RAGGED) {
+            for (; nb + D <= my_units; nb += D) {
+#pragma unroll
+                for (int n = 0; n < D; n += 2) {
+                    unit_pair(qc[n], qc[n + 1], operand_b(nb + n, nb + n + 1), tslot, width);
+                    __builtin_amdgcn_sched_barrier(0);
+                    qc[n] = load_idx<B>(qcur + (size_t)unit_at(nb + n + D) * step_c + lane_c);
+                    qc[n + 1] = load_idx<B>(qcur + (size_t)unit_at(nb + n + 1 + D) * step_c + lane_c);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (!has_next && output_ends) __builtin_amdgcn_s_setprio(1);
+            const int left = my_units - nb;
+#pragma unroll
+            for (int n = 0; n < D; n += 2) {
+                if (n + 1 < left) unit_pair(qc[n], qc[n + 1], operand_b(nb + n, nb + n + 1), tslot, width);
+                else if (n < left) unit_products(qc[n], qc[n], operand_b_alone(nb + n), tslot, width, 0u, 0u, std::true_type());
+            }
+            if (has_next) {
+#pragma unroll
+                for (int n = 0; n < DN; ++n) qn[n] = load_idx<BN>(qnext + (size_t)unit_at(n) * step_n + lane_n);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (!has_next && output_ends) __builtin_amdgcn_s_setprio(0);
+            return;
+        }
         for (; nb + 2 * D <= my_units; nb += D) {            // every refill exists
 #pragma unroll
             for (int n = 0; n < D; n += 2) {
@@ -956,7 +1011,7 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
             if (second) {
 #pragma unroll
                 for (int n = 0; n < DB; ++n) {
-                    q2[n] = load_idx<BB>(qb_cur + (size_t)n * stepB + lane0B);
+                    q2[n] = load_idx<BB>(qb_cur + (size_t)unit_at(n) * stepB + lane0B);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -1102,5 +1157,12 @@ flute_status launch_gemv_pair_1bit(const GemvParams &p, int pair, int grid_x, in
                                    size_t lds_bytes, bool lut_bf16, hipStream_t stream);
 flute_status launch_gemv_pair_wide(const GemvParams &p, int pair, int grid_x, int nw, int pf,
                                    size_t lds_bytes, bool lut_bf16, hipStream_t stream);
+
+// The launches of the instantiations for K ranges that do not divide (their own translation units).
+// pair as above, 0: one 4-bit width (p.slices > 0: a walking grid).
+flute_status launch_gemv_ragged_a(const GemvParams &p, int pair, int grid_x, int nw, size_t lds_bytes, bool lut_bf16,
+                                  hipStream_t stream);
+flute_status launch_gemv_ragged_b(const GemvParams &p, int pair, int grid_x, int nw, size_t lds_bytes, bool lut_bf16,
+                                  hipStream_t stream);
 
 }  // namespace flute

@@ -62,6 +62,44 @@ flute_status launch_pair(const GemvParams &p, int grid_x, int nw, int pf, size_t
 }
 
 
+// K ranges whose loads the wavefronts cannot share evenly.
+template <int LPGL, int NW, bool BF16, bool WALK, int BA, int BB>
+flute_status launch_ragged_grid(const GemvParams &p, int grid_x, size_t lds_bytes, hipStream_t stream) {
+    static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
+    if (!attr_done) {
+        FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)gemv4_kernel<LPGL, NW, 4, BF16, WALK, BA, BB, false, false, true>,
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsPerCU));
+        attr_done = true;
+    }
+    hipLaunchKernelGGL((gemv4_kernel<LPGL, NW, 4, BF16, WALK, BA, BB, false, false, true>), dim3(grid_x, p.split),
+                       dim3(NW * 64), lds_bytes, stream, p);
+    FLUTE_HIP_CHECK(hipGetLastError());
+    return FLUTE_OK;
+}
+
+// p.slices > 0: a walking grid (four wavefronts, one width)
+template <bool BF16, int BA, int BB>
+flute_status launch_ragged(const GemvParams &p, int grid_x, int nw, size_t lds_bytes, hipStream_t stream) {
+    if constexpr (BA == 4 && BB == 4) {
+        if (p.slices > 0) {
+            switch (p.lpg_log2) {
+                case 4: return launch_ragged_grid<4, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
+                case 5: return launch_ragged_grid<5, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
+                default: return launch_ragged_grid<6, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
+            }
+        }
+    }
+    switch (nw * 10 + p.lpg_log2) {
+        case 44: return launch_ragged_grid<4, 4, BF16, false, BA, BB>(p, grid_x, lds_bytes, stream);
+        case 45: return launch_ragged_grid<5, 4, BF16, false, BA, BB>(p, grid_x, lds_bytes, stream);
+        case 46: return launch_ragged_grid<6, 4, BF16, false, BA, BB>(p, grid_x, lds_bytes, stream);
+        case 84: return launch_ragged_grid<4, 8, BF16, false, BA, BB>(p, grid_x, lds_bytes, stream);
+        case 85: return launch_ragged_grid<5, 8, BF16, false, BA, BB>(p, grid_x, lds_bytes, stream);
+        case 86: return launch_ragged_grid<6, 8, BF16, false, BA, BB>(p, grid_x, lds_bytes, stream);
+        default: return FLUTE_ERR_UNSUPPORTED;       // (not reached: the caller checks the shape)
+    }
+}
+
 }  // namespace
 
 }  // namespace flute

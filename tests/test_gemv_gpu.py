@@ -633,3 +633,49 @@ def test_residual_coefficients_of_every_form(rank, K, form):
     y = _run(w, x, signs=signs, awq=awq, **extra)
     assert rel_l2(y.cpu(), _exact(w, xr)) <= TOL
     assert torch.equal(y, _run(w, x, signs=signs, awq=awq, **extra))
+
+
+@pytest.mark.parametrize("bits,bits2,act,lut", [
+    (4, 0, torch.float16, torch.float16), (4, 4, torch.bfloat16, torch.bfloat16), (4, 1, torch.float16, torch.float16),
+    (1, 4, torch.bfloat16, torch.float16), (3, 3, torch.float16, torch.float16), (2, 4, torch.bfloat16, torch.float16),
+    (2, 3, torch.float16, torch.float16), (3, 0, torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("N,K,gs,block", [
+    (128, 320, 128, None),     # five loads of a 32-row slice over four wavefronts
+    (256, 896, 256, None),     # fourteen tiles: seven loads of two
+    (1024, 1472, 128, None),   # 23 tiles over eight wavefronts, two and three loads each
+    (384, 1216, 128, 64),      # 19 tiles, blocks of a unit rotated in the wavefront
+    (256, 2880, 512, 0),       # 45 tiles, the whole row rotated
+    (256, 12352, 128, None),   # 193 tiles: more pieces of x than a wavefront holds at once
+])
+def test_ragged_k_ranges(tuning_env, N, K, gs, block, bits, bits2, act, lut):
+    """K ranges that the wavefronts cannot share evenly: against the oracle at the reference's
+    rounding point, repeats bit identical, and against the general kernel, whose fp32 sums run in
+    another order (each is within one rounding of the exact row: 2^-8 of a bfloat16 value)."""
+    w = make_weight(N, K, bits, gs, seed=N + K + bits, bits2=bits2, rank=8, bias=True, lut_dtype=lut, act_dtype=act,
+                    device=DEV)
+    x = make_x(1, K, seed=3, dtype=act)
+    signs = None if block is None else O.rotation_signs(K, 5)
+    extra = {"rot_block": block} if block else {}
+    y = _run(w, x, signs=signs, **extra).cpu()
+    assert torch.equal(y, _run(w, x, signs=signs, **extra).cpu())
+    if block is None:
+        assert rel_l2(y, _exact(w, x).to(act)) <= TOL
+    tuning_env("FLUTE_GEMV_NO_FAST", "1")
+    assert rel_l2(y, _run(w, x, signs=signs, **extra).cpu()) <= (TOL if act == torch.float16 else 4 * TOL)
+
+
+def test_ragged_k_ranges_keep_infinite_weights():
+    """A load without a partner is multiplied by zeros on both sides: an infinite LUT value gives an
+    infinity wherever its code meets a nonzero activation and nothing anywhere else."""
+    N, K = 256, 960
+    w = make_weight(N, K, 4, 128, seed=3, device=DEV)
+    w["lut"][0, 15] = w["lut_d"][0, 15] = float("inf")
+    x = torch.zeros(1, K, dtype=torch.float16)
+    x[0, K - 1] = 1.0
+    idx = w["idx"][:, K - 1].long()
+    want = w["lut"].float()[torch.arange(N) // 128, idx]
+    has_inf = (w["idx"][:128] == 15).any(dim=1)
+    y = _run(w, x).cpu()[0].float()
+    assert torch.equal(y[128:], want[128:])
+    # (rows of the first group: inf * 0 = NaN in the exact sum too)
+    assert bool(torch.isnan(y[:128])[has_inf].all()) and torch.equal(y[:128][~has_inf], want[:128][~has_inf])
