@@ -141,14 +141,58 @@ __device__ __forceinline__ void store_cols8(const FhtParams &p, int64_t orow, in
     }
 }
 
-// One workgroup per row, eight consecutive columns a thread and step.  The first nine stages stay in
+// One workgroup per row, eight consecutive columns a thread and piece, all segments of the row side by
+// side (transform_row).  What bounds it: for few rows the chain load -> stages -> barriers -> store, so
+// a row's values and multipliers are one memory round trip; for many rows the loads and stores.  P pieces
+// of eight columns a thread in as few registers as K needs, so a CU holds several rows.
+template <int P>
+__global__ void __launch_bounds__(kFhtThreads) fht_row_kernel(const FhtParams p) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x;
+    const int64_t row = (int64_t)blockIdx.x * p.ldx;
+    const int64_t orow = (int64_t)blockIdx.x * p.ldo;
+    if (p.ap && (int)blockIdx.x >= p.ap_M) {           // padding row of the operand image
+        const uint16_t zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (int j = tid * 8; j < p.K; j += kFhtThreads * 8)
+            store_operand_order(p, blockIdx.x, j, zero);
+        return;
+    }
+    uint32_t top = 0;
+    float sg[P][8];
+    transform_row<8, P>(
+        (float *)lds, p.K, p.block, tid, kFhtThreads,
+        [&](int h, int j, float (&f)[8]) {
+            float sc[8];
+            load_cols8(p, row, j, f, sg[h], sc);
+        },
+        [&](int h, int j, float (&f)[8], int nst) {
+            float sc[8];
+            if (p.awq) load_mul8(p.awq, j, p.vec_mul, sc);
+            store_cols8(p, orow, j, inv_sqrt_pow2(nst), f, sg[h], sc, top);
+        });
+    if (p.shift) {
+        __shared__ uint32_t slots[kFhtThreads / 64];
+        top = workgroup_max(top, slots, tid, kFhtThreads);
+        if (tid == 0) p.shift[blockIdx.x] = bf16_row_shift(top);
+    }
+}
+
+template <int P>
+flute_status launch_row(const FhtParams &p, int rows, size_t lds_bytes, hipStream_t stream) {
+    static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
+    if (!attr_done) {
+        FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)fht_row_kernel<P>, hipFuncAttributeMaxDynamicSharedMemorySize, 98304));
+        attr_done = true;
+    }
+    hipLaunchKernelGGL(fht_row_kernel<P>, dim3(rows), dim3(kFhtThreads), lds_bytes, stream, p);
+    FLUTE_HIP_CHECK(hipGetLastError());
+    return FLUTE_OK;
+}
+
+// Rows beyond 16384 columns: their segments (chunks of blocks) one after the other, eight consecutive
+// columns a thread and step.  The first nine stages stay in
 // registers (fht_head: between a thread's columns, then between lanes), the rest are one or two
-// passes over an fp32 buffer in LDS; blocks and segments of up to 512 columns never touch it.  What
-// bounds it: for few rows the chain load -> stages -> barriers -> store, so a row's values and
-// multipliers are one memory round trip; for many rows the loads and stores.  Eight wavefronts of
-// one step each keep 4096 columns in few registers, so a CU holds several rows: the earlier form,
-// four wavefronts of two steps, took 204 registers, its form for 8192 columns 270.  Before and now:
-// 1 x 4096 5.3 -> 3.9 us, 1 x 12288 12.1 -> 8.1, 1000 x 4096 12.1 -> 8.9, 1024 x 12288 38.4 -> 22.1.
+// passes over an fp32 buffer in LDS; blocks and segments of up to 512 columns never touch it.
 __global__ void __launch_bounds__(kFhtThreads) fht_kernel(const FhtParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
     float *buf = (float *)lds;
@@ -259,6 +303,15 @@ flute_status fht_launch(const void *x, int64_t ldx, const float *signs, const fl
     }
     const int rows = operand ? operand->mblk_pad * 16 : M;
     if (rows == 0) return FLUTE_OK;
+    if (K <= transform_reach(8, 4, kFhtThreads)) {
+        lds_bytes = lds_bytes ? (size_t)K * 4 : 0;
+        switch ((K + kFhtThreads * 8 - 1) / (kFhtThreads * 8)) {
+            case 1: return launch_row<1>(p, rows, lds_bytes, stream);
+            case 2: return launch_row<2>(p, rows, lds_bytes, stream);
+            case 3: return launch_row<3>(p, rows, lds_bytes, stream);
+            default: return launch_row<4>(p, rows, lds_bytes, stream);
+        }
+    }
     static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
     if (!attr_done) {
         FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)fht_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 98304));

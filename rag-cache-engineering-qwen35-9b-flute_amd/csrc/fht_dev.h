@@ -14,6 +14,8 @@
 // instead of one per stage.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace flute {
@@ -152,6 +154,189 @@ __device__ __forceinline__ void fht_tail(float *buf, int count, int nst, int sh0
     else if (rem == 2) fht_pass<2>(buf, count, sh0, tid, nthreads);
     else if (rem == 1) fht_pass<1>(buf, count, sh0, tid, nthreads);
     if (rem > 0) __syncthreads();
+}
+
+// ---- a whole row at once -----------------------------------------------------------------------
+// The same stage for wavefronts whose lanes are all active, shared out over the two pipes: 1, 2 and 8
+// are row permutations of the vector pipe, 4 goes through ds_swizzle, and for 16 and 32 two values
+// change halves with each other (v_permlane16_swap, v_permlane32_swap), so that sum and difference
+// are each formed once, for half the lanes of either, and change back.
+template <int M, int N>
+__device__ __forceinline__ void stage_all_lanes(float (&f)[N], int lane) {
+    if constexpr (M == 16 || M == 32) {
+#pragma unroll
+        for (int q = 0; q < N; q += 2) {
+            auto swap = [](float a, float b) {
+                const uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+                if constexpr (M == 32) return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+                else return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+            };
+            const auto in = swap(f[q], f[q + 1]);
+            const float a = __uint_as_float(in[0]), c = __uint_as_float(in[1]);
+            const auto out = swap(a + c, a - c);
+            f[q] = __uint_as_float(out[0]);
+            f[q + 1] = __uint_as_float(out[1]);
+        }
+    } else {
+        const float sgn = (lane & M) ? -1.0f : 1.0f;
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const int own = __float_as_int(f[q]);
+            int other;
+            if constexpr (M == 1) other = __builtin_amdgcn_mov_dpp(own, 0xb1, 0xf, 0xf, false);
+            else if constexpr (M == 2) other = __builtin_amdgcn_mov_dpp(own, 0x4e, 0xf, 0xf, false);
+            else if constexpr (M == 8) other = __builtin_amdgcn_mov_dpp(own, 0x128, 0xf, 0xf, false);
+            else other = __builtin_amdgcn_ds_swizzle(own, (M << 10) | 0x1f);
+            f[q] = fmaf(f[q], sgn, __int_as_float(other));
+        }
+    }
+}
+
+// Stages of the transform that column j of a row of K takes part in: its block's, or those of its
+// descending power-of-two segment (the highest bit in which j and K differ: K has it, j has not).
+__device__ __forceinline__ int column_stages(int j, int K, int block) {
+    return 31 - __builtin_clz((unsigned)(block > 0 ? block : K ^ j));
+}
+
+// Stage `s` for the lanes whose columns take part in it.
+template <int M, int N>
+__device__ __forceinline__ void stage_some_lanes(float (&f)[N], int lane, bool takes) {
+    float g[N];
+#pragma unroll
+    for (int q = 0; q < N; ++q) g[q] = f[q];
+    stage_all_lanes<M>(g, lane);
+#pragma unroll
+    for (int q = 0; q < N; ++q) f[q] = takes ? g[q] : f[q];
+}
+
+// Where transform_row keeps column i in LDS: 16-byte pieces stay whole, and pieces that a thread's
+// neighbours access together lie on different banks, as do the consecutive columns of a pass.
+__device__ __forceinline__ int row_slot(int i) { return i ^ ((i >> 3) & 4); }
+
+// R stages of length 2^SH0 (512 or 1024 columns, or sixteen times that) and up over the 2^nst columns
+// from `off` on (a multiple of 2^nst).  Bits of a column above row_slot's reach are apart from it, so
+// the columns of a group lie at constant distances from the first: one address, the rest immediates.
+template <int R, int SH0>
+__device__ __forceinline__ void row_pass(float *buf, int off, int nst, int tid, int nthreads) {
+    constexpr int E = 1 << R;
+    static_assert(SH0 >= 9, "above the slots' permutation");
+    const int groups = 1 << (nst - R);
+#pragma unroll 1
+    for (int g = tid; g < groups; g += nthreads) {
+        float *const at = buf + row_slot(off + (((g >> SH0) << (SH0 + R)) | (g & ((1 << SH0) - 1))));
+        float v[E];
+#pragma unroll
+        for (int j = 0; j < E; ++j) v[j] = at[j << SH0];
+        stages_in_thread(v);
+#pragma unroll
+        for (int j = 0; j < E; ++j) at[j << SH0] = v[j];
+    }
+}
+
+// Columns of a row that transform_row reaches with P pieces of N columns a thread.
+constexpr int transform_reach(int N, int P, int nthreads) { return N * P * nthreads; }
+
+// Transform of a whole row of K columns (K and the block multiples of 32, K up to transform_reach),
+// all its segments side by side: thread `tid` holds the N consecutive columns at (h * nthreads + tid) * N
+// for h = 0 ... P - 1, load(h, j, f) fetches them and store(h, j, f, stages) gets them back.  The
+// first stages stay in registers, the rest are one or two passes over `buf` (K floats of LDS, needed
+// for blocks and segments beyond 64 * N columns), with two or three barriers whatever the number of
+// segments.  Every value goes through the same single roundings as in the buffered butterfly.
+// Called by all threads; on return no wavefront reads another's columns in the buffer any more.
+// What bounds it, for one row: vector instructions of one CU (about thirty a column over 64 lanes) and
+// the trip to memory in front.  Segments one after the other (a chain of loads, barriers and passes
+// each), eight dword accesses a thread and column-wise addresses: 1 x 12288 9.0 -> 7.6 us, 800 x 11072
+// 22.8 -> 20.0, 1000 x 4096 9.2 -> 8.1; the fused prologue, one token: 11072 -> 4096 22.5 -> 14.4 us
+// (with the ragged GEMV), 12288 -> 4096, (3, 3) bits 17.2 -> 15.9.
+template <int N, int P, class Load, class Store>
+__device__ __forceinline__ void transform_row(float *buf, int K, int block, int tid, int nthreads, Load load, Store store) {
+    constexpr int own = N == 8 ? 3 : 4, sh = own + 6;
+    static_assert(N == 8 || N == 16, "columns of a thread");
+    const int lane = tid & 63;
+    float f[P][N];
+#pragma unroll
+    for (int h = 0; h < P; ++h)
+        if (h * nthreads * N < K) load(h, min((h * nthreads + tid) * N, K - N), f[h]);
+#pragma unroll
+    for (int h = 0; h < P; ++h) {
+        if (h * nthreads * N >= K) break;               // uniform
+        const int nst = column_stages(min((h * nthreads + tid) * N, K - N), K, block);
+        stages_in_thread(f[h]);
+        stage_all_lanes<1>(f[h], lane);
+        if (__all(nst >= sh)) {
+            stage_all_lanes<2>(f[h], lane);
+            stage_all_lanes<4>(f[h], lane);
+            stage_all_lanes<8>(f[h], lane);
+            stage_all_lanes<16>(f[h], lane);
+            stage_all_lanes<32>(f[h], lane);
+        } else {
+            stage_some_lanes<2>(f[h], lane, nst > own + 1);
+            stage_some_lanes<4>(f[h], lane, nst > own + 2);
+            stage_some_lanes<8>(f[h], lane, nst > own + 3);
+            stage_some_lanes<16>(f[h], lane, nst > own + 4);
+            stage_some_lanes<32>(f[h], lane, nst > own + 5);
+        }
+    }
+    const int top = column_stages(0, K, block);         // the longest segment is the first
+    if (top > sh) {
+#pragma unroll
+        for (int h = 0; h < P; ++h) {
+            const int j = (h * nthreads + tid) * N;
+            if (j < K && column_stages(j, K, block) > sh) {
+                // (j + q and j agree above bit 3: the pieces' slots differ as the columns do)
+#pragma unroll
+                for (int q = 0; q < N; q += 4)
+                    *(float4 *)(buf + (row_slot(j) ^ q)) = make_float4(f[h][q], f[h][q + 1], f[h][q + 2], f[h][q + 3]);
+            }
+        }
+        __syncthreads();
+        auto level = [&](auto first, int nst, int off) {
+            constexpr int SH0 = decltype(first)::value;
+            switch (min(nst - SH0, 4)) {
+                case 4: row_pass<4, SH0>(buf, off, nst, tid, nthreads); break;
+                case 3: row_pass<3, SH0>(buf, off, nst, tid, nthreads); break;
+                case 2: row_pass<2, SH0>(buf, off, nst, tid, nthreads); break;
+                default: row_pass<1, SH0>(buf, off, nst, tid, nthreads); break;
+            }
+        };
+        auto levels = [&](auto first) {
+            constexpr int SH0 = decltype(first)::value;
+            if (block > 0) {
+                for (int off = 0; off < K; off += block) level(first, top, off);
+            } else {
+                for (int b = top, off = 0; b > SH0; --b) {
+                    if (!((K >> b) & 1)) continue;
+                    level(first, b, off);
+                    off += 1 << b;
+                }
+            }
+        };
+        levels(std::integral_constant<int, sh>());
+        if (top > sh + 4) {
+            __syncthreads();
+            levels(std::integral_constant<int, sh + 4>());
+        }
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < P; ++h) {
+            const int j = (h * nthreads + tid) * N;
+            if (j < K && column_stages(j, K, block) > sh) {
+#pragma unroll
+                for (int q = 0; q < N; q += 4) {
+                    const float4 v = *(const float4 *)(buf + (row_slot(j) ^ q));
+                    f[h][q] = v.x;
+                    f[h][q + 1] = v.y;
+                    f[h][q + 2] = v.z;
+                    f[h][q + 3] = v.w;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < P; ++h) {
+        const int j = (h * nthreads + tid) * N;
+        if (j < K) store(h, j, f[h], column_stages(j, K, block));
+    }
 }
 
 }  // namespace flute

@@ -6,6 +6,7 @@
 
 #include <atomic>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -528,6 +529,23 @@ flute_status make_plan(const flute_linear *segs, int count, const void *x, void 
                 for (int i = 0; i < count; ++i) std::swap(p.seg[i].st[0], p.seg[i].st[1]);
                 plan->pair = 14;
             }
+        }
+    }
+    // A fused rotation transforms its slice at once where a thread's pieces reach it (an unsplit row, or
+    // blocks beyond those that stay in a wavefront) and the fp32 slice in LDS costs no workgroup a CU
+    // would otherwise hold.
+    p.rot_whole = 0;
+    if (any_fused_rot && (fht_block > 256 || (fht_block == 0 && split == 1)) &&
+        kc <= transform_reach(8, kRotPieces, waves * 64)) {
+        const auto total = [&](size_t head) {
+            return ((head + 255) & ~(size_t)255) + ((kc * 2 + 15) & ~15) + kGemvRedBytes + 16 + 8 * 4;
+        };
+        const size_t whole = std::max(tab_bytes, (size_t)kc * 4), now = std::max(tab_bytes, scratch);
+        const long per_cu = std::min<long>(((long)col * split + kNumCU - 1) / kNumCU, 16 / waves);
+        const long holds = std::min<long>(per_cu, kLdsPerCU / total(now));
+        if (kLdsPerCU / total(whole) >= (size_t)std::max(holds, 1L)) {
+            p.rot_whole = 1;
+            scratch = std::max(scratch, (size_t)kc * 4);
         }
     }
     size_t region0 = tab_bytes > scratch ? tab_bytes : scratch;

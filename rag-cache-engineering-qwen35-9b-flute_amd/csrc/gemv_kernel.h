@@ -87,6 +87,8 @@ struct GemvParams {
     int lds_x;              // LDS byte offsets
     int lds_red;            // row sums [2][8][32] fp32, ticket flag (16 B), 8 words for a row maximum
     int slices;             // > 0: a workgroup walks the row slices blockIdx.x, + gridDim.x, ... below this
+    int rot_whole;          // a fused rotation transforms its slice at once (transform_row); the scratch at the start
+                            // of LDS holds it
     int xcd_runs;           // lean kernel, one column space: workgroup b takes slice (b % 8) * (grid / 8) + b / 8
 };
 
@@ -552,6 +554,7 @@ __device__ __forceinline__ void rotate_segment_fast(const uint16_t *x, const flo
 // bfloat16 activations in front of a float16 LUT are scaled by a power of two on the
 // way (normalise_staged_row); the shift is returned and is 0 otherwise.
 // Ends with the slice complete and the scratch free (barrier included).
+constexpr int kRotPieces = 4;       // eight columns each that a thread holds of a slice transformed at once
 template <bool BF16>
 __device__ int stage_x(const GemvParams &p, const uint16_t *x, const float *signs,
                        const float *awq, uint8_t *lds, int k0, int kc, int tid, int nthreads) {
@@ -573,6 +576,35 @@ __device__ int stage_x(const GemvParams &p, const uint16_t *x, const float *sign
     float *buf = (float *)lds;
     if (p.fht_block > 0 && p.fht_block <= 256) {
         rotate_blocks_inwave<BF16>(x, signs, awq, xs, k0, kc, p.fht_block, p.act_bf16, tid, nthreads);
+        return finish();
+    }
+    if (p.rot_whole) {
+        // (k0 is a multiple of the block, or 0)
+        constexpr int P = kRotPieces;
+        float sg[P][8];
+        transform_row<8, P>(
+            buf, kc, p.fht_block, tid, nthreads,
+            [&](int h, int j, float (&f)[8]) {
+                load_act8(x, k0 + j, p.act_bf16, f);
+                load_f8(signs, k0 + j, sg[h]);
+                if (awq) {
+                    float sc[8];
+                    load_f8(awq, k0 + j, sc);
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) f[q] *= sc[q];
+                }
+            },
+            [&](int h, int j, float (&f)[8], int nst) {
+                const float inv = inv_sqrt_pow2(nst);
+                float sc[8];
+                if (awq) load_f8(awq, k0 + j, sc);
+                uint32_t o[4];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) f[q] = f[q] * sg[h][q] * inv;
+                pack_act8(f, awq ? sc : nullptr, p.act_bf16, o);
+                *(uint4 *)(xs + j) = make_uint4(o[0], o[1], o[2], o[3]);
+            });
+        __syncthreads();                               // the scratch is free
         return finish();
     }
     if (p.fht_block > 0) {

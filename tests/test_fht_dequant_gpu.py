@@ -72,6 +72,31 @@ def test_fht_every_segment_length_bit_exact(M, K):
         assert torch.equal(ya, O.fht_adjoint_reference(x, signs))
 
 
+@pytest.mark.parametrize("K", [160, 992, 2432, 4064, 8160, 11072, 16352, 16416])
+def test_fht_rows_of_many_segments_bit_exact(K):
+    """All segments of a row are transformed side by side: wavefronts whose lanes lie in several of
+    them, one to four pieces a thread, the last partly empty, passes over segments of different length
+    at once; beyond 16384 columns one after the other.  The reference's bits, in place too."""
+    signs = O.rotation_signs(K, 11)
+    for dtype in (torch.float32, torch.float16):
+        x = make_x(3, K, seed=K, dtype=dtype)
+        want = O.fht_reference(x, signs)
+        xd = x.to(DEV)
+        assert torch.equal(fht.fht_apply(xd, signs.to(DEV), backend="kernel").cpu(), want)
+        ya = fht.fht_adjoint(xd, signs.to(DEV), backend="kernel").cpu()
+        assert torch.equal(ya, O.fht_adjoint_reference(x, signs))
+        fht.fht_apply_(xd, signs.to(DEV), backend="kernel")
+        assert torch.equal(xd.cpu(), want)
+
+
+@pytest.mark.parametrize("K,block", [(12288, 4096), (16384, 1024), (6144, 2048), (16384, 16384), (24576, 8192)])
+def test_fht_long_blocks_bit_exact(K, block):
+    x = make_x(2, K, seed=block, dtype=torch.float32)
+    signs = O.rotation_signs(K, 3)
+    y = fx._C.fht_forward(x.to(DEV), signs.to(DEV), block=block).cpu()
+    assert torch.equal(y, O.block_fht_reference(x, block, signs))
+
+
 @pytest.mark.parametrize("block", [32, 64, 128, 256, 512, 2048])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_fht_every_block_size_bit_exact(block, dtype):

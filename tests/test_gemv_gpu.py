@@ -679,3 +679,20 @@ def test_ragged_k_ranges_keep_infinite_weights():
     assert torch.equal(y[128:], want[128:])
     # (rows of the first group: inf * 0 = NaN in the exact sum too)
     assert bool(torch.isnan(y[:128])[has_inf].all()) and torch.equal(y[:128][~has_inf], want[:128][~has_inf])
+
+
+@pytest.mark.parametrize("N,K,block,split", [
+    (256, 11072, 0, 0),       # 8192 + 2048 + 512 + 256 + 64 columns
+    (1024, 4992, 0, 0),       # 4096 + 512 + 256 + 128
+    (128, 12288, 4096, 0), (256, 8192, 512, 2), (512, 2048, 1024, 0), (256, 20480, 0, 0)])
+def test_fused_rotation_at_once_is_bit_identical_to_rotate_then_gemv(N, K, block, split):
+    import fht
+    for act in (torch.float16, torch.bfloat16):
+        w = make_weight(N, K, 4, 128, seed=K, act_dtype=act, device=DEV)
+        x = make_x(1, K, seed=9, dtype=act)
+        signs = O.rotation_signs(K, 5)
+        rotated = fx._C.fht_forward(x.to(DEV), signs.to(DEV), block=block) if block else \
+            fht.fht_apply(x.to(DEV), signs.to(DEV), backend="kernel")
+        extra = {"rot_block": block} if block else {}
+        y = _run(w, x, signs=signs, split=split, **extra)
+        assert rel_l2(y.cpu(), _run(w, rotated, split=split).cpu()) <= (0 if act == torch.float16 else 4 * TOL)
