@@ -19,15 +19,17 @@ namespace {
 // What has to be known before a GEMV launch can finish a row: the rotated input of every weight
 // that carries a residual, and the residual coefficients xb[r] = sum_k x[k] * resB[r][k] (fp32, x
 // rotated and rounded to the activation type where the weight is rotated).  One launch for all
-// weights of a call: eight residual rows per workgroup, one per wavefront, and every workgroup
-// transforms the input itself (a few microseconds of one CU) instead of waiting for another launch
-// to do it.  The butterflies are fht_dev.h's in the same order, so the rotated row has the bits of
-// flute_fht; a lane's sum runs over its columns in ascending order, then a fixed tree.
-// What bounds it: latency.  The row, its multipliers and the first 4096 columns of a residual row
-// are requested together; what follows is LDS passes between barriers.  Rotated q/k/v of rank 16,
-// K = 4096: three rotations of 5.2 us and three coefficient launches of 8.9 us, six launches in a
-// row, against one of 7.4 us; the whole call 50.5 -> 22.1 us.
-constexpr int kPreThreads = 512, kPreRows = kPreThreads / 64;
+// weights of a call, and every workgroup transforms the input itself (a few microseconds of one CU)
+// instead of waiting for another launch to do it.  The butterflies are fht_dev.h's in the same order,
+// so the rotated row has the bits of flute_fht; a lane's sum runs over its columns in ascending order,
+// then a fixed tree, then over the wavefronts of the residual row in order.
+// What bounds it: latency.  The row, its multipliers and a wavefront's first columns of its residual
+// row are requested together; what follows is LDS passes between barriers, then a step of eight
+// columns a lane for every 512 * (8 / rows) columns, rows = residual rows per workgroup, as few as
+// leave a workgroup per CU.  (One wavefront a residual row, eight rows a workgroup: rotated q/k/v of
+// rank 16, K = 4096, 7.2 us, now 6.0; rank 16, K = 11520, not rotated, 10.8, now 4.0; rank 8, K = 12288,
+// rotated, the call 26.7, now 21.2.)
+constexpr int kPreThreads = 512, kPreWaves = kPreThreads / 64;
 
 struct PreSeg {
     const uint16_t *resB;
@@ -43,6 +45,7 @@ struct PreParams {
     PreSeg seg[kGemvMaxSegs];
     const uint16_t *x;
     int nsegs, K, act_bf16, rot_block;
+    int rows;               // residual rows per workgroup: 1, 2, 4 or 8
 };
 
 __device__ __forceinline__ void pre_unpack8(const uint4 raw, int bf16, float (&f)[8]) {
@@ -73,8 +76,12 @@ __device__ __forceinline__ void pre_mul8(const float *p, int vec, float (&f)[8])
     }
 }
 
+// WHOLE: rows that transform_row reaches (buf holds K floats); else, segment by segment, the longest
+// segment or chunk of blocks.
+template <bool WHOLE>
 __global__ void __launch_bounds__(kPreThreads) gemv_pre_kernel(const PreParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
+    __shared__ float sums[kPreWaves];
     float *const buf = (float *)lds;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -82,40 +89,88 @@ __global__ void __launch_bounds__(kPreThreads) gemv_pre_kernel(const PreParams p
     while (si + 1 < p.nsegs && (int)blockIdx.x >= p.seg[si + 1].block0) ++si;
     const PreSeg &w = p.seg[si];
     const int part = blockIdx.x - w.block0;
-    const int r = part * kPreRows + wave;               // this wavefront's residual row
+    const int share = kPreWaves / p.rows;               // wavefronts of a residual row
+    const int r = part * p.rows + wave / share, c = wave % share;
     const bool mine = r < w.R;
     const uint16_t *const row = w.resB + (size_t)(mine ? r : 0) * p.K;
-    constexpr int AHEAD = 8;                            // steps of 512 columns requested up front
+    // columns of this lane: (h * share + c) * 512 + lane * 8, h = 0, 1, ...
+    const int col0 = c * 512 + lane * 8, step = share * 512;
+    constexpr int AHEAD = 4;                            // steps requested up front
     uint4 first[AHEAD];
     if (mine) {
 #pragma unroll
-        for (int h = 0; h < AHEAD; ++h) {
-            const int k = h * 512 + lane * 8;
-            first[h] = pre_load8(row + (k < p.K ? k : 0), w.vec_b);
-        }
+        for (int h = 0; h < AHEAD; ++h)
+            if (h * step < p.K) first[h] = pre_load8(row + min(col0 + h * step, p.K - 8), w.vec_b);
     }
     float acc = 0.0f;
-    // products of the columns [off, off + count), x from `get`
+    // products of this lane's columns in [off, off + count), x from `get`
     auto dot = [&](int off, int count, auto get) {
         if (!mine) return;
-        auto step = [&](int j, const uint4 raw) {
+        auto take = [&](int k, const uint4 raw) {
             float b[8], x[8];
             pre_unpack8(raw, p.act_bf16, b);
-            get(j, x);
+            get(k, x);
 #pragma unroll
             for (int q = 0; q < 8; ++q) acc = fmaf(x[q], b[q], acc);
         };
-        int j = lane * 8;
-        if (off == 0) {
 #pragma unroll
-            for (int h = 0; h < AHEAD; ++h)
-                if (h * 512 + lane * 8 < count) step(h * 512 + lane * 8, first[h]);
-            j += AHEAD * 512;
+        for (int h = 0; h < AHEAD; ++h) {
+            const int k = col0 + h * step;
+            if (k >= off && k < off + count) take(k, first[h]);
         }
-        for (; j < count; j += 512) step(j, pre_load8(row + off + j, w.vec_b));
+        int k = col0 + AHEAD * step;
+        if (k < off) k += (off - k + step - 1) / step * step;
+        for (; k < off + count; k += step) take(k, pre_load8(row + k, w.vec_b));
+    };
+    // eight finished columns of the rotated row: rounded to the activation type, kept in fp32 at `to`
+    auto rotated = [&](int k, float (&t)[8], const float (&sg)[8], float inv, float (&back)[8]) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) t[q] = t[q] * sg[q] * inv;
+        if (w.awq) {
+            float sc[8];
+            pre_mul8(w.awq + k, w.vec_m, sc);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) t[q] = t[q] / sc[q];
+        }
+        uint16_t o[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            o[q] = round_act(t[q], p.act_bf16);
+            back[q] = p.act_bf16 ? bf2f(o[q]) : h2f(o[q]);
+        }
+        if (w.xrot && part == 0)
+            *(uint4 *)(w.xrot + k) =
+                make_uint4((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16),
+                           (uint32_t)o[4] | ((uint32_t)o[5] << 16), (uint32_t)o[6] | ((uint32_t)o[7] << 16));
     };
     if (w.signs == nullptr) {
-        dot(0, p.K, [&](int j, float (&x)[8]) { pre_unpack8(*(const uint4 *)(p.x + j), p.act_bf16, x); });
+        dot(0, p.K, [&](int k, float (&x)[8]) { pre_unpack8(*(const uint4 *)(p.x + k), p.act_bf16, x); });
+    } else if constexpr (WHOLE) {
+        float sg[4][8];
+        transform_row<8, 4>(
+            buf, p.K, p.rot_block, tid, kPreThreads,
+            [&](int h, int j, float (&f)[8]) {
+                pre_unpack8(*(const uint4 *)(p.x + j), p.act_bf16, f);
+                pre_mul8(w.signs + j, w.vec_m, sg[h]);
+                if (w.awq) {
+                    float s[8];
+                    pre_mul8(w.awq + j, w.vec_m, s);
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) f[q] *= s[q];
+                }
+            },
+            [&](int h, int j, float (&f)[8], int nst) {
+                float b[8];
+                rotated(j, f, sg[h], inv_sqrt_pow2(nst), b);
+                *(float4 *)(buf + (row_slot(j) ^ 0)) = make_float4(b[0], b[1], b[2], b[3]);
+                *(float4 *)(buf + (row_slot(j) ^ 4)) = make_float4(b[4], b[5], b[6], b[7]);
+            });
+        __syncthreads();
+        dot(0, p.K, [&](int k, float (&x)[8]) {
+            const float4 a = *(const float4 *)(buf + row_slot(k)), b = *(const float4 *)(buf + (row_slot(k) ^ 4));
+            x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
+            x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
+        });
     } else {
         for (int off = 0; off < p.K;) {
             int count, nst;
@@ -127,12 +182,6 @@ __global__ void __launch_bounds__(kPreThreads) gemv_pre_kernel(const PreParams p
                 count = 1 << nst;
             }
             const float inv = inv_sqrt_pow2(nst);
-            // eight consecutive columns a thread and step: their first stages in registers
-            // (multipliers of the first step travel with the row)
-            float sg[8], sc[8];
-            const int j0 = tid * 8 < count ? tid * 8 : 0;
-            pre_mul8(w.signs + off + j0, w.vec_m, sg);
-            if (w.awq) pre_mul8(w.awq + off + j0, w.vec_m, sc);
             for (int j = tid * 8; j < count; j += kPreThreads * 8) {
                 float f[8];
                 pre_unpack8(*(const uint4 *)(p.x + off + j), p.act_bf16, f);
@@ -150,32 +199,18 @@ __global__ void __launch_bounds__(kPreThreads) gemv_pre_kernel(const PreParams p
             __syncthreads();
             fht_tail(buf, count, nst, 9, tid, kPreThreads);
             for (int j = tid * 8; j < count; j += kPreThreads * 8) {
-                if (j != tid * 8) {
-                    pre_mul8(w.signs + off + j, w.vec_m, sg);
-                    if (w.awq) pre_mul8(w.awq + off + j, w.vec_m, sc);
-                }
+                float sg[8], t[8], b[8];
+                pre_mul8(w.signs + off + j, w.vec_m, sg);
                 const int s0 = fht_slot(j);
-                float t[8];
 #pragma unroll
-                for (int q = 0; q < 8; ++q) t[q] = buf[s0 ^ q] * sg[q] * inv;
-                if (w.awq) {
+                for (int q = 0; q < 8; ++q) t[q] = buf[s0 ^ q];
+                rotated(off + j, t, sg, inv, b);
 #pragma unroll
-                    for (int q = 0; q < 8; ++q) t[q] = t[q] / sc[q];
-                }
-                uint16_t o[8];
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    o[q] = round_act(t[q], p.act_bf16);
-                    buf[s0 ^ q] = p.act_bf16 ? bf2f(o[q]) : h2f(o[q]);
-                }
-                if (w.xrot && part == 0)
-                    *(uint4 *)(w.xrot + off + j) =
-                        make_uint4((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16),
-                                   (uint32_t)o[4] | ((uint32_t)o[5] << 16), (uint32_t)o[6] | ((uint32_t)o[7] << 16));
+                for (int q = 0; q < 8; ++q) buf[s0 ^ q] = b[q];
             }
             __syncthreads();
-            dot(off, count, [&](int j, float (&x)[8]) {
-                const int s0 = fht_slot(j);
+            dot(off, count, [&](int k, float (&x)[8]) {
+                const int s0 = fht_slot(k - off);
 #pragma unroll
                 for (int q = 0; q < 8; ++q) x[q] = buf[s0 ^ q];
             });
@@ -183,10 +218,14 @@ __global__ void __launch_bounds__(kPreThreads) gemv_pre_kernel(const PreParams p
             if (off < p.K) __syncthreads();             // the next segment reuses the buffer
         }
     }
-    if (mine) {
 #pragma unroll
-        for (int m = 32; m > 0; m >>= 1) acc += __shfl_xor(acc, m);
-        if (lane == 0) w.xb[r] = acc;
+    for (int m = 32; m > 0; m >>= 1) acc += __shfl_xor(acc, m);
+    if (lane == 0) sums[wave] = acc;
+    __syncthreads();
+    if (lane == 0 && c == 0 && mine) {
+        float total = sums[wave];
+        for (int i = 1; i < share; ++i) total += sums[wave + i];
+        w.xb[r] = total;
     }
 }
 
@@ -197,6 +236,7 @@ struct Plan {
     GemvParams p;
     int pair;               // 10 * b1 + b2 when the widths are a pair the lean kernel serves with two tables, else 0
     bool k_group;           // the LUT is grouped along K (single weight, lean kernel only)
+    bool lean;              // the lean kernel serves the launch (make_plan lays the tables out for it)
     size_t lds_bytes;
     int grid_x;
     int threads;
@@ -275,6 +315,54 @@ void choose_shape(int rows, int G, int split_req, int *rw, int *split, int *wave
         wv = eight ? 8 : (units >= 4 ? 4 : (units >= 2 ? 2 : 1));
     }
     *waves = wv;
+}
+
+// 10 * b1 + b2 of a launch that the lean kernel takes with two tables, 0: one 4-bit width, -1: neither.
+int lean_pair(const flute_linear *segs, int count) {
+    const int b1 = segs[0].b1;
+    int b2 = 0;
+    bool four = true, same = true;
+    for (int i = 0; i < count; ++i) {
+        four &= segs[i].b1 == 4 && (segs[i].b2 == 0 || segs[i].b2 == 4);
+        same &= segs[i].b1 == b1;
+        if (segs[i].b2 > 0) {
+            if (b2 == 0) b2 = segs[i].b2;
+            same &= segs[i].b2 == b2;
+        }
+    }
+    if (four) return 0;
+    if (!same) return -1;
+    // a single narrow stream ((3, 0) is one of upstream's pairs): the two-table instantiation
+    // of its width with the second table unused
+    if (b2 == 0) b2 = b1 == 3 ? 3 : (b1 == 2 ? 3 : 4);
+    const int code = 10 * b1 + b2;
+    return code == 41 || code == 14 || code == 33 || code == 24 || code == 23 ? code : -1;
+}
+
+// LDS bytes of its tables: 4^b entries of 128 bytes a stream, of which a launch of one width has one;
+// a 1-bit stream's nibble table has 16 entries of 256 bytes.
+size_t lean_table_bytes(int pair) {
+    const auto tab = [](int b) { return b == 1 ? (size_t)16 * 256 : ((size_t)1 << (2 * b)) * 128; };
+    return pair == 0 ? tab(4) : tab(pair / 10) + tab(pair % 10);
+}
+
+// Whether the lean kernel takes a launch: widths as above, one LUT group per half tile (its row
+// slices lie in one half), LUT rows that can be read through the scalar cache, gate and up with one
+// input and rotation (the activations are staged once), a load or more per wavefront, and LDS for the
+// tables (32 KB, two-table pairs 36 KB at most) beside the activations.
+bool lean_serves(const flute_linear *segs, int count, int gs_tiles, int rw, int waves, int silu_mul) {
+    if (lean_pair(segs, count) < 0 || tuning().gemv_no_fast || !(waves == 4 || waves == 8)) return false;
+    for (int i = 0; i < count; ++i) {
+        if (segs[i].group_size < 64 || ((uintptr_t)segs[i].lut1 & 3) || (segs[i].b2 && ((uintptr_t)segs[i].lut2 & 3)))
+            return false;
+    }
+    if (silu_mul) {
+        const flute_linear &g = segs[0], &u = segs[1];
+        if (g.signs != u.signs || g.awq != u.awq || (g.signs && (g.R > 0) != (u.R > 0))) return false;
+    }
+    const int gpi = 32 / rw;
+    return gs_tiles % gpi == 0 && gs_tiles / gpi >= waves &&
+           36 * 1024 + gs_tiles * 128 + kGemvRedBytes + 1024 <= kLdsPerCU;
 }
 
 // Fill a launch plan for `count` weights that share x.  silu_mul couples
@@ -364,11 +452,24 @@ flute_status make_plan(const flute_linear *segs, int count, const void *x, void 
                       "a LUT grouped along K (K/split must be a multiple of 512 whose LUT rows fit a "
                       "workgroup's staging); try another split", who, K, split);
     }
+    // A lean launch whose tables and activations let fewer workgroups stay on a CU than its narrow
+    // slices need (a long K range over many rows): 32-row slices instead of a second round.  One
+    // token, 16-row slices and these: 11264 -> 12288, (4, 1) bits 41.7 -> 25.9 us, 12288 -> 12288 20.9
+    // -> 18.0, (2, 4) bits 33.4 -> 31.2; where all are resident either width measures the same.
+    if (rw < 32 && tuning().gemv_rw == 0 && !k_group && lean_serves(segs, count, G / split, rw, waves, silu_mul)) {
+        const size_t lds = lean_table_bytes(lean_pair(segs, count)) + (size_t)(G / split) * 128 + kGemvRedBytes + 512;
+        const long holds = std::min<long>(waves == 4 ? 3 : 1, (long)(kLdsPerCU / lds));
+        if ((long)(rows / rw) * split > holds * kNumCU) {
+            rw = 32;
+            waves = G / split >= 16 && (long)(rows / 32) * split <= kNumCU ? 8 : 4;
+        }
+    }
     FLUTE_REQUIRE((G / split) % (32 / rw) == 0, FLUTE_ERR_UNSUPPORTED,
                   "%s: K/64/split = %d is not a whole number of wavefront loads", who, G / split);
     const int gs_tiles = G / split;
     const int kc = gs_tiles * 64;
     const int spt = 128 / rw;
+    plan->lean = !k_group && lean_serves(segs, count, gs_tiles, rw, waves, silu_mul);
 
     bool any_fused_rot = false;
     const int fht_block = segs[0].rot_block;
@@ -385,14 +486,10 @@ flute_status make_plan(const flute_linear *segs, int count, const void *x, void 
         long wgs = 0;
         for (int i = 0; i < (silu_mul ? 1 : count); ++i) wgs += (long)(segs[i].N / rw) * split;
         long per_cu = (wgs + kNumCU - 1) / kNumCU;
-        // The lean all-4-bit kernel needs the full 32 KB table and is built for three
-        // workgroups per CU; grids of many rounds gain more from it than from a fourth
-        // resident workgroup with a half-size table in the general kernel (4096 -> 248320:
-        // 104 us against 127 us).
-        bool lean = true;
-        for (int i = 0; i < count; ++i)
-            lean &= segs[i].b1 == 4 && (segs[i].b2 == 0 || segs[i].b2 == 4) && segs[i].group_size >= 128;
-        if (per_cu > (lean ? 3 : 4)) per_cu = lean ? 3 : 4;
+        // The lean kernel needs the full 32 KB table and is built for three workgroups per CU; grids
+        // of many rounds gain more from it than from a fourth resident workgroup with a half-size
+        // table in the general kernel (4096 -> 248320: 104 us against 127 us).
+        if (per_cu > (plan->lean ? 3 : 4)) per_cu = plan->lean ? 3 : 4;
         if (per_cu < 1) per_cu = 1;
         const long fixed = kc * 2 + 4096;
         budget = 14;
@@ -447,7 +544,7 @@ flute_status make_plan(const flute_linear *segs, int count, const void *x, void 
             sg.awq = w.awq;
             any_fused_rot |= w.signs != nullptr;
         }
-        const int ngrp_log2 = k_group || w.group_size >= 128 ? 0 : ilog2(128 / w.group_size);
+        const int ngrp_log2 = k_group || plan->lean || w.group_size >= 128 ? 0 : ilog2(128 / w.group_size);
         for (int st = 0; st < sg.nstreams; ++st) {
             GemvStream &gs = sg.st[st];
             gs.q = (const uint8_t *)(st ? w.q2 : w.q1);
@@ -456,7 +553,7 @@ flute_status make_plan(const flute_linear *segs, int count, const void *x, void 
             int es = budget - entries_log2(gs.bits) - ngrp_log2;
             if (es > 7) es = 7;             // 32 replicas cover the 32 LDS banks
             if (es < entry_bytes_log2(gs.bits)) es = entry_bytes_log2(gs.bits);
-            if (k_group) es = 7;            // (no table: the lean kernel's LUT rows, sized below)
+            if (k_group || plan->lean) es = 7;   // (k_group: no table but the lean kernel's LUT rows, sized below)
             gs.es = es;
             const size_t tb = k_group ? (size_t)(kc / 128) * (rw * 64 + (rw / 8) * 64)
                                       : ((size_t)1 << (entries_log2(gs.bits) + es)) << ngrp_log2;
@@ -496,29 +593,11 @@ flute_status make_plan(const flute_linear *segs, int count, const void *x, void 
     // the launcher may still send the launch to the general kernel, which needs less.
     plan->pair = 0;
     plan->k_group = k_group;
-    if (!k_group) {
-        int b1 = segs[0].b1, b2 = 0;
-        bool ok = true;
-        for (int i = 0; i < count; ++i) {
-            ok &= segs[i].b1 == b1 && segs[i].group_size >= 128;
-            if (segs[i].b2 > 0) {
-                if (b2 == 0) b2 = segs[i].b2;
-                ok &= segs[i].b2 == b2;
-            }
-        }
-        int code = 10 * b1 + b2;
-        // a single narrow stream ((3, 0) is one of upstream's pairs): the two-table instantiation
-        // of its width with the second table unused
-        if (b2 == 0 && b1 < 4) {
-            b2 = b1 == 3 ? 3 : (b1 == 2 ? 3 : 4);
-            code = 10 * b1 + b2;
-        }
-        if (ok && (code == 41 || code == 14 || code == 33 || code == 24 || code == 23)) {
+    if (plan->lean) {
+        const int code = lean_pair(segs, count);
+        if (code) {
             plan->pair = code;
-            // (4^b entries of 128 bytes; a 1-bit stream's nibble table: 16 entries of 256 bytes)
-            auto tab = [](int b) { return b == 1 ? (size_t)16 * 256 : ((size_t)1 << (2 * b)) * 128; };
-            const size_t both = tab(b1) + tab(b2);
-            if (both > tab_bytes) tab_bytes = both;
+            if (lean_table_bytes(code) > tab_bytes) tab_bytes = lean_table_bytes(code);
             // (4, 1) where every weight has both streams: the kernel walks the 1-bit stream first
             // (the sum of the two streams does not depend on their order beyond fp32 rounding, and
             // the order is fixed, so results stay deterministic).  With the narrow stream in front
@@ -535,7 +614,7 @@ flute_status make_plan(const flute_linear *segs, int count, const void *x, void 
     // blocks beyond those that stay in a wavefront) and the fp32 slice in LDS costs no workgroup a CU
     // would otherwise hold.
     p.rot_whole = 0;
-    if (any_fused_rot && (fht_block > 256 || (fht_block == 0 && split == 1)) &&
+    if (plan->lean && any_fused_rot && (fht_block > 256 || (fht_block == 0 && split == 1)) &&
         kc <= transform_reach(8, kRotPieces, waves * 64)) {
         const auto total = [&](size_t head) {
             return ((head + 255) & ~(size_t)255) + ((kc * 2 + 15) & ~15) + kGemvRedBytes + 16 + 8 * 4;
@@ -641,12 +720,6 @@ int pick_prefetch(const Plan &plan, int nw) {
     return u % 4 == 0 ? 4 : 2;
 }
 
-// What the lean kernel takes besides: any whole number of loads, one or more per wavefront.
-bool ragged_fits(const Plan &plan, int nw) {
-    const int gpi = 64 >> plan.p.lpg_log2;
-    return (nw == 4 || nw == 8) && plan.p.gs_tiles % gpi == 0 && plan.p.gs_tiles / gpi >= nw;
-}
-
 template <int LPGL, int NW, bool BF16>
 flute_status launch_fast4_pf(Plan &plan, hipStream_t stream) {
     switch (pick_prefetch(plan, NW)) {
@@ -665,13 +738,9 @@ template <bool BF16>
 flute_status launch_width(Plan &plan, hipStream_t stream) {
     // one width for the whole launch -> the instantiation specialised for it
     int bits = plan.p.seg[0].st[0].bits;
-    int es = plan.p.seg[0].st[0].es;
-    bool one_group = true;
     for (int i = 0; i < plan.p.nsegs; ++i) {
-        one_group &= plan.p.seg[i].gs >= 128;
         for (int st = 0; st < plan.p.seg[i].nstreams; ++st) {
             if (plan.p.seg[i].st[st].bits != bits) bits = 0;
-            if (plan.p.seg[i].st[st].es != es) es = 0;
         }
     }
     const int nw = plan.threads / 64;
@@ -679,16 +748,6 @@ flute_status launch_width(Plan &plan, hipStream_t stream) {
     plan.p.xcd_runs = tuning().gemv_xcd != 0;
     for (int i = 0; i < plan.p.nsegs; ++i)
         if (((plan.p.seg[i].N >> 7) * (256 >> plan.p.lpg_log2)) % 8 != 0) plan.p.xcd_runs = 0;
-    // the lean kernel stages the activations once: gate and up must share input and rotation
-    const bool one_input = !plan.p.silu_mul ||
-                           (plan.p.seg[0].xsrc == plan.p.seg[1].xsrc &&
-                            plan.p.seg[0].signs == plan.p.seg[1].signs &&
-                            plan.p.seg[0].awq == plan.p.seg[1].awq);
-    // the lean kernel reads LUT rows through the scalar cache: dword-aligned LUTs only
-    bool luts_aligned = true;
-    for (int i = 0; i < plan.p.nsegs; ++i)
-        for (int st = 0; st < plan.p.seg[i].nstreams; ++st)
-            luts_aligned &= ((uintptr_t)plan.p.seg[i].st[st].lut & 3) == 0;
     if (plan.k_group) {
         // only the lean kernel knows this form: no general-kernel route
         const int pf = pick_prefetch(plan, nw);
@@ -699,43 +758,37 @@ flute_status launch_width(Plan &plan, hipStream_t stream) {
         plan.p.slices = 0;
         return launch_gemv_kgroup(plan.p, plan.grid_x, nw, pf, plan.lds_bytes, BF16, stream);
     }
-    if (bits == 4 && one_group && one_input && es == 7 && (nw == 4 || nw == 8) && luts_aligned &&
-        pick_prefetch(plan, nw) != 0 && tuning().gemv_no_fast == 0) {
-        switch (plan.p.lpg_log2) {
-            case 4: return launch_fast4_shape<4, BF16>(plan, nw, stream);
-            case 5: return launch_fast4_shape<5, BF16>(plan, nw, stream);
-            default: return launch_fast4_shape<6, BF16>(plan, nw, stream);
-        }
-    }
-    const bool lean = one_group && one_input && es == 7 && luts_aligned && tuning().gemv_no_fast == 0;
-    // K ranges that do not divide into equal, even numbers of loads: the lean kernel's ragged form, which
-    // is the faster one wherever it fits.  One token, the general kernel and this one, the launch alone:
-    //   3968 -> 2 x 11520, (1, 4) bits   30.0 -> 22.8 us      11520 -> 3968             25.7 -> 16.2
-    //   2944 -> 2 x 11904, rotated       23.5 -> 19.0         11904 -> 2944, rotated    20.6 -> 17.4
-    //   1152 -> 2 x 4480, (2, 4) bits    19.2 -> 14.8         4480 -> 1152              12.8 -> 9.1
-    //   2432 -> 2 x 2304, (3, 3), rotated 20.8 -> 16.1        4032 -> 2048, 512, 512    9.5 -> 6.4
-    //   2112 -> 144000: the call 57.9 -> 33.1 (a walking grid), (3, 3) bits 81.3 -> 64.2
-    if (lean && (bits == 4 || plan.pair) && pick_prefetch(plan, nw) == 0 && ragged_fits(plan, nw)) {
-        plan.p.slices = 0;
-        int gx = plan.grid_x;
-        if (bits == 4 && nw == 4)
-            if (const int resident = walking_grid(plan)) gx = resident;
-        const int pair = bits == 4 ? 0 : plan.pair;
-        return (pair == 0 || pair == 14 || pair == 41)
-                   ? launch_gemv_ragged_a(plan.p, pair, gx, nw, plan.lds_bytes, BF16, stream)
-                   : launch_gemv_ragged_b(plan.p, pair, gx, nw, plan.lds_bytes, BF16, stream);
-    }
-    if (plan.pair && one_group && one_input && es == 7 && luts_aligned &&
-        (nw == 4 || (nw == 8 && plan.p.lpg_log2 <= 5)) && pick_prefetch(plan, nw) != 0 &&
-        tuning().gemv_no_fast == 0) {
+    if (plan.lean) {
         int pf = pick_prefetch(plan, nw);
-        // a 1-bit stream with loads that come in eights: the deep ring (launch_pair's pf 8)
-        const int u = (plan.p.gs_tiles / (64 >> plan.p.lpg_log2)) / nw;
-        if (pf == 4 && plan.pair == 14 && u % 8 == 0 && tuning().gemv4_pf == 0) pf = 8;
+        if (plan.pair == 0 && pf != 0) {
+            switch (plan.p.lpg_log2) {
+                case 4: return launch_fast4_shape<4, BF16>(plan, nw, stream);
+                case 5: return launch_fast4_shape<5, BF16>(plan, nw, stream);
+                default: return launch_fast4_shape<6, BF16>(plan, nw, stream);
+            }
+        }
         plan.p.slices = 0;
-        return (plan.pair == 41 || plan.pair == 14)
-                   ? launch_gemv_pair_1bit(plan.p, plan.pair, plan.grid_x, nw, pf, plan.lds_bytes, BF16, stream)
-                   : launch_gemv_pair_wide(plan.p, plan.pair, plan.grid_x, nw, pf, plan.lds_bytes, BF16, stream);
+        if (pf != 0 && (nw == 4 || plan.p.lpg_log2 <= 5)) {
+            // a 1-bit stream with loads that come in eights: the deep ring (launch_pair's pf 8)
+            const int u = (plan.p.gs_tiles / (64 >> plan.p.lpg_log2)) / nw;
+            if (pf == 4 && plan.pair == 14 && u % 8 == 0 && tuning().gemv4_pf == 0) pf = 8;
+            return (plan.pair == 41 || plan.pair == 14)
+                       ? launch_gemv_pair_1bit(plan.p, plan.pair, plan.grid_x, nw, pf, plan.lds_bytes, BF16, stream)
+                       : launch_gemv_pair_wide(plan.p, plan.pair, plan.grid_x, nw, pf, plan.lds_bytes, BF16, stream);
+        }
+        // K ranges that do not divide into equal, even numbers of loads: the lean kernel's ragged form, which
+        // is the faster one wherever it fits.  One token, the general kernel and this one, the launch alone:
+        //   3968 -> 2 x 11520, (1, 4) bits   30.0 -> 22.8 us      11520 -> 3968             25.7 -> 16.2
+        //   2944 -> 2 x 11904, rotated       23.5 -> 19.0         11904 -> 2944, rotated    20.6 -> 17.4
+        //   1152 -> 2 x 4480, (2, 4) bits    19.2 -> 14.8         4480 -> 1152              12.8 -> 9.1
+        //   2432 -> 2 x 2304, (3, 3), rotated 20.8 -> 16.1        4032 -> 2048, 512, 512    9.5 -> 6.4
+        //   2112 -> 144000: the call 57.9 -> 33.1 (a walking grid), (3, 3) bits 81.3 -> 64.2
+        int gx = plan.grid_x;
+        if (plan.pair == 0 && nw == 4)
+            if (const int resident = walking_grid(plan)) gx = resident;
+        return (plan.pair == 0 || plan.pair == 14 || plan.pair == 41)
+                   ? launch_gemv_ragged_a(plan.p, plan.pair, gx, nw, plan.lds_bytes, BF16, stream)
+                   : launch_gemv_ragged_b(plan.p, plan.pair, gx, nw, plan.lds_bytes, BF16, stream);
     }
     switch (bits) {
         case 4: return launch_typed<BF16, 4>(plan, stream);
@@ -799,6 +852,12 @@ flute_status launch(Plan &plan, int act_dtype, hipStream_t stream, float *fixed_
         pp.K = plan.p.K;
         pp.act_bf16 = plan.p.act_bf16;
         pp.rot_block = plan.rot_block;
+        // as few residual rows per workgroup as leave one per CU
+        int ranks = 0;
+        for (int i = 0; i < plan.npre; ++i) ranks += plan.pre[i].R;
+        pp.rows = 1;
+        while (pp.rows < kPreWaves && ranks > kNumCU * pp.rows) pp.rows *= 2;
+        const bool whole = plan.p.K <= transform_reach(8, 4, kPreThreads);
         int blocks = 0;
         size_t lds = 0;
         for (int i = 0; i < plan.npre; ++i) {
@@ -806,16 +865,16 @@ flute_status launch(Plan &plan, int act_dtype, hipStream_t stream, float *fixed_
             uint16_t *const xr = xrot_base + pre.xrot_off;
             float *const xb = xb_base + pre.xb_off;
             if (pre.signs) {
-                const size_t cols = plan.rot_block > 0
-                                        ? (size_t)(plan.p.K <= 16384 ? plan.p.K : (16384 / plan.rot_block) * plan.rot_block)
-                                        : (size_t)make_segments(plan.p.K, 0).len[0];
+                const size_t cols = whole ? (size_t)plan.p.K
+                                    : plan.rot_block > 0 ? (size_t)(16384 / plan.rot_block) * plan.rot_block
+                                                         : (size_t)make_segments(plan.p.K, 0).len[0];
                 FLUTE_REQUIRE(cols <= 16384 && plan.p.K <= 65504, FLUTE_ERR_UNSUPPORTED,
                               "flute_gemv: the rotation of K=%d columns is not served", plan.p.K);
                 lds = cols * 4;
                 plan.p.seg[pre.seg].xsrc = xr;
             }
             if (pre.R > 0) plan.p.seg[pre.seg].xb = xb;
-            const int rowblocks = (pre.R + kPreRows - 1) / kPreRows;
+            const int rowblocks = (pre.R + pp.rows - 1) / pp.rows;
             if (rowblocks == 0 && pre.share >= 0) continue;      // another weight's rotation is all it needs
             PreSeg &g = pp.seg[pp.nsegs++];
             g.resB = pre.resB;
@@ -830,7 +889,14 @@ flute_status launch(Plan &plan, int act_dtype, hipStream_t stream, float *fixed_
             blocks += rowblocks ? rowblocks : 1;
         }
         if (blocks) {
-            hipLaunchKernelGGL(gemv_pre_kernel, dim3(blocks), dim3(kPreThreads), lds, stream, pp);
+            static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
+            if (!attr_done) {
+                for (const void *k : {(const void *)gemv_pre_kernel<true>, (const void *)gemv_pre_kernel<false>})
+                    FLUTE_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 16384 * 4));
+                attr_done = true;
+            }
+            if (whole) hipLaunchKernelGGL(gemv_pre_kernel<true>, dim3(blocks), dim3(kPreThreads), lds, stream, pp);
+            else hipLaunchKernelGGL(gemv_pre_kernel<false>, dim3(blocks), dim3(kPreThreads), lds, stream, pp);
             FLUTE_HIP_CHECK(hipGetLastError());
         }
     }

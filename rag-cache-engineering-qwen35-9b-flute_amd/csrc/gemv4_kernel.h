@@ -1,5 +1,5 @@
 // Lean specialisation of the M = 1 LUT GEMV for the common case: every stream
-// 4 bits wide and one LUT group per 128-row tile (group_size >= 128).  Same
+// 4 bits wide and one LUT group per half tile (group_size >= 64).  Same
 // ownership, table format and K-split protocol as gemv_kernel.h; what differs is
 // how a looked-up weight pair meets the activations.
 //
@@ -384,7 +384,9 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
         const int sg = so_ == 1 ? 1 : si0;
         const GemvStream st = kp->seg[sg].st[si_];
         const int t = sl_ / SPT, cg0 = (sl_ % SPT) * (RW >> 3);
-        const int grp = min((t * 128) >> __builtin_ctz(kp->seg[sg].gs), kp->seg[sg].lut_rows - 1);
+        // (the rows of a slice lie in one half of the tile: groups of 64 rows are one LUT row, too)
+        const int first = t * 128 + ((sl_ % SPT) >= SPT / 2 ? 64 : 0);
+        const int grp = min(first >> __builtin_ctz(kp->seg[sg].gs), kp->seg[sg].lut_rows - 1);
         const int B = si_ ? BB : BA;
         qr = st.q + ((size_t)t * G + g_lo) * (1024u * B) + (uint32_t)cg0 * (64u * B);
         lutp = st.lut + ((size_t)grp << B);
@@ -699,7 +701,7 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
             q[n] = load_idx<BA>(qrow + (size_t)unit_at(n) * step + lane0);
             __builtin_amdgcn_sched_barrier(0);
         }
-        xshift = stage_x<BF16>(p, staged_x, staged_signs, staged_awq, lds, k0, kc, tid, NT);
+        xshift = stage_x<BF16, true>(p, staged_x, staged_signs, staged_awq, lds, k0, kc, tid, NT);
         slab_issue();
         write_tables(lrow, lrowB, second0);
         __builtin_amdgcn_sched_barrier(0);

@@ -87,7 +87,7 @@ struct GemvParams {
     int lds_x;              // LDS byte offsets
     int lds_red;            // row sums [2][8][32] fp32, ticket flag (16 B), 8 words for a row maximum
     int slices;             // > 0: a workgroup walks the row slices blockIdx.x, + gridDim.x, ... below this
-    int rot_whole;          // a fused rotation transforms its slice at once (transform_row); the scratch at the start
+    int rot_whole;          // lean kernel: a fused rotation transforms its slice at once (transform_row); the scratch at the start
                             // of LDS holds it
     int xcd_runs;           // lean kernel, one column space: workgroup b takes slice (b % 8) * (grid / 8) + b / 8
 };
@@ -554,8 +554,10 @@ __device__ __forceinline__ void rotate_segment_fast(const uint16_t *x, const flo
 // bfloat16 activations in front of a float16 LUT are scaled by a power of two on the
 // way (normalise_staged_row); the shift is returned and is 0 otherwise.
 // Ends with the slice complete and the scratch free (barrier included).
+// LEAN: the lean kernel's; the general kernel has no registers for a slice at once (it spilled 25 to 159
+// of them with transform_row inside, and unrotated launches paid for that too: 10.7 -> 21.6 us).
 constexpr int kRotPieces = 4;       // eight columns each that a thread holds of a slice transformed at once
-template <bool BF16>
+template <bool BF16, bool LEAN = false>
 __device__ int stage_x(const GemvParams &p, const uint16_t *x, const float *signs,
                        const float *awq, uint8_t *lds, int k0, int kc, int tid, int nthreads) {
     uint16_t *xs = (uint16_t *)(lds + p.lds_x);
@@ -578,7 +580,7 @@ __device__ int stage_x(const GemvParams &p, const uint16_t *x, const float *sign
         rotate_blocks_inwave<BF16>(x, signs, awq, xs, k0, kc, p.fht_block, p.act_bf16, tid, nthreads);
         return finish();
     }
-    if (p.rot_whole) {
+    if (LEAN && p.rot_whole) {
         // (k0 is a multiple of the block, or 0)
         constexpr int P = kRotPieces;
         float sg[P][8];

@@ -696,3 +696,33 @@ def test_fused_rotation_at_once_is_bit_identical_to_rotate_then_gemv(N, K, block
         extra = {"rot_block": block} if block else {}
         y = _run(w, x, signs=signs, split=split, **extra)
         assert rel_l2(y.cpu(), _run(w, rotated, split=split).cpu()) <= (0 if act == torch.float16 else 4 * TOL)
+
+
+@pytest.mark.parametrize("rank", [1, 3, 16, 100, 256])
+@pytest.mark.parametrize("K,block", [(64, None), (4160, None), (12288, None), (2432, 0), (4096, 128), (20480, 0), (24576, 8192)])
+def test_residual_coefficients_of_one_token(K, block, rank):
+    """Residual rows shared by one to eight wavefronts, columns beyond those requested up front, rows
+    transformed at once and segment by segment.  The coefficients are fp32 sums of exact products, so
+    the outputs stay within one rounding of the oracle's: TOL."""
+    N = 128
+    w = make_weight(N, K, 4, 128, seed=K + rank, rank=rank, device=DEV)
+    x = make_x(1, K, seed=rank)
+    signs = None if block is None else O.rotation_signs(K, 5)
+    extra = {"rot_block": block} if block else {}
+    y = _run(w, x, signs=signs, **extra).cpu()
+    xr = x if block is None else (O.block_fht_reference(x, block, signs) if block else O.fht_reference(x, signs))
+    assert rel_l2(y, _exact(w, xr).half()) <= TOL
+
+
+@pytest.mark.parametrize("bits,bits2", [(4, 0), (4, 4), (4, 1), (1, 4), (3, 3), (2, 4), (2, 3), (3, 0), (1, 0)])
+@pytest.mark.parametrize("N,K", [(128, 1024), (256, 1216), (384, 4096), (4096, 8192), (25600, 1024)])
+def test_groups_of_64_rows(tuning_env, N, K, bits, bits2):
+    """A slice of 8, 16 or 32 rows lies in one half of its tile, so groups of 64 rows are one LUT row a
+    slice: N = 128 ... 25600 takes slices of each width and, for one 4-bit width, a grid that walks over
+    the slices of both halves.  Against the oracle and, in the rounding of the output, the general kernel."""
+    w = make_weight(N, K, bits, 64, seed=N + K + bits, bits2=bits2, device=DEV)
+    x = make_x(1, K, seed=4)
+    y = _run(w, x).cpu()
+    assert rel_l2(y, _exact(w, x).half()) <= TOL
+    tuning_env("FLUTE_GEMV_NO_FAST", "1")
+    assert rel_l2(y, _run(w, x).cpu()) <= TOL
