@@ -116,31 +116,56 @@ CoeffPlan plan_coeff(const flute_linear *ws, int count, int M) {
     return c;
 }
 
-flute_status launch_coeff(const CoeffPlan &plan, const flute_linear *ws, int count, const void *A, int64_t lda,
-                          float *const *xb, int M, int is_bf16, float *part, int *tickets, hipStream_t stream) {
+// The pre-pass of rows of A: coefficients of `count` weights (those with a residual; plan NULL: none)
+// and what `image` asks for (blocks 0: nothing), in one launch.
+flute_status launch_pre(const CoeffPlan *plan, const flute_linear *ws, int count, const void *A, int64_t lda,
+                        float *const *xb, int M, int is_bf16, float *part, int *tickets, const ImageParams &image,
+                        hipStream_t stream) {
     CoeffParams p = {};
-    p.A = (const uint16_t *)A;
-    p.lda = lda;
-    p.M = M;
-    p.K = ws[0].K;
-    p.aligned = ((uintptr_t)A & 15) == 0 && lda % 8 == 0;
-    p.kper = (p.K / 32 + plan.slices - 1) / plan.slices * 32;
-    p.part = part;
-    p.tickets = tickets;
     int n = 0, ranks = 0;
-    for (int i = 0; i < count; ++i) {
-        if (ws[i].R == 0) continue;
-        p.resB[n] = (const uint16_t *)ws[i].resB;
-        p.xb[n] = xb[i];
-        p.R[n] = ws[i].R;
-        p.rank0[n++] = ranks;
-        p.aligned &= ((uintptr_t)ws[i].resB & 15) == 0;
-        ranks += (ws[i].R + 15) / 16;
+    if (plan) {
+        p.A = (const uint16_t *)A;
+        p.lda = lda;
+        p.M = M;
+        p.K = ws[0].K;
+        p.aligned = ((uintptr_t)A & 15) == 0 && lda % 8 == 0;
+        p.kper = (p.K / 32 + plan->slices - 1) / plan->slices * 32;
+        p.rows = plan->rows;
+        p.ranks = plan->ranks;
+        p.slices = plan->slices;
+        p.part = part;
+        p.tickets = tickets;
+        for (int i = 0; i < count; ++i) {
+            if (ws[i].R == 0) continue;
+            p.resB[n] = (const uint16_t *)ws[i].resB;
+            p.xb[n] = xb[i];
+            p.R[n] = ws[i].R;
+            p.rank0[n++] = ranks;
+            p.aligned &= ((uintptr_t)ws[i].resB & 15) == 0;
+            ranks += (ws[i].R + 15) / 16;
+        }
     }
     for (; n < kGemmMaxSegs; ++n) p.rank0[n] = INT_MAX;
-    const dim3 grid(plan.rows, plan.ranks, plan.slices);
-    if (is_bf16) hipLaunchKernelGGL(gemm_coeff_kernel<true>, grid, dim3(1024), 0, stream, p);
-    else hipLaunchKernelGGL(gemm_coeff_kernel<false>, grid, dim3(1024), 0, stream, p);
+    // Coefficients and the search for scales are work for sixteen wavefronts; a small image alone is
+    // spread over the chip in workgroups of four.  A share of the image is four rows, or a 1 KB block a
+    // wavefront; workgroups beyond those resident at once would only queue (4096 x 12288: 512 workgroups
+    // of sixteen wavefronts 33 us, 2048 39, 6144 44; 2048 of four 36).
+    const int64_t ncoeff = (int64_t)p.rows * p.ranks * p.slices;
+    const int waves = ncoeff || image.find || (int64_t)image.blocks * image.segs > 32 * kNumCU ? 16 : 4;
+    const int64_t shares = image.find ? (int64_t)image.blocks * 4 : ((int64_t)image.blocks * image.segs + waves - 1) / waves;
+    const int64_t grid = ncoeff + std::min<int64_t>(shares, 32 / waves * kNumCU);
+    FLUTE_REQUIRE(grid <= 0x7fffffff, FLUTE_ERR_UNSUPPORTED, "flute_gemm: %lld workgroups exceed the grid", (long long)grid);
+    if (grid == 0) return FLUTE_OK;
+    const dim3 threads(64 * waves);
+    if (is_bf16) hipLaunchKernelGGL(gemm_pre_kernel<true>, dim3((unsigned)grid), threads, 0, stream, p, image);
+    else hipLaunchKernelGGL(gemm_pre_kernel<false>, dim3((unsigned)grid), threads, 0, stream, p, image);
+    FLUTE_HIP_CHECK(hipGetLastError());
+    return FLUTE_OK;
+}
+
+// Scales of bfloat16 rows by a launch of their own (rows that gemm_pre_kernel does not look through).
+flute_status launch_rowshift(const void *rows, int64_t ld, int M, int K, int *shift, hipStream_t stream) {
+    hipLaunchKernelGGL(gemm_rowshift_kernel, dim3(M), dim3(256), 0, stream, (const uint16_t *)rows, ld, K, shift);
     FLUTE_HIP_CHECK(hipGetLastError());
     return FLUTE_OK;
 }
@@ -269,12 +294,21 @@ flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *c
     const size_t shift_floats = scale_rows ? up4(M) : 0;
     size_t xb_floats = 0, part_xb = 0, want_tickets = 0;
     int tiles = 0;
+    // the weights of each image side by side, and their coefficients
+    flute_linear of[kWideMaxSegs][kWideMaxSegs];
+    int members[kWideMaxSegs][kWideMaxSegs], ofs[kWideMaxSegs] = {};
+    CoeffPlan coeff[kWideMaxSegs];
     for (int i = 0; i < count; ++i) {
+        const int k = image_of[i];
+        members[k][ofs[k]] = i;
+        of[k][ofs[k]++] = ws[i];
         xb_floats += up4((size_t)M * ws[i].R);
-        const CoeffPlan c = plan_coeff(ws + i, 1, M);
-        part_xb = std::max(part_xb, c.floats());
-        want_tickets = std::max(want_tickets, c.tickets());
         tiles += ws[i].N / 128;
+    }
+    for (int k = 0; k < images; ++k) {
+        coeff[k] = plan_coeff(of[k], ofs[k], M);
+        part_xb = std::max(part_xb, coeff[k].floats());
+        want_tickets = std::max(want_tickets, coeff[k].tickets());
     }
     const size_t part_floats = slices > 1 ? (size_t)slices * mtiles * tiles * plan.rows * 128 : 0;
     size_t total = part_floats + xb_floats + part_xb + 64;
@@ -289,49 +323,63 @@ flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *c
 
     const u4_t *image[kWideMaxSegs];
     const int *shift[kWideMaxSegs];
-    const void *rows[kWideMaxSegs];
-    int64_t ldr[kWideMaxSegs];
-    for (int k = 0; k < images; ++k) {
-        const flute_linear &w = ws[owner[k]];
-        rows[k] = A;
-        ldr[k] = lda;
-        if (w.signs) {
-            // (the rotation knows its rows' largest exponents)
-            int *const row_shift = scale_rows ? (int *)(next + rot_floats) : nullptr;
-            st = fht_launch(A, lda, w.signs, w.awq, next, K, M, K, act_dtype, 0, w.rot_block, stream, nullptr, row_shift);
-            if (st != FLUTE_OK) return st;
-            rows[k] = next;
-            ldr[k] = K;
-            next += rot_floats;
-        }
-        shift[k] = nullptr;
-        if (scale_rows && w.signs) {
-            shift[k] = (const int *)next;
-            next += shift_floats;
-        } else if (scale_rows) {
-            hipLaunchKernelGGL(gemm_rowshift_kernel, dim3(M), dim3(256), 0, stream, (const uint16_t *)rows[k], ldr[k], K,
-                               (int *)next);
-            FLUTE_HIP_CHECK(hipGetLastError());
-            shift[k] = (const int *)next;
-            next += shift_floats;
-        }
-        const int64_t blocks = (int64_t)(2 * G) * ((M + 15) / 16);
-        const int grid = (int)((blocks + 3) / 4 < 8192 ? (blocks + 3) / 4 : 8192);
-        hipLaunchKernelGGL(gemm_image_kernel, dim3(grid), dim3(256), 0, stream, (const uint16_t *)rows[k], (u4_t *)next, M,
-                           ldr[k], 2 * G, mblk, out_bf16, (int)(lut_dtype == FLUTE_BF16),
-                           (int)(((uintptr_t)rows[k] & 15) == 0 && ldr[k] % 8 == 0), shift[k]);
-        FLUTE_HIP_CHECK(hipGetLastError());
-        image[k] = (const u4_t *)next;
-        next += image_floats;
-    }
     float *xb[kWideMaxSegs] = {};
     for (int i = 0; i < count; ++i) {
         if (ws[i].R == 0) continue;
         xb[i] = next;
         next += up4((size_t)M * ws[i].R);
-        // (weights of different rotations have different rows: one launch each)
-        st = launch_coeff(plan_coeff(ws + i, 1, M), ws + i, 1, rows[image_of[i]], ldr[image_of[i]], xb + i, M, out_bf16,
-                          xb_part, tickets, stream);
+    }
+    for (int k = 0; k < images; ++k) {
+        const flute_linear &w = ws[owner[k]];
+        const void *rows = A;
+        int64_t ldr = lda;
+        int *row_shift = nullptr;
+        if (w.signs) {
+            // (the rotation knows its rows' largest exponents)
+            row_shift = scale_rows ? (int *)(next + rot_floats) : nullptr;
+            st = fht_launch(A, lda, w.signs, w.awq, next, K, M, K, act_dtype, 0, w.rot_block, stream, nullptr, row_shift);
+            if (st != FLUTE_OK) return st;
+            rows = next;
+            ldr = K;
+            next += rot_floats;
+        } else if (scale_rows) {
+            row_shift = (int *)next;
+        }
+        if (scale_rows) next += shift_floats;
+        shift[k] = row_shift;
+        image[k] = (const u4_t *)next;
+        ImageParams im = {};
+        im.A = (const uint16_t *)rows;
+        im.Ap = (u4_t *)next;
+        im.lda = ldr;
+        im.rowshift = row_shift;
+        im.M = M;
+        im.segs = 2 * G;
+        im.blocks = (M + 15) / 16;
+        im.mblk = mblk;
+        im.in_bf16 = out_bf16;
+        im.out_bf16 = lut_dtype == FLUTE_BF16;
+        im.wide = 1;
+        next += image_floats;
+        const bool find = scale_rows && !w.signs, rows16 = ((uintptr_t)rows & 15) == 0 && ldr % 8 == 0;
+        im.find = find && rows16 && K <= find_reach();
+        if (find && !im.find) {
+            st = launch_rowshift(rows, ldr, M, K, row_shift, stream);
+            if (st != FLUTE_OK) return st;
+        }
+        if (!rows16) {
+            const int64_t blocks = (int64_t)im.segs * im.blocks;
+            const int grid = (int)((blocks + 3) / 4 < 8192 ? (blocks + 3) / 4 : 8192);
+            hipLaunchKernelGGL(gemm_image_kernel, dim3(grid), dim3(256), 0, stream, im.A, im.Ap, M, ldr, im.segs, mblk,
+                               im.in_bf16, im.out_bf16, (const int *)row_shift);
+            FLUTE_HIP_CHECK(hipGetLastError());
+            im.blocks = 0;
+        }
+        // (weights of different rotations have different rows: a launch each)
+        float *to[kWideMaxSegs];
+        for (int j = 0; j < ofs[k]; ++j) to[j] = xb[members[k][j]];
+        st = launch_pre(coeff[k].ranks ? &coeff[k] : nullptr, of[k], ofs[k], rows, ldr, to, M, out_bf16, xb_part, tickets,
+                        im, stream);
         if (st != FLUTE_OK) return st;
     }
     WideParams p = {};
@@ -464,13 +512,6 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
     p.Ap = Ap;
     int *rowshift = scale_rows
         ? (int *)(base + p_floats + xb_floats + ap_floats + rot_floats) : nullptr;
-    auto launch_rowshift = [&](const void *rows, int64_t ld) -> flute_status {
-        hipLaunchKernelGGL(gemm_rowshift_kernel, dim3(M), dim3(256), 0, stream,
-                           (const uint16_t *)rows, ld, w->K, rowshift);
-        FLUTE_HIP_CHECK(hipGetLastError());
-        p.rowshift = rowshift;
-        return FLUTE_OK;
-    };
     // One block of rows per wavefront: the kernel reads A itself (16-byte pieces of a row, put into
     // operand order in registers), so the pre-pass launch is dropped.  Needs 16-byte aligned rows;
     // rotated rows are read the same way (the rotation can write the image itself, but only without a
@@ -492,35 +533,43 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
             if (st != FLUTE_OK) return st;
             A = Arot;
             lda = w->K;
-            p.rowshift = rowshift;                      // (the rotation knows its rows' largest exponents)
-        } else if (scale_rows) {
-            st = launch_rowshift(A, lda);
+        }
+        p.rowshift = rowshift;                          // (the rotation knows its rows' largest exponents)
+        const bool rows16 = ((uintptr_t)A & 15) == 0 && lda % 8 == 0, find = scale_rows && !w->signs;
+        ImageParams im = {};
+        im.A = (const uint16_t *)A;
+        im.lda = lda;
+        im.rowshift = rowshift;
+        im.M = M;
+        im.segs = 2 * p.G;
+        im.mblk = p.mblk_pad;
+        im.in_bf16 = act_dtype == FLUTE_BF16;
+        im.out_bf16 = w->lut_dtype == FLUTE_BF16;
+        im.block_xor = block_xor;
+        im.find = find && rows16 && w->K <= find_reach();
+        if (find && !im.find) {
+            st = launch_rowshift(A, lda, M, w->K, rowshift, stream);
             if (st != FLUTE_OK) return st;
         }
-        const int64_t total = (int64_t)p.G * 2 * p.mblk_pad * 64;
-        const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
-        const bool rows16 = ((uintptr_t)A & 15) == 0 && lda % 8 == 0;
         if (direct && rows16) {
             p.A8 = (const u4_t *)A;
             p.lda8 = lda / 8;
             p.a_bf16 = act_dtype == FLUTE_BF16;
+            im.blocks = im.find ? (M + 15) / 16 : 0;    // (the scales alone)
         } else if (rows16) {
-            // 16-byte aligned rows: one coalesced 16-byte load per thread and a transpose
-            // inside each quad (M = 256, K = 4096: 2.2 us against 5.2 us for the gathers)
-            hipLaunchKernelGGL(gemm_prep_quad_kernel, dim3(blocks), dim3(256), 0, stream,
-                               (const uint16_t *)A, Ap, M, lda, p.G, p.mblk_pad,
-                               (int)(act_dtype == FLUTE_BF16), (int)(w->lut_dtype == FLUTE_BF16),
-                               rowshift, (const uint32_t *)w->lut1,
-                               (int)(((size_t)w->lut_rows << w->b1) * 2 / 64), block_xor);
+            im.Ap = Ap;
+            im.blocks = p.mblk_pad;
+            im.warm = (const uint32_t *)w->lut1;
+            im.warm_lines = (int)(((size_t)w->lut_rows << w->b1) * 2 / 64);
         } else {
+            const int64_t total = (int64_t)p.G * 2 * p.mblk_pad * 64;
+            const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
             hipLaunchKernelGGL(gemm_prep_kernel, dim3(blocks), dim3(256), 0, stream,
                                (const uint16_t *)A, Ap, M, lda, p.G, p.mblk_pad,
                                (int)(act_dtype == FLUTE_BF16), (int)(w->lut_dtype == FLUTE_BF16),
                                (int)((((uintptr_t)A & 3) == 0) && (lda % 2 == 0)), rowshift, block_xor);
+            FLUTE_HIP_CHECK(hipGetLastError());
         }
-        FLUTE_HIP_CHECK(hipGetLastError());
-    }
-    if (any_res) {
         float *next = xb + coeff.floats(), *to[kGemmMaxSegs] = {};
         for (int i = 0; i < count; ++i) {
             if (ws[i].R == 0) continue;
@@ -529,7 +578,7 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
             p.seg[i].vec_res = ws[i].R % 8 == 0 && ((uintptr_t)ws[i].resA & 15) == 0 && ((uintptr_t)next & 15) == 0;
             next += ((size_t)M * ws[i].R + 3) & ~(size_t)3;
         }
-        st = launch_coeff(coeff, ws, count, A, lda, to, M, p.out_bf16, xb, tickets, stream);
+        st = launch_pre(any_res ? &coeff : nullptr, ws, count, A, lda, to, M, p.out_bf16, xb, tickets, im, stream);
         if (st != FLUTE_OK) return st;
     }
 

@@ -93,7 +93,8 @@ struct GemmParams {
     const int *rowshift;   // [M] or NULL: row m of the operands holds A[m] * 2^-rowshift[m]
 };
 
-// Activation pre-pass: Ap[g][j][mb][lane][slot] in the LUT's 16-bit type.
+// Activation pre-pass of rows that are not 16-byte aligned (others: gemm_pre_kernel):
+// Ap[g][j][mb][lane][slot] in the LUT's 16-bit type.
 // block_xor: the mode of image_block_xor (common.h).
 static __global__ void __launch_bounds__(256) gemm_prep_kernel(const uint16_t *A, u4_t *Ap, int M,
                                                         int64_t lda, int G, int mblk,
@@ -136,80 +137,15 @@ static __global__ void __launch_bounds__(256) gemm_prep_kernel(const uint16_t *A
     }
 }
 
-// The same image for 16-byte aligned rows, without gathers: a thread loads one 16-byte piece
-// (eight consecutive k) of a row, the four threads that share a 32-k segment transpose their
-// 4 x 4 dwords among themselves (thread q ends up with dword q of every piece, which is
-// operand kg = q), and each stores one operand.  A wavefront owns one (segment, 16-row block):
-// it reads sixteen 64-byte pieces of rows and writes one whole 1 KB block of the image.
+// Lane J of this lane's quad.
 template <int J>
 __device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, J * 0x55, 0xf, 0xf, true);
 }
-static __global__ void __launch_bounds__(256) gemm_prep_quad_kernel(const uint16_t *A, u4_t *Ap, int M,
-                                                             int64_t lda, int G, int mblk,
-                                                             int in_bf16, int out_bf16,
-                                                             const int *rowshift,
-                                                             const uint32_t *warm, int warm_lines,
-                                                             int block_xor) {
-    // The launch that follows starts with a chain of dependent loads (its arguments, then the
-    // LUT rows): one thread per 64-byte line touches the LUT here, so that the rows come from
-    // the memory-side cache there instead of from memory.
-    {
-        const int line = blockIdx.x * blockDim.x + threadIdx.x;
-        if (line < warm_lines) {
-            const uint32_t seen = __builtin_nontemporal_load(warm + (size_t)line * 16);
-            asm volatile("" ::"v"(seen));
-        }
-    }
-    const int segs = 2 * G;                             // 32-k segments per row
-    const int64_t total = (int64_t)mblk * 16 * segs * 4;
-    // the four threads of a quad share their row and their loop bound
-    for (int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; o < total;
-         o += (int64_t)gridDim.x * blockDim.x) {
-        const int q = (int)(o & 3);
-        const int64_t wv = o >> 6;
-        int gj, mblock;
-        if (total >> 6 <= 0x7fffffff) {                 // uniform; a 64-bit division costs some hundred instructions
-            gj = (int)((uint32_t)wv % (uint32_t)segs);
-            mblock = (int)((uint32_t)wv / (uint32_t)segs);
-        } else {
-            gj = (int)(wv % segs);
-            mblock = (int)(wv / segs);
-        }
-        const int m = mblock * 16 + (int)((o >> 2) & 15);
-        u4_t raw = {0u, 0u, 0u, 0u};
-        if (m < M) {
-            raw = *(const u4_t *)(A + (int64_t)m * lda + gj * 32 + q * 8);
-            if (in_bf16 != out_bf16) {
-                const int shift = rowshift ? rowshift[m] : 0;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint16_t lo = (uint16_t)(raw[e] & 0xffffu), hi = (uint16_t)(raw[e] >> 16);
-                    const float flo = ldexpf(in_bf16 ? bf2f(lo) : h2f(lo), -shift);
-                    const float fhi = ldexpf(in_bf16 ? bf2f(hi) : h2f(hi), -shift);
-                    raw[e] = (uint32_t)round_act(flo, out_bf16) | ((uint32_t)round_act(fhi, out_bf16) << 16);
-                }
-            }
-        }
-        // piece j of a segment holds its dwords 4j .. 4j + 3; operand kg is the dwords
-        // {kg, kg + 4, kg + 8, kg + 12} = element kg of the pieces 0 .. 3
-        u4_t out;
-#define FLUTE_TAKE(J)                                                                          \
-        {                                                                                      \
-            const uint32_t b0 = quad_bcast<J>(raw[0]), b1 = quad_bcast<J>(raw[1]);             \
-            const uint32_t b2 = quad_bcast<J>(raw[2]), b3 = quad_bcast<J>(raw[3]);             \
-            out[J] = (q & 2) ? ((q & 1) ? b3 : b2) : ((q & 1) ? b1 : b0);                      \
-        }
-        FLUTE_TAKE(0) FLUTE_TAKE(1) FLUTE_TAKE(2) FLUTE_TAKE(3)
-#undef FLUTE_TAKE
-        Ap[((int64_t)gj * mblk + ((m >> 4) ^ image_block_xor(gj >> 1, block_xor))) * 64 + q * 16 + (m & 15)] = out;
-    }
-}
-
-// The activation image of the many-row kernel (wide_piece) from rows: a wavefront moves one 1 KB block,
-// sixteen rows by 64 bytes, so that every line of the image is written whole by one instruction.
+// The activation image of the many-row kernel (wide_piece) from rows that are not 16-byte aligned (others:
+// gemm_pre_kernel): a wavefront moves one 1 KB block, sixteen rows by 64 bytes.
 static __global__ void __launch_bounds__(256) gemm_image_kernel(const uint16_t *A, u4_t *Ap, int M, int64_t lda, int segs,
-                                                         int mblk, int in_bf16, int out_bf16, int aligned,
+                                                         int mblk, int in_bf16, int out_bf16,
                                                          const int *rowshift) {
     const int lane = threadIdx.x & 63;
     const int64_t blocks = (int64_t)segs * ((M + 15) >> 4);          // (16-row block, 32-k segment)
@@ -225,12 +161,8 @@ static __global__ void __launch_bounds__(256) gemm_image_kernel(const uint16_t *
         const int m = min(mb * 16 + (lane >> 2), M - 1); // rows past the end repeat the last: nobody stores their products
         const uint16_t *src = A + (int64_t)m * lda + seg * 32 + (lane & 3) * 8;
         u4_t v;
-        if (aligned) {
-            v = *(const u4_t *)src;
-        } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = (uint32_t)src[2 * e] | ((uint32_t)src[2 * e + 1] << 16);
-        }
+        for (int e = 0; e < 4; ++e) v[e] = (uint32_t)src[2 * e] | ((uint32_t)src[2 * e + 1] << 16);
         if (in_bf16 != out_bf16) {
             const int shift = rowshift ? rowshift[m] : 0;
 #pragma unroll
@@ -267,7 +199,7 @@ static __global__ void __launch_bounds__(256) gemm_rowshift_kernel(const uint16_
 // xb[m, r] = sum_k A[m, k] * resB[r, k] in fp32: sixteen rows by sixteen ranks per workgroup on the
 // matrix cores, sixteen wavefronts taking the 32-k pieces of K in turn, their sums added in wavefront
 // order.  K is what there is to spread: a call of few rows has few such blocks, and a wavefront's
-// loads (sixteen rows each) are a chain of trips to memory; gridDim.z slices of K leave their sums in
+// loads (sixteen rows each) are a chain of trips to memory; `slices` slices of K leave their sums in
 // `part`, and the last arrival of a block adds them in slice order.  M = 48, K = 12288, R = 16: 22.8
 // us in one slice, 6.3 in sixteen.
 struct CoeffParams {
@@ -275,20 +207,22 @@ struct CoeffParams {
     const uint16_t *resB[kGemmMaxSegs];
     float *xb[kGemmMaxSegs];
     int R[kGemmMaxSegs];
-    int rank0[kGemmMaxSegs];   // first block of ranks (blockIdx.y) of each weight; past the last one INT_MAX
+    int rank0[kGemmMaxSegs];   // first block of ranks of each weight; past the last one INT_MAX
     int64_t lda;
     int M, K, aligned, kper;
+    int rows, ranks, slices;   // blocks
     float *part;
     int *tickets;
 };
 template <bool BF16>
-__global__ void __launch_bounds__(1024) gemm_coeff_kernel(const CoeffParams p) {
-    __shared__ f4_t red[16][64];
+__device__ __forceinline__ void coeff_block(const CoeffParams &p, int index, f4_t (&red)[16][64]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int si = ((int)blockIdx.y >= p.rank0[1]) + ((int)blockIdx.y >= p.rank0[2]) + ((int)blockIdx.y >= p.rank0[3]);
-    const int M = p.M, K = p.K, R = p.R[si], rb = blockIdx.y - p.rank0[si], aligned = p.aligned;
+    const int bz = index / (p.rows * p.ranks), in_slice = index - bz * (p.rows * p.ranks);
+    const int by = in_slice / p.rows, bx = in_slice - by * p.rows;
+    const int si = (by >= p.rank0[1]) + (by >= p.rank0[2]) + (by >= p.rank0[3]);
+    const int M = p.M, K = p.K, R = p.R[si], rb = by - p.rank0[si], aligned = p.aligned;
     float *const xb = p.xb[si];
-    const int m = min((int)blockIdx.x * 16 + (lane & 15), M - 1), rr = min(rb * 16 + (lane & 15), R - 1);
+    const int m = min(bx * 16 + (lane & 15), M - 1), rr = min(rb * 16 + (lane & 15), R - 1);
     const uint16_t *a = p.A + (int64_t)m * p.lda + (lane >> 4) * 8, *b = p.resB[si] + (int64_t)rr * K + (lane >> 4) * 8;
     auto load8 = [&](const uint16_t *p) {
         u4_t v;
@@ -298,18 +232,18 @@ __global__ void __launch_bounds__(1024) gemm_coeff_kernel(const CoeffParams p) {
         return v;
     };
     f4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const int k0 = blockIdx.z * p.kper, k1 = min(k0 + p.kper, K);
+    const int k0 = bz * p.kper, k1 = min(k0 + p.kper, K);
 #pragma unroll 4
     for (int k = k0 + wave * 32; k < k1; k += 512) acc = mfma16<BF16>(load8(b + k), load8(a + k), acc);
     red[wave][lane] = acc;
     __syncthreads();
     if (wave == 0) {
         for (int w = 1; w < 16; ++w) acc += red[w][lane];
-        if (gridDim.z > 1) {
-            const int block = blockIdx.y * gridDim.x + blockIdx.x, Z = gridDim.z;
-            const int64_t step = (int64_t)gridDim.x * gridDim.y * 256;       // floats of one slice
+        if (p.slices > 1) {
+            const int block = in_slice, Z = p.slices;
+            const int64_t step = (int64_t)p.rows * p.ranks * 256;            // floats of one slice
             float *const mine = p.part + (int64_t)block * 256 + lane * 4;
-            ws_store16(mine + blockIdx.z * step, acc);
+            ws_store16(mine + bz * step, acc);
             ws_stores_done();
             int old = 0;
             if (lane == 0) old = __hip_atomic_fetch_add(p.tickets + block, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -324,10 +258,143 @@ __global__ void __launch_bounds__(1024) gemm_coeff_kernel(const CoeffParams p) {
                 for (int i = 0; i < 4; ++i) acc += v[i];
             }
         }
-        const int mo = blockIdx.x * 16 + (lane & 15), r0 = rb * 16 + (lane >> 4) * 4;
+        const int mo = bx * 16 + (lane & 15), r0 = rb * 16 + (lane >> 4) * 4;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (mo < M && r0 + e < R) xb[(int64_t)mo * R + r0 + e] = acc[e];
+    }
+}
+
+// What a launch over rows of A (16-byte aligned) has to have in front of it, in one launch: the operand
+// image, the power-of-two scale of every row (bfloat16 rows in front of float16 operands), the residual
+// coefficients.  The first workgroups take the coefficients, the longest chain of the three; the others
+// a share of the image each.  As launches of their own: M = 48, K = 12288, rank 16 image 4.2 and
+// coefficients 6.9 us one after the other; M = 509, K = 12288, bfloat16 rows, scales 3.1 and image 6.8.
+struct ImageParams {
+    const uint16_t *A;
+    u4_t *Ap;                  // or NULL: only the scales are wanted
+    int64_t lda;
+    int *rowshift;             // [M] or NULL; find: written here, else read
+    const uint32_t *warm;      // LUT rows the launch behind reads first: one touch per 64-byte line
+    int M, segs;               // rows, 32-k segments of a row
+    int blocks;                // 16-row blocks to write
+    int mblk;                  // 16-row blocks the image holds per segment
+    int in_bf16, out_bf16;
+    int wide;                  // 1: pieces as they are (wide_piece), rows past the end repeat the last; 0: operands of
+                               // gemm_kernel.h, rows past the end zero
+    int block_xor;             // wide == 0: mode of image_block_xor
+    int find;                  // look for the scales first (a workgroup then takes four whole rows)
+    int warm_lines;
+};
+
+constexpr int kPieceMax = 8;   // 16-byte pieces of a row quarter that a thread holds where it looks for scales
+constexpr int find_reach() { return kPieceMax * 64 * 32; }       // columns
+
+__device__ __forceinline__ u4_t image_convert(u4_t raw, int in_bf16, int out_bf16, int shift) {
+    if (in_bf16 != out_bf16) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint16_t lo = (uint16_t)(raw[e] & 0xffffu), hi = (uint16_t)(raw[e] >> 16);
+            const float flo = ldexpf(in_bf16 ? bf2f(lo) : h2f(lo), -shift);
+            const float fhi = ldexpf(in_bf16 ? bf2f(hi) : h2f(hi), -shift);
+            raw[e] = (uint32_t)round_act(flo, out_bf16) | ((uint32_t)round_act(fhi, out_bf16) << 16);
+        }
+    }
+    return raw;
+}
+
+// Piece q (lane & 3) of 32-k segment `seg` of row m into the image; the four lanes of a quad hold the
+// pieces of one row's segment.
+__device__ __forceinline__ void image_store(const ImageParams &p, int m, int seg, u4_t raw) {
+    const int q = threadIdx.x & 3;
+    u4_t out = raw;
+    int mb = m >> 4;
+    if (!p.wide) {                                      // uniform
+        // piece j of a segment holds its dwords 4j .. 4j + 3; operand kg is the dwords
+        // {kg, kg + 4, kg + 8, kg + 12} = element kg of the pieces 0 .. 3
+#define FLUTE_TAKE(J)                                                                          \
+        {                                                                                      \
+            const uint32_t b0 = quad_bcast<J>(raw[0]), b1 = quad_bcast<J>(raw[1]);             \
+            const uint32_t b2 = quad_bcast<J>(raw[2]), b3 = quad_bcast<J>(raw[3]);             \
+            out[J] = (q & 2) ? ((q & 1) ? b3 : b2) : ((q & 1) ? b1 : b0);                      \
+        }
+        FLUTE_TAKE(0) FLUTE_TAKE(1) FLUTE_TAKE(2) FLUTE_TAKE(3)
+#undef FLUTE_TAKE
+        mb ^= image_block_xor(seg >> 1, p.block_xor);
+    }
+    p.Ap[((int64_t)seg * p.mblk + mb) * 64 + q * 16 + (m & 15)] = out;
+}
+
+template <bool BF16>
+__global__ void __launch_bounds__(1024) gemm_pre_kernel(const CoeffParams c, const ImageParams p) {
+    __shared__ f4_t red[16][64];
+    const int ncoeff = c.rows * c.ranks * c.slices;
+    if ((int)blockIdx.x < ncoeff) {
+        coeff_block<BF16>(c, blockIdx.x, red);
+        return;
+    }
+    const int b = blockIdx.x - ncoeff, nb = gridDim.x - ncoeff, tid = threadIdx.x, lane = tid & 63;
+    {
+        const int line = b * (int)blockDim.x + tid;
+        if (line < p.warm_lines) {
+            const uint32_t seen = __builtin_nontemporal_load(p.warm + (size_t)line * 16);
+            asm volatile("" ::"v"(seen));
+        }
+    }
+    // a row past the end: the last one again (wide) or zeros
+    auto load = [&](int m, int seg) -> u4_t {
+        if (m >= p.M && !p.wide) return u4_t{0u, 0u, 0u, 0u};
+        return *(const u4_t *)(p.A + (int64_t)min(m, p.M - 1) * p.lda + seg * 32 + (lane & 3) * 8);
+    };
+    if (p.find) {
+        // four rows by all segments: a quad per segment and row, 64 quads of a row side by side
+        const int r = (tid >> 2) & 3, s0 = tid >> 4;
+        uint32_t *const slots = (uint32_t *)red;        // [wave][row]
+        for (int m4 = b * 4; m4 < p.blocks * 16; m4 += nb * 4) {
+            const int m = m4 + r;
+            u4_t raw[kPieceMax];
+            uint32_t e = 0;
+#pragma unroll
+            for (int i = 0; i < kPieceMax; ++i)
+                if (s0 + i * 64 < p.segs) raw[i] = load(m, s0 + i * 64);
+#pragma unroll
+            for (int i = 0; i < kPieceMax; ++i)
+                if (s0 + i * 64 < p.segs) e = max(e, bf16_max_exp8(make_uint4(raw[i][0], raw[i][1], raw[i][2], raw[i][3])));
+            e = dpp_max<0xB1>(e);                       // the quad
+            e = dpp_max<0x4E>(e);
+            e = max(e, (uint32_t)__shfl_xor((int)e, 16));
+            e = max(e, (uint32_t)__shfl_xor((int)e, 32));
+            __syncthreads();                            // (the rows before are done with the slots)
+            if ((lane & 3) == 0 && lane < 16) slots[(tid >> 6) * 4 + r] = e;
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < 16; ++w) e = max(e, slots[w * 4 + r]);
+            const int shift = bf16_row_shift(e);
+            if ((tid & ~12) == 0 && m < p.M) p.rowshift[m] = shift;
+            if (p.Ap) {
+#pragma unroll
+                for (int i = 0; i < kPieceMax; ++i)
+                    if (s0 + i * 64 < p.segs) image_store(p, m, s0 + i * 64, image_convert(raw[i], p.in_bf16, p.out_bf16, shift));
+            }
+        }
+        return;
+    }
+    // a wavefront moves one 1 KB block of the image, sixteen rows by 64 bytes, at a time
+    const int waves = blockDim.x >> 6;
+    const int64_t total = (int64_t)p.blocks * p.segs;
+    for (int64_t w = (int64_t)b * waves + (tid >> 6); w < total; w += (int64_t)nb * waves) {
+        int mb, seg;
+        if (total <= 0x7fffffff) {                      // uniform; a 64-bit division costs some hundred instructions
+            mb = (int)((uint32_t)w / (uint32_t)p.segs);
+            seg = (int)((uint32_t)w - (uint32_t)mb * (uint32_t)p.segs);
+        } else {
+            mb = (int)(w / p.segs);
+            seg = (int)(w - (int64_t)mb * p.segs);
+        }
+        const int m = mb * 16 + (lane >> 2);
+        const u4_t raw = load(m, seg);
+        const int shift = p.rowshift ? p.rowshift[min(m, p.M - 1)] : 0;
+        image_store(p, m, seg, image_convert(raw, p.in_bf16, p.out_bf16, shift));
     }
 }
 

@@ -502,3 +502,25 @@ def test_gemm_residual_of_infinite_operands(tuning_env, rows):
     assert torch.isinf(want[5]).any() and torch.isinf(want[:, 17]).any()
     assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(torch.isinf(y), torch.isinf(want))
     assert torch.equal(torch.sign(y[torch.isinf(y)]), torch.sign(want[torch.isinf(want)]))
+
+
+@pytest.mark.parametrize("M,K,rows", [(2, 64, None), (17, 2048, "32"), (33, 12288, "32"), (70, 4160, "64"), (300, 1088, "256"),
+                                      (513, 16384, "512"), (40, 16448, "32"), (9, 20480, None)])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("rank", [0, 20])
+def test_gemm_pre_pass_of_scaled_rows(tuning_env, M, K, rows, offset, rank):
+    """Row scales, image and coefficients of bfloat16 rows over a float16 LUT in one launch: rows of
+    every magnitude, the last group of four partly past the end, K at and beyond what a workgroup holds
+    of four rows, rows that are not 16-byte aligned (the kernels of their own).  Products are exact in
+    fp32 and scales powers of two, so a row is off by its one rounding to bfloat16: 2^-9 of a value."""
+    if rows:
+        tuning_env("FLUTE_GEMM_ROWS", rows)
+    N = 256
+    w = make_weight(N, K, 4, 128, seed=M + K, rank=rank, act_dtype=torch.bfloat16, device=DEV)
+    x = make_x(M, K, seed=5, dtype=torch.bfloat16) * (2.0 ** torch.randint(-60, 60, (M, 1))).to(torch.bfloat16)
+    flat = torch.zeros(M * K + 8, dtype=torch.bfloat16, device=DEV)
+    xd = flat[offset:offset + M * K].reshape(M, K)
+    xd.copy_(x)
+    y = _dual(w, xd).cpu().double()
+    want = _exact(w, x).double()
+    assert bool(((y - want).norm(dim=1) <= 2.0 ** -8 * want.norm(dim=1)).all())
