@@ -352,6 +352,7 @@ size_t lean_table_bytes(int pair) {
 // tables (32 KB, two-table pairs 36 KB at most) beside the activations.
 bool lean_serves(const flute_linear *segs, int count, int gs_tiles, int rw, int waves, int silu_mul) {
     if (lean_pair(segs, count) < 0 || tuning().gemv_no_fast || !(waves == 4 || waves == 8)) return false;
+    if (tuning().gemv_table_log2 >= 12 && tuning().gemv_table_log2 < 15) return false;   // (smaller tables are asked for)
     for (int i = 0; i < count; ++i) {
         if (segs[i].group_size < 64 || ((uintptr_t)segs[i].lut1 & 3) || (segs[i].b2 && ((uintptr_t)segs[i].lut2 & 3)))
             return false;
