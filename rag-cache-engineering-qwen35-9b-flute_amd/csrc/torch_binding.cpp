@@ -7,7 +7,8 @@
 //   qgemm_gemv_splitk_fht_stream            (src/bindings.cpp:277-354)
 //   qgemm_gemv_multi, qgemm_gemv_mlp        (src/bindings.cpp:368-384)
 //   qgemm_cutlass_streaming, qgemm_dual_stream   (src/bindings.cpp:245-270)
-//   qgemm_linear, qgemm_linear_multi, embedding_rows   (what a module's forward calls; no upstream counterpart)
+//   qgemm_linear, qgemm_linear_multi, embedding_rows, operand_addresses
+//                                           (what a module's forward calls; no upstream counterpart)
 //
 // Same positional signatures, same conventions (empty tensor = absent operand, N from the
 // blob's byte count, RuntimeError on every contract violation, fresh outputs, launches on the
@@ -449,6 +450,46 @@ std::pair<Tensor, bool> embedding_rows(const Tensor &ids, const Tensor &indices,
     return {out, in_range != 0};
 }
 
+// Addresses of what the members' launches read, seven to a member in a fixed order, 0 for what is absent:
+// palettized_modules._operand_ptrs as it stands there (the dictionaries that a module's attribute lookup
+// ends in, in its order, then the lookup itself).
+pybind11::tuple operand_addresses(const pybind11::sequence &members) {
+    namespace py = pybind11;
+    static PyObject *const names[] = {PyUnicode_InternFromString("indices"), PyUnicode_InternFromString("lut"),
+                                      PyUnicode_InternFromString("indices2"), PyUnicode_InternFromString("lut2"),
+                                      PyUnicode_InternFromString("resA"), PyUnicode_InternFromString("resB"),
+                                      PyUnicode_InternFromString("bias")};
+    static PyObject *const buffers = PyUnicode_InternFromString("_buffers"), *const parameters = PyUnicode_InternFromString("_parameters");
+    const size_t count = members.size();
+    py::tuple out(7 * count);
+    for (size_t i = 0; i < count; ++i) {
+        const py::object m = members[i];
+        PyObject *places[3] = {nullptr, nullptr, nullptr};
+        PyObject **const own = _PyObject_GetDictPtr(m.ptr());
+        if (own && *own) {
+            PyObject *const b = PyDict_GetItemWithError(*own, buffers), *const p = PyDict_GetItemWithError(*own, parameters);
+            if (b && p && PyDict_Check(b) && PyDict_Check(p)) {          // a module
+                places[0] = *own;
+                places[1] = b;
+                places[2] = p;
+            }
+        }
+        for (int n = 0; n < 7; ++n) {
+            py::object t;
+            for (PyObject *place : places) {
+                if (!place) continue;
+                if (PyObject *const found = PyDict_GetItemWithError(place, names[n])) {
+                    t = py::reinterpret_borrow<py::object>(found);
+                    break;
+                }
+            }
+            if (!t) t = py::getattr(m, names[n], py::none());
+            out[7 * i + n] = THPVariable_Check(t.ptr()) ? py::int_((size_t)THPVariable_Unpack(t.ptr()).data_ptr()) : py::int_(0);
+        }
+    }
+    return out;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -468,6 +509,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("rot_block") = 0);
     m.def("qgemm_linear", &qgemm_linear);
     m.def("embedding_rows", &embedding_rows);
+    m.def("operand_addresses", &operand_addresses);
     m.def("qgemm_linear_multi", &qgemm_linear_multi);
     m.def("qgemm_gemv_multi", &qgemm_gemv_multi, py::arg("A"), py::arg("seg_table"),
           py::arg("lut_dtype") = py::none(), py::arg("split") = 0);

@@ -563,3 +563,41 @@ def test_gemm_rows_names_the_kernel_of_a_call(monkeypatch):
     finally:
         monkeypatch.undo()
         _lib.lib.flute_reload_tuning()
+
+
+def test_operand_addresses_compiled_and_not(monkeypatch):
+    """The compiled walk over the members' operands finds what the attribute lookup finds: buffers,
+    parameters, attributes of the object in front of either, classes without a module's dictionaries."""
+    import palettized_modules as pm
+    pm._flute()
+    if pm._fx._C.native is None:
+        pytest.skip("the compiled binding is not built")
+    ind, lut = torch.zeros(128 * 64 // 2, dtype=torch.uint8), torch.zeros(1, 16, dtype=torch.float16)
+
+    def layer(**kw):
+        return pm.PalettizedLinear(indices=ind.clone(), lut=lut.clone(), bitwidth=4, group_size=128, N=128, K=64, **kw)
+    plain, biased, shadowed, bare = layer(), layer(bias=torch.zeros(128)), layer(), type("Bare", (), {})()
+    shadowed.__dict__["lut"] = torch.zeros(1, 16, dtype=torch.bfloat16)
+    biased._buffers.pop("indices")
+    biased.indices = torch.nn.Parameter(ind.float())
+    bare.indices, bare.lut, bare.resA = ind, None, "not a tensor"
+    members = (plain, biased, shadowed, bare)
+    with_native = pm._operand_ptrs(members)
+    monkeypatch.setattr(pm, "_fx", None)
+    assert pm._operand_ptrs(members) == with_native and with_native[7] == biased.indices.data_ptr()
+    assert with_native[15] == shadowed.__dict__["lut"].data_ptr() and with_native[21:] == (ind.data_ptr(), 0, 0, 0, 0, 0, 0)
+    monkeypatch.undo()
+    before = pm._operand_ptrs([plain])
+    plain.lut = plain.lut.clone()
+    assert pm._operand_ptrs([plain]) != before
+
+
+def test_environment_switches_are_seen_at_once(monkeypatch):
+    import palettized_modules as pm
+    assert not pm._env_on("FLUTE_NO_SPLITK")
+    monkeypatch.setenv("FLUTE_NO_SPLITK", " 1 ")
+    assert pm._env_on("FLUTE_NO_SPLITK")
+    monkeypatch.setenv("FLUTE_NO_SPLITK", "0")
+    assert not pm._env_on("FLUTE_NO_SPLITK")
+    monkeypatch.setattr("os.environ", {"FLUTE_NO_SPLITK": "true"})
+    assert pm._env_on("FLUTE_NO_SPLITK")
