@@ -254,6 +254,26 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     constexpr int tab2 = FewTable<B1>::bytes, stage0 = tab2 + FewTable<B2>::bytes;
     constexpr int stage_wave = FewTable<B1>::stage + FewTable<B2>::stage;
     const uint32_t stage = lds0 + stage0 + (uint32_t)wave * stage_wave;
+    // (the residual's first sixteen ranks in front of all: what comes behind them can still be counted)
+    const bool residual = w.R > 0 && p.z_base + z == 0;
+    uint16_t res_a[4] = {0, 0, 0, 0};
+    float res_x[MB][4];
+    const uint16_t *const res_row = w.resA + (int64_t)(t * 128 + (rho >> 3) * 64 + wave * 8 + (rho & 7)) * w.R;
+    auto residual_load = [&](int r0) {
+        const int k0 = r0 + kg * 4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            res_a[e] = k0 + e < w.R ? res_row[k0 + e] : (uint16_t)0;
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+                res_x[mb][e] = k0 + e < w.R ? w.xb[(int64_t)min((mb0 + mb) * 16 + rho, p.M - 1) * w.R + k0 + e] : 0.0f;
+        }
+    };
+    if (residual) residual_load(0);
+    int unscale[MB];                                    // (with a residual: sums leave the loop's scale at once)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+        unscale[mb] = w.R > 0 && p.rowshift ? p.rowshift[min((mb0 + mb) * 16 + rho, p.M - 1)] : 0;
     FewLut<B1> lut1;
     FewLut<B2 ? B2 : 1> lut2;
     FewStream<B1> s1;
@@ -317,6 +337,43 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
         --left;
     }
     __builtin_amdgcn_s_setprio(0);
+
+    // ---- residual: + xb @ resA^T, in fp32 products onto the sums of the first slice ----------------
+    // Wavefront i takes the outputs of accumulator i, sixteen ranks a step, of which lane group kg holds
+    // four (the order of ranks is free as long as both operands agree): a few loads a lane, requested
+    // with the first loads of one slice, where the threads of the last arrival read eight rows of resA
+    // each behind the exchange (M = 48, 4096 <- 12288, (4, 1) bits, rank 16: the call 31.2 us, now 28.9;
+    // M = 64, bfloat16 rows, 12288 <- 4096, 4 bits: 23.7 and 22.0; M = 8: 18.1 and 17.8).  Sums of rows that are held scaled are
+    // scaled back ahead of it, in every slice: a residual may be of another magnitude than its row, and
+    // is added at its own.
+    if (w.R > 0 && p.rowshift) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[mb][i][q] = ldexpf(acc[mb][i][q], unscale[mb]);
+    }
+    if (residual) {
+        f4_t sum[MB];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) sum[mb] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int r0 = 0; r0 < w.R; r0 += 16) {
+            if (r0 > 0) residual_load(r0);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    sum[mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(p.out_bf16 ? bf2f(res_a[e]) : h2f(res_a[e]),
+                                                                  res_x[mb][e], sum[mb], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (i != wave) continue;                    // uniform
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) acc[mb][i] += sum[mb];
+        }
+    }
 
     // ---- sums of the eight wavefronts ---------------------------------------------------------
     // Four outputs of one row = one f4: accumulator i of lane (kg, rho) holds row rho, outputs
@@ -387,40 +444,14 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
             for (int q = 0; q < 4; ++q) y[4 * e + q] = sum[e][q];
     }
 
-    // ---- epilogue: scale back, residual, bias, one rounding, store --------------------------------
+    // ---- epilogue: scale back, bias, one rounding, store ------------------------------------------
     const int m = blockIdx.y * (16 * MB) + ml;
     if (m >= p.M) return;
     const int n0 = t * 128 + n_in;
-    if (p.rowshift) {                                   // exact
+    if (p.rowshift && w.R == 0) {                       // exact
         const int sh = p.rowshift[m];
 #pragma unroll
         for (int e = 0; e < PW; ++e) y[e] = ldexpf(y[e], sh);
-    }
-    if (w.R > 0 && w.vec_res) {                         // eight ranks a step, all its loads at once
-        const float *xr = w.xb + (size_t)m * w.R;
-        for (int r0 = 0; r0 < w.R; r0 += 8) {
-            u4_t a[PW];
-#pragma unroll
-            for (int e = 0; e < PW; ++e) a[e] = *(const u4_t *)(w.resA + (int64_t)(n0 + e) * w.R + r0);
-            const f4_t c0 = *(const f4_t *)(xr + r0), c1 = *(const f4_t *)(xr + r0 + 4);
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const float c = r < 4 ? c0[r & 3] : c1[r & 3];
-#pragma unroll
-                for (int e = 0; e < PW; ++e) {
-                    const uint16_t h = (uint16_t)(a[e][r >> 1] >> (16 * (r & 1)));
-                    y[e] = fmaf(c, p.out_bf16 ? bf2f(h) : h2f(h), y[e]);
-                }
-            }
-        }
-    } else if (w.R > 0) {
-        const float *xr = w.xb + (size_t)m * w.R;
-        for (int r = 0; r < w.R; ++r) {
-            const float c = xr[r];
-#pragma unroll
-            for (int e = 0; e < PW; ++e)
-                y[e] = fmaf(c, load_act(w.resA, (int64_t)(n0 + e) * w.R + r, p.out_bf16), y[e]);
-        }
     }
     if (w.bias) {
 #pragma unroll

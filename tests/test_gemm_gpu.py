@@ -524,3 +524,23 @@ def test_gemm_pre_pass_of_scaled_rows(tuning_env, M, K, rows, offset, rank):
     y = _dual(w, xd).cpu().double()
     want = _exact(w, x).double()
     assert bool(((y - want).norm(dim=1) <= 2.0 ** -8 * want.norm(dim=1)).all())
+
+
+@pytest.mark.parametrize("M", [3, 16, 17, 40])
+@pytest.mark.parametrize("rank", [1, 15, 17, 256])
+@pytest.mark.parametrize("exponent", [-100, 0, 100])
+def test_gemm_few_rows_residual_far_from_its_row(M, rank, exponent):
+    """Rows held scaled by 2^exponent, a residual 2^-exponent of them and a zero LUT: the residual is
+    added at its own magnitude (scaled with its row it would leave the range of fp32).  fp32 sums over K and
+    the ranks are off by (K + rank) * 2^-24 of the sum of magnitudes, the rounding by 2^-9 of a value."""
+    N, K, act = 256, 1088, torch.bfloat16
+    w = make_weight(N, K, 4, 128, seed=M + rank, act_dtype=act, device=DEV)
+    g = torch.Generator().manual_seed(M * rank)
+    x = torch.ldexp(torch.randn(M, K, generator=g), torch.tensor(exponent)).to(act)
+    resB = torch.ldexp(torch.randn(rank, K, generator=g), torch.tensor(-exponent)).to(act)
+    resA = torch.ldexp(torch.randn(N, rank, generator=g), torch.tensor(-exponent // 2)).to(act)
+    y = fx.qgemm_linear(x.to(DEV), w["blob_d"], w["lut_d"] * 0, 4, None, None, 0, resB.to(DEV), resA.to(DEV),
+                        None, 128, None, None).cpu().double()
+    xb, a = x.double() @ resB.double().t(), resA.double().t()
+    magnitude = (x.double().abs() @ resB.double().abs().t()) @ a.abs()
+    assert bool(((y - xb @ a).abs() <= 2.0 ** -8 * (xb @ a).abs() + (K + rank) * 2.0 ** -24 * magnitude).all())
