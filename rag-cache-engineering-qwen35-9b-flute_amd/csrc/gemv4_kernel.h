@@ -272,7 +272,6 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
     static_assert(PF % 2 == 0 && PF >= PF0, "loads are consumed in pairs");
     static_assert(!WALK || NW == 4, "the alternating sum areas of a walking grid are sized for four wavefronts");
     constexpr bool TWO = !(BA == 4 && BB == 4);     // two resident tables
-    static_assert(!TWO || !WALK, "walking grids: the (4, 4) kernel");
     static_assert(!KG || (!TWO && !WALK), "K-grouped LUTs: one 4-bit stream, one slice per workgroup");
     static_assert(!DEEP || (TWO && PF == 4 && BA == 1), "the deep ring is for a 1-bit first stream");
     static_assert(!RAGGED || (!KG && !DEEP), "ragged K ranges: tables along N, rings of PF loads");
@@ -987,7 +986,61 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
     const auto WB = std::integral_constant<int, BB>();
 
     int par = 0;                                    // walking: the partial sums alternate between two areas
-    if constexpr (TWO) {
+    if constexpr (TWO && WALK) {
+        // ---- two resident tables, one output, a slice after the other: the barriers and the two sum
+        //      areas are those of the one-table walk below ------------------------------------------
+        const bool second = second0;
+        const uint16_t *lutB = nullptr;
+        const uint8_t *qb_cur = qrow;
+        if (second) pass_ptrs(sl, 0, 1, qb_cur, lutB);
+        bool same_tables = false;                   // this slice's LUT rows are those of the one before
+        for (bool first = true;; first = false) {
+            if (!first && !same_tables) write_tables(lrow, lrowB, second);
+            const int nsl = sl + sl_step;
+            const bool more = nsl < sl_end;
+            const uint8_t *qa_next = qrow, *qb_next = qb_cur;
+            const uint16_t *luta = lut, *lutb = lutB;
+            bool next_same = false;
+            if (more) {
+                pass_ptrs(nsl, 0, 0, qa_next, luta);
+                if (second) pass_ptrs(nsl, 0, 1, qb_next, lutb);
+                next_same = luta == lut && lutb == lutB;
+                if (!next_same) {
+                    load_lut_row<BA>(luta, lrow);
+                    if (second) load_lut_row<BB>(lutb, lrowB);
+                }
+            }
+            if (second) {
+#pragma unroll
+                for (int n = 0; n < DB; ++n) {
+                    q2[n] = load_idx<BB>(qb_cur + (size_t)unit_at(n) * stepB + lane0B);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (!same_tables) __syncthreads();
+            if (second) {
+                k_loop(q, qrow, lane0, step, slotA, WA, q2, qb_cur, lane0B, stepB, WB, false, false);
+                k_loop(q2, qb_cur, lane0B, stepB, slotB, WB, q, qa_next, lane0, step, WA, more);
+            } else {
+                k_loop(q, qrow, lane0, step, slotA, WA, q, qa_next, lane0, step, WA, more);
+            }
+            end_of_output(0, par);
+            if (!more) break;
+            __syncthreads();
+            if (tid < RW) {
+                float yv[2];
+                fold_rows(yv, par);
+                finish_rows(sl, yv);
+            }
+            sl = nsl;
+            par ^= 1;
+            same_tables = next_same;
+            qrow = qa_next;
+            qb_cur = qb_next;
+            lut = luta;
+            lutB = lutb;
+        }
+    } else if constexpr (TWO) {
         // ---- two resident tables: per output, [both tables] barrier, loop A, loop B ----------
         for (so = 0; so < nout; ++so) {
             const int sg = so == 1 ? 1 : si0;

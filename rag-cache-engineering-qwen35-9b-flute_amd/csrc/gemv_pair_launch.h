@@ -13,19 +13,19 @@ namespace flute {
 
 namespace {
 
-// The lean kernel with two resident tables (mixed widths); no walking grid.  Eight wavefronts
+// The lean kernel with two resident tables (mixed widths).  Eight wavefronts
 // come with 8- or 16-row slices only (choose_shape).
-template <int LPGL, int NW, int PF, bool BF16, int BA, int BB, bool DEEP = false>
+template <int LPGL, int NW, int PF, bool BF16, int BA, int BB, bool DEEP = false, bool WALK = false>
 flute_status launch_pair_grid(const GemvParams &p, int grid_x, size_t lds_bytes, hipStream_t stream) {
     static std::atomic<bool> attr_done{false};
     if (!attr_done) {
         FLUTE_HIP_CHECK(hipFuncSetAttribute(
-            (const void *)gemv4_kernel<LPGL, NW, PF, BF16, false, BA, BB, false, DEEP>,
+            (const void *)gemv4_kernel<LPGL, NW, PF, BF16, WALK, BA, BB, false, DEEP>,
             hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsPerCU));
         attr_done = true;
     }
     dim3 grid(grid_x, p.split);
-    hipLaunchKernelGGL((gemv4_kernel<LPGL, NW, PF, BF16, false, BA, BB, false, DEEP>), grid, dim3(NW * 64),
+    hipLaunchKernelGGL((gemv4_kernel<LPGL, NW, PF, BF16, WALK, BA, BB, false, DEEP>), grid, dim3(NW * 64),
                        lds_bytes, stream, p);
     FLUTE_HIP_CHECK(hipGetLastError());
     return FLUTE_OK;
@@ -35,6 +35,22 @@ flute_status launch_pair_grid(const GemvParams &p, int grid_x, size_t lds_bytes,
 template <bool BF16, int BA, int BB>
 flute_status launch_pair(const GemvParams &p, int grid_x, int nw, int pf, size_t lds_bytes, hipStream_t stream) {
     constexpr bool NARROW = BA == 1;                 // the deep ring: for a 1-bit stream in front
+    if (p.slices > 0) {                              // a walking grid (pf 4 or 8: the caller checks)
+        if constexpr (NARROW) {
+            if (pf == 8) {
+                switch (p.lpg_log2) {
+                    case 4: return launch_pair_grid<4, 4, 4, BF16, BA, BB, true, true>(p, grid_x, lds_bytes, stream);
+                    case 5: return launch_pair_grid<5, 4, 4, BF16, BA, BB, true, true>(p, grid_x, lds_bytes, stream);
+                    default: return launch_pair_grid<6, 4, 4, BF16, BA, BB, true, true>(p, grid_x, lds_bytes, stream);
+                }
+            }
+        }
+        switch (p.lpg_log2) {
+            case 4: return launch_pair_grid<4, 4, 4, BF16, BA, BB, false, true>(p, grid_x, lds_bytes, stream);
+            case 5: return launch_pair_grid<5, 4, 4, BF16, BA, BB, false, true>(p, grid_x, lds_bytes, stream);
+            default: return launch_pair_grid<6, 4, 4, BF16, BA, BB, false, true>(p, grid_x, lds_bytes, stream);
+        }
+    }
     switch (nw * 100 + p.lpg_log2 * 10 + pf) {
         case 442: return launch_pair_grid<4, 4, 2, BF16, BA, BB>(p, grid_x, lds_bytes, stream);
         case 444: return launch_pair_grid<4, 4, 4, BF16, BA, BB>(p, grid_x, lds_bytes, stream);
@@ -77,16 +93,14 @@ flute_status launch_ragged_grid(const GemvParams &p, int grid_x, size_t lds_byte
     return FLUTE_OK;
 }
 
-// p.slices > 0: a walking grid (four wavefronts, one width)
+// p.slices > 0: a walking grid (four wavefronts)
 template <bool BF16, int BA, int BB>
 flute_status launch_ragged(const GemvParams &p, int grid_x, int nw, size_t lds_bytes, hipStream_t stream) {
-    if constexpr (BA == 4 && BB == 4) {
-        if (p.slices > 0) {
-            switch (p.lpg_log2) {
-                case 4: return launch_ragged_grid<4, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
-                case 5: return launch_ragged_grid<5, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
-                default: return launch_ragged_grid<6, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
-            }
+    if (p.slices > 0) {
+        switch (p.lpg_log2) {
+            case 4: return launch_ragged_grid<4, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
+            case 5: return launch_ragged_grid<5, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
+            default: return launch_ragged_grid<6, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
         }
     }
     switch (nw * 10 + p.lpg_log2) {

@@ -726,3 +726,19 @@ def test_groups_of_64_rows(tuning_env, N, K, bits, bits2):
     assert rel_l2(y, _exact(w, x).half()) <= TOL
     tuning_env("FLUTE_GEMV_NO_FAST", "1")
     assert rel_l2(y, _run(w, x).cpu()) <= TOL
+
+
+@pytest.mark.parametrize("bits,bits2", [(4, 1), (1, 4), (3, 3), (2, 4), (2, 3), (3, 0), (1, 0)])
+@pytest.mark.parametrize("N,K,gs,rank", [(16640, 1024, 128, 3), (33024, 2048, 64, 0), (33024, 704, 256, 0), (33152, 1088, 128, 0)])
+def test_resident_grid_walking_with_two_tables(tuning_env, N, K, gs, rank, bits, bits2):
+    """Width pairs and narrow streams on a walking grid (one workgroup a CU forces it at these sizes):
+    two to five slices each, side by side and strided, tables kept and rebuilt, the ring of eight 1-bit
+    loads, ragged K ranges.  A row's sums are formed as without walking: the same bits."""
+    w = make_weight(N, K, bits, gs, seed=N + K + bits, bits2=bits2, rank=rank, bias=rank > 0, device=DEV)
+    x = make_x(1, K, seed=9)
+    tuning_env("FLUTE_GEMV4_WALK", "0")
+    plain = _run(w, x)
+    tuning_env("FLUTE_GEMV4_WALK", "1")
+    walked = _run(w, x)
+    assert torch.equal(plain, walked)
+    assert rel_l2(walked.cpu(), _exact(w, x).half()) <= TOL
