@@ -92,7 +92,14 @@ GemmShape choose_gemm_shape(int M, int tiles, int G, int b1, int b2, double &us)
         us = few1;
         return {1, 8, 1, 1};
     }
-    if (few2 < other) {
+    // The estimate of 64 rows is 4 us and more short where the two are close and a workgroup has few
+    // tiles (less with more: M = 256 and 512, 12288 -> 4096 stay).  64 and 32 rows: M = 225,
+    // 5248 -> 2816 29.2 / 23.3 us; M = 300, 6912 -> 1792 32.2 / 27.6; M = 39, 1664 -> 12288 18.2 / 14.5;
+    // M = 672, 10432 -> 896 43.2 / 40.1; (3, 3) bits, M = 218, 1408 -> 6912 42.5 / 29.1.
+    const GemmShape shape = other_shape(M, tiles);
+    const double short_by = shape.mw == 1
+        ? std::min(4.0, std::max(0.0, 8.0 - G / slices_of_k((int64_t)tiles * ((M + 63) / 64), G, shape) / 16.0)) : 0.0;
+    if (few2 < other + short_by) {
         us = few2;
         return {2, 8, 1, 1};
     }
