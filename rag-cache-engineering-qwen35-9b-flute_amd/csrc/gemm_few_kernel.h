@@ -193,6 +193,13 @@ struct FewStream {
 template <>
 struct FewStream<0> {};
 
+// Rows held scaled by 2^-shift that carry a residual: their sums are scaled back to 2^-few_lift of their
+// magnitude ahead of the residual, and by the rest in the epilogue.  Partial sums of such a row stay
+// below 2^(shift + 34) (operands below 2, two float16 LUT values, K up to 2^16), so up to shift 92 they
+// fit fp32 as they are; beyond, they may leave its range where the row's sum does not, and are kept
+// 2^36 smaller, as is the residual (which loses bits below 2^-90 there, next to a row of 2^93 or more).
+__device__ __forceinline__ int few_lift(int shift) { return shift > 92 ? 36 : 0; }
+
 // B2 == 0: one stream (launches of one stream each may share a fold, p.z_base and p.ztotal).
 // SEGS: several weights in the launch.
 template <int MB, bool BF16, int B1, int B2, bool SEGS>
@@ -345,14 +352,14 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     // each behind the exchange (M = 48, 4096 <- 12288, (4, 1) bits, rank 16: the call 31.2 us, now 28.9;
     // M = 64, bfloat16 rows, 12288 <- 4096, 4 bits: 23.7 and 22.0; M = 8: 18.1 and 17.8).  Sums of rows that are held scaled are
     // scaled back ahead of it, in every slice: a residual may be of another magnitude than its row, and
-    // is added at its own.
+    // is added at its own (few_lift).
     if (w.R > 0 && p.rowshift) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
             for (int i = 0; i < 8; ++i)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) acc[mb][i][q] = ldexpf(acc[mb][i][q], unscale[mb]);
+                for (int q = 0; q < 4; ++q) acc[mb][i][q] = ldexpf(acc[mb][i][q], unscale[mb] - few_lift(unscale[mb]));
     }
     if (residual) {
         f4_t sum[MB];
@@ -371,7 +378,9 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
         for (int i = 0; i < 8; ++i) {
             if (i != wave) continue;                    // uniform
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb) acc[mb][i] += sum[mb];
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[mb][i][q] += ldexpf(sum[mb][q], -few_lift(unscale[mb]));
         }
     }
 
@@ -448,8 +457,8 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     const int m = blockIdx.y * (16 * MB) + ml;
     if (m >= p.M) return;
     const int n0 = t * 128 + n_in;
-    if (p.rowshift && w.R == 0) {                       // exact
-        const int sh = p.rowshift[m];
+    if (p.rowshift) {                                   // exact
+        const int sh = w.R == 0 ? p.rowshift[m] : few_lift(p.rowshift[m]);
 #pragma unroll
         for (int e = 0; e < PW; ++e) y[e] = ldexpf(y[e], sh);
     }

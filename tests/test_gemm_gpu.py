@@ -544,3 +544,26 @@ def test_gemm_few_rows_residual_far_from_its_row(M, rank, exponent):
     xb, a = x.double() @ resB.double().t(), resA.double().t()
     magnitude = (x.double().abs() @ resB.double().abs().t()) @ a.abs()
     assert bool(((y - xb @ a).abs() <= 2.0 ** -8 * (xb @ a).abs() + (K + rank) * 2.0 ** -24 * magnitude).all())
+
+
+@pytest.mark.parametrize("M,rows,slices", [(3, "16", "1"), (17, "16", "2"), (40, "32", "1"), (40, "32", "2")])
+def test_gemm_few_rows_residual_of_rows_at_the_end_of_the_range(tuning_env, M, rows, slices):
+    """Rows of 2^127 whose partial sums leave the range of fp32 and whose sums do not: the odd tiles of K
+    take back what the even ones add, up to one element of half the size.  fp32 sums over K and the ranks
+    are off by (K + rank) * 2^-24 of the sum of magnitudes, the rounding by 2^-9 of a value."""
+    tuning_env("FLUTE_GEMM_ROWS", rows)
+    tuning_env("FLUTE_GEMM_KSPLIT", slices)
+    N, K, rank, act = 256, 1024, 8, torch.bfloat16
+    w = make_weight(N, K, 4, 128, seed=M, act_dtype=act, device=DEV)
+    sign = 1.0 - 2.0 * (torch.arange(K) // 64 % 2)
+    x = (sign * 2.0 ** 127).repeat(M, 1).to(act)
+    x[:, 0] = 2.0 ** 126
+    g = torch.Generator().manual_seed(M)
+    resB = torch.ldexp(torch.randn(rank, K, generator=g), torch.tensor(-127)).to(act)
+    resA = torch.ldexp(torch.randn(N, rank, generator=g), torch.tensor(117)).to(act)
+    y = fx.qgemm_linear(x.to(DEV), w["blob_d"], torch.ones_like(w["lut_d"]), 4, None, None, 0, resB.to(DEV),
+                        resA.to(DEV), None, 128, None, None).cpu().double()
+    xb, a = x.double() @ resB.double().t(), resA.double().t()
+    want = x.double().sum(dim=1, keepdim=True) + xb @ a
+    magnitude = (x.double().abs() @ resB.double().abs().t()) @ a.abs()
+    assert bool(((y - want).abs() <= 2.0 ** -8 * want.abs() + (K + rank) * 2.0 ** -24 * magnitude).all())
