@@ -483,7 +483,14 @@ pybind11::tuple operand_addresses(const pybind11::sequence &members) {
                     break;
                 }
             }
-            if (!t) t = py::getattr(m, names[n], py::none());
+            if (!t) {                                                    // (only what is not there counts as absent)
+                t = py::reinterpret_steal<py::object>(PyObject_GetAttr(m.ptr(), names[n]));
+                if (!t) {
+                    if (!PyErr_ExceptionMatches(PyExc_AttributeError)) throw py::error_already_set();
+                    PyErr_Clear();
+                    t = py::none();
+                }
+            }
             out[7 * i + n] = THPVariable_Check(t.ptr()) ? py::int_((size_t)THPVariable_Unpack(t.ptr()).data_ptr()) : py::int_(0);
         }
     }

@@ -592,6 +592,28 @@ def test_operand_addresses_compiled_and_not(monkeypatch):
     assert pm._operand_ptrs([plain]) != before
 
 
+def test_operand_addresses_pass_errors_on(monkeypatch):
+    """An operand that is not there has address 0; one whose lookup fails is an error, compiled and not."""
+    import palettized_modules as pm
+    pm._flute()
+
+    class Failing:
+        @property
+        def lut2(self):
+            raise RuntimeError("not loaded yet")
+
+    class Absent:
+        @property
+        def lut2(self):
+            raise AttributeError("lut2")
+
+    for fx in (pm._fx, None):
+        monkeypatch.setattr(pm, "_fx", fx)
+        assert pm._operand_ptrs([Absent()]) == (0,) * 7
+        with pytest.raises(RuntimeError, match="not loaded yet"):
+            pm._operand_ptrs([Failing()])
+
+
 def test_environment_switches_are_seen_at_once(monkeypatch):
     import palettized_modules as pm
     assert not pm._env_on("FLUTE_NO_SPLITK")
