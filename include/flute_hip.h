@@ -280,6 +280,13 @@ int flute_pick_split(int N, int K);
 int64_t flute_gemv_lds_bytes(const flute_linear *w, int split);
 
 /*
+ * The output rows of a workgroup, 8, 16 or 32, and its wavefronts (`waves` may be NULL) in the launch that
+ * serves 1...4 weights over one token; -1 for descriptors it would refuse.  Host arithmetic under the
+ * tuning variables in force.
+ */
+int flute_gemv_rows(const flute_linear *ws, int count, int *waves);
+
+/*
  * The argument checks of a binding, once.  Upstream's bindings check the tensors they are handed
  * (dtype, rank, shape against K and the blob's byte count, contiguity, device) before they build
  * a launch (src/bindings.cpp:230-546, src/kernel_gemv.cu:379-474); so must any binding of this

@@ -257,6 +257,19 @@ struct Plan {
     int rot_block;
 };
 
+// Wavefronts of a workgroup of `rw` rows: eight when each still has two loads or more and the grid is
+// at most one workgroup per CU, or two per CU of eight-row workgroups with a long K range
+// (measured: 384 eight-row workgroups at K >= 8192 gain 2-10 % from eight, 512
+// sixteen- or 32-row ones lose 3-8 %).  Otherwise four, fewer for very short K.
+int choose_waves(int rows, int G, int split, int rw) {
+    const int forced = tuning().gemv_waves;
+    if (forced == 1 || forced == 2 || forced == 4 || forced == 8) return forced;
+    const int units = (G / split) / (32 / rw);
+    const long wgs = (long)(rows / rw) * split;
+    const bool eight = units >= 16 && (wgs <= kNumCU || (wgs <= 2 * kNumCU && units >= 32 && rw == 8));
+    return eight ? 8 : (units >= 4 ? 4 : (units >= 2 ? 2 : 1));
+}
+
 // Shape of the launch for `rows` output rows over G tiles of K.  A workgroup
 // owns `rw` rows.  The library's own policy splits K only where a workgroup's K range
 // would be very long over few rows: the exchange between workgroups (partial sums
@@ -302,19 +315,7 @@ void choose_shape(int rows, int G, int split_req, int *rw, int *split, int *wave
     }
     *rw = best_rw;
     *split = sp;
-    int wv = tuning().gemv_waves;
-    if (wv != 1 && wv != 2 && wv != 4 && wv != 8) {
-        // Eight wavefronts when each still has two loads or more and the grid is at most
-        // one workgroup per CU, or two per CU of eight-row workgroups with a long K range
-        // (measured: 384 eight-row workgroups at K >= 8192 gain 2-10 % from eight, 512
-        // sixteen- or 32-row ones lose 3-8 %).  Otherwise four, fewer for very short K.
-        const int units = (G / sp) / (32 / best_rw);
-        const long wgs = (long)(rows / best_rw) * sp;
-        const bool eight = units >= 16 && (wgs <= kNumCU || (wgs <= 2 * kNumCU && units >= 32 &&
-                                                             best_rw == 8));
-        wv = eight ? 8 : (units >= 4 ? 4 : (units >= 2 ? 2 : 1));
-    }
-    *waves = wv;
+    *waves = choose_waves(rows, G, sp, best_rw);
 }
 
 // 10 * b1 + b2 of a launch that the lean kernel takes with two tables, 0: one 4-bit width, -1: neither.
@@ -457,12 +458,12 @@ flute_status make_plan(const flute_linear *segs, int count, const void *x, void 
     // slices need (a long K range over many rows): 32-row slices instead of a second round.  One
     // token, 16-row slices and these: 11264 -> 12288, (4, 1) bits 41.7 -> 25.9 us, 12288 -> 12288 20.9
     // -> 18.0, (2, 4) bits 33.4 -> 31.2; where all are resident either width measures the same.
-    if (rw < 32 && tuning().gemv_rw == 0 && !k_group && lean_serves(segs, count, G / split, rw, waves, silu_mul)) {
+    if (tuning().gemv_rw == 0 && rw < 32 && !k_group && lean_serves(segs, count, G / split, rw, waves, silu_mul)) {
         const size_t lds = lean_table_bytes(lean_pair(segs, count)) + (size_t)(G / split) * 128 + kGemvRedBytes + 512;
         const long holds = std::min<long>(waves == 4 ? 3 : 1, (long)(kLdsPerCU / lds));
         if ((long)(rows / rw) * split > holds * kNumCU) {
             rw = 32;
-            waves = G / split >= 16 && (long)(rows / 32) * split <= kNumCU ? 8 : 4;
+            waves = choose_waves(rows, G, split, rw);
         }
     }
     FLUTE_REQUIRE((G / split) % (32 / rw) == 0, FLUTE_ERR_UNSUPPORTED,
@@ -1047,6 +1048,19 @@ int flute_pick_split(int N, int K) {
     int rw, split, waves;
     choose_shape(N, K / 64, 0, &rw, &split, &waves);
     return split;
+}
+
+int flute_gemv_rows(const flute_linear *ws, int count, int *waves) {
+    if (!ws || count < 1 || count > kGemvMaxSegs) return -1;
+    Plan plan;
+    alignas(16) char dummy[16] = {};                        // never dereferenced
+    void *outs[kGemvMaxSegs];
+    for (void *&o : outs) o = dummy;
+    if (make_plan(ws, count, dummy, outs, ws[0].lut_dtype == FLUTE_BF16 ? FLUTE_BF16 : FLUTE_F16, 0, 0, "flute_gemv_rows",
+                  &plan) != FLUTE_OK)
+        return -1;
+    if (waves) *waves = plan.threads / 64;
+    return 1 << (plan.p.lpg_log2 - 1);
 }
 
 int64_t flute_gemv_lds_bytes(const flute_linear *w, int split) {

@@ -106,6 +106,7 @@ SYMBOLS = {
     "flute_embedding": (_I, [_LP, _P, ctypes.c_int64, _P, _P]),
     "flute_embedding_checked": (_I, [_LP, _P, ctypes.c_int64, _P, _P, ctypes.POINTER(_I)]),
     "flute_pick_split": (_I, [_I, _I]),
+    "flute_gemv_rows": (_I, [_LP, _I, ctypes.POINTER(_I)]),
     "flute_gemv_lds_bytes": (ctypes.c_int64, [_LP, _I]),
     "flute_validate": (_I, [_LP, _I]),
     "flute_release_workspaces": (None, []),

@@ -40,6 +40,19 @@ def gemm_rows(M, *shapes):
     """Rows of A per workgroup that the library takes for weights (N, K, bits, bits2, gs) together:
     16 ... 128 the small-M kernel, 256 or 512 the many-row kernel."""
     from flute_extended import _lib
+    return _lib.lib.flute_gemm_rows(_weights(shapes), len(shapes), M)
+
+
+def gemv_rows(*shapes):
+    """(output rows, wavefronts) of a workgroup in the one-token launch of weights (N, K, bits, bits2, gs)."""
+    import ctypes
+    from flute_extended import _lib
+    waves = ctypes.c_int(0)
+    return _lib.lib.flute_gemv_rows(_weights(shapes), len(shapes), ctypes.byref(waves)), waves.value
+
+
+def _weights(shapes):
+    from flute_extended import _lib
     ws = (_lib.FluteLinear * len(shapes))()
     for w, (N, K, bits, bits2, gs) in zip(ws, shapes):
         w.N, w.K, w.b1, w.b2, w.group_size, w.lut_rows = N, K, bits, bits2, gs, -(-N // gs)
@@ -49,7 +62,7 @@ def gemm_rows(M, *shapes):
         if bits2:
             w.q2 = w.lut2 = 16
             w.q2_bytes = N * K * bits2 // 8
-    return _lib.lib.flute_gemm_rows(ws, len(shapes), M)
+    return ws
 
 
 def make_x(M, K, seed=1, dtype=torch.float16):

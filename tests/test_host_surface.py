@@ -565,6 +565,22 @@ def test_gemm_rows_names_the_kernel_of_a_call(monkeypatch):
         _lib.lib.flute_reload_tuning()
 
 
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("N,K,bits,bits2", [(2176, 8192, 4, 0), (3072, 12288, 3, 3), (6144, 12288, 4, 1), (12288, 12288, 4, 0)])
+def test_gemv_rows_keeps_forced_wavefronts(monkeypatch, N, K, bits, bits2, waves):
+    """FLUTE_GEMV_WAVES is what runs, also where the launch takes wider slices than its rows ask for."""
+    from _util import gemv_rows
+    from flute_extended import _lib
+    monkeypatch.setenv("FLUTE_GEMV_WAVES", str(waves))
+    _lib.lib.flute_reload_tuning()
+    try:
+        rows, got = gemv_rows((N, K, bits, bits2, 128))
+        assert rows in (8, 16, 32) and got == waves
+    finally:
+        monkeypatch.undo()
+        _lib.lib.flute_reload_tuning()
+
+
 def test_operand_addresses_compiled_and_not(monkeypatch):
     """The compiled walk over the members' operands finds what the attribute lookup finds: buffers,
     parameters, attributes of the object in front of either, classes without a module's dictionaries."""
