@@ -258,9 +258,8 @@ struct Plan {
 };
 
 // Wavefronts of a workgroup of `rw` rows: eight when each still has two loads or more and the grid is
-// at most one workgroup per CU, or two per CU of eight-row workgroups with a long K range
-// (measured: 384 eight-row workgroups at K >= 8192 gain 2-10 % from eight, 512
-// sixteen- or 32-row ones lose 3-8 %).  Otherwise four, fewer for very short K.
+// at most one workgroup per CU, or two per CU of eight-row workgroups with a long K range (the general
+// kernel; the lean one takes wider slices there, see make_plan).  Otherwise four, fewer for very short K.
 int choose_waves(int rows, int G, int split, int rw) {
     const int forced = tuning().gemv_waves;
     if (forced == 1 || forced == 2 || forced == 4 || forced == 8) return forced;
@@ -454,15 +453,19 @@ flute_status make_plan(const flute_linear *segs, int count, const void *x, void 
                       "a LUT grouped along K (K/split must be a multiple of 512 whose LUT rows fit a "
                       "workgroup's staging); try another split", who, K, split);
     }
-    // A lean launch whose tables and activations let fewer workgroups stay on a CU than its narrow
-    // slices need (a long K range over many rows): 32-row slices instead of a second round.  One
-    // token, 16-row slices and these: 11264 -> 12288, (4, 1) bits 41.7 -> 25.9 us, 12288 -> 12288 20.9
-    // -> 18.0, (2, 4) bits 33.4 -> 31.2; where all are resident either width measures the same.
+    // A lean launch of which fewer workgroups stay on a CU than its narrow slices need: wider slices
+    // instead of a second round.  Four wavefronts (tables and activations of a long K range over many rows
+    // leave no room for three workgroups): 32 rows.  One token, 16-row slices and these: 11264 -> 12288, (4, 1)
+    // bits 41.7 -> 25.9 us, 12288 -> 12288 20.9 -> 18.0, (2, 4) bits 33.4 -> 31.2; where all are resident either
+    // width measures the same.  Eight wavefronts (the registers leave room for one workgroup; 257 to 512 eight-row
+    // ones): 16 rows, which are one per CU and fill half of the chip or more; 32 rows leave up to three quarters
+    // of it idle.  The launch alone with 8, 16 and 32 rows: 8192 -> 3072, 4 bits 7.9 / 5.9 / 7.5 us, (3, 3) 11.5 /
+    // 8.7 / 13.0; 12288 -> 2176, (4, 1) 9.5 / 9.5 / 14.8; 12288 -> 3968, rotated, (2, 4) 19.9 / 16.4 / 21.9.
     if (tuning().gemv_rw == 0 && rw < 32 && !k_group && lean_serves(segs, count, G / split, rw, waves, silu_mul)) {
         const size_t lds = lean_table_bytes(lean_pair(segs, count)) + (size_t)(G / split) * 128 + kGemvRedBytes + 512;
         const long holds = std::min<long>(waves == 4 ? 3 : 1, (long)(kLdsPerCU / lds));
         if ((long)(rows / rw) * split > holds * kNumCU) {
-            rw = 32;
+            rw = waves == 8 ? 2 * rw : 32;
             waves = choose_waves(rows, G, split, rw);
         }
     }

@@ -565,6 +565,27 @@ def test_gemm_rows_names_the_kernel_of_a_call(monkeypatch):
         _lib.lib.flute_reload_tuning()
 
 
+@pytest.mark.parametrize("bits,bits2", [(4, 0), (4, 1), (3, 3), (2, 4), (3, 0)])
+@pytest.mark.parametrize("K", [8192, 11520, 12288, 16384])
+def test_gemv_rows_of_long_k_ranges(K, bits, bits2):
+    """257 to 512 eight-row workgroups of eight wavefronts, of which a CU holds one, become 16-row ones: at
+    most one per CU, on half of the 256 CUs or more.  Launches of four wavefronts widen to 32 rows."""
+    from _util import gemv_rows
+    from flute_extended import _lib
+    _lib.lib.flute_reload_tuning()
+    for N in range(128, 4097, 128):
+        rows, waves = gemv_rows((N, K, bits, bits2, 128))
+        groups = N // rows
+        if N <= 2048:
+            assert (rows, waves) == (8, 8)
+        else:
+            assert rows == 16 and waves == 8 and 128 <= groups <= 256
+    if 4 in (bits, bits2):                                               # 768 workgroups, two per CU at most
+        assert gemv_rows((12288, 12288, bits, bits2, 128))[0] == 32
+    if bits == 4:                                                        # groups of 32 rows: the general kernel
+        assert gemv_rows((2176, K, bits, bits2, 32)) == (8, 8)
+
+
 @pytest.mark.parametrize("waves", [4, 8])
 @pytest.mark.parametrize("N,K,bits,bits2", [(2176, 8192, 4, 0), (3072, 12288, 3, 3), (6144, 12288, 4, 1), (12288, 12288, 4, 0)])
 def test_gemv_rows_keeps_forced_wavefronts(monkeypatch, N, K, bits, bits2, waves):
