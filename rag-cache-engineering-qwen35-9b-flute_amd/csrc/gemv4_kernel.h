@@ -430,7 +430,13 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
             return;
         }
         if (tid < (1 << (2 * B))) {
-            const uint32_t v = lut_value(row, tid & ((1 << B) - 1)) | (lut_value(row, tid >> B) << 16);
+            uint32_t v;
+            if constexpr (B == 2) {                 // four values: a shift (selects become an array in scratch memory)
+                const uint64_t four = (uint64_t)row[0] | ((uint64_t)row[1] << 32);
+                v = (uint32_t)(four >> (16 * (tid & 3)) & 0xffffu) | ((uint32_t)(four >> (16 * (tid >> 2))) << 16);
+            } else {
+                v = lut_value(row, tid & ((1 << B) - 1)) | (lut_value(row, tid >> B) << 16);
+            }
             const uint4 v4 = make_uint4(v, v, v, v);
             uint8_t *ent = lds + base + tid * STRIDE;
 #pragma unroll

@@ -49,7 +49,7 @@ def _kernels():
     return found
 
 
-@pytest.mark.parametrize("kernel", ["gemm_few_kernel"])
+@pytest.mark.parametrize("kernel", ["gemm_few_kernel", "gemv4_kernel"])
 def test_lookup_kernels_use_no_scratch_memory(kernel):
     """Tables, codes and sums live in registers and LDS: a kernel with a private segment fetches some of
     them from memory (a local array with a runtime index, or registers spilled)."""
