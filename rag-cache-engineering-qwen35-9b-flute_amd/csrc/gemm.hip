@@ -38,8 +38,10 @@ int slices_of_k(int64_t units, int G, const GemmShape &shape) {
     return ks;
 }
 
-// Width pairs (the wider first) that the few-row kernel takes in one launch: those of deployed weights.
-bool few_takes(int b1, int b2) { return b1 == 3 ? b2 >= 2 : b1 == 4 ? b2 <= 2 : false; }
+// Width pairs (the wider first) that the few-row kernel takes in one launch: all but (4, 4), whose tables
+// and staged codes take 192 KB of LDS (a launch per stream, M = 8, 4096 -> 4096 16.3 us; the kernel before it,
+// which took both with half of the tables' replicas, 20.9).
+bool few_takes(int b1, int b2) { return !(b1 == 4 && b2 == 4); }
 
 // Microseconds of a call (one round = a workgroup per CU; `turns` = K tiles of a wavefront), fitted to
 // measurements on tiles of 16 and 32 rows: a fixed part, the pre-pass for 32 rows (16-row workgroups
@@ -493,7 +495,7 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
     // ---- workspace: [partial images][xb][Ap] -----------------------------------------
     const size_t image = (size_t)shape.mw * shape.mb * 8 * 64 * 4;
     // Two streams where no kernel takes both (four blocks of rows per wavefront: they do not fit the
-    // register file; widths that no deployed weight has): one launch per stream, both write partial
+    // register file; twice 4 bits): one launch per stream, both write partial
     // tiles and the last workgroup of the second launch folds everything, exactly as a K split does.
     const bool per_stream = p.nstreams == 2 && !(few && few_takes(p.bits[0], p.bits[1]));
     const int zparts = ksplit * (per_stream ? 2 : 1);

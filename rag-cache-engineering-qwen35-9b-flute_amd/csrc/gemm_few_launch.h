@@ -31,10 +31,15 @@ flute_status launch_few_bits(const GemmParams &p, dim3 grid, hipStream_t stream)
         case 8 * 2: return launch_few<MB, BF16, 2, 0, SEGS>(p, grid, stream);
         case 8 * 3: return launch_few<MB, BF16, 3, 0, SEGS>(p, grid, stream);
         case 8 * 4: return launch_few<MB, BF16, 4, 0, SEGS>(p, grid, stream);
+        case 8 * 1 + 1: return launch_few<MB, BF16, 1, 1, SEGS>(p, grid, stream);
+        case 8 * 2 + 1: return launch_few<MB, BF16, 2, 1, SEGS>(p, grid, stream);
+        case 8 * 2 + 2: return launch_few<MB, BF16, 2, 2, SEGS>(p, grid, stream);
+        case 8 * 3 + 1: return launch_few<MB, BF16, 3, 1, SEGS>(p, grid, stream);
         case 8 * 3 + 2: return launch_few<MB, BF16, 3, 2, SEGS>(p, grid, stream);
         case 8 * 3 + 3: return launch_few<MB, BF16, 3, 3, SEGS>(p, grid, stream);
         case 8 * 4 + 1: return launch_few<MB, BF16, 4, 1, SEGS>(p, grid, stream);
         case 8 * 4 + 2: return launch_few<MB, BF16, 4, 2, SEGS>(p, grid, stream);
+        case 8 * 4 + 3: return launch_few<MB, BF16, 4, 3, SEGS>(p, grid, stream);
     }
     set_error("flute_gemm: no few-row kernel for widths (%d, %d)", p.bits[0], p.bits[1]);
     return FLUTE_ERR_UNSUPPORTED;

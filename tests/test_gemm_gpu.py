@@ -141,7 +141,8 @@ def test_gemm_dual_stream_fp16(M, N, K, bits, gs, bits2, rank, bias):
     assert torch.equal(y, _dual(w, x).cpu())
 
 
-@pytest.mark.parametrize("bits,bits2", [(4, 0), (3, 0), (2, 0), (1, 0), (4, 1), (1, 4), (3, 3), (2, 4), (3, 2), (4, 4), (1, 2)])
+@pytest.mark.parametrize("bits,bits2", [(4, 0), (3, 0), (2, 0), (1, 0), (4, 1), (1, 4), (3, 3), (2, 4), (3, 2), (4, 4), (1, 2),
+                                        (1, 1), (2, 2), (1, 3), (4, 3)])
 @pytest.mark.parametrize("M,N,K,gs,rows,slices", [
     (1, 128, 64, 128, "16", None),      # one tile of K: seven wavefronts without one
     (16, 256, 576, 16, "16", "2"),      # nine tiles in slices of five and four

@@ -56,3 +56,16 @@ def test_lookup_kernels_use_no_scratch_memory(kernel):
     kernels = {n: k for n, k in _kernels().items() if kernel in n}
     assert kernels
     assert not {n: k[".private_segment_fixed_size"] for n, k in kernels.items() if k[".private_segment_fixed_size"]}
+
+
+def test_few_row_kernel_takes_width_pairs_in_one_launch():
+    """Every pair of widths, the wider first, in 16- and 32-row workgroups, both LUT types, one weight and
+    several; not (4, 4), whose tables and codes exceed a CU's LDS."""
+    kernels = _kernels()
+    for rows in (1, 2):
+        for bf16 in (0, 1):
+            for segs in (0, 1):
+                for b1 in (1, 2, 3, 4):
+                    for b2 in range(b1 + 1):
+                        name = f"_ZN5flute15gemm_few_kernelILi{rows}ELb{bf16}ELi{b1}ELi{b2}ELb{segs}EEEvNS_10GemmParamsE"
+                        assert (name in kernels) == ((b1, b2) != (4, 4)), name
