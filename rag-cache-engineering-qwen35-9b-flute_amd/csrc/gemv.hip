@@ -778,13 +778,14 @@ flute_status launch_width(Plan &plan, hipStream_t stream) {
             const int u = (plan.p.gs_tiles / (64 >> plan.p.lpg_log2)) / nw;
             if (pf == 4 && plan.pair == 14 && u % 8 == 0 && tuning().gemv4_pf == 0) pf = 8;
             // Grids beyond the resident workgroups walk here too (one weight: gate and up are never that
-            // wide), both tables kept while the slices share their LUT rows.  The call, one workgroup per
+            // wide; 32-row slices: choose_shape has no more workgroups of narrower ones than are resident),
+            // both tables kept while the slices share their LUT rows.  The call, one workgroup per
             // slice and walking:
             //   4096 -> 151936, (4, 1) bits  90.2 -> 79.5 us       4096 -> 248320, 3 bits        93.8 -> 86.3
             //   4096 -> 128000, (2, 4)       87.6 -> 82.5          4096 -> 51200, (1, 4), rotated 42.4 -> 33.1
             //   4096 -> 167552, (3, 3)      111.8 -> 110.2         1024 -> 51200, (3, 3)         17.5 -> 14.3
             int gx = plan.grid_x;
-            if (nw == 4 && pf >= 4 && plan.p.nsegs == 1)
+            if (nw == 4 && pf >= 4 && plan.p.nsegs == 1 && plan.p.lpg_log2 == 6)
                 if (const int resident = walking_grid(plan)) gx = resident;
             return (plan.pair == 41 || plan.pair == 14)
                        ? launch_gemv_pair_1bit(plan.p, plan.pair, gx, nw, pf, plan.lds_bytes, BF16, stream)
@@ -792,7 +793,7 @@ flute_status launch_width(Plan &plan, hipStream_t stream) {
         }
         // K ranges that do not divide into equal, even numbers of loads: the lean kernel's ragged form, which
         // is the faster one wherever it fits.  One token, the general kernel and this one, the launch alone:
-        //   3968 -> 2 x 11520, (1, 4) bits   30.0 -> 22.8 us      11520 -> 3968             25.7 -> 16.2
+        //   3968 -> 2 x 11520, (1, 4) bits   30.0 -> 22.8 us      11520 -> 3968             25.7 -> 11.1
         //   2944 -> 2 x 11904, rotated       23.5 -> 19.0         11904 -> 2944, rotated    20.6 -> 17.4
         //   1152 -> 2 x 4480, (2, 4) bits    19.2 -> 14.8         4480 -> 1152              12.8 -> 9.1
         //   2432 -> 2 x 2304, (3, 3), rotated 20.8 -> 16.1        4032 -> 2048, 512, 512    9.5 -> 6.4
@@ -800,7 +801,7 @@ flute_status launch_width(Plan &plan, hipStream_t stream) {
         // and of the pairs' walking grid, the call: 3008 -> 100352, (2, 3) bits 58.6 -> 52.8, 3 bits 35.2 -> 30.2;
         // 1600 -> 90112, (4, 1) 28.9 -> 26.6
         int gx = plan.grid_x;
-        if (nw == 4 && (plan.pair == 0 || plan.p.nsegs == 1))
+        if (nw == 4 && (plan.pair == 0 || plan.p.nsegs == 1) && plan.p.lpg_log2 == 6)
             if (const int resident = walking_grid(plan)) gx = resident;
         return (plan.pair == 0 || plan.pair == 14 || plan.pair == 41)
                    ? launch_gemv_ragged_a(plan.p, plan.pair, gx, nw, plan.lds_bytes, BF16, stream)

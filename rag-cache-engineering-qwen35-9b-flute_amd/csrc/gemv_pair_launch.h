@@ -35,21 +35,13 @@ flute_status launch_pair_grid(const GemvParams &p, int grid_x, size_t lds_bytes,
 template <bool BF16, int BA, int BB>
 flute_status launch_pair(const GemvParams &p, int grid_x, int nw, int pf, size_t lds_bytes, hipStream_t stream) {
     constexpr bool NARROW = BA == 1;                 // the deep ring: for a 1-bit stream in front
-    if (p.slices > 0) {                              // a walking grid (pf 4 or 8: the caller checks)
+    if (p.slices > 0) {                              // a walking grid (32-row slices, pf 4 or 8: the caller checks)
         if constexpr (NARROW) {
-            if (pf == 8) {
-                switch (p.lpg_log2) {
-                    case 4: return launch_pair_grid<4, 4, 4, BF16, BA, BB, true, true>(p, grid_x, lds_bytes, stream);
-                    case 5: return launch_pair_grid<5, 4, 4, BF16, BA, BB, true, true>(p, grid_x, lds_bytes, stream);
-                    default: return launch_pair_grid<6, 4, 4, BF16, BA, BB, true, true>(p, grid_x, lds_bytes, stream);
-                }
-            }
+            if (pf == 8) return launch_pair_grid<6, 4, 4, BF16, BA, BB, true, true>(p, grid_x, lds_bytes, stream);
         }
-        switch (p.lpg_log2) {
-            case 4: return launch_pair_grid<4, 4, 4, BF16, BA, BB, false, true>(p, grid_x, lds_bytes, stream);
-            case 5: return launch_pair_grid<5, 4, 4, BF16, BA, BB, false, true>(p, grid_x, lds_bytes, stream);
-            default: return launch_pair_grid<6, 4, 4, BF16, BA, BB, false, true>(p, grid_x, lds_bytes, stream);
-        }
+        if constexpr (!(BA == 4 && BB == 1))         // (of one weight, the 1-bit stream comes first)
+            return launch_pair_grid<6, 4, 4, BF16, BA, BB, false, true>(p, grid_x, lds_bytes, stream);
+        return FLUTE_ERR_UNSUPPORTED;                // (not reached: several weights do not walk)
     }
     switch (nw * 100 + p.lpg_log2 * 10 + pf) {
         case 442: return launch_pair_grid<4, 4, 2, BF16, BA, BB>(p, grid_x, lds_bytes, stream);
@@ -93,15 +85,12 @@ flute_status launch_ragged_grid(const GemvParams &p, int grid_x, size_t lds_byte
     return FLUTE_OK;
 }
 
-// p.slices > 0: a walking grid (four wavefronts)
+// p.slices > 0: a walking grid (four wavefronts, 32-row slices)
 template <bool BF16, int BA, int BB>
 flute_status launch_ragged(const GemvParams &p, int grid_x, int nw, size_t lds_bytes, hipStream_t stream) {
     if (p.slices > 0) {
-        switch (p.lpg_log2) {
-            case 4: return launch_ragged_grid<4, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
-            case 5: return launch_ragged_grid<5, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
-            default: return launch_ragged_grid<6, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
-        }
+        if constexpr (!(BA == 4 && BB == 1)) return launch_ragged_grid<6, 4, BF16, true, BA, BB>(p, grid_x, lds_bytes, stream);
+        return FLUTE_ERR_UNSUPPORTED;                // (not reached, as above)
     }
     switch (nw * 10 + p.lpg_log2) {
         case 44: return launch_ragged_grid<4, 4, BF16, false, BA, BB>(p, grid_x, lds_bytes, stream);
