@@ -504,7 +504,6 @@ __device__ __forceinline__ u4_t quad_transpose(u4_t v, int lane) {
     return out;
 }
 
-// One stream of B1-bit codes.
 // Block mb of an activation half: 16 bytes per lane at src + mb KB, as a statement the compiler
 // does not take for a load (no wait of its own follows).
 __device__ __forceinline__ void lean_load16(u4_t &dst, const u4_t *src, int mb) {
@@ -516,14 +515,16 @@ __device__ __forceinline__ void lean_load16(u4_t &dst, const u4_t *src, int mb) 
     }
 }
 
-// LEAN (four blocks per wavefront, one 4-bit stream, one LUT group per tile): every vector memory
+// One stream of B1-bit codes, four blocks of rows per wavefront (fewer rows: gemm_few_kernel.h).
+// LEAN (one 4-bit stream, one LUT group per tile): every vector memory
 // instruction of the kernel is written out and so is every wait for one.  The tile goes straight
 // into LDS (global_load_lds_dwordx4), which frees the sixteen registers a tile in flight would
 // hold; the compiler cannot count such loads next to its own (it answers one in flight with
 // vmcnt(0) in front of the next use of any loaded register), hence all or nothing.
 template <int MB, int KW, int MW, bool BF16, int B1, bool PERM = false, bool LEAN = false, bool SEGS = false>
 __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) {
-    static_assert(!LEAN || (PERM && MB >= 2 && B1 == 4), "lean loop: fast path, operand image");
+    static_assert(MB == 4 && KW * MW == 8, "64 or 128 rows");
+    static_assert(!LEAN || (PERM && B1 == 4), "lean loop: fast path, operand image");
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int NT = 64 * KW * MW;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -620,7 +621,6 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
         uint32_t lv;
         asm volatile("global_load_ushort %0, %1, off" : "=&v"(lv) : "v"(lp) : "memory");
         lean_tile(0);                                  // tile 0
-        static_assert(MB == 4 || MB == 2, "operands of a half");
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) lean_load16(A0[mb], ap, mb);
 #pragma unroll
@@ -780,12 +780,8 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
                     __builtin_amdgcn_sched_barrier(0);
                 };
                 auto wait_half = [&](u4_t (&Aj)[MB], auto younger) {
-                    if constexpr (MB == 4)
-                        asm volatile("s_waitcnt vmcnt(%4)" : "+v"(Aj[0]), "+v"(Aj[1]), "+v"(Aj[2]), "+v"(Aj[3])
-                                     : "n"(decltype(younger)::value) : "memory");
-                    else
-                        asm volatile("s_waitcnt vmcnt(%2)" : "+v"(Aj[0]), "+v"(Aj[1])
-                                     : "n"(decltype(younger)::value) : "memory");
+                    asm volatile("s_waitcnt vmcnt(%4)" : "+v"(Aj[0]), "+v"(Aj[1]), "+v"(Aj[2]), "+v"(Aj[3])
+                                 : "n"(decltype(younger)::value) : "memory");
                 };
                 // (the same in every lane: a scalar count gives a scalar loop)
                 left = __builtin_amdgcn_readfirstlane(left);
@@ -939,45 +935,43 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
     // hold the same block and the odd one gives its sums to the even one.  The same bytes cross
     // LDS as in the tree and the sums are the same (every addition commutes), but all eight
     // wavefronts move them, barriers go, and four or eight wavefronts write the totals tile.
-    const bool scattered = MB == 4 && KW * MW == 8 && p.scatter != 0;
-    if constexpr (MB == 4 && KW * MW == 8) {
-        if (scattered) {
-            constexpr int P1 = KW == 4 ? 2 : 4, P2 = KW == 4 ? 1 : 2;   // partners of the two hand-overs
-            f4_t *mine1 = red + (size_t)wave * 1024;
-            const f4_t *theirs1 = red + (size_t)(wave ^ P1) * 1024;
+    const bool scattered = p.scatter != 0;
+    if (scattered) {
+        constexpr int P1 = KW == 4 ? 2 : 4, P2 = KW == 4 ? 1 : 2;   // partners of the two hand-overs
+        f4_t *mine1 = red + (size_t)wave * 1024;
+        const f4_t *theirs1 = red + (size_t)(wave ^ P1) * 1024;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                mine1[i * 64 + lane] = acc[2][i];
-                mine1[(8 + i) * 64 + lane] = acc[3][i];
+        for (int i = 0; i < 8; ++i) {
+            mine1[i * 64 + lane] = acc[2][i];
+            mine1[(8 + i) * 64 + lane] = acc[3][i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            acc[0][i] += theirs1[i * 64 + lane];
+            acc[1][i] += theirs1[(8 + i) * 64 + lane];
+        }
+        __syncthreads();
+        // second hand-over: behind the region the totals tile takes (17 * 4 KB from the start)
+        f4_t *mine2 = red + 4352 + (size_t)wave * 512;
+        const f4_t *theirs2 = red + 4352 + (size_t)(wave ^ P2) * 512;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) mine2[i * 64 + lane] = acc[1][i];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[0][i] += theirs2[i * 64 + lane];
+        if constexpr (KW == 8) {
+            // k ways kw and kw ^ 1 hold the same block: between the (smaller) totals tile
+            // and the second hand-over's areas
+            f4_t *pair3 = red + 2176 + (size_t)(wave >> 1) * 512;
+            if (kw & 1) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) pair3[i * 64 + lane] = acc[0][i];
             }
             __syncthreads();
+            if (!(kw & 1)) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                acc[0][i] += theirs1[i * 64 + lane];
-                acc[1][i] += theirs1[(8 + i) * 64 + lane];
-            }
-            __syncthreads();
-            // second hand-over: behind the region the totals tile takes (17 * 4 KB from the start)
-            f4_t *mine2 = red + 4352 + (size_t)wave * 512;
-            const f4_t *theirs2 = red + 4352 + (size_t)(wave ^ P2) * 512;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) mine2[i * 64 + lane] = acc[1][i];
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < 8; ++i) acc[0][i] += theirs2[i * 64 + lane];
-            if constexpr (KW == 8) {
-                // k ways kw and kw ^ 1 hold the same block: between the (smaller) totals tile
-                // and the second hand-over's areas
-                f4_t *pair3 = red + 2176 + (size_t)(wave >> 1) * 512;
-                if (kw & 1) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) pair3[i * 64 + lane] = acc[0][i];
-                }
-                __syncthreads();
-                if (!(kw & 1)) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) acc[0][i] += pair3[i * 64 + lane];
-                }
+                for (int i = 0; i < 8; ++i) acc[0][i] += pair3[i * 64 + lane];
             }
         }
     }
