@@ -179,32 +179,26 @@ flute_status launch_rowshift(const void *rows, int64_t ld, int M, int K, int *sh
     return FLUTE_OK;
 }
 
-// LDS plan of one launch: pair tables (+ staging on the fast path), sized against the
-// reduction tree and the totals tile that reuse the same memory afterwards.
-// A single 4-bit stream with at most two LUT groups per 128-row tile gets 64-lane
-// replication (256 bytes per entry, 64 KB per group, first table at LDS offset 0: the
-// layout the one-instruction address needs).  Everything else: as much replication as
-// the budget allows, 32 lanes at most.
+// LDS plan of one launch of gemm_kernel, one stream: the pair table (+ staging on the fast path), sized
+// against the reduction tree and the totals tile that reuse the same memory afterwards.
+// 4 bits with at most two LUT groups per 128-row tile get 64-lane replication (256 bytes per entry,
+// 64 KB per group, table at LDS offset 0: the layout the one-instruction address needs).  Everything
+// else: as much replication as the budget allows, 32 lanes at most.
 int plan_lds(GemmParams &p, const GemmShape &shape) {
     const int ngrp = p.seg[0].gs >= 128 ? 1 : 128 / p.seg[0].gs;
-    const bool perm = p.nstreams == 1 && p.bits[0] == 4 && ngrp <= 2 &&
-                      !tuning().gemm_no_perm;
-    const int table_budget = 96 * 1024 / p.nstreams;
-    int lds_tables = 0;
-    for (int s = 0; s < p.nstreams; ++s) {
-        const int entries = ngrp << (2 * p.bits[s]);
-        int rl = 5;
-        while (rl > 0 && (entries << rl) * 4 > table_budget) --rl;
-        if (perm) rl = 6;
-        p.rep_log2[s] = rl;
-        p.tab_off[s] = lds_tables;
-        lds_tables += (entries << rl) * 4;
-    }
+    const bool perm = p.bits[0] == 4 && ngrp <= 2 && !tuning().gemm_no_perm;
+    const int table_budget = 96 * 1024, entries = ngrp << (2 * p.bits[0]);
+    int rl = 5;
+    while (rl > 0 && (entries << rl) * 4 > table_budget) --rl;
+    if (perm) rl = 6;
+    p.rep_log2[0] = rl;
+    p.tab_off[0] = 0;
+    int lds_tables = (entries << rl) * 4;
     p.lean = 0;
-    if (perm) {                                  // per-wavefront tile staging behind the tables
-        // four blocks per wavefront and one LUT group per tile: the lean loop, whose tiles go
-        // straight into two staging buffers per wavefront
-        p.lean = shape.mb == 4 && ngrp == 1 && !tuning().gemm_no_lean;
+    if (perm) {                                  // per-wavefront tile staging behind the table
+        // one LUT group per tile: the lean loop, whose tiles go straight into two staging buffers
+        // per wavefront
+        p.lean = ngrp == 1 && !tuning().gemm_no_lean;
         p.stage_off = lds_tables;
         lds_tables += shape.kw * shape.mw * (p.lean ? 8192 : 4096);
         if (p.lean) {                            // one progress word per wavefront
