@@ -497,11 +497,18 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
     const CoeffPlan coeff = plan_coeff(ws, count, M);
     size_t xb_floats = any_res ? coeff.floats() : 0;
     for (int i = 0; i < count; ++i) xb_floats += ((size_t)M * ws[i].R + 3) & ~(size_t)3;
-    const size_t ap_floats = (size_t)p.G * 2 * p.mblk_pad * 64 * 4;
     const size_t rot_floats = w->signs ? ((size_t)M * w->K / 2 + 4) & ~(size_t)3 : 0;
     // bfloat16 activations presented as float16 operands: one power-of-two scale per row
     const bool scale_rows = act_dtype == FLUTE_BF16 && w->lut_dtype == FLUTE_F16;
     const size_t shift_floats = scale_rows ? ((size_t)M + 3) & ~(size_t)3 : 0;
+    // One block of rows per wavefront: the kernel reads A itself (16-byte pieces of a row, put into
+    // operand order in registers), so the pre-pass launch is dropped, and the image with it.  Needs
+    // 16-byte aligned rows; rotated rows are read the same way (the rotation can write the image itself,
+    // but only without a residual and row scales).
+    const bool image_of_rotation = w->signs && !any_res && !scale_rows;
+    const bool rows16 = w->signs || (((uintptr_t)A & 15) == 0 && lda % 8 == 0);
+    const bool direct = shape.mb == 1 && !tuning().gemm_no_direct && rows16 && !image_of_rotation;
+    const size_t ap_floats = direct ? 0 : (size_t)p.G * 2 * p.mblk_pad * 64 * 4;
     float *base = nullptr;
     int *tickets = nullptr;
     const size_t want_tickets = std::max((size_t)units, any_res ? coeff.tickets() : 0) + 1;
@@ -515,12 +522,7 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
     p.Ap = Ap;
     int *rowshift = scale_rows
         ? (int *)(base + p_floats + xb_floats + ap_floats + rot_floats) : nullptr;
-    // One block of rows per wavefront: the kernel reads A itself (16-byte pieces of a row, put into
-    // operand order in registers), so the pre-pass launch is dropped.  Needs 16-byte aligned rows;
-    // rotated rows are read the same way (the rotation can write the image itself, but only without a
-    // residual and row scales).
-    const bool direct = shape.mb == 1 && !tuning().gemm_no_direct;
-    if (w->signs && !any_res && !scale_rows) {
+    if (image_of_rotation) {
         // the rotation writes the operand image itself: one launch instead of two
         FhtOperandOut image_out = {(uint32_t *)Ap, p.mblk_pad, (int)(w->lut_dtype == FLUTE_BF16), block_xor};
         st = fht_launch(A, lda, w->signs, w->awq, nullptr, 0, M, w->K, act_dtype, 0, w->rot_block,
@@ -530,7 +532,7 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
         if (w->signs) {
             // the residual coefficients and the row scales need the rotated rows as rows:
             // rotated copy first, then the ordinary pre-pass on it
-            void *Arot = (void *)(Ap + (size_t)p.G * 2 * p.mblk_pad * 64);
+            void *Arot = (void *)((float *)Ap + ap_floats);
             st = fht_launch(A, lda, w->signs, w->awq, Arot, w->K, M, w->K, act_dtype, 0,
                             w->rot_block, stream, nullptr, rowshift);
             if (st != FLUTE_OK) return st;
@@ -538,7 +540,7 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
             lda = w->K;
         }
         p.rowshift = rowshift;                          // (the rotation knows its rows' largest exponents)
-        const bool rows16 = ((uintptr_t)A & 15) == 0 && lda % 8 == 0, find = scale_rows && !w->signs;
+        const bool find = scale_rows && !w->signs;
         ImageParams im = {};
         im.A = (const uint16_t *)A;
         im.lda = lda;
@@ -554,7 +556,7 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
             st = launch_rowshift(A, lda, M, w->K, rowshift, stream);
             if (st != FLUTE_OK) return st;
         }
-        if (direct && rows16) {
+        if (direct) {
             p.A8 = (const u4_t *)A;
             p.lda8 = lda / 8;
             p.a_bf16 = act_dtype == FLUTE_BF16;
