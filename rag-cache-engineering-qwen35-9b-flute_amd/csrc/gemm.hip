@@ -90,7 +90,9 @@ GemmShape choose_gemm_shape(int M, int tiles, int G, int b1, int b2, double &us)
     if (v == 64) return {4, 8, 1, 1};
     if (v == 128) return {4, 4, 2, 1};
     const double few1 = few_us(1, M, tiles, G, b1, b2), few2 = few_us(2, M, tiles, G, b1, b2);
-    if (M <= 16 || (few1 <= few2 && few1 < other)) {
+    // (row blocks that gridDim.y holds)
+    const bool fits1 = M <= 65535 * 16, fits2 = M <= 65535 * 32;
+    if (M <= 16 || (fits1 && few1 <= few2 && few1 < other)) {
         us = few1;
         return {1, 8, 1, 1};
     }
@@ -101,7 +103,7 @@ GemmShape choose_gemm_shape(int M, int tiles, int G, int b1, int b2, double &us)
     const GemmShape shape = other_shape(M, tiles);
     const double short_by = shape.mw == 1
         ? std::min(4.0, std::max(0.0, 8.0 - G / slices_of_k((int64_t)tiles * ((M + 63) / 64), G, shape) / 16.0)) : 0.0;
-    if (few2 < other + short_by) {
+    if (fits2 && few2 < other + short_by) {
         us = few2;
         return {2, 8, 1, 1};
     }

@@ -602,6 +602,17 @@ def test_gemv_rows_keeps_forced_wavefronts(monkeypatch, N, K, bits, bits2, waves
         _lib.lib.flute_reload_tuning()
 
 
+@pytest.mark.parametrize("bits,bits2", [(1, 1), (4, 0), (4, 1), (4, 4)])
+@pytest.mark.parametrize("N,K", [(128, 64), (1024, 4096), (12288, 65472)])
+def test_gemm_rows_of_millions_of_rows_fit_the_grid(N, K, bits, bits2):
+    """16- and 32-row workgroups are taken while the grid holds their row blocks (65535): a call of more
+    rows that a wider shape serves is not refused for the estimate of a narrow one."""
+    from _util import gemm_rows
+    for M in (1 << 20, (1 << 20) + 1, 1 << 21, 65535 * 128):
+        rows = gemm_rows(M, (N, K, bits, bits2, 128))
+        assert rows >= 256 or -(-M // rows) <= 65535
+
+
 def test_operand_addresses_compiled_and_not(monkeypatch):
     """The compiled walk over the members' operands finds what the attribute lookup finds: buffers,
     parameters, attributes of the object in front of either, classes without a module's dictionaries."""
