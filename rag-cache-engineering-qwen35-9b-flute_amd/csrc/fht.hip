@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(kFhtThreads) fht_row_kernel(const FhtParams p)
     }
     uint32_t top = 0;
     float sg[P][8];
-    transform_row<8, P>(
+    transform_row<P>(
         (float *)lds, p.K, p.block, tid, kFhtThreads,
         [&](int h, int j, float (&f)[8]) {
             float sc[8];
@@ -303,7 +303,7 @@ flute_status fht_launch(const void *x, int64_t ldx, const float *signs, const fl
     }
     const int rows = operand ? operand->mblk_pad * 16 : M;
     if (rows == 0) return FLUTE_OK;
-    if (K <= transform_reach(8, 4, kFhtThreads)) {
+    if (K <= transform_reach(4, kFhtThreads)) {
         lds_bytes = lds_bytes ? (size_t)K * 4 : 0;
         switch ((K + kFhtThreads * 8 - 1) / (kFhtThreads * 8)) {
             case 1: return launch_row<1>(p, rows, lds_bytes, stream);

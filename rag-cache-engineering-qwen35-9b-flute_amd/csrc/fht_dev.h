@@ -213,7 +213,7 @@ __device__ __forceinline__ void stage_some_lanes(float (&f)[N], int lane, bool t
 // neighbours access together lie on different banks, as do the consecutive columns of a pass.
 __device__ __forceinline__ int row_slot(int i) { return i ^ ((i >> 3) & 4); }
 
-// R stages of length 2^SH0 (512 or 1024 columns, or sixteen times that) and up over the 2^nst columns
+// R stages of length 2^SH0 (512 columns, or sixteen times that) and up over the 2^nst columns
 // from `off` on (a multiple of 2^nst).  Bits of a column above row_slot's reach are apart from it, so
 // the columns of a group lie at constant distances from the first: one address, the rest immediates.
 template <int R, int SH0>
@@ -233,14 +233,14 @@ __device__ __forceinline__ void row_pass(float *buf, int off, int nst, int tid, 
     }
 }
 
-// Columns of a row that transform_row reaches with P pieces of N columns a thread.
-constexpr int transform_reach(int N, int P, int nthreads) { return N * P * nthreads; }
+// Columns of a row that transform_row reaches with P pieces of eight columns a thread.
+constexpr int transform_reach(int P, int nthreads) { return 8 * P * nthreads; }
 
 // Transform of a whole row of K columns (K and the block multiples of 32, K up to transform_reach),
-// all its segments side by side: thread `tid` holds the N consecutive columns at (h * nthreads + tid) * N
+// all its segments side by side: thread `tid` holds the eight consecutive columns at (h * nthreads + tid) * 8
 // for h = 0 ... P - 1, load(h, j, f) fetches them and store(h, j, f, stages) gets them back.  The
 // first stages stay in registers, the rest are one or two passes over `buf` (K floats of LDS, needed
-// for blocks and segments beyond 64 * N columns), with two or three barriers whatever the number of
+// for blocks and segments beyond 512 columns), with two or three barriers whatever the number of
 // segments.  Every value goes through the same single roundings as in the buffered butterfly.
 // Called by all threads; on return no wavefront reads another's columns in the buffer any more.
 // What bounds it, for one row: vector instructions of one CU (about thirty a column over 64 lanes) and
@@ -248,10 +248,9 @@ constexpr int transform_reach(int N, int P, int nthreads) { return N * P * nthre
 // each), eight dword accesses a thread and column-wise addresses: 1 x 12288 9.0 -> 7.6 us, 800 x 11072
 // 22.8 -> 20.0, 1000 x 4096 9.2 -> 8.1; the fused prologue, one token: 11072 -> 4096 22.5 -> 14.4 us
 // (with the ragged GEMV), 12288 -> 4096, (3, 3) bits 17.2 -> 15.9.
-template <int N, int P, class Load, class Store>
+template <int P, class Load, class Store>
 __device__ __forceinline__ void transform_row(float *buf, int K, int block, int tid, int nthreads, Load load, Store store) {
-    constexpr int own = N == 8 ? 3 : 4, sh = own + 6;
-    static_assert(N == 8 || N == 16, "columns of a thread");
+    constexpr int N = 8, own = 3, sh = own + 6;         // columns of a thread; stages in it, in a wavefront
     const int lane = tid & 63;
     float f[P][N];
 #pragma unroll

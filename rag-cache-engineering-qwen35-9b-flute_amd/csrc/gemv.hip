@@ -147,7 +147,7 @@ __global__ void __launch_bounds__(kPreThreads) gemv_pre_kernel(const PreParams p
         dot(0, p.K, [&](int k, float (&x)[8]) { pre_unpack8(*(const uint4 *)(p.x + k), p.act_bf16, x); });
     } else if constexpr (WHOLE) {
         float sg[4][8];
-        transform_row<8, 4>(
+        transform_row<4>(
             buf, p.K, p.rot_block, tid, kPreThreads,
             [&](int h, int j, float (&f)[8]) {
                 pre_unpack8(*(const uint4 *)(p.x + j), p.act_bf16, f);
@@ -620,7 +620,7 @@ flute_status make_plan(const flute_linear *segs, int count, const void *x, void 
     // would otherwise hold.
     p.rot_whole = 0;
     if (plan->lean && any_fused_rot && (fht_block > 256 || (fht_block == 0 && split == 1)) &&
-        kc <= transform_reach(8, kRotPieces, waves * 64)) {
+        kc <= transform_reach(kRotPieces, waves * 64)) {
         const auto total = [&](size_t head) {
             return ((head + 255) & ~(size_t)255) + ((kc * 2 + 15) & ~15) + kGemvRedBytes + 16 + 8 * 4;
         };
@@ -874,7 +874,7 @@ flute_status launch(Plan &plan, int act_dtype, hipStream_t stream, float *fixed_
         for (int i = 0; i < plan.npre; ++i) ranks += plan.pre[i].R;
         pp.rows = 1;
         while (pp.rows < kPreWaves && ranks > kNumCU * pp.rows) pp.rows *= 2;
-        const bool whole = plan.p.K <= transform_reach(8, 4, kPreThreads);
+        const bool whole = plan.p.K <= transform_reach(4, kPreThreads);
         int blocks = 0;
         size_t lds = 0;
         for (int i = 0; i < plan.npre; ++i) {

@@ -584,7 +584,7 @@ __device__ int stage_x(const GemvParams &p, const uint16_t *x, const float *sign
         // (k0 is a multiple of the block, or 0)
         constexpr int P = kRotPieces;
         float sg[P][8];
-        transform_row<8, P>(
+        transform_row<P>(
             buf, kc, p.fht_block, tid, nthreads,
             [&](int h, int j, float (&f)[8]) {
                 load_act8(x, k0 + j, p.act_bf16, f);
