@@ -49,6 +49,9 @@ bool few_takes(int b1, int b2) { return !(b1 == 4 && b2 == 4); }
 // M = 32, 4096 -> 12288, 16 and 32 rows: 4 bits 14.6 / 16.0, (4, 1) bits 19.6 / 18.5, (3, 3) 24.7 / 21.1;
 // M = 64: 27.5 / 17.1, 36.4 / 23.5, 46.6 / 28.3; M = 64, 12288 -> 4096: 22.2 / 19.6, 29.6 / 24.5,
 // 37.9 / 28.4; M = 128, 4096 -> 4096: 15.5 / 16.1, 20.6 / 19.5, 25.7 / 22.0.
+// (A residual's launch in front of 16-row workgroups is not in it.  Where the choice misses: M = 22,
+// 6912 -> 4224, (2, 3) bits, rank 16: 16 rows 28.4, 32 rows 23.4; M = 233, 1408 -> 8448, twice 1 bit: the
+// many-row kernel 30.7, 16 rows 25.2; over 58 other random shapes it is within 3 % of the best of six.)
 double few_us(int mb, int M, int tiles, int G, int b1, int b2) {
     static const double tile_us[5] = {0.0, 0.6, 0.75, 1.2, 1.15};
     const GemmShape shape = {mb, 8, 1, 1};

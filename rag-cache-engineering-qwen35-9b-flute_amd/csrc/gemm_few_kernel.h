@@ -5,10 +5,11 @@
 // Workgroup = eight wavefronts on one 128-row tile of the weight; wavefront w takes the K tiles w,
 // w + 8, ... of the workgroup's slice of K, for MB blocks of 16 rows of A, both streams of a tile one
 // after the other on the same activations.  What bounds it: such a launch is a few trips to memory and
-// through LDS around a loop of a few microseconds (M = 48, 12288 -> 4096, four slices of K: 5 us of
-// loop in a launch of 18), so a second stream costs its loop here and not a launch of its own, and the
-// eight wavefronts' sums cross LDS once, every thread adding the eight terms of the outputs it then
-// stores, instead of a tree of three steps with two barriers each and a totals tile behind it.
+// through LDS around a loop of a few microseconds (M = 48, 12288 -> 4096, four slices of K, six tiles a
+// wavefront: 4 bits 8 us of loop in a launch of 16, (4, 1) bits 13 of 22), so a second stream costs its
+// loop here and not a launch of its own, and the eight wavefronts' sums cross LDS once, every thread
+// adding the eight terms of the outputs it then stores, instead of a tree of three steps with two
+// barriers each and a totals tile behind it.
 #pragma once
 
 #include "gemm_kernel.h"
