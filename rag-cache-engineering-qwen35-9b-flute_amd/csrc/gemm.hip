@@ -214,7 +214,10 @@ int plan_lds(GemmParams &p, const GemmShape &shape) {
     }
     const int slot_bytes = shape.mb * 8 * 64 * 16;
     const int lds_reduce = (shape.kw / 2) * shape.mw * slot_bytes;
-    const int lds_tile = shape.mw * shape.mb * 16 * 132 * 4 + 16;   // totals tile + ticket flag
+    const int rows = shape.mw * shape.mb * 16;
+    bool residual = false;
+    for (const GemmSeg &g : p.seg) residual |= g.R > 0;
+    const int lds_tile = gemm_residual_offset(rows) + (residual ? rows * 132 * 4 : 0);
     int lds = lds_tables > lds_reduce ? lds_tables : lds_reduce;
     if (lds_tile > lds) lds = lds_tile;
     // the hand-overs between the k ways: eight 16 KB areas, then eight of 8 KB behind the totals tile
@@ -585,7 +588,7 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
             if (ws[i].R == 0) continue;
             to[i] = next;
             p.seg[i].xb = next;
-            p.seg[i].vec_res = ws[i].R % 8 == 0 && ((uintptr_t)ws[i].resA & 15) == 0 && ((uintptr_t)next & 15) == 0;
+            p.seg[i].vec_res = ws[i].R % 4 == 0 && ((uintptr_t)ws[i].resA & 7) == 0 && ((uintptr_t)next & 15) == 0;
             next += ((size_t)M * ws[i].R + 3) & ~(size_t)3;
         }
         st = launch_pre(any_res ? &coeff : nullptr, ws, count, A, lda, to, M, p.out_bf16, xb, tickets, im, stream);

@@ -48,6 +48,10 @@ static __device__ long long *g_gemm_stamps = nullptr;
 #endif
 constexpr int kGemmMaxSegs = 4;
 
+// LDS of gemm_kernel behind its loop: the totals of `rows` rows as fp32 rows of 132, a ticket flag, and (a
+// residual) as many rows again.
+constexpr int gemm_residual_offset(int rows) { return rows * 132 * 4 + 16; }
+
 // One weight of a launch.
 struct GemmSeg {
     const uint8_t *q[2];
@@ -58,7 +62,7 @@ struct GemmSeg {
     const uint16_t *bias;  // [N] activation dtype
     int64_t ldc;
     int gs, lut_rows, R;
-    int vec_res;           // R % 8 == 0 and rows of resA and xb allow 16-byte loads
+    int vec_res;           // R % 4 == 0 and rows of resA and xb allow loads of four ranks
     int vec_store;         // C rows allow 16-byte stores
 };
 
@@ -1001,6 +1005,57 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
     constexpr int ROWS = MW * MB * 16;                  // rows of C this workgroup owns
     constexpr int LDT = 128 + 4;                        // padded row: conflict-free both ways
     float *tile = (float *)smem;
+    // Residual, xb @ resA^T, as a tile of its own behind the totals' (gemm_residual_offset): fp32 products on
+    // the matrix cores, sixteen ranks a step, of which lane group kg holds four (the order of ranks is free
+    // as long as both operands agree); wavefront i takes the outputs 16 * i ... + 15 of every row.  resA and
+    // xb are read once each; every thread reading the eight rows of resA behind its outputs and adding rank by
+    // rank: M = 1271, 1344 -> 3200, 3 bits, rank 16, the launch 40.6 us, now 27; M = 256,
+    // 4096 -> 12288, 4 bits, rank 16, the call 54.5 and 42.4; M = 300, 4096 -> 4096 39.8 and 32.8.
+    float *const rtile = (float *)(smem + gemm_residual_offset(ROWS));
+    auto residual_tile = [&] {
+        constexpr int BLOCKS = ROWS / 16;
+        f4_t sum[BLOCKS];
+#pragma unroll
+        for (int b = 0; b < BLOCKS; ++b) sum[b] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        const uint16_t *const ra = w.resA + (int64_t)(t * 128 + wave * 16 + rho) * w.R;
+#pragma unroll 1
+        for (int r0 = 0; r0 < w.R; r0 += 16) {
+            const int k0 = r0 + kg * 4;
+            uint32_t h[2] = {0u, 0u};
+            f4_t x[BLOCKS];
+#pragma unroll
+            for (int b = 0; b < BLOCKS; ++b) x[b] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            if (w.vec_res) {                            // uniform
+                if (k0 < w.R) {
+                    const uint2 raw = *(const uint2 *)(ra + k0);
+                    h[0] = raw.x;
+                    h[1] = raw.y;
+#pragma unroll
+                    for (int b = 0; b < BLOCKS; ++b)
+                        x[b] = *(const f4_t *)(w.xb + (int64_t)min((int)blockIdx.y * ROWS + b * 16 + rho, p.M - 1) * w.R + k0);
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (k0 + e >= w.R) continue;
+                    h[e >> 1] |= (uint32_t)ra[k0 + e] << (16 * (e & 1));
+#pragma unroll
+                    for (int b = 0; b < BLOCKS; ++b)
+                        x[b][e] = w.xb[(int64_t)min((int)blockIdx.y * ROWS + b * 16 + rho, p.M - 1) * w.R + k0 + e];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint16_t one = (uint16_t)(h[e >> 1] >> (16 * (e & 1)));
+                const float a = p.out_bf16 ? bf2f(one) : h2f(one);
+#pragma unroll
+                for (int b = 0; b < BLOCKS; ++b)
+                    sum[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, x[b][e], sum[b], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < BLOCKS; ++b) *(f4_t *)(rtile + (b * 16 + rho) * LDT + wave * 16 + kg * 4) = sum[b];
+    };
     if (scattered) {                                    // the totals of block x(kw) are in accumulator 0
         if (KW == 4 || !(kw & 1)) {
 #pragma unroll
@@ -1020,6 +1075,7 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
                 *(f4_t *)(tile + row * LDT + n0) = acc[mb][i];
             }
     }
+    if (w.R > 0 && p.ztotal == 1) residual_tile();      // (of several slices the last arrival forms it)
     __syncthreads();
 
     FLUTE_STAMP(5);
@@ -1050,6 +1106,10 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
         if (!*flag) return;
         if (tid == 0)
             __hip_atomic_store(p.tickets + unit, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (w.R > 0) {
+            residual_tile();
+            __syncthreads();
+        }
     }
 
     // ---- epilogue: residual, bias, one rounding, store -------------------------------
@@ -1095,32 +1155,13 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
 #pragma unroll
             for (int e = 0; e < 8; ++e) y[e] = ldexpf(y[e], sh);
         }
-        if (w.R > 0 && w.vec_res) {
-            // eight ranks a step, ten 16-byte loads at once instead of a chain of 2-byte ones
-            // (M = 48, rank 16, 12288 -> 4096: the launch that folds the partial tiles 46.1 -> 22.6 us)
-            const float *xr = w.xb + (size_t)m * w.R;
-            for (int r0 = 0; r0 < w.R; r0 += 8) {
-                u4_t a[8];
+        if (w.R > 0) {
+            const f4_t lo = *(const f4_t *)(rtile + ml * LDT + n8 * 8);
+            const f4_t hi = *(const f4_t *)(rtile + ml * LDT + n8 * 8 + 4);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) a[e] = *(const u4_t *)(w.resA + (int64_t)(n0 + e) * w.R + r0);
-                const f4_t c0 = *(const f4_t *)(xr + r0), c1 = *(const f4_t *)(xr + r0 + 4);
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    const float c = r < 4 ? c0[r & 3] : c1[r & 3];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const uint16_t h = (uint16_t)(a[e][r >> 1] >> (16 * (r & 1)));
-                        y[e] = fmaf(c, p.out_bf16 ? bf2f(h) : h2f(h), y[e]);
-                    }
-                }
-            }
-        } else if (w.R > 0) {
-            const float *xr = w.xb + (size_t)m * w.R;
-            for (int r = 0; r < w.R; ++r) {
-                const float c = xr[r];
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    y[e] = fmaf(c, load_act(w.resA, (int64_t)(n0 + e) * w.R + r, p.out_bf16), y[e]);
+            for (int e = 0; e < 4; ++e) {
+                y[e] += lo[e];
+                y[4 + e] += hi[e];
             }
         }
         if (w.bias) {
