@@ -226,19 +226,47 @@ __device__ __forceinline__ void coeff_block(const CoeffParams &p, int index, f4_
     const int si = (by >= p.rank0[1]) + (by >= p.rank0[2]) + (by >= p.rank0[3]);
     const int M = p.M, K = p.K, R = p.R[si], rb = by - p.rank0[si], aligned = p.aligned;
     float *const xb = p.xb[si];
-    const int m = min(bx * 16 + (lane & 15), M - 1), rr = min(rb * 16 + (lane & 15), R - 1);
-    const uint16_t *a = p.A + (int64_t)m * p.lda + (lane >> 4) * 8, *b = p.resB[si] + (int64_t)rr * K + (lane >> 4) * 8;
-    auto load8 = [&](const uint16_t *p) {
-        u4_t v;
-        if (aligned) return *(const u4_t *)p;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = (uint32_t)p[2 * e] | ((uint32_t)p[2 * e + 1] << 16);
-        return v;
-    };
     f4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const int k0 = bz * p.kper, k1 = min(k0 + p.kper, K);
-#pragma unroll 4
-    for (int k = k0 + wave * 32; k < k1; k += 512) acc = mfma16<BF16>(load8(b + k), load8(a + k), acc);
+    const int k0 = bz * p.kper + wave * 32, k1 = min(bz * p.kper + p.kper, K);
+    // Rows that allow it are loaded as four lanes to the 64 bytes of a row: a lane per row and piece, the order
+    // of the matrix operands, is 64 accesses of the address path an instruction and not 16, and that path
+    // bounds these workgroups; the lanes are put in order behind the load (ds_bpermute).  The pre-pass of
+    // M = 98, K = 1536, three weights of rank 16 4.5 us, before 7.2; M = 86, K = 1792 4.7, before 6.0; M = 48, K = 12288 6.4, before 6.8.
+    if (aligned) {                                      // uniform
+        const int m = min(bx * 16 + (lane >> 2), M - 1), rr = min(rb * 16 + (lane >> 2), R - 1);
+        const uint16_t *a = p.A + (int64_t)m * p.lda + (lane & 3) * 8, *b = p.resB[si] + (int64_t)rr * K + (lane & 3) * 8;
+        const int from = ((lane & 15) * 4 + (lane >> 4)) << 2;
+        auto ordered = [&](u4_t v) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)v[e]);
+            return v;
+        };
+        constexpr int U = 4;                            // steps whose loads go out together
+        for (int k = k0; k < k1; k += 512 * U) {
+            u4_t va[U], vb[U];
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                if (k + 512 * i >= k1) break;           // uniform
+                va[i] = *(const u4_t *)(a + k + 512 * i);
+                vb[i] = *(const u4_t *)(b + k + 512 * i);
+            }
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                if (k + 512 * i >= k1) break;
+                acc = mfma16<BF16>(ordered(vb[i]), ordered(va[i]), acc);
+            }
+        }
+    } else {
+        const int m = min(bx * 16 + (lane & 15), M - 1), rr = min(rb * 16 + (lane & 15), R - 1);
+        const uint16_t *a = p.A + (int64_t)m * p.lda + (lane >> 4) * 8, *b = p.resB[si] + (int64_t)rr * K + (lane >> 4) * 8;
+        auto load8 = [&](const uint16_t *p) {
+            u4_t v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (uint32_t)p[2 * e] | ((uint32_t)p[2 * e + 1] << 16);
+            return v;
+        };
+        for (int k = k0; k < k1; k += 512) acc = mfma16<BF16>(load8(b + k), load8(a + k), acc);
+    }
     red[wave][lane] = acc;
     __syncthreads();
     if (wave == 0) {
