@@ -434,6 +434,15 @@ flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *c
     return FLUTE_OK;
 }
 
+// Whether 16-row workgroups that read A themselves look for their rows' scales too, instead of a launch in front
+// (3 us of the device and as much of the host): every workgroup reads whole rows for it, sixteen of 12288 columns
+// in about those 3 us.  The launch in front and this, us a call: M = 8, 4096 -> 12288 14.6 / 12.5; M = 16 14.9 / 13.5;
+// M = 2, 12288 -> 1024 13.8 / 11.3; M = 16, 12288 -> 4096 16.0 / 16.0; M = 6, 1152 -> 512, (2, 3) bits 12.0 / 10.2.
+bool few_finds(int M, int K, int64_t workgroups) {
+    const int64_t rounds = (workgroups + kNumCU - 1) / kNumCU;
+    return rounds * std::min(M, 16) * K <= 16 * 12288;
+}
+
 // Up to four weights of one width pair, group size and rotation over the same rows of A through the
 // small-M kernel, in the given shape: one launch of each pre-pass and one (per stream) of the kernel.
 flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *const *C, const int64_t *ldc, int M,
@@ -548,11 +557,13 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
             lda = w->K;
         }
         p.rowshift = rowshift;                          // (the rotation knows its rows' largest exponents)
-        const bool find = scale_rows && !w->signs;
+        p.find = direct && scale_rows && !w->signs && !any_res && few_finds(M, w->K, units * ksplit);
+        if (p.find) p.rowshift = nullptr;
+        const bool find = scale_rows && !w->signs && !p.find;
         ImageParams im = {};
         im.A = (const uint16_t *)A;
         im.lda = lda;
-        im.rowshift = rowshift;
+        im.rowshift = p.find ? nullptr : rowshift;
         im.M = M;
         im.segs = 2 * p.G;
         im.mblk = p.mblk_pad;

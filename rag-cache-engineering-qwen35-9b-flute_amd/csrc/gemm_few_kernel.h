@@ -38,6 +38,10 @@ constexpr int few_lds_bytes() {
     return loop > sums ? loop : sums;
 }
 
+// Bytes of a launch: behind the above, the scales of sixteen rows that a workgroup looks for itself.
+template <int B1, int B2, int MB>
+constexpr int few_lds_total() { return few_lds_bytes<B1, B2, MB>() + (MB == 1 ? 64 : 0); }
+
 // What a thread contributes to a table: the LUT values its entries are made of, requested with the
 // kernel's first loads; `build` waits for them only.
 template <int B>
@@ -233,7 +237,8 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     const bool direct = MB == 1 && p.A8 != nullptr;
     const int a_row = mb0 * 16 + rho;
     const bool a_row_valid = a_row < p.M;
-    const int a_shift = direct && p.rowshift && a_row_valid ? p.rowshift[a_row] : 0;
+    const bool find = MB == 1 && p.find;
+    int a_shift = direct && p.rowshift && a_row_valid ? p.rowshift[a_row] : 0;
     const int64_t jstep = direct ? 4 : (int64_t)p.mblk_pad * 64, gstep = direct ? 8 : 2 * jstep;
     const u4_t *ap = (direct ? p.A8 + (int64_t)(a_row_valid ? a_row : 0) * p.lda8 + kg : p.Ap + (int64_t)mb0 * 64 + lane) +
                      (int64_t)g_first * gstep;
@@ -303,7 +308,29 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     __builtin_amdgcn_sched_barrier(0);
     lut1.build(smem, lane, wave);
     if constexpr (B2 > 0) lut2.build(smem + tab2, lane, wave);
+    // bfloat16 rows in front of a float16 LUT: each wavefront looks two of the workgroup's rows through for
+    // their scales (few_finds).
+    int *const found = (int *)(smem + few_lds_bytes<B1, B2, MB>());
+    if constexpr (MB == 1) {
+        if (find) {
+            const int pieces = p.G * 8;                 // of a row
+            for (int r = wave; r < 16 && mb0 * 16 + r < p.M; r += 8) {
+                const u4_t *const row = p.A8 + (int64_t)(mb0 * 16 + r) * p.lda8;
+                uint32_t e = 0;
+                for (int i = 0; i < pieces; i += 512) { // (past the end: the last piece again)
+                    u4_t v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = row[min(i + u * 64 + lane, pieces - 1)];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) e = max(e, bf16_max_exp8(make_uint4(v[u][0], v[u][1], v[u][2], v[u][3])));
+                }
+                e = wavefront_max(e);
+                if (lane == 0) found[r] = bf16_row_shift(e);
+            }
+        }
+    }
     __syncthreads();
+    if (find && a_row_valid) a_shift = found[rho];
 
     f4_t acc[MB][8];
 #pragma unroll
@@ -461,8 +488,8 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     const int m = blockIdx.y * (16 * MB) + ml;
     if (m >= p.M) return;
     const int n0 = t * 128 + n_in;
-    if (p.rowshift) {                                   // exact
-        const int sh = w.R == 0 ? p.rowshift[m] : few_lift(p.rowshift[m]);
+    if (p.rowshift || find) {                           // exact
+        const int sh = find ? found[ml] : w.R == 0 ? p.rowshift[m] : few_lift(p.rowshift[m]);
 #pragma unroll
         for (int e = 0; e < PW; ++e) y[e] = ldexpf(y[e], sh);
     }

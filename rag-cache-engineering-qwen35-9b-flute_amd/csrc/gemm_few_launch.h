@@ -11,7 +11,7 @@ namespace flute {
 
 template <int MB, bool BF16, int B1, int B2, bool SEGS>
 flute_status launch_few(const GemmParams &p, dim3 grid, hipStream_t stream) {
-    constexpr int lds = few_lds_bytes<B1, B2, MB>();
+    constexpr int lds = few_lds_total<B1, B2, MB>();
     static_assert(lds <= kLdsPerCU, "tables, staging or sums exceed a CU's LDS");
     static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
     if (!attr_done) {

@@ -94,6 +94,7 @@ struct GemmParams {
     const u4_t *A8;        // 16-row workgroups: A itself, rows of lda8 16-byte pieces, no pre-pass (or NULL)
     int64_t lda8;
     int a_bf16;            // dtype of A there
+    int find;              // A8 of one type and a LUT of the other: workgroups look for their rows' scales themselves
     const int *rowshift;   // [M] or NULL: row m of the operands holds A[m] * 2^-rowshift[m]
 };
 

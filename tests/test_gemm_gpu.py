@@ -130,6 +130,29 @@ DUAL = [
 ]
 
 
+@pytest.mark.parametrize("M,K", [(2, 64), (15, 448), (16, 512), (17, 576), (33, 4160), (16, 12288), (16, 12352), (5, 16448)])
+def test_gemm_scales_found_by_the_workgroups_match_the_pre_pass(tuning_env, M, K):
+    """bfloat16 rows in front of a float16 LUT in 16-row workgroups, below and above the size up to which
+    the workgroups look for the scales themselves: the same bits as with the scales of the pre-pass."""
+    tuning_env("FLUTE_GEMM_ROWS", "16")
+    w = make_weight(256, K, 4, 128, seed=K, device=DEV)
+    x = make_x(M, K, seed=M, dtype=torch.bfloat16)
+    x[0] *= 1e30
+    x[M // 2] *= 1e-30
+    x[M - 1] = 0
+    if M > 4:
+        x[3, K - 1] = float("inf")
+
+    def run():
+        return fx.qgemm_per_group_lut(x.to(DEV), w["blob_d"], w["lut_d"], bitwidth=4, group_size=128,
+                                      indices_layout="idx4")
+    direct = run()
+    tuning_env("FLUTE_GEMM_NO_DIRECT", "1")
+    assert torch.equal(direct.nan_to_num(7.0), run().nan_to_num(7.0))
+    ok = torch.isfinite(x).all(dim=1)
+    assert rel_l2(direct.cpu()[ok][1:], _exact(w, x)[ok][1:].bfloat16()) <= TOL
+
+
 @pytest.mark.parametrize("M,N,K,bits,gs,bits2,rank,bias", DUAL)
 def test_gemm_dual_stream_fp16(M, N, K, bits, gs, bits2, rank, bias):
     w = make_weight(N, K, bits, gs, seed=M + N + bits2, bits2=bits2, rank=rank, bias=bias,
