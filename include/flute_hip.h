@@ -198,6 +198,16 @@ flute_status flute_gemm_multi(const flute_linear *ws, int count, const void *A, 
  */
 int flute_gemm_rows(const flute_linear *ws, int count, int M);
 
+/*
+ * C = h @ W^T (+ residual, bias) with h = silu(gate) * up, formed (fp32 inside, one rounding to the activation
+ * type) on the way to the operand image, for calls that have one: flute_gemm_takes_silu says so for a
+ * descriptor and M, others are refused (FLUTE_ERR_UNSUPPORTED; flute_silu_mul and flute_gemm serve them, to
+ * the same bits).  gate and up: 16-byte aligned rows of lda elements (a multiple of 8).
+ */
+int flute_gemm_takes_silu(const flute_linear *w, int M, int act_dtype);
+flute_status flute_gemm_silu(const flute_linear *w, const void *gate, const void *up, void *C, int M, int64_t lda,
+                             int64_t ldc, int act_dtype, void *stream);
+
 /* h = silu(g) * u over `count` 16-bit values (a multiple of 8), all 16-byte aligned; h may be g or u. */
 flute_status flute_silu_mul(const void *g, const void *u, void *h, int64_t count, int act_dtype,
                             void *stream);

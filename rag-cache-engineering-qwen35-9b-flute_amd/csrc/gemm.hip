@@ -131,14 +131,15 @@ CoeffPlan plan_coeff(const flute_linear *ws, int count, int M) {
 }
 
 // The pre-pass of rows of A: coefficients of `count` weights (those with a residual; plan NULL: none)
-// and what `image` asks for (blocks 0: nothing), in one launch.
+// and what `image` asks for (blocks 0: nothing), in one launch.  image.up: the rows are silu(A) * up.
 flute_status launch_pre(const CoeffPlan *plan, const flute_linear *ws, int count, const void *A, int64_t lda,
-                        float *const *xb, int M, int is_bf16, float *part, int *tickets, const ImageParams &image,
+                        float *const *xb, int M, int is_bf16, float *part, int *tickets, ImageParams image,
                         hipStream_t stream) {
     CoeffParams p = {};
     int n = 0, ranks = 0;
     if (plan) {
         p.A = (const uint16_t *)A;
+        p.up = image.up;
         p.lda = lda;
         p.M = M;
         p.K = ws[0].K;
@@ -166,13 +167,23 @@ flute_status launch_pre(const CoeffPlan *plan, const flute_linear *ws, int count
     // of sixteen wavefronts 33 us, 2048 39, 6144 44; 2048 of four 36).
     const int64_t ncoeff = (int64_t)p.rows * p.ranks * p.slices;
     const int waves = ncoeff || image.find || (int64_t)image.blocks * image.segs > 32 * kNumCU ? 16 : 4;
-    const int64_t shares = image.find ? (int64_t)image.blocks * 4 : ((int64_t)image.blocks * image.segs + waves - 1) / waves;
+    // (whole rows: two a workgroup where four leave CUs without one.  The block 2048/8192 on 300 rows 80.5 us with
+    // four, 74.9 with two; 509 rows, 12288 -> 4096 64.2 and 63.1)
+    if (image.find) image.find = (int64_t)image.blocks * 4 < kNumCU ? 2 : 4;
+    const int64_t shares = image.find ? (int64_t)image.blocks * (16 / image.find)
+                                      : ((int64_t)image.blocks * image.segs + waves - 1) / waves;
     const int64_t grid = ncoeff + std::min<int64_t>(shares, 32 / waves * kNumCU);
     FLUTE_REQUIRE(grid <= 0x7fffffff, FLUTE_ERR_UNSUPPORTED, "flute_gemm: %lld workgroups exceed the grid", (long long)grid);
     if (grid == 0) return FLUTE_OK;
-    const dim3 threads(64 * waves);
-    if (is_bf16) hipLaunchKernelGGL(gemm_pre_kernel<true>, dim3((unsigned)grid), threads, 0, stream, p, image);
-    else hipLaunchKernelGGL(gemm_pre_kernel<false>, dim3((unsigned)grid), threads, 0, stream, p, image);
+    const dim3 threads(64 * waves), blocks((unsigned)grid);
+    if (image.up) {
+        if (is_bf16) hipLaunchKernelGGL((gemm_pre_kernel<true, true>), blocks, threads, 0, stream, p, image);
+        else hipLaunchKernelGGL((gemm_pre_kernel<false, true>), blocks, threads, 0, stream, p, image);
+    } else if (is_bf16) {
+        hipLaunchKernelGGL((gemm_pre_kernel<true, false>), blocks, threads, 0, stream, p, image);
+    } else {
+        hipLaunchKernelGGL((gemm_pre_kernel<false, false>), blocks, threads, 0, stream, p, image);
+    }
     FLUTE_HIP_CHECK(hipGetLastError());
     return FLUTE_OK;
 }
@@ -280,8 +291,9 @@ WidePlan choose_wide(int M, int tiles, int G, int streams, double us_others) {
 
 // Up to four weights over the same rows of A in one launch: C[i] = A @ W[i]^T (+ residual, bias).  They
 // share their widths, LUT's type and K.
+// up: the rows are silu(A) * up (rows that takes_silu allows, of one stride).
 flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *const *C, const int64_t *ldc, int M,
-                       int64_t lda, int act_dtype, WidePlan plan, hipStream_t stream) {
+                       int64_t lda, int act_dtype, WidePlan plan, hipStream_t stream, const void *up = nullptr) {
     const int K = ws[0].K, G = K / 64, lut_dtype = ws[0].lut_dtype;
     const int out_bf16 = act_dtype == FLUTE_BF16;
     const bool scale_rows = act_dtype == FLUTE_BF16 && lut_dtype == FLUTE_F16;
@@ -361,6 +373,7 @@ flute_status gemm_wide(const flute_linear *ws, int count, const void *A, void *c
         image[k] = (const u4_t *)next;
         ImageParams im = {};
         im.A = (const uint16_t *)rows;
+        im.up = (const uint16_t *)up;
         im.Ap = (u4_t *)next;
         im.lda = ldr;
         im.rowshift = row_shift;
@@ -445,8 +458,9 @@ bool few_finds(int M, int K, int64_t workgroups) {
 
 // Up to four weights of one width pair, group size and rotation over the same rows of A through the
 // small-M kernel, in the given shape: one launch of each pre-pass and one (per stream) of the kernel.
+// up: as gemm_wide's.
 flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *const *C, const int64_t *ldc, int M,
-                       int64_t lda, int act_dtype, const GemmShape &shape, hipStream_t stream) {
+                       int64_t lda, int act_dtype, const GemmShape &shape, hipStream_t stream, const void *up = nullptr) {
     const flute_linear *w = ws;                         // what they share
     flute_status st;
     GemmParams p = {};
@@ -562,6 +576,7 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
         const bool find = scale_rows && !w->signs && !p.find;
         ImageParams im = {};
         im.A = (const uint16_t *)A;
+        im.up = (const uint16_t *)up;
         im.lda = lda;
         im.rowshift = p.find ? nullptr : rowshift;
         im.M = M;
@@ -670,6 +685,13 @@ GemmPlan plan_gemm(const flute_linear *ws, int count, int M) {
     return plan;
 }
 
+// Whether a call forms silu(gate) * up on its way to the operand image: calls that have one, of rows that are not
+// rotated (the rotation wants the rows themselves, as do coefficients of factors that are not aligned).
+bool takes_silu(const flute_linear &w, const GemmPlan &plan, int act_dtype) {
+    return !w.signs && ((uintptr_t)w.resB & 15) == 0 && (plan.wide.rows || plan.shape.mb > 1) &&
+           (w.K <= find_reach() || (act_dtype == FLUTE_BF16) == (w.lut_dtype == FLUTE_BF16));
+}
+
 }  // namespace
 }  // namespace flute
 
@@ -703,6 +725,29 @@ extern "C" flute_status flute_gemm(const flute_linear *w, const void *A, void *C
     const GemmPlan plan = plan_gemm(w, 1, M);
     if (plan.wide.rows) return gemm_wide(w, 1, A, &C, &ldc, M, lda, act_dtype, plan.wide, stream);
     return gemm_rows(w, 1, A, &C, &ldc, M, lda, act_dtype, plan.shape, stream);
+}
+
+extern "C" int flute_gemm_takes_silu(const flute_linear *w, int M, int act_dtype) {
+    if (!w || M < 1 || validate_linear(w, 1, "flute_gemm_takes_silu") != FLUTE_OK) return 0;
+    return takes_silu(*w, plan_gemm(w, 1, M), act_dtype);
+}
+
+extern "C" flute_status flute_gemm_silu(const flute_linear *w, const void *gate, const void *up, void *C, int M,
+                                        int64_t lda, int64_t ldc, int act_dtype, void *stream) {
+    flute_status st = validate_linear(w, 1, "flute_gemm_silu");
+    if (st != FLUTE_OK) return st;
+    FLUTE_REQUIRE(act_dtype == FLUTE_F16 || act_dtype == FLUTE_BF16, FLUTE_ERR_INVALID,
+                  "flute_gemm_silu: activations must be float16 or bfloat16");
+    FLUTE_REQUIRE(M >= 0, FLUTE_ERR_INVALID, "flute_gemm_silu: M must be >= 0 (got %d)", M);
+    if (M == 0) return FLUTE_OK;
+    FLUTE_REQUIRE(gate && up && C && lda >= w->K && ldc >= w->N && lda % 8 == 0 && (((uintptr_t)gate | (uintptr_t)up) & 15) == 0 &&
+                      ((uintptr_t)C & 1) == 0,
+                  FLUTE_ERR_INVALID, "flute_gemm_silu: gate and up must be 16-byte aligned rows, C rows of N or more");
+    const GemmPlan plan = plan_gemm(w, 1, M);
+    FLUTE_REQUIRE(takes_silu(*w, plan, act_dtype), FLUTE_ERR_UNSUPPORTED,
+                  "flute_gemm_silu: this call has no operand image (flute_gemm_takes_silu); use flute_silu_mul and flute_gemm");
+    if (plan.wide.rows) return gemm_wide(w, 1, gate, &C, &ldc, M, lda, act_dtype, plan.wide, (hipStream_t)stream, up);
+    return gemm_rows(w, 1, gate, &C, &ldc, M, lda, act_dtype, plan.shape, (hipStream_t)stream, up);
 }
 
 extern "C" flute_status flute_gemm_multi(const flute_linear *ws, int count, const void *A, void *const *C,
@@ -740,20 +785,7 @@ __global__ void __launch_bounds__(256) silu_mul_kernel(const uint16_t *g, const 
                                                        int bf16) {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < pieces; i += (int64_t)gridDim.x * 256) {
         const u4_t a = *(const u4_t *)(g + i * 8), b = *(const u4_t *)(u + i * 8);
-        u4_t o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            uint32_t r = 0;
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const uint16_t x = (uint16_t)(a[e] >> (16 * s)), y = (uint16_t)(b[e] >> (16 * s));
-                const float f = bf16 ? bf2f(x) : h2f(x);
-                const float t = f / (1.0f + expf(-f)) * (bf16 ? bf2f(y) : h2f(y));
-                r |= (uint32_t)round_act(t, bf16) << (16 * s);
-            }
-            o[e] = r;
-        }
-        *(u4_t *)(h + i * 8) = o;
+        *(u4_t *)(h + i * 8) = bf16 ? silu_mul8<true>(a, b) : silu_mul8<false>(a, b);
     }
 }
 

@@ -29,6 +29,25 @@ __device__ __forceinline__ f4_t mfma16(u4_t w, u4_t a, f4_t acc) {
                                                       __builtin_bit_cast(h8_t, a), acc, 0, 0, 0);
 }
 
+// silu(a) * b of eight 16-bit values: fp32 inside, one rounding.
+template <bool BF16>
+__device__ __forceinline__ u4_t silu_mul8(u4_t a, u4_t b) {
+    u4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        uint32_t r = 0;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const uint16_t x = (uint16_t)(a[e] >> (16 * s)), y = (uint16_t)(b[e] >> (16 * s));
+            const float f = BF16 ? bf2f(x) : h2f(x);
+            const float t = f / (1.0f + expf(-f)) * (BF16 ? bf2f(y) : h2f(y));
+            r |= (uint32_t)round_act(t, BF16) << (16 * s);
+        }
+        o[e] = r;
+    }
+    return o;
+}
+
 // Partial sums cross workgroups (and so the per-XCD L2s) inside one launch: they are
 // written through and read around the L2 with device-scope (sc1) accesses, the same
 // instructions a relaxed agent-scope atomic compiles to, but 16 bytes at a time.

@@ -209,6 +209,7 @@ static __global__ void __launch_bounds__(256) gemm_rowshift_kernel(const uint16_
 // us in one slice, 6.3 in sixteen.
 struct CoeffParams {
     const uint16_t *A;
+    const uint16_t *up;        // (SILU) as ImageParams
     const uint16_t *resB[kGemmMaxSegs];
     float *xb[kGemmMaxSegs];
     int R[kGemmMaxSegs];
@@ -219,7 +220,7 @@ struct CoeffParams {
     float *part;
     int *tickets;
 };
-template <bool BF16>
+template <bool BF16, bool SILU>
 __device__ __forceinline__ void coeff_block(const CoeffParams &p, int index, f4_t (&red)[16][64]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int bz = index / (p.rows * p.ranks), in_slice = index - bz * (p.rows * p.ranks);
@@ -236,6 +237,7 @@ __device__ __forceinline__ void coeff_block(const CoeffParams &p, int index, f4_
     if (aligned) {                                      // uniform
         const int m = min(bx * 16 + (lane >> 2), M - 1), rr = min(rb * 16 + (lane >> 2), R - 1);
         const uint16_t *a = p.A + (int64_t)m * p.lda + (lane & 3) * 8, *b = p.resB[si] + (int64_t)rr * K + (lane & 3) * 8;
+        const uint16_t *up = SILU ? p.up + (int64_t)m * p.lda + (lane & 3) * 8 : nullptr;
         const int from = ((lane & 15) * 4 + (lane >> 4)) << 2;
         auto ordered = [&](u4_t v) {
 #pragma unroll
@@ -244,16 +246,18 @@ __device__ __forceinline__ void coeff_block(const CoeffParams &p, int index, f4_
         };
         constexpr int U = 4;                            // steps whose loads go out together
         for (int k = k0; k < k1; k += 512 * U) {
-            u4_t va[U], vb[U];
+            u4_t va[U], vb[U], vu[SILU ? U : 1];
 #pragma unroll
             for (int i = 0; i < U; ++i) {
                 if (k + 512 * i >= k1) break;           // uniform
                 va[i] = *(const u4_t *)(a + k + 512 * i);
                 vb[i] = *(const u4_t *)(b + k + 512 * i);
+                if constexpr (SILU) vu[i] = *(const u4_t *)(up + k + 512 * i);
             }
 #pragma unroll
             for (int i = 0; i < U; ++i) {
                 if (k + 512 * i >= k1) break;
+                if constexpr (SILU) va[i] = silu_mul8<BF16>(va[i], vu[i]);
                 acc = mfma16<BF16>(ordered(vb[i]), ordered(va[i]), acc);
             }
         }
@@ -305,6 +309,7 @@ __device__ __forceinline__ void coeff_block(const CoeffParams &p, int index, f4_
 // coefficients 6.9 us one after the other; M = 509, K = 12288, bfloat16 rows, scales 3.1 and image 6.8.
 struct ImageParams {
     const uint16_t *A;
+    const uint16_t *up;        // (SILU) an element of the rows is silu(A's) * this one, rounded; rows as A's
     u4_t *Ap;                  // or NULL: only the scales are wanted
     int64_t lda;
     int *rowshift;             // [M] or NULL; find: written here, else read
@@ -316,12 +321,12 @@ struct ImageParams {
     int wide;                  // 1: pieces as they are (wide_piece), rows past the end repeat the last; 0: operands of
                                // gemm_kernel.h, rows past the end zero
     int block_xor;             // wide == 0: mode of image_block_xor
-    int find;                  // look for the scales first (a workgroup then takes four whole rows)
+    int find;                  // look for the scales first: the rows (2 or 4) that a workgroup then takes whole, or 0
     int warm_lines;
 };
 
 constexpr int kPieceMax = 8;   // 16-byte pieces of a row quarter that a thread holds where it looks for scales
-constexpr int find_reach() { return kPieceMax * 64 * 32; }       // columns
+constexpr int find_reach() { return kPieceMax * 64 * 32; }       // columns, four rows a workgroup
 
 __device__ __forceinline__ u4_t image_convert(u4_t raw, int in_bf16, int out_bf16, int shift) {
     if (in_bf16 != out_bf16) {
@@ -358,12 +363,61 @@ __device__ __forceinline__ void image_store(const ImageParams &p, int m, int seg
     p.Ap[((int64_t)seg * p.mblk + mb) * 64 + q * 16 + (m & 15)] = out;
 }
 
-template <bool BF16>
+// ROWS rows by all segments: a quad per segment and row, 256 / ROWS quads of a row side by side.
+template <bool BF16, bool SILU, int ROWS>
+__device__ __forceinline__ void find_rows(const ImageParams &p, int b, int nb, uint32_t *slots) {
+    constexpr int STEP = 256 / ROWS, PIECES = kPieceMax * ROWS / 4;
+    const int tid = threadIdx.x, lane = tid & 63, r = (tid >> 2) & (ROWS - 1), s0 = tid / (4 * ROWS);
+    for (int m0 = b * ROWS; m0 < p.blocks * 16; m0 += nb * ROWS) {
+        const int m = m0 + r;
+        const int64_t at = (int64_t)min(m, p.M - 1) * p.lda + (lane & 3) * 8;
+        u4_t raw[PIECES];
+        uint32_t e = 0;
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+            if (s0 + i * STEP < p.segs) raw[i] = *(const u4_t *)(p.A + at + (s0 + i * STEP) * 32);
+        if constexpr (SILU) {
+            u4_t up[PIECES];
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i)
+                if (s0 + i * STEP < p.segs) up[i] = *(const u4_t *)(p.up + at + (s0 + i * STEP) * 32);
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i)
+                if (s0 + i * STEP < p.segs) raw[i] = silu_mul8<BF16>(raw[i], up[i]);
+        }
+        if (m >= p.M && !p.wide) {
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i) raw[i] = u4_t{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+            if (s0 + i * STEP < p.segs) e = max(e, bf16_max_exp8(make_uint4(raw[i][0], raw[i][1], raw[i][2], raw[i][3])));
+        e = dpp_max<0xB1>(e);                           // the quad
+        e = dpp_max<0x4E>(e);
+        if constexpr (ROWS == 2) e = max(e, (uint32_t)__shfl_xor((int)e, 8));
+        e = max(e, (uint32_t)__shfl_xor((int)e, 16));
+        e = max(e, (uint32_t)__shfl_xor((int)e, 32));
+        __syncthreads();                                // (the rows before are done with the slots)
+        if ((lane & 3) == 0 && lane < 4 * ROWS) slots[(tid >> 6) * 4 + r] = e;      // [wave][row]
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < 16; ++w) e = max(e, slots[w * 4 + r]);
+        const int shift = bf16_row_shift(e);
+        if (tid < 4 * ROWS && (tid & 3) == 0 && m < p.M) p.rowshift[m] = shift;
+        if (p.Ap) {
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i)
+                if (s0 + i * STEP < p.segs) image_store(p, m, s0 + i * STEP, image_convert(raw[i], p.in_bf16, p.out_bf16, shift));
+        }
+    }
+}
+
+template <bool BF16, bool SILU>
 __global__ void __launch_bounds__(1024) gemm_pre_kernel(const CoeffParams c, const ImageParams p) {
     __shared__ f4_t red[16][64];
     const int ncoeff = c.rows * c.ranks * c.slices;
     if ((int)blockIdx.x < ncoeff) {
-        coeff_block<BF16>(c, blockIdx.x, red);
+        coeff_block<BF16, SILU>(c, blockIdx.x, red);
         return;
     }
     const int b = blockIdx.x - ncoeff, nb = gridDim.x - ncoeff, tid = threadIdx.x, lane = tid & 63;
@@ -375,41 +429,10 @@ __global__ void __launch_bounds__(1024) gemm_pre_kernel(const CoeffParams c, con
         }
     }
     // a row past the end: the last one again (wide) or zeros
-    auto load = [&](int m, int seg) -> u4_t {
-        if (m >= p.M && !p.wide) return u4_t{0u, 0u, 0u, 0u};
-        return *(const u4_t *)(p.A + (int64_t)min(m, p.M - 1) * p.lda + seg * 32 + (lane & 3) * 8);
-    };
+    auto offset = [&](int m, int seg) { return (int64_t)min(m, p.M - 1) * p.lda + seg * 32 + (lane & 3) * 8; };
     if (p.find) {
-        // four rows by all segments: a quad per segment and row, 64 quads of a row side by side
-        const int r = (tid >> 2) & 3, s0 = tid >> 4;
-        uint32_t *const slots = (uint32_t *)red;        // [wave][row]
-        for (int m4 = b * 4; m4 < p.blocks * 16; m4 += nb * 4) {
-            const int m = m4 + r;
-            u4_t raw[kPieceMax];
-            uint32_t e = 0;
-#pragma unroll
-            for (int i = 0; i < kPieceMax; ++i)
-                if (s0 + i * 64 < p.segs) raw[i] = load(m, s0 + i * 64);
-#pragma unroll
-            for (int i = 0; i < kPieceMax; ++i)
-                if (s0 + i * 64 < p.segs) e = max(e, bf16_max_exp8(make_uint4(raw[i][0], raw[i][1], raw[i][2], raw[i][3])));
-            e = dpp_max<0xB1>(e);                       // the quad
-            e = dpp_max<0x4E>(e);
-            e = max(e, (uint32_t)__shfl_xor((int)e, 16));
-            e = max(e, (uint32_t)__shfl_xor((int)e, 32));
-            __syncthreads();                            // (the rows before are done with the slots)
-            if ((lane & 3) == 0 && lane < 16) slots[(tid >> 6) * 4 + r] = e;
-            __syncthreads();
-#pragma unroll
-            for (int w = 0; w < 16; ++w) e = max(e, slots[w * 4 + r]);
-            const int shift = bf16_row_shift(e);
-            if ((tid & ~12) == 0 && m < p.M) p.rowshift[m] = shift;
-            if (p.Ap) {
-#pragma unroll
-                for (int i = 0; i < kPieceMax; ++i)
-                    if (s0 + i * 64 < p.segs) image_store(p, m, s0 + i * 64, image_convert(raw[i], p.in_bf16, p.out_bf16, shift));
-            }
-        }
+        if (p.find == 2) find_rows<BF16, SILU, 2>(p, b, nb, (uint32_t *)red);
+        else find_rows<BF16, SILU, 4>(p, b, nb, (uint32_t *)red);
         return;
     }
     // a wavefront moves one 1 KB block of the image, sixteen rows by 64 bytes, at a time
@@ -425,7 +448,11 @@ __global__ void __launch_bounds__(1024) gemm_pre_kernel(const CoeffParams c, con
             seg = (int)(w - (int64_t)mb * p.segs);
         }
         const int m = mb * 16 + (lane >> 2);
-        const u4_t raw = load(m, seg);
+        u4_t raw = {0u, 0u, 0u, 0u};
+        if (m < p.M || p.wide) {
+            raw = *(const u4_t *)(p.A + offset(m, seg));
+            if constexpr (SILU) raw = silu_mul8<BF16>(raw, *(const u4_t *)(p.up + offset(m, seg)));
+        }
         const int shift = p.rowshift ? p.rowshift[min(m, p.M - 1)] : 0;
         image_store(p, m, seg, image_convert(raw, p.in_bf16, p.out_bf16, shift));
     }

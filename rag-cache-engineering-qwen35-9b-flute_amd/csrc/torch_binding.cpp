@@ -7,7 +7,7 @@
 //   qgemm_gemv_splitk_fht_stream            (src/bindings.cpp:277-354)
 //   qgemm_gemv_multi, qgemm_gemv_mlp        (src/bindings.cpp:368-384)
 //   qgemm_cutlass_streaming, qgemm_dual_stream   (src/bindings.cpp:245-270)
-//   qgemm_linear, qgemm_linear_multi, embedding_rows, operand_addresses
+//   qgemm_linear, qgemm_linear_multi, qgemm_linear_mlp, embedding_rows, operand_addresses
 //                                           (what a module's forward calls; no upstream counterpart)
 //
 // Same positional signatures, same conventions (empty tensor = absent operand, N from the
@@ -377,47 +377,83 @@ Tensor qgemm_linear(const Tensor &A, const Tensor &indices, const Tensor &lut, i
                 held(bias), gs, signs, awq);
 }
 
-// Several layers on the same rows, each (indices, lut, b1, indices2, lut2, b2, resB, resA, bias, gs,
-// signs, s) with None for what it has not: their outputs side by side, or silu(first) * second.
+// The layers of a call on several rows, each (indices, lut, b1, indices2, lut2, b2, resB, resA, bias, gs,
+// signs, s) with None for what it has not.
+Described described(const char *who, const Tensor &A, int64_t K, const pybind11::tuple &l) {
+    const auto opt = [](const pybind11::handle &h) {
+        return h.is_none() ? c10::optional<Tensor>() : c10::optional<Tensor>(h.cast<Tensor>());
+    };
+    const auto held = [](const pybind11::handle &h) { return h.is_none() ? Tensor() : h.cast<Tensor>(); };
+    TORCH_CHECK(l.size() == 12, who, ": a layer has 12 operands");
+    return describe(who, A, K, l[0].cast<Tensor>(), l[1].cast<Tensor>(), l[2].cast<int64_t>(), held(l[3]), held(l[4]),
+                    l[5].cast<int64_t>(), held(l[6]), held(l[7]), held(l[8]), l[9].cast<int64_t>(), opt(l[10]), opt(l[11]),
+                    0, kGsAll, 256);
+}
+
+// The first `count` layers on the rows of A: outputs of one row side by side, or one below the other
+// (`stacked`, layers of equal N).
+Tensor gemm_layers(const char *who, const Tensor &A, const Shape2 &s, const std::vector<pybind11::tuple> &layers,
+                   size_t count, bool stacked) {
+    std::vector<Described> d;
+    std::vector<flute_linear> ws;
+    int64_t total = 0;
+    for (size_t i = 0; i < count; ++i) {
+        d.push_back(described(who, A, s.K, layers[i]));
+        ws.push_back(d.back().w);
+        total += d.back().N;
+    }
+    TORCH_CHECK(!stacked || d[0].N == d[1].N, who, ": gate and up must agree in N");
+    const Tensor out = stacked ? torch::empty({2, s.M, d[0].N}, A.options()) : torch::empty({s.M, total}, A.options());
+    std::vector<void *> C;
+    std::vector<int64_t> ldc;
+    char *at = (char *)out.data_ptr();
+    for (const Described &one : d) {
+        C.push_back(at);
+        at += 2 * one.N * (stacked ? s.M : 1);
+        ldc.push_back(stacked ? one.N : total);
+    }
+    check_status(flute_gemm_multi(ws.data(), (int)ws.size(), A.data_ptr(), C.data(), ldc.data(), (int)s.M, s.K, act_code(A),
+                                  stream_of(A)));
+    return out;
+}
+
+// Several layers on the same rows: their outputs side by side, or silu(first) * second.
 // Layers of one rotation (the same signs and s at the same address) share the rotated rows.
 Tensor qgemm_linear_multi(const Tensor &A_in, const std::vector<pybind11::tuple> &layers, bool silu_mul) {
     const char *who = "qgemm_linear_multi";
     const Shape2 s = check_2d_input(who, A_in, false);
     TORCH_CHECK(!layers.empty() && layers.size() <= 4 && (!silu_mul || layers.size() == 2), who,
                 ": 1..4 layers, two for silu_mul");
-    const auto opt = [](const pybind11::handle &h) {
-        return h.is_none() ? c10::optional<Tensor>() : c10::optional<Tensor>(h.cast<Tensor>());
-    };
-    const auto held = [&](const pybind11::handle &h) { return h.is_none() ? Tensor() : h.cast<Tensor>(); };
     const Tensor A = aligned16(A_in);
     c10::DeviceGuard guard(A.device());
-    std::vector<Described> d;
-    std::vector<flute_linear> ws;
-    int64_t total = 0;
-    for (const pybind11::tuple &l : layers) {
-        TORCH_CHECK(l.size() == 12, who, ": a layer has 12 operands");
-        d.push_back(describe(who, A, s.K, l[0].cast<Tensor>(), l[1].cast<Tensor>(), l[2].cast<int64_t>(), held(l[3]),
-                             held(l[4]), l[5].cast<int64_t>(), held(l[6]), held(l[7]), held(l[8]), l[9].cast<int64_t>(),
-                             opt(l[10]), opt(l[11]), 0, kGsAll, 256));
-        ws.push_back(d.back().w);
-        total += d.back().N;
-    }
-    TORCH_CHECK(!silu_mul || d[0].N == d[1].N, who, ": gate and up must agree in N");
-    const Tensor out = silu_mul ? torch::empty({2, s.M, d[0].N}, A.options()) : torch::empty({s.M, total}, A.options());
-    std::vector<void *> C;
-    std::vector<int64_t> ldc;
-    char *at = (char *)out.data_ptr();
-    for (const Described &one : d) {
-        C.push_back(at);
-        at += 2 * one.N * (silu_mul ? s.M : 1);
-        ldc.push_back(silu_mul ? one.N : total);
-    }
-    check_status(flute_gemm_multi(ws.data(), (int)ws.size(), A.data_ptr(), C.data(), ldc.data(), (int)s.M, s.K, act_code(A),
-                                  stream_of(A)));
+    const Tensor out = gemm_layers(who, A, s, layers, layers.size(), silu_mul);
     if (!silu_mul) return out;
-    const Tensor h = torch::empty({s.M, d[0].N}, A.options());
-    check_status(flute_silu_mul(C[0], C[1], h.data_ptr(), s.M * d[0].N, act_code(A), stream_of(A)));
+    const Tensor g = out.select(0, 0), u = out.select(0, 1), h = torch::empty_like(g);
+    check_status(flute_silu_mul(g.data_ptr(), u.data_ptr(), h.data_ptr(), g.numel(), act_code(A), stream_of(A)));
     return h;
+}
+
+// A gated block on several rows: down(silu(gate(A)) * up(A)) of the layers gate, up and down.
+Tensor qgemm_linear_mlp(const Tensor &A_in, const std::vector<pybind11::tuple> &layers) {
+    const char *who = "qgemm_linear_mlp";
+    const Shape2 s = check_2d_input(who, A_in, false);
+    TORCH_CHECK(layers.size() == 3, who, ": three layers: gate, up, down");
+    const Tensor A = aligned16(A_in);
+    c10::DeviceGuard guard(A.device());
+    const Tensor out = gemm_layers(who, A, s, layers, 2, true);
+    const Tensor g = out.select(0, 0), u = out.select(0, 1);
+    const int64_t K = g.size(1);
+    const Described d = described(who, g, K, layers[2]);
+    const Tensor C = torch::empty({s.M, d.N}, A.options());
+    const int act = act_code(A);
+    void *const stream = stream_of(A);
+    if (flute_gemm_takes_silu(&d.w, (int)s.M, act)) {
+        check_status(flute_gemm_silu(&d.w, g.data_ptr(), u.data_ptr(), C.data_ptr(), (int)s.M, K, d.N, act, stream));
+    } else {
+        check_status(flute_silu_mul(g.data_ptr(), u.data_ptr(), g.data_ptr(), g.numel(), act, stream));
+        check_status(flute_gemm(&d.w, g.data_ptr(), C.data_ptr(), (int)s.M, K, d.N, act, stream));
+    }
+    return C;
 }
 
 // Rows `ids` (int64, contiguous, flat) of a table, and whether every id lay in it (true where
@@ -518,6 +554,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("embedding_rows", &embedding_rows);
     m.def("operand_addresses", &operand_addresses);
     m.def("qgemm_linear_multi", &qgemm_linear_multi);
+    m.def("qgemm_linear_mlp", &qgemm_linear_mlp);
     m.def("qgemm_gemv_multi", &qgemm_gemv_multi, py::arg("A"), py::arg("seg_table"),
           py::arg("lut_dtype") = py::none(), py::arg("split") = 0);
     m.def("qgemm_gemv_mlp", &qgemm_gemv_mlp, py::arg("A"), py::arg("seg_table"), py::arg("C"),

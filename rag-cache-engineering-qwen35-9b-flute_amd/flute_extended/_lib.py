@@ -97,6 +97,8 @@ SYMBOLS = {
     "flute_gemm_multi": (_I, [_LP, _I, _P, ctypes.POINTER(_P), ctypes.POINTER(ctypes.c_int64), _I,
                               ctypes.c_int64, _I, _P]),
     "flute_gemm_rows": (_I, [_LP, _I, _I]),
+    "flute_gemm_takes_silu": (_I, [_LP, _I, _I]),
+    "flute_gemm_silu": (_I, [_LP, _P, _P, _P, _I, ctypes.c_int64, ctypes.c_int64, _I, _P]),
     "flute_silu_mul": (_I, [_P, _P, _P, ctypes.c_int64, _I, _P]),
     "flute_gemm": (_I, [_LP, _P, _P, _I, ctypes.c_int64, ctypes.c_int64, _I, _P]),
     "flute_gemm_debug_simple": (_I, [_P, ctypes.c_int64, _I, _P, _I, _I, _I, _I, _I, _I, _P, _P, _I,

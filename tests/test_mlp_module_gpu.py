@@ -394,6 +394,29 @@ def test_layers_on_the_same_rows_in_one_call(monkeypatch, M, spec, act, rot):
         assert qkv(x).requires_grad and mlp(x).requires_grad
 
 
+@pytest.mark.parametrize("rows", [16, 32, 64, 128, 256, 512])
+@pytest.mark.parametrize("M", [2, 33, 530])
+@pytest.mark.parametrize("K,N,spec,act", [
+    (256, 1152, dict(rank=16), torch.bfloat16), (128, 2176, dict(rank=5, bias=True), torch.float16),
+    (512, 640, dict(lut_dtype=torch.bfloat16, bits2=1), torch.bfloat16)])
+def test_block_in_one_call_equals_its_parts(tuning_env, rows, M, K, N, spec, act):
+    """silu(gate) * up formed on the way to the operand image, in every shape of the down projection's
+    launch, whole and ragged row blocks, scaled rows (two and four a workgroup) and coefficients: the bits of the
+    product as a tensor and the down projection of it."""
+    gate, up = (_modules(make_weight(N, K, seed=i))[1] for i in range(2))
+    if "lut_dtype" in spec:
+        gate, up = (_modules(make_weight(N, K, seed=i, lut_dtype=spec["lut_dtype"]))[1] for i in range(2))
+    down = _modules(make_weight(K, N, seed=3, act_dtype=act, **spec))[1]
+    x = make_x(M, K, seed=6, dtype=act)
+    x[M // 2] *= 100.0
+    x = x.to(DEV)
+    with torch.no_grad():
+        tuning_env("FLUTE_GEMM_ROWS", str(rows))
+        h = pm._rows_together((gate, up), x, True)
+        want, got = down(h), pm.FusedPalettizedMLP(gate, up, down, torch.nn.SiLU())(x)
+    assert torch.equal(got, want)
+
+
 def test_layers_wrapped_on_the_object_are_called_one_by_one():
     """A forward set on one object (placement libraries wrap modules so) is called, as torch would."""
     K = 1024
