@@ -49,28 +49,252 @@ __device__ __forceinline__ float to_f(uint32_t h, int bf16) {
     return bf16 ? bf2f((uint16_t)h) : h2f((uint16_t)h);
 }
 
-// One workgroup per requested row, sixteen consecutive columns a thread.  What bounds it: the chain
+// The grid's first workgroup looks all ids over and leaves its verdict in host memory, 1 = every id lies in the
+// table, 2 = some do not.
+__device__ __forceinline__ void check_ids(const EmbParams &p, int64_t count, int *check) {
+    __shared__ int bad;
+    const int tid = threadIdx.x;
+    if (tid == 0) bad = 0;
+    __syncthreads();
+    int mine = 0;
+    for (int64_t i = tid; i < count; i += 8 * kEmbThreads) {
+        int64_t id[8];                                  // (past the end: the last one again)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) id[u] = p.ids[i + u * kEmbThreads < count ? i + u * kEmbThreads : count - 1];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) mine |= id[u] < 0 || id[u] >= p.N;
+    }
+    if (mine) bad = 1;
+    __syncthreads();
+    if (tid == 0) __hip_atomic_store(check, bad ? 2 : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Rows of up to 4096 columns: one workgroup per requested row, sixteen consecutive columns a thread, all segments
+// of a rotated row side by side.  What bounds it: for few rows the chain id -> codes -> values -> butterfly -> store,
+// for many vector and LDS instructions, so widths and types are decided outside the loops over the values, the LUT
+// row lies in LDS as fp32 (16-bit LDS reads take four times a dword's), the codes of a stream are requested together,
+// stages between lanes exchange halves in registers, the ones above cross LDS once, and stores are
+// contiguous.  In a graph, the kernel below and this one, us: 1000 rows of 4096 columns, 4 bits, rotated 13.8 / 9.9, plain
+// 11.0 / 8.5; 4000 rotated 45.1 / 25; 2000 of 3136, (1, 4) bits, rotated 32.5 / 17.5; 64 rotated 6.5 / 4.4.
+constexpr int kEmbRow = kEmbThreads * 16;
+// Dynamic LDS of a wavefront: its 1024 columns in fp32 (rotated), or as it stores them.
+__host__ __device__ constexpr int emb_wave_bytes(bool rotated) { return rotated ? 4096 : 2048; }
+
+// Codes of the columns k ... k + 15 of a row as chunks c4 = 0 ... 3 (from = the row's place in its tile row).
+template <int B>
+__device__ __forceinline__ void row_codes(const uint8_t *from, int k, int d, uint32_t (&c)[4]) {
+    const uint8_t *const at = from + (size_t)(k >> 6) * (1024 * B) + ((k >> 4) & 3) * (4 * B);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint8_t *const q = at + i * 16 * B;
+        if constexpr (B == 4) c[i] = *(const uint16_t *)(q + 2 * d);
+        else if constexpr (B == 3) c[i] = ((uint32_t)q[d] | ((uint32_t)q[d + 1] << 8)) >> (4 * d);
+        else if constexpr (B == 2) c[i] = q[d];
+        else c[i] = (uint32_t)*q >> (4 * d);
+    }
+}
+// Their values out of the LUT row, fp32 in LDS.
+template <int B>
+__device__ __forceinline__ void row_values(const float *lut, const uint32_t (&c)[4], float (&f)[16]) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const int i = (j >> 1) & 3, shift = 2 * (j >> 3) + (j & 1);         // in codes
+        f[j] = lut[__builtin_amdgcn_ubfe(c[i], B * shift, B)];
+    }
+}
+
+template <bool BF16, bool ROT>
+__global__ void __launch_bounds__(kEmbThreads) embedding_row_kernel(const EmbParams p, int64_t count, int *check) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    float *const buf = (float *)lds;                    // (ROT, segments beyond 1024 columns)
+    __shared__ float luts[2][16];
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (check && blockIdx.x == 0) {
+        check_ids(p, count, check);
+        return;
+    }
+    const int64_t row = (int64_t)blockIdx.x - (check ? 1 : 0);
+    const int64_t n64 = p.ids[row];
+    uint16_t *const out = p.out + (size_t)row * p.K;
+    if (n64 < 0 || n64 >= p.N) {                        // refused on the host; never read out of range
+        for (int k = tid; k < p.K; k += kEmbThreads) out[k] = 0;
+        return;
+    }
+    const int n = (int)n64, G = p.K >> 6;
+    const int wx = (n >> 6) & 1, v = (n >> 4) & 3, d = (n >> 3) & 1, r8 = n & 7;
+    const bool mine = tid * 16 < p.K;
+    const int k = min(tid * 16, p.K - 16);
+    uint32_t c[2][4];
+    auto codes = [&](int s) {
+        const int b = p.bits[s];
+        const uint8_t *const from = p.q[s] + (size_t)(n >> 7) * G * (1024 * b) + (wx * 32 + r8 * 4) * (16 * b) + b * v;
+        switch (b) {                                    // uniform, around all of a stream's loads
+            case 4: row_codes<4>(from, k, d, c[s]); break;
+            case 3: row_codes<3>(from, k, d, c[s]); break;
+            case 2: row_codes<2>(from, k, d, c[s]); break;
+            default: row_codes<1>(from, k, d, c[s]); break;
+        }
+    };
+    auto act = [](uint16_t h) { return BF16 ? bf2f(h) : h2f(h); };
+    float sg[ROT ? 16 : 1];
+    if constexpr (ROT) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sg[e] = p.signs[k + e];
+    }
+    codes(0);
+    if (p.nstreams == 2) codes(1);
+    {
+        const int grp = min(n / p.gs, p.lut_rows - 1), s = tid >> 4, e = tid & 15;
+        if (tid < 32 && s < p.nstreams && e < (1 << p.bits[s])) luts[s][e] = act(p.lut[s][((size_t)grp << p.bits[s]) + e]);
+    }
+    __syncthreads();                                    // the LUT rows are in
+    float f[16];
+    auto values = [&](int s, float (&t)[16]) {
+        switch (p.bits[s]) {
+            case 4: row_values<4>(luts[s], c[s], t); break;
+            case 3: row_values<3>(luts[s], c[s], t); break;
+            case 2: row_values<2>(luts[s], c[s], t); break;
+            default: row_values<1>(luts[s], c[s], t); break;
+        }
+    };
+    values(0, f);
+    if (p.nstreams == 2) {
+        float t[16];
+        values(1, t);
+        // the 16-bit add of the module: exact sum, one rounding to the LUT's type
+#pragma unroll
+        for (int j = 0; j < 16; ++j) f[j] = act(round_act(f[j] + t[j], BF16));
+    }
+    if (p.R > 0) {
+        float sum[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) sum[j] = 0.0f;
+        for (int r = 0; r < p.R; ++r) {
+            const float a = act(p.resA[(size_t)n * p.R + r]);
+            const uint16_t *const b = p.resB + (size_t)r * p.K + k;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) sum[j] = fmaf(a, act(b[j]), sum[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) f[j] += sum[j];
+    }
+    auto pair = [](float a, float b) { return (uint32_t)round_act(a, BF16) | ((uint32_t)round_act(b, BF16) << 16); };
+    // A wavefront's 1024 columns out, sixteen bytes a lane side by side: its lanes' 32 bytes change places through
+    // LDS on the way (as two stores 32 bytes apart: 1000 plain rows of 4096 columns 11.5 us, 8.5).
+    // (the wavefront's own part of the dynamic memory, which the stages across wavefronts use otherwise)
+    auto store16 = [&] {
+        if ((tid >> 6) * 1024 >= p.K) return;           // a whole wavefront past the end
+        uint4 *const at = (uint4 *)(lds + (tid >> 6) * emb_wave_bytes(ROT));
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            at[2 * lane + (h ^ ((lane >> 2) & 1))] = make_uint4(pair(f[8 * h], f[8 * h + 1]), pair(f[8 * h + 2], f[8 * h + 3]),
+                                                                pair(f[8 * h + 4], f[8 * h + 5]), pair(f[8 * h + 6], f[8 * h + 7]));
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int i = h * 64 + lane, col = (tid >> 6) * 1024 + i * 8;
+            if (col >= p.K) continue;
+            const uint4 o = at[i ^ ((i >> 3) & 1)];
+            if (p.vec_out) {
+                *(uint4 *)(out + col) = o;
+            } else {
+                const uint32_t w[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) *(uint32_t *)(out + col + 2 * e) = w[e];
+            }
+        }
+    };
+    if constexpr (!ROT) {
+        store16();
+    } else {
+        // the adjoint transform: ten stages within a wavefront (1024 columns), the one or two above across
+        // wavefronts through LDS
+        const int nst = column_stages(k, p.K, p.block);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) f[e] *= sg[e];
+        stages_in_thread(f);
+        if (__all(nst >= 10)) {
+            stage_all_lanes<1>(f, lane);
+            stage_all_lanes<2>(f, lane);
+            stage_all_lanes<4>(f, lane);
+            stage_all_lanes<8>(f, lane);
+            stage_all_lanes<16>(f, lane);
+            stage_all_lanes<32>(f, lane);
+        } else {
+            stage_some_lanes<1>(f, lane, nst > 4);
+            stage_some_lanes<2>(f, lane, nst > 5);
+            stage_some_lanes<4>(f, lane, nst > 6);
+            stage_some_lanes<8>(f, lane, nst > 7);
+            stage_some_lanes<16>(f, lane, nst > 8);
+            stage_some_lanes<32>(f, lane, nst > 9);
+        }
+        const float inv = inv_sqrt_pow2(nst);
+        const int top = column_stages(0, p.K, p.block); // the longest segment is the first
+        // (a segment beyond 1024 columns takes whole wavefronts)
+        if (__any(mine && nst <= 10)) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) f[e] *= inv;
+            store16();
+        } else if (mine) {
+            // piece q of thread t (16 bytes) lies at t * 4 + (q ^ (t >> 1 & 3)): writers side by side, and readers
+            // of consecutive pieces, meet different banks
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *(float4 *)(buf + tid * 16 + ((q ^ ((tid >> 1) & 3)) << 2)) = make_float4(f[4 * q], f[4 * q + 1], f[4 * q + 2], f[4 * q + 3]);
+        }
+        if (top <= 10) return;                          // uniform
+        __syncthreads();
+        // Four columns of each of the 2^T chunks of 1024 a thread: the stages between chunks, and a store of
+        // eight bytes a lane side by side.
+        auto across = [&](auto stages, int chunk0) {
+            constexpr int T = decltype(stages)::value, E = 1 << T;
+            float w[4][E];
+#pragma unroll
+            for (int h = 0; h < E; ++h) {
+                const int t = (chunk0 + h) * 64 + (tid >> 2);
+                const float4 x = *(const float4 *)(buf + t * 16 + (((tid & 3) ^ ((t >> 1) & 3)) << 2));
+                w[0][h] = x.x; w[1][h] = x.y; w[2][h] = x.z; w[3][h] = x.w;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) stages_in_thread(w[q]);
+            const float scale = inv_sqrt_pow2(10 + T);
+#pragma unroll
+            for (int h = 0; h < E; ++h) {
+                uint16_t *const to = out + (chunk0 + h) * 1024 + tid * 4;
+                const uint32_t lo = pair(w[0][h] * scale, w[1][h] * scale), hi = pair(w[2][h] * scale, w[3][h] * scale);
+                if (p.vec_out) {
+                    *(uint2 *)to = make_uint2(lo, hi);
+                } else {
+                    *(uint32_t *)to = lo;
+                    *(uint32_t *)(to + 2) = hi;
+                }
+            }
+        };
+        if (top == 12) {
+            across(std::integral_constant<int, 2>(), 0);
+        } else {
+            across(std::integral_constant<int, 1>(), 0);
+            if (p.block == 2048 && p.K == 4096) across(std::integral_constant<int, 1>(), 2);
+        }
+    }
+}
+
+// Longer rows.  One workgroup per requested row, sixteen consecutive columns a thread.  What bounds it: the chain
 // id -> codes -> values -> butterfly -> store, so everything a phase needs is requested together
 // (the LUT row goes to LDS beside the codes and signs, a value costs one LDS read) and the first ten
 // stages of the butterfly stay in registers.  (One pair at a time, byte loads of the codes and trips
 // to memory for the LUT, all stages in LDS: 15.2 us for 1000 rotated rows of 4096 columns, 4 bits,
 // against 13.6; the check of the ids as five launches and a copy before it: 71 us a call against 27.)
-// check != NULL: the first workgroup of the grid looks all ids over instead and leaves its verdict
-// in host memory, 1 = every id lies in the table, 2 = some do not.
+// check != NULL: the first workgroup of the grid looks all ids over instead (check_ids).
 __global__ void __launch_bounds__(kEmbThreads) embedding_kernel(const EmbParams p, int64_t count, int *check) {
     extern __shared__ __align__(16) uint8_t lds[];
     float *buf = (float *)lds;
     __shared__ uint16_t luts[2][16];
     const int tid = threadIdx.x;
     if (check && blockIdx.x == 0) {
-        __shared__ int bad;
-        if (tid == 0) bad = 0;
-        __syncthreads();
-        int mine = 0;
-        for (int64_t i = tid; i < count; i += kEmbThreads) mine |= p.ids[i] < 0 || p.ids[i] >= p.N;
-        if (mine) bad = 1;
-        __syncthreads();
-        if (tid == 0) __hip_atomic_store(check, bad ? 2 : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        check_ids(p, count, check);
         return;
     }
     const int64_t at = (int64_t)blockIdx.x - (check ? 1 : 0);
@@ -282,6 +506,19 @@ flute_status embedding(const flute_linear *w, const int64_t *ids, int64_t count,
         } else {
             lds = (size_t)make_segments(w->K, 0).len[0] * 4;
         }
+    }
+    const dim3 grid((unsigned)(count + (check ? 1 : 0))), threads(kEmbThreads);
+    if (w->K <= kEmbRow) {
+        const int form = 2 * p.bf16 + (w->signs != nullptr);
+        lds = (size_t)((w->K + 1023) / 1024) * emb_wave_bytes(w->signs != nullptr);
+        if (form == 3) hipLaunchKernelGGL((embedding_row_kernel<true, true>), grid, threads, lds, stream, p, count, check);
+        else if (form == 2) hipLaunchKernelGGL((embedding_row_kernel<true, false>), grid, threads, lds, stream, p, count, check);
+        else if (form == 1) hipLaunchKernelGGL((embedding_row_kernel<false, true>), grid, threads, lds, stream, p, count, check);
+        else hipLaunchKernelGGL((embedding_row_kernel<false, false>), grid, threads, lds, stream, p, count, check);
+        FLUTE_HIP_CHECK(hipGetLastError());
+        return FLUTE_OK;
+    }
+    if (w->signs) {
         static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
         if (!attr_done) {
             FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)embedding_kernel,
@@ -289,8 +526,7 @@ flute_status embedding(const flute_linear *w, const int64_t *ids, int64_t count,
             attr_done = true;
         }
     }
-    hipLaunchKernelGGL(embedding_kernel, dim3((unsigned)(count + (check ? 1 : 0))), dim3(kEmbThreads), lds, stream, p,
-                       count, check);
+    hipLaunchKernelGGL(embedding_kernel, grid, threads, lds, stream, p, count, check);
     FLUTE_HIP_CHECK(hipGetLastError());
     return FLUTE_OK;
 }

@@ -147,6 +147,38 @@ def test_hip_gather_column_edges(K, bits, bits2, block):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K,block", [(1024, 0), (1088, 0), (3072, 0), (3136, 0), (4032, 0), (4096, 0), (4096, 1024), (4096, 2048),
+                                     (2048, 2048), (4096, 4096), (4160, 0)])
+@pytest.mark.parametrize("dtype,bits2", [(torch.float16, 0), (torch.bfloat16, 3)])
+def test_rotated_rows_of_every_mix_of_segments(K, block, dtype, bits2):
+    """Segments in one wavefront, across two and four, several beside each other, and the rows the longer kernel
+    takes: the rotation of the gathered rows, also into rows of four-byte alignment."""
+    import ctypes
+    import flute_extended as fx
+    from flute_extended import _C, _lib
+    N = 256
+    w = make_weight(N, K, 4, 128, seed=K, bits2=bits2, lut_dtype=dtype, device=DEV)
+    ids = torch.arange(0, N, 7, device=DEV)
+    signs = O.rotation_signs(K, 3).to(DEV)
+    kw = dict(indices2=w["blob2_d"], lut2=w["lut2_d"], bitwidth2=bits2) if bits2 else {}
+    args = (ids, w["blob_d"], w["lut_d"], N, K, 4, 128)
+    y = fx.embedding_gather(*args, signs=signs, rot_block=block, **kw)
+    row = fx.embedding_gather(*args, **kw)
+    want = _C.fht_backward(row.float(), signs, block).to(dtype)
+    # (odd numbers of stages scale by a multiple of sqrt(2), a product the kernel may round once with the type:
+    # a unit in the last place where the fp32 product lies at a tie)
+    off = (y.float() - want.float()).abs()
+    assert bool((off <= want.float().abs() * torch.finfo(dtype).eps).all()) and int((off > 0).sum()) <= 1e-3 * off.numel()
+    like = torch.empty(1, K, dtype=dtype, device=DEV)
+    none = torch.empty(0, dtype=dtype, device=DEV)
+    d, _, keep = _C._describe("test", like, K, w["blob_d"], w["lut_d"], 4, w.get("blob2_d"), w.get("lut2_d"), bits2, none, none,
+                              none, 128, signs, None, block)
+    out = torch.zeros(ids.numel() * K + 2, dtype=dtype, device=DEV)
+    _lib.check(_lib.lib.flute_embedding(ctypes.byref(d), ids.data_ptr(), ids.numel(), out.data_ptr() + 4, _C._stream_of(out)))
+    assert torch.equal(out[2:].view(-1, K), y)
+
+
+@pytest.mark.gpu
 def test_ids_are_checked_by_the_launch():
     """One id outside the table anywhere, the first and the last one included, is refused, from
     several threads at a time; the next good call is served."""
