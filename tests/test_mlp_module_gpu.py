@@ -485,3 +485,106 @@ def test_several_weights_in_many_row_workgroups(tuning_env, rows, slices, M, spe
     assert pm.ROUTE_CENSUS["gemm_multi"] == 2 and torch.equal(y, again)
     assert rel_l2(y.cpu(), want.cpu()) <= rounding
     assert rel_l2(y.cpu(), torch.cat([p[0](x) for p in pairs], dim=-1)) <= 2 * rounding    # half a unit each
+
+
+def _both_ways(monkeypatch, compiled, block, x):
+    """(output, census) of a call through the compiled forward, which has to take it, and through Python's."""
+    with torch.no_grad():
+        block(x)                                        # (copies and tables that the module keeps)
+        pm.ROUTE_CENSUS.clear()
+        one = compiled(block, x)
+        assert one is not None
+        taken = dict(pm.ROUTE_CENSUS)
+        pm.ROUTE_CENSUS.clear()
+        with monkeypatch.context() as patch:
+            patch.setattr(pm, "_forwards", None)
+            two = block(x)
+        assert taken == pm.ROUTE_CENSUS and one.shape == two.shape and torch.equal(one, two)
+
+
+@pytest.mark.skipif(fx._C.native is None, reason="the compiled binding is not built or switched off")
+@pytest.mark.parametrize("shape", [(1,), (1, 1), (2,), (1, 17), (3, 2, 5)])
+@pytest.mark.parametrize("spec,act,rot", [
+    (dict(), torch.float16, None), (dict(bits2=1, rank=8, bias=True), torch.bfloat16, None),
+    (dict(bits=3, gs=64, rank=16), torch.float16, "same"), (dict(bits=2, bits2=4, gs=16), torch.float16, "awq"),
+    (dict(lut_dtype=torch.bfloat16, rank=64), torch.bfloat16, "different")])
+def test_compiled_forwards_equal_the_python_ones(monkeypatch, shape, spec, act, rot):
+    K, F = 256, 384
+
+    def member(n, k, seed):
+        kw = {}
+        if rot:
+            kw = dict(rotation_seed=seed if rot == "different" else 5, rotation_k=k)
+        if rot == "awq":
+            kw["awq_scale"] = torch.rand(k, generator=torch.Generator().manual_seed(1)) + 0.5
+        return _modules(make_weight(n, k, seed=seed, act_dtype=act, **spec), **kw)[1]
+    x = make_x(int(torch.tensor(shape).prod()), K, seed=3, dtype=act).view(*shape, K).to(DEV)
+    gate, up, down = member(F, K, 1), member(F, K, 2), member(K, F, 3)
+    pm._flute()
+    fw = pm._forwards
+    _both_ways(monkeypatch, fw.linear, gate, x)
+    if len(shape) < 3 or shape[0] > 1:
+        _both_ways(monkeypatch, fw.qkv, pm.SplitQKV(gate, up, member(128, K, 4)), x)
+        _both_ways(monkeypatch, fw.mlp, pm.FusedPalettizedMLP(gate, up, down, torch.nn.SiLU()), x)
+    w = make_weight(256, K, seed=7, lut_dtype=spec.get("lut_dtype", torch.float16), bits2=spec.get("bits2", 0))
+    table = pm.PalettizedEmbedding(w["blob"], w["lut"], 4, 128, 256, K, indices2=w["blob2"], lut2=w["lut2"], reference=False,
+                                   bitwidth2=w["bits2"] or None, **(dict(rotation_seed=1, rotation_k=K) if rot else {})).to(DEV)
+    _both_ways(monkeypatch, fw.embedding, table, torch.randint(0, 256, shape, device=DEV))
+
+
+@pytest.mark.skipif(fx._C.native is None, reason="the compiled binding is not built or switched off")
+@pytest.mark.parametrize("M", [1, 20])
+def test_compiled_forwards_leave_other_calls_to_python(monkeypatch, M):
+    """Conversions, switches, subclasses, watchers and derivatives: the compiled forwards answer None."""
+    from torch.autograd import forward_ad
+    K = 256
+    pm._flute()
+    fw = pm._forwards
+
+    def layer(n=256, **spec):
+        return _modules(make_weight(n, K, seed=n, rank=8, bias=True, **spec))[1]
+    a, b, c = layer(), layer(), layer()
+    qkv, mlp = pm.SplitQKV(a, b, c), pm.FusedPalettizedMLP(a, b, c, torch.nn.SiLU())
+    x = make_x(M, K, seed=3).to(DEV)
+
+    def refused(which=("linear", "qkv", "mlp"), x=x):
+        blocks = dict(linear=a, qkv=qkv, mlp=mlp)
+        return [fw.__getattribute__(n)(blocks[n], x) is None for n in which] == [True] * len(which)
+    with torch.no_grad():
+        for block in (a, qkv, mlp):
+            block(x)
+        assert not refused(("linear",)) and not refused(("qkv",)) and not refused(("mlp",))
+        for name in ("FLUTE_NO_FHT_FUSE", "FLUTE_NO_MERGE", "FLUTE_ROTATION", "FLUTE_NO_SPLITK", "FLUTE_NO_WIDE_PREF"):
+            monkeypatch.setenv(name, "0")
+            assert refused()
+            monkeypatch.delenv(name)
+        assert refused(x=x.float()) and refused(x=x.cpu()) and refused(x=x[:0]) and refused(x=x[:, :64].contiguous())
+        assert refused(x=x.clone().requires_grad_(True))
+        for watch in (lambda m: m.register_forward_hook(lambda *a: None), lambda m: m.register_forward_pre_hook(lambda *a: None)):
+            handle = watch(c)
+            assert refused(("mlp",)) and (M == 1 or refused(("qkv",)))
+            handle.remove()
+        if M > 1:
+            with forward_ad.dual_level():
+                assert refused()
+            mlp.act_fn = torch.nn.GELU()
+            assert refused(("mlp",))
+            mlp.act_fn = torch.nn.SiLU()
+        kept = a.resA
+        a.resA = a.resA.float()
+        assert refused()
+        a.resA = kept
+        c.__class__ = type("Other", (pm.PalettizedLinear,), {})
+        assert refused(("mlp",)) and (M == 1 or refused(("qkv",)))
+        c.__class__ = pm.PalettizedLinear
+        a.lut = a.lut.clone()                           # the decode tables hold the old one's address
+        assert M > 1 or refused(("qkv", "mlp"))
+        block(x), qkv(x), mlp(x)
+        assert not refused(("linear",)) and not refused(("qkv",)) and not refused(("mlp",))
+        w = make_weight(256, K, seed=7)
+        table = pm.PalettizedEmbedding(w["blob"], w["lut"], 4, 128, 256, K, reference=False).to(DEV)
+        ids = torch.arange(5, device=DEV)
+        assert fw.embedding(table, ids) is not None and fw.embedding(table, ids.int()) is None
+        assert fw.embedding(table, ids + 256) is None and fw.embedding(table, ids.cpu()) is None
+    if M > 1:
+        assert a.bias.requires_grad and refused()       # with gradients on
