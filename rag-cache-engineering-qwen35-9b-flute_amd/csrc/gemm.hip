@@ -44,11 +44,11 @@ int slices_of_k(int64_t units, int G, const GemmShape &shape) {
 bool few_takes(int b1, int b2) { return !(b1 == 4 && b2 == 4); }
 
 // Microseconds of a call (one round = a workgroup per CU; `turns` = K tiles of a wavefront), fitted to
-// measurements on tiles of 16 and 32 rows: a fixed part, the pre-pass for 32 rows (16-row workgroups
-// read A themselves) and, per round, prologue, sums and epilogue, then what a wavefront's tile costs.
-// M = 32, 4096 -> 12288, 16 and 32 rows: 4 bits 14.6 / 16.0, (4, 1) bits 19.6 / 18.5, (3, 3) 24.7 / 21.1;
-// M = 64: 27.5 / 17.1, 36.4 / 23.5, 46.6 / 28.3; M = 64, 12288 -> 4096: 22.2 / 19.6, 29.6 / 24.5,
-// 37.9 / 28.4; M = 128, 4096 -> 4096: 15.5 / 16.1, 20.6 / 19.5, 25.7 / 22.0.
+// measurements on tiles of 16 and 32 rows: a fixed part, what some calls of 32 rows have in front (few_reads)
+// and, per round, prologue, sums and epilogue, then what a wavefront's tile costs.
+// M = 32, 4096 -> 12288, 16 and 32 rows: 4 bits 13.2 / 14.4, (3, 3) bits, M = 24 23.6 / 20.2; M = 64: 25.6 / 17.1;
+// M = 48, 12288 -> 4096: 19.0 / 17.8, (4, 1) bits, bfloat16 rows 31.3 / 27.1; M = 128, 4096 -> 4096: 13.1 / 14.1;
+// M = 200: 24.0 / 16.6; M = 300, 4096 -> 1024 12.6 / 13.1; M = 100, 2048 -> 8192, (4, 1) bits 21.0 / 15.5.
 // (A residual's launch in front of 16-row workgroups is not in it.  Where the choice misses: M = 22,
 // 6912 -> 4224, (2, 3) bits, rank 16: 16 rows 28.4, 32 rows 23.4; M = 233, 1408 -> 8448, twice 1 bit: the
 // many-row kernel 30.7, 16 rows 25.2; over 58 other random shapes it is within 3 % of the best of six.)
@@ -60,7 +60,7 @@ double few_us(int mb, int M, int tiles, int G, int b1, int b2) {
     const int64_t rounds = (units * ks + kNumCU - 1) / kNumCU;
     const double tile = (tile_us[b1] + tile_us[b2]) * (mb == 1 ? 1.0 : 1.09);
     const double launches = b2 && !few_takes(std::max(b1, b2), std::min(b1, b2)) ? 2.0 : 1.0;
-    return (mb == 1 ? 1.5 : 5.0) + rounds * ((mb == 1 ? 4.0 : 5.0) * launches + tile * turns) +
+    return (mb == 1 ? 1.5 : 3.5) + rounds * ((mb == 1 ? 4.0 : 5.0) * launches + tile * turns) +
            (ks > 1 ? (mb == 1 ? 0.5 : 0.75) * ks * launches : 0.0);
 }
 
@@ -99,13 +99,13 @@ GemmShape choose_gemm_shape(int M, int tiles, int G, int b1, int b2, double &us)
         us = few1;
         return {1, 8, 1, 1};
     }
-    // The estimate of 64 rows is 4 us and more short where the two are close and a workgroup has few
+    // The estimate of 64 rows is up to 2.5 us short where the two are close and a workgroup has few
     // tiles (less with more: M = 256 and 512, 12288 -> 4096 stay).  64 and 32 rows: M = 225,
     // 5248 -> 2816 29.2 / 23.3 us; M = 300, 6912 -> 1792 32.2 / 27.6; M = 39, 1664 -> 12288 18.2 / 14.5;
     // M = 672, 10432 -> 896 43.2 / 40.1; (3, 3) bits, M = 218, 1408 -> 6912 42.5 / 29.1.
     const GemmShape shape = other_shape(M, tiles);
     const double short_by = shape.mw == 1
-        ? std::min(4.0, std::max(0.0, 8.0 - G / slices_of_k((int64_t)tiles * ((M + 63) / 64), G, shape) / 16.0)) : 0.0;
+        ? std::min(2.5, std::max(-1.5, 6.5 - G / slices_of_k((int64_t)tiles * ((M + 63) / 64), G, shape) / 16.0)) : -1.5;
     if (fits2 && few2 < other + short_by) {
         us = few2;
         return {2, 8, 1, 1};
@@ -456,6 +456,19 @@ bool few_finds(int M, int K, int64_t workgroups) {
     return rounds * std::min(M, 16) * K <= 16 * 12288;
 }
 
+// Whether workgroups of few rows read A themselves.  Sixteen rows always do.  Thirty-two do where that leaves no
+// launch in front, and where a launch that only looks for scales in few, long rows is the shorter for it; beside
+// coefficients the image costs nothing, and rows of one type in front of a LUT of the other cost each turn of
+// the loop their conversions (0.3 us).  The image and A itself, us a call: M = 64, 4096 -> 12288 18.1 / 17.2;
+// M = 200, 4096 -> 4096 19.5 / 16.6; M = 24, 4096 -> 12288, (3, 3) bits 22.0 / 20.2; bfloat16 rows, float16 LUT: M = 48,
+// 12288 -> 4096, (4, 1) bits 29.0 / 27.0; M = 64, 4096 -> 12288, eight turns, 20.0 / 21.3, rotated 22.2 / 22.8; M = 24, four
+// turns, (4, 1) bits, rotated 23.1 / 21.6; M = 64, 12288 -> 12288, 24 turns, 43.6 / 46.3; residual of rank 16, M = 48, 12288 -> 4096, (4, 1) bits 28.9 / 30.7.
+bool few_reads(const GemmShape &shape, bool residual, bool scale_rows, bool rotated, int K, int gper) {
+    if (shape.mb == 1) return true;
+    if (residual) return false;
+    return !scale_rows || ((rotated || K > 8192) && (gper + 7) / 8 <= 6);
+}
+
 // Up to four weights of one width pair, group size and rotation over the same rows of A through the
 // small-M kernel, in the given shape: one launch of each pre-pass and one (per stream) of the kernel.
 // up: as gemm_wide's.
@@ -532,13 +545,14 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
     // bfloat16 activations presented as float16 operands: one power-of-two scale per row
     const bool scale_rows = act_dtype == FLUTE_BF16 && w->lut_dtype == FLUTE_F16;
     const size_t shift_floats = scale_rows ? ((size_t)M + 3) & ~(size_t)3 : 0;
-    // One block of rows per wavefront: the kernel reads A itself (16-byte pieces of a row, put into
+    // Few rows: the kernel reads A itself where that pays (16-byte pieces of a row, put into
     // operand order in registers), so the pre-pass launch is dropped, and the image with it.  Needs
     // 16-byte aligned rows; rotated rows are read the same way (the rotation can write the image itself,
     // but only without a residual and row scales).
     const bool image_of_rotation = w->signs && !any_res && !scale_rows;
     const bool rows16 = w->signs || (((uintptr_t)A & 15) == 0 && lda % 8 == 0);
-    const bool direct = shape.mb == 1 && !tuning().gemm_no_direct && rows16 && !image_of_rotation;
+    const bool direct = few && few_reads(shape, any_res, scale_rows, w->signs != nullptr, w->K, p.gper) && !up &&
+                        !tuning().gemm_no_direct && rows16 && (w->signs ? w->K : lda) <= few_lda() && !image_of_rotation;
     const size_t ap_floats = direct ? 0 : (size_t)p.G * 2 * p.mblk_pad * 64 * 4;
     float *base = nullptr;
     int *tickets = nullptr;
@@ -571,7 +585,7 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
             lda = w->K;
         }
         p.rowshift = rowshift;                          // (the rotation knows its rows' largest exponents)
-        p.find = direct && scale_rows && !w->signs && !any_res && few_finds(M, w->K, units * ksplit);
+        p.find = direct && shape.mb == 1 && scale_rows && !w->signs && !any_res && few_finds(M, w->K, units * ksplit);
         if (p.find) p.rowshift = nullptr;
         const bool find = scale_rows && !w->signs && !p.find;
         ImageParams im = {};

@@ -90,4 +90,32 @@ __device__ __forceinline__ void ws_load16x8(const float *p, int64_t step, f4_t (
         : "memory");
 }
 
+// Dword b of the lane whose bits (5, 4) are a changes places with dword a of the one whose are b.
+__device__ __forceinline__ void transpose_lanes16(uint32_t (&q)[4]) {
+    auto p = __builtin_amdgcn_permlane32_swap(q[0], q[2], false, false);
+    q[0] = p[0]; q[2] = p[1];
+    p = __builtin_amdgcn_permlane32_swap(q[1], q[3], false, false);
+    q[1] = p[0]; q[3] = p[1];
+    p = __builtin_amdgcn_permlane16_swap(q[0], q[1], false, false);
+    q[0] = p[0]; q[1] = p[1];
+    p = __builtin_amdgcn_permlane16_swap(q[2], q[3], false, false);
+    q[2] = p[0]; q[3] = p[1];
+}
+
+// The same between the four lanes of a quad.
+__device__ __forceinline__ void transpose_quad(uint32_t (&q)[4], int lane) {
+    auto swap = [](uint32_t &lo, uint32_t &hi, auto ctrl, bool odd) {
+        const uint32_t l = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo, decltype(ctrl)::value, 0xf, 0xf, true);
+        const uint32_t h = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi, decltype(ctrl)::value, 0xf, 0xf, true);
+        hi = odd ? hi : l;
+        lo = odd ? h : lo;
+    };
+    const std::integral_constant<int, 0x4e> by2;        // quad_perm [2, 3, 0, 1]
+    const std::integral_constant<int, 0xb1> by1;        // quad_perm [1, 0, 3, 2]
+    swap(q[0], q[2], by2, lane & 2);
+    swap(q[1], q[3], by2, lane & 2);
+    swap(q[0], q[1], by1, lane & 1);
+    swap(q[2], q[3], by1, lane & 1);
+}
+
 }  // namespace flute

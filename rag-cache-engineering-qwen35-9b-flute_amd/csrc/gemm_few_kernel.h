@@ -173,30 +173,6 @@ struct FewStream {
             return w;
         }
     }
-    // Half a tile: eight operands, MB products each.  The lookups run two pairs of operands ahead of
-    // the products that consume them, so that LDS latency hides behind matrix work.
-    template <int MB, bool BF16>
-    __device__ __forceinline__ void half(int j, const u4_t (&Aj)[MB], f4_t (&acc)[MB][8]) const {
-        constexpr int AHEAD = 2;
-        u4_t W[AHEAD + 1][2];
-#pragma unroll
-        for (int v = 0; v < AHEAD; ++v)
-#pragma unroll
-            for (int d = 0; d < 2; ++d) W[v][d] = operand(j, v, d);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            if (v + AHEAD < 4)
-#pragma unroll
-                for (int d = 0; d < 2; ++d) W[(v + AHEAD) % (AHEAD + 1)][d] = operand(j, v + AHEAD, d);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int d = 0; d < 2; ++d)
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb)
-                    acc[mb][v * 2 + d] = mfma16<BF16>(W[v % (AHEAD + 1)][d], Aj[mb], acc[mb][v * 2 + d]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
 };
 template <>
 struct FewStream<0> {};
@@ -210,9 +186,13 @@ __device__ __forceinline__ int few_lift(int shift) { return shift > 92 ? 36 : 0;
 
 // B2 == 0: one stream (launches of one stream each may share a fold, p.z_base and p.ztotal).
 // SEGS: several weights in the launch.
-template <int MB, bool BF16, int B1, int B2, bool SEGS>
+// FORM: 1: 16 rows, of A or of the image; 2: 32 rows of the image; 3: 32 rows of A.  (Forms of their own: what 32
+// rows need to read A themselves costs the image's launches 0.6 us where they step over it, and a loop for each in
+// one kernel costs more, in registers and in code that every launch fetches.)
+template <int FORM, bool BF16, int B1, int B2, bool SEGS>
 __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
-    static_assert(MB == 1 || MB == 2, "16 or 32 rows");
+    static_assert(FORM >= 1 && FORM <= 3, "16 or 32 rows");
+    constexpr int MB = FORM == 1 ? 1 : 2;
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int KW = 8, NT = 512;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -232,36 +212,53 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     // unconditional like everyone's, and the compiler can count them.
     const int g_first = left > 0 ? g0 : gbeg;
 
-    // ---- activations: the image (its blocks are padded to whole workgroups), or A itself (MB == 1 and
-    // rows of whole 16-byte pieces), whose pieces are put into operand order in registers ----------
-    const bool direct = MB == 1 && p.A8 != nullptr;
-    const int a_row = mb0 * 16 + rho;
-    const bool a_row_valid = a_row < p.M;
+    // ---- activations: A itself where its rows are whole 16-byte pieces, put into operand order in registers,
+    // or the image (its blocks are padded to whole workgroups) ------------------------------------------
+    const bool direct = FORM == 3 || (FORM == 1 && p.A8 != nullptr);
     const bool find = MB == 1 && p.find;
-    int a_shift = direct && p.rowshift && a_row_valid ? p.rowshift[a_row] : 0;
-    const int64_t jstep = direct ? 4 : (int64_t)p.mblk_pad * 64, gstep = direct ? 8 : 2 * jstep;
-    const u4_t *ap = (direct ? p.A8 + (int64_t)(a_row_valid ? a_row : 0) * p.lda8 + kg : p.Ap + (int64_t)mb0 * 64 + lane) +
-                     (int64_t)g_first * gstep;
-    auto load_a = [&](u4_t (&Aj)[MB], const u4_t *src) {
+    // Four lanes to the 64 bytes of a row, as the address path likes it (lane per row and piece: 64 accesses an
+    // instruction, not 16), in the order of rows that to_operand leaves as 0 ... 15.  Rows beyond M repeat the
+    // last: nobody stores their outputs.
+    const int load_row = ((lane >> 2) & 3) * 4 + (lane >> 4);
+    int a_row[MB], a_shift[MB];
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) Aj[mb] = src[mb * 64];
+    for (int mb = 0; mb < MB; ++mb) {
+        a_row[mb] = min((mb0 + mb) * 16 + load_row, p.M - 1);
+        a_shift[mb] = 0;
+    }
+    // (uniform base, 32-bit offsets of a lane: few_lda bounds the stride)
+    const int64_t jstep = direct ? 4 : (int64_t)p.mblk_pad * 64, gstep = direct ? 8 : 2 * jstep;
+    const u4_t *ap = (direct ? p.A8 + (int64_t)mb0 * 16 * p.lda8 : p.Ap + (int64_t)mb0 * 64) + (int64_t)g_first * gstep;
+    uint32_t a_ofs[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+        a_ofs[mb] = direct ? ((uint32_t)(a_row[mb] - mb0 * 16) * (uint32_t)p.lda8 + (lane & 3)) * 16 : mb * 1024 + lane * 16;
+    auto load_a = [&](u4_t (&Aj)[MB], int64_t ofs) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) Aj[mb] = *(const u4_t *)((const char *)(ap + ofs) + a_ofs[mb]);
     };
-    // (rows beyond M are zero; the activations are presented in the LUT's 16-bit type)
+    // A lane has loaded piece lane & 3 of its row, eight consecutive k; the matrix cores want lane kg * 16 + rho to
+    // hold the pairs (2*kg, 2*kg + 1) of all four pieces of row rho, in the LUT's 16-bit type: dwords change
+    // places with the lane's upper two bits, then with the lower two.
     auto to_operand = [&](u4_t (&T)[MB]) {
         if (!direct) return;
-        if constexpr (MB == 1) {
-            u4_t raw = T[0];
-            if (!a_row_valid) raw = u4_t{0u, 0u, 0u, 0u};
-            if (p.a_bf16 != (int)BF16) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint16_t lo16 = (uint16_t)(raw[q] & 0xffffu), hi16 = (uint16_t)(raw[q] >> 16);
-                    const float flo = ldexpf(p.a_bf16 ? bf2f(lo16) : h2f(lo16), -a_shift);
-                    const float fhi = ldexpf(p.a_bf16 ? bf2f(hi16) : h2f(hi16), -a_shift);
-                    raw[q] = (uint32_t)round_act(flo, BF16) | ((uint32_t)round_act(fhi, BF16) << 16);
+        for (int mb = 0; mb < MB; ++mb) {
+            uint32_t q[4] = {T[mb][0], T[mb][1], T[mb][2], T[mb][3]};
+            if constexpr (!BF16) {
+                if (p.a_bf16) {
+                    typedef float f2_t __attribute__((ext_vector_type(2)));
+                    typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        q[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(
+                            (f2_t{ldexpf(__builtin_bit_cast(float, q[e] << 16), -a_shift[mb]),
+                                  ldexpf(__builtin_bit_cast(float, q[e] & 0xffff0000u), -a_shift[mb])}), h2_t));
                 }
             }
-            T[0] = quad_transpose(raw, lane);
+            transpose_lanes16(q);
+            transpose_quad(q, lane);
+            T[mb] = u4_t{q[0], q[1], q[2], q[3]};
         }
     };
 
@@ -303,34 +300,35 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     __builtin_amdgcn_sched_barrier(0);
     s1.load();
     if constexpr (B2 > 0) s2.load();
-    load_a(A0, ap);
-    load_a(A1, ap + jstep);
+    load_a(A0, 0);
+    load_a(A1, jstep);
     __builtin_amdgcn_sched_barrier(0);
+    if (direct && p.rowshift)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) a_shift[mb] = p.rowshift[a_row[mb]];
     lut1.build(smem, lane, wave);
     if constexpr (B2 > 0) lut2.build(smem + tab2, lane, wave);
     // bfloat16 rows in front of a float16 LUT: each wavefront looks two of the workgroup's rows through for
     // their scales (few_finds).
     int *const found = (int *)(smem + few_lds_bytes<B1, B2, MB>());
-    if constexpr (MB == 1) {
-        if (find) {
-            const int pieces = p.G * 8;                 // of a row
-            for (int r = wave; r < 16 && mb0 * 16 + r < p.M; r += 8) {
-                const u4_t *const row = p.A8 + (int64_t)(mb0 * 16 + r) * p.lda8;
-                uint32_t e = 0;
-                for (int i = 0; i < pieces; i += 512) { // (past the end: the last piece again)
-                    u4_t v[8];
+    if (find) {
+        const int pieces = p.G * 8;                     // of a row
+        for (int r = wave; r < 16 && mb0 * 16 + r < p.M; r += 8) {
+            const u4_t *const row = p.A8 + (int64_t)(mb0 * 16 + r) * p.lda8;
+            uint32_t e = 0;
+            for (int i = 0; i < pieces; i += 512) {     // (past the end: the last piece again)
+                u4_t v[8];
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) v[u] = row[min(i + u * 64 + lane, pieces - 1)];
+                for (int u = 0; u < 8; ++u) v[u] = row[min(i + u * 64 + lane, pieces - 1)];
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) e = max(e, bf16_max_exp8(make_uint4(v[u][0], v[u][1], v[u][2], v[u][3])));
-                }
-                e = wavefront_max(e);
-                if (lane == 0) found[r] = bf16_row_shift(e);
+                for (int u = 0; u < 8; ++u) e = max(e, bf16_max_exp8(make_uint4(v[u][0], v[u][1], v[u][2], v[u][3])));
             }
+            e = wavefront_max(e);
+            if (lane == 0) found[r] = bf16_row_shift(e);
         }
     }
     __syncthreads();
-    if (find && a_row_valid) a_shift = found[rho];
+    if (find) a_shift[0] = found[a_row[0] & 15];
 
     f4_t acc[MB][8];
 #pragma unroll
@@ -349,28 +347,59 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
         s1.load();
         if constexpr (B2 > 0) s2.load();
     };
-    if (left > 0) next_codes(left > 1);
+    // A turn is one run of operand pairs (half a tile: four of the first stream, four of the second), MB products
+    // an operand.  The lookups run two pairs ahead of the products that consume them, from one half and
+    // stream into the next, and the next tile's codes leave the staging behind the last of them, so that LDS
+    // latency hides behind matrix work.
+    constexpr int STREAMS = B2 > 0 ? 2 : 1, HALF = 4 * STREAMS, PAIRS = 2 * HALF, AHEAD = 2;
+    u4_t W[AHEAD + 1][2];
+    auto lookup = [&](int u) {
+        const int j = u / HALF, v = u & 3;
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            if constexpr (B2 > 0) W[u % (AHEAD + 1)][d] = (u & 4) ? s2.operand(j, v, d) : s1.operand(j, v, d);
+            else W[u % (AHEAD + 1)][d] = s1.operand(j, v, d);
+        }
+    };
+    auto get_codes = [&]() {
+        s1.get();
+        if constexpr (B2 > 0) s2.get();
+    };
+    if (left > 0) {
+        next_codes(left > 1);
+        get_codes();
+    }
     while (left > 0) {
         // the two wavefronts of a SIMD (w and w + 4) take turns at the higher priority
         if ((left + (wave >> 2)) & 1) __builtin_amdgcn_s_setprio(1);
         else __builtin_amdgcn_s_setprio(0);
-        s1.get();
-        if constexpr (B2 > 0) s2.get();
-        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) lookup(u);
         to_operand(A0);
-        s1.template half<MB, BF16>(0, A0, acc);
-        if constexpr (B2 > 0) s2.template half<MB, BF16>(0, A0, acc);
-        if (left > 1) ap += KW * gstep;
-        load_a(A0, ap);
-        // issue order activations -> codes: the wait for these activations at the top of the next
-        // round then does not include the codes'
-        __builtin_amdgcn_sched_barrier(0);
-        next_codes(left > 2);
-        __builtin_amdgcn_sched_barrier(0);
-        to_operand(A1);
-        s1.template half<MB, BF16>(1, A1, acc);
-        if constexpr (B2 > 0) s2.template half<MB, BF16>(1, A1, acc);
-        load_a(A1, ap + jstep);
+#pragma unroll
+        for (int u = 0; u < PAIRS; ++u) {
+            if (u + AHEAD < PAIRS) lookup(u + AHEAD);
+            if (u + AHEAD == PAIRS) get_codes();
+            if (u == HALF) {
+                if (left > 1) ap += KW * gstep;
+                load_a(A0, 0);
+                // issue order activations -> codes: the wait for these activations at the top of the next
+                // round then does not include the codes'
+                __builtin_amdgcn_sched_barrier(0);
+                next_codes(left > 2);
+                __builtin_amdgcn_sched_barrier(0);
+                to_operand(A1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+                    acc[mb][(u & 3) * 2 + d] = mfma16<BF16>(W[u % (AHEAD + 1)][d], u < HALF ? A0[mb] : A1[mb],
+                                                            acc[mb][(u & 3) * 2 + d]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        load_a(A1, jstep);
         __builtin_amdgcn_sched_barrier(0);
         --left;
     }

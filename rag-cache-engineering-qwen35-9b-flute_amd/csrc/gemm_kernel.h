@@ -91,12 +91,15 @@ struct GemmParams {
     int z_base, ztotal;    // partial tiles: this launch writes [z_base, z_base + gridDim.z) of
                            // ztotal (several launches, one per stream, may share a fold)
     int out_bf16;          // dtype of C, resA, bias
-    const u4_t *A8;        // 16-row workgroups: A itself, rows of lda8 16-byte pieces, no pre-pass (or NULL)
+    const u4_t *A8;        // few rows: A itself, rows of lda8 16-byte pieces, no pre-pass (or NULL)
     int64_t lda8;
     int a_bf16;            // dtype of A there
     int find;              // A8 of one type and a LUT of the other: workgroups look for their rows' scales themselves
     const int *rowshift;   // [M] or NULL: row m of the operands holds A[m] * 2^-rowshift[m]
 };
+
+// Strides of A (elements) at which the offsets of a few-row workgroup's lanes within its rows fit 32 bits.
+constexpr int64_t few_lda() { return (int64_t)1 << 25; }
 
 // Activation pre-pass of rows that are not 16-byte aligned (others: gemm_pre_kernel):
 // Ap[g][j][mb][lane][slot] in the LUT's 16-bit type.
@@ -538,30 +541,6 @@ __device__ __forceinline__ void half_mma(const uint32_t (&Q)[4 * B], int j, cons
                     mfma16<BF16>(W[v % (AHEAD + 1)][d], Aj[mb], acc[mb][v * 2 + d]);
         __builtin_amdgcn_sched_barrier(0);
     }
-}
-
-// A itself instead of the image (16-row workgroups, gemm_few_kernel.h): a lane has loaded eight consecutive k of its row
-// (piece c = lane >> 4 of the 32-k half tile), the matrix cores want the pairs
-// (2*kg, 2*kg + 1) of all four pieces.  With the four lanes that share a row (16 apart)
-// this is a 4 x 4 transpose of dwords: in round r every lane offers dword (kg + r) & 3 and
-// reads the offer of piece (kg - r) & 3, which is that piece's dword kg.
-__device__ __forceinline__ u4_t quad_transpose(u4_t v, int lane) {
-    const int kg = lane >> 4;
-    u4_t out = v;                                      // round 0: own piece, dword kg stays
-#pragma unroll
-    for (int r = 1; r < 4; ++r) {
-        const int give = (kg + r) & 3, take = (kg - r) & 3;
-        const uint32_t offer = (give & 2) ? ((give & 1) ? v[3] : v[2]) : ((give & 1) ? v[1] : v[0]);
-        const uint32_t got = (uint32_t)__builtin_amdgcn_ds_bpermute(
-            (take * 16 + (lane & 15)) << 2, (int)offer);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) out[q] = (take == q) ? got : out[q];
-    }
-    // out[q] for q != kg now holds piece q's dword kg; the own piece contributes v[kg] at q = kg
-    const uint32_t own = (kg & 2) ? ((kg & 1) ? v[3] : v[2]) : ((kg & 1) ? v[1] : v[0]);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) out[q] = (kg == q) ? own : out[q];
-    return out;
 }
 
 // Block mb of an activation half: 16 bytes per lane at src + mb KB, as a statement the compiler

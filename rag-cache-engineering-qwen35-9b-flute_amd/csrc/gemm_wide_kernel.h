@@ -51,18 +51,6 @@ struct WideParams {
     int *tickets;
 };
 
-// Dword b of the lane whose bits (5, 4) are a changes places with dword a of the one whose are b.
-__device__ __forceinline__ void transpose_lanes16(uint32_t (&q)[4]) {
-    auto p = __builtin_amdgcn_permlane32_swap(q[0], q[2], false, false);
-    q[0] = p[0]; q[2] = p[1];
-    p = __builtin_amdgcn_permlane32_swap(q[1], q[3], false, false);
-    q[1] = p[0]; q[3] = p[1];
-    p = __builtin_amdgcn_permlane16_swap(q[0], q[1], false, false);
-    q[0] = p[0]; q[1] = p[1];
-    p = __builtin_amdgcn_permlane16_swap(q[2], q[3], false, false);
-    q[2] = p[0]; q[3] = p[1];
-}
-
 typedef const __attribute__((address_space(1))) uint8_t *GlobalBytes;
 typedef const __attribute__((address_space(1))) u4_t *GlobalQuad;
 typedef const __attribute__((address_space(1))) uint32_t *GlobalWord;

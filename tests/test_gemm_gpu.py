@@ -117,6 +117,49 @@ def test_gemm_direct_activations_match_the_pre_pass(tuning_env, M, N, K, gs, act
     assert torch.equal(_dual(w, shifted[1:].reshape(M, K)), y)
 
 
+@pytest.mark.parametrize("M,K,bits,bits2,act,lut,rot", [
+    (17, 64, 4, 0, torch.float16, torch.float16, False),           # one row in the second block, one tile of K
+    (32, 576, 3, 3, torch.bfloat16, torch.bfloat16, False),        # more wavefronts with a second tile than without
+    (33, 1088, 4, 3, torch.float16, torch.float16, False),         # a workgroup with a single row
+    (63, 1024, 2, 0, torch.bfloat16, torch.bfloat16, True),
+    (40, 8256, 4, 1, torch.bfloat16, torch.float16, False),        # scales from a launch in front
+    (48, 1024, 1, 4, torch.bfloat16, torch.float16, True),         # scales from the rotation
+])
+def test_gemm_32_row_workgroups_read_the_rows_themselves(tuning_env, M, K, bits, bits2, act, lut, rot):
+    """32-row workgroups on the rows of A and on the operand image: equal bits, at any stride of the rows."""
+    tuning_env("FLUTE_GEMM_ROWS", "32")
+    w = make_weight(256, K, bits, 128, seed=M + K, bits2=bits2, lut_dtype=lut, act_dtype=act, bias=True, device=DEV)
+    signs = O.rotation_signs(K, 3).to(DEV) if rot else None
+    wide = torch.full((M, K + 24), float("nan"), dtype=act, device=DEV)
+    x = make_x(M, K, seed=M, dtype=act).to(DEV)
+    x[0] *= 1e3
+    x[M - 1] = 0
+    wide[:, 8:K + 8] = x
+    import ctypes
+    from flute_extended import _lib
+    kind = lambda t: _lib.BF16 if t == torch.bfloat16 else _lib.F16
+    d = _lib.FluteLinear()
+    d.q1, d.lut1, d.q1_bytes, d.b1 = w["blob_d"].data_ptr(), w["lut_d"].data_ptr(), w["blob_d"].numel(), bits
+    if bits2:
+        d.q2, d.lut2, d.q2_bytes, d.b2 = w["blob2_d"].data_ptr(), w["lut2_d"].data_ptr(), w["blob2_d"].numel(), bits2
+    d.N, d.K, d.group_size, d.lut_rows, d.lut_dtype, d.bias = 256, K, 128, 2, kind(lut), w["bias_d"].data_ptr()
+    if rot:
+        d.signs = signs.data_ptr()
+
+    def run(a):
+        C = torch.zeros(M, 256, dtype=act, device=DEV)
+        assert _lib.lib.flute_gemm(ctypes.byref(d), a.data_ptr(), C.data_ptr(), M, a.stride(0), 256, kind(act),
+                                   torch.cuda.current_stream().cuda_stream) == 0, _lib.last_error()
+        return C
+
+    rows = run(x)
+    assert torch.equal(run(wide[:, 8:K + 8]), rows)
+    tuning_env("FLUTE_GEMM_NO_DIRECT", "1")
+    assert torch.equal(run(x), rows)
+    if not rot:
+        assert rel_l2(rows.cpu(), _exact(w, x.cpu()).to(act)) <= (TOL if act == torch.float16 else TOL_BF16)
+
+
 DUAL = [
     # M, N, K, bits, gs, bits2, rank, bias
     (8, 512, 1024, 4, 128, 1, 0, False),
