@@ -49,9 +49,7 @@ bool few_takes(int b1, int b2) { return !(b1 == 4 && b2 == 4); }
 // M = 32, 4096 -> 12288, 16 and 32 rows: 4 bits 13.2 / 14.4, (3, 3) bits, M = 24 23.6 / 20.2; M = 64: 25.6 / 17.1;
 // M = 48, 12288 -> 4096: 19.0 / 17.8, (4, 1) bits, bfloat16 rows 31.3 / 27.1; M = 128, 4096 -> 4096: 13.1 / 14.1;
 // M = 200: 24.0 / 16.6; M = 300, 4096 -> 1024 12.6 / 13.1; M = 100, 2048 -> 8192, (4, 1) bits 21.0 / 15.5.
-// (A residual's launch in front of 16-row workgroups is not in it.  Where the choice misses: M = 22,
-// 6912 -> 4224, (2, 3) bits, rank 16: 16 rows 28.4, 32 rows 23.4; M = 233, 1408 -> 8448, twice 1 bit: the
-// many-row kernel 30.7, 16 rows 25.2; over 58 other random shapes it is within 3 % of the best of six.)
+// (A launch in front of 16-row workgroups is not in it.)
 double few_us(int mb, int M, int tiles, int G, int b1, int b2) {
     static const double tile_us[5] = {0.0, 0.6, 0.75, 1.2, 1.15};
     const GemmShape shape = {mb, 8, 1, 1};
@@ -458,16 +456,19 @@ bool few_finds(int M, int K, int64_t workgroups) {
 
 // Whether workgroups of few rows read A themselves.  Sixteen rows always do.  Thirty-two do where that leaves no
 // launch in front, and where a launch that only looks for scales in few, long rows is the shorter for it; beside
-// coefficients the image costs nothing, and rows of one type in front of a LUT of the other cost each turn of
+// coefficients of more ranks (few_coeff) the image costs nothing, and rows of one type in front of a LUT of the other cost each turn of
 // the loop their conversions (0.3 us).  The image and A itself, us a call: M = 64, 4096 -> 12288 18.1 / 17.2;
 // M = 200, 4096 -> 4096 19.5 / 16.6; M = 24, 4096 -> 12288, (3, 3) bits 22.0 / 20.2; bfloat16 rows, float16 LUT: M = 48,
 // 12288 -> 4096, (4, 1) bits 29.0 / 27.0; M = 64, 4096 -> 12288, eight turns, 20.0 / 21.3, rotated 22.2 / 22.8; M = 24, four
-// turns, (4, 1) bits, rotated 23.1 / 21.6; M = 64, 12288 -> 12288, 24 turns, 43.6 / 46.3; residual of rank 16, M = 48, 12288 -> 4096, (4, 1) bits 28.9 / 30.7.
-bool few_reads(const GemmShape &shape, bool residual, bool scale_rows, bool rotated, int K, int gper) {
+// turns, (4, 1) bits, rotated 23.1 / 21.6; M = 64, 12288 -> 12288, 24 turns, 43.6 / 46.3; coefficients in front, M = 48, 12288 -> 4096,
+// (4, 1) bits 28.9 / 30.7.
+bool few_reads(const GemmShape &shape, bool scale_rows, bool rotated, int K, int gper) {
     if (shape.mb == 1) return true;
-    if (residual) return false;
     return !scale_rows || ((rotated || K > 8192) && (gper + 7) / 8 <= 6);
 }
+
+// Residuals whose coefficients the few-row kernel can form: one operand of ranks.
+bool few_coeff(const flute_linear &w) { return w.R > 0 && w.R <= 16 && ((uintptr_t)w.resB & 15) == 0; }
 
 // Up to four weights of one width pair, group size and rotation over the same rows of A through the
 // small-M kernel, in the given shape: one launch of each pre-pass and one (per stream) of the kernel.
@@ -538,25 +539,35 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
     const bool per_stream = p.nstreams == 2 && !(few && few_takes(p.bits[0], p.bits[1]));
     const int zparts = ksplit * (per_stream ? 2 : 1);
     const size_t p_floats = zparts > 1 ? (size_t)zparts * units * image : 0;
-    const CoeffPlan coeff = plan_coeff(ws, count, M);
-    size_t xb_floats = any_res ? coeff.floats() : 0;
-    for (int i = 0; i < count; ++i) xb_floats += ((size_t)M * ws[i].R + 3) & ~(size_t)3;
-    const size_t rot_floats = w->signs ? ((size_t)M * w->K / 2 + 4) & ~(size_t)3 : 0;
     // bfloat16 activations presented as float16 operands: one power-of-two scale per row
     const bool scale_rows = act_dtype == FLUTE_BF16 && w->lut_dtype == FLUTE_F16;
+    const bool rows16 = w->signs || (((uintptr_t)A & 15) == 0 && lda % 8 == 0);
+    const bool reads = few && rows16 && (w->signs ? w->K : lda) <= few_lda() && !up && !tuning().gemm_no_direct;
+    p.find = reads && shape.mb == 1 && scale_rows && !w->signs && few_finds(M, w->K, units * ksplit);
+    // Residuals of up to 16 ranks whose rows the kernel reads, and needs nothing else of a launch in front for: it
+    // forms their coefficients beside its products (gemm_few_kernel.h).
+    bool coeff_in = reads && !per_stream && few_reads(shape, scale_rows, w->signs != nullptr, w->K, p.gper) &&
+                    (!scale_rows || w->signs || p.find);
+    for (int i = 0; i < count; ++i) coeff_in &= few_coeff(ws[i]);
+    const bool coeff_pre = any_res && !coeff_in;
+    p.find &= !coeff_pre;
+    for (int i = 0; i < count; ++i) p.seg[i].resB = coeff_in ? (const uint16_t *)ws[i].resB : nullptr;
+    const CoeffPlan coeff = plan_coeff(ws, count, M);
+    size_t xb_floats = coeff_pre ? coeff.floats() : 0;
+    for (int i = 0; i < count && coeff_pre; ++i) xb_floats += ((size_t)M * ws[i].R + 3) & ~(size_t)3;
+    const size_t rot_floats = w->signs ? ((size_t)M * w->K / 2 + 4) & ~(size_t)3 : 0;
     const size_t shift_floats = scale_rows ? ((size_t)M + 3) & ~(size_t)3 : 0;
     // Few rows: the kernel reads A itself where that pays (16-byte pieces of a row, put into
     // operand order in registers), so the pre-pass launch is dropped, and the image with it.  Needs
     // 16-byte aligned rows; rotated rows are read the same way (the rotation can write the image itself,
     // but only without a residual and row scales).
     const bool image_of_rotation = w->signs && !any_res && !scale_rows;
-    const bool rows16 = w->signs || (((uintptr_t)A & 15) == 0 && lda % 8 == 0);
-    const bool direct = few && few_reads(shape, any_res, scale_rows, w->signs != nullptr, w->K, p.gper) && !up &&
-                        !tuning().gemm_no_direct && rows16 && (w->signs ? w->K : lda) <= few_lda() && !image_of_rotation;
+    const bool direct = reads && !image_of_rotation &&
+                        (coeff_pre ? shape.mb == 1 : few_reads(shape, scale_rows, w->signs != nullptr, w->K, p.gper));
     const size_t ap_floats = direct ? 0 : (size_t)p.G * 2 * p.mblk_pad * 64 * 4;
     float *base = nullptr;
     int *tickets = nullptr;
-    const size_t want_tickets = std::max((size_t)units, any_res ? coeff.tickets() : 0) + 1;
+    const size_t want_tickets = std::max((size_t)units, coeff_pre ? coeff.tickets() : 0) + 1;
     st = get_workspace(p_floats + xb_floats + ap_floats + rot_floats + shift_floats + 64, want_tickets, stream, &base,
                        &tickets);
     if (st != FLUTE_OK) return st;
@@ -585,7 +596,6 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
             lda = w->K;
         }
         p.rowshift = rowshift;                          // (the rotation knows its rows' largest exponents)
-        p.find = direct && shape.mb == 1 && scale_rows && !w->signs && !any_res && few_finds(M, w->K, units * ksplit);
         if (p.find) p.rowshift = nullptr;
         const bool find = scale_rows && !w->signs && !p.find;
         ImageParams im = {};
@@ -625,13 +635,13 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
         }
         float *next = xb + coeff.floats(), *to[kGemmMaxSegs] = {};
         for (int i = 0; i < count; ++i) {
-            if (ws[i].R == 0) continue;
+            if (ws[i].R == 0 || coeff_in) continue;
             to[i] = next;
             p.seg[i].xb = next;
             p.seg[i].vec_res = ws[i].R % 4 == 0 && ((uintptr_t)ws[i].resA & 7) == 0 && ((uintptr_t)next & 15) == 0;
             next += ((size_t)M * ws[i].R + 3) & ~(size_t)3;
         }
-        st = launch_pre(any_res ? &coeff : nullptr, ws, count, A, lda, to, M, p.out_bf16, xb, tickets, im, stream);
+        st = launch_pre(coeff_pre ? &coeff : nullptr, ws, count, A, lda, to, M, p.out_bf16, xb, tickets, im, stream);
         if (st != FLUTE_OK) return st;
     }
 
@@ -700,8 +710,12 @@ GemmPlan plan_gemm(const flute_linear *ws, int count, int M) {
 }
 
 // Whether a call forms silu(gate) * up on its way to the operand image: calls that have one, of rows that are not
-// rotated (the rotation wants the rows themselves, as do coefficients of factors that are not aligned).
+// rotated (the rotation wants the rows themselves, as do coefficients of factors that are not aligned, and
+// the few-row kernel where it forms the coefficients: their sums have an order of their own).
 bool takes_silu(const flute_linear &w, const GemmPlan &plan, int act_dtype) {
+    if (!plan.wide.rows && plan.shape.mb == 2 && few_coeff(w) && !tuning().gemm_no_direct &&
+        (act_dtype == FLUTE_BF16) == (w.lut_dtype == FLUTE_BF16) && few_takes(std::max(w.b1, w.b2), std::min(w.b1, w.b2)))
+        return false;
     return !w.signs && ((uintptr_t)w.resB & 15) == 0 && (plan.wide.rows || plan.shape.mb > 1) &&
            (w.K <= find_reach() || (act_dtype == FLUTE_BF16) == (w.lut_dtype == FLUTE_BF16));
 }

@@ -38,9 +38,13 @@ constexpr int few_lds_bytes() {
     return loop > sums ? loop : sums;
 }
 
-// Bytes of a launch: behind the above, the scales of sixteen rows that a workgroup looks for itself.
-template <int B1, int B2, int MB>
-constexpr int few_lds_total() { return few_lds_bytes<B1, B2, MB>() + (MB == 1 ? 64 : 0); }
+// Bytes of a launch: behind the above, the scales of sixteen rows that a workgroup looks for itself, and every
+// wavefront's residual coefficients.
+template <int B1, int B2, int FORM>
+constexpr int few_lds_total() {
+    constexpr int MB = FORM == 1 || FORM == 4 ? 1 : 2;
+    return few_lds_bytes<B1, B2, MB>() + (MB == 1 ? 64 : 0) + (FORM >= 4 ? 8 * MB * 64 * 16 : 0);
+}
 
 // What a thread contributes to a table: the LUT values its entries are made of, requested with the
 // kernel's first loads; `build` waits for them only.
@@ -186,13 +190,15 @@ __device__ __forceinline__ int few_lift(int shift) { return shift > 92 ? 36 : 0;
 
 // B2 == 0: one stream (launches of one stream each may share a fold, p.z_base and p.ztotal).
 // SEGS: several weights in the launch.
-// FORM: 1: 16 rows, of A or of the image; 2: 32 rows of the image; 3: 32 rows of A.  (Forms of their own: what 32
-// rows need to read A themselves costs the image's launches 0.6 us where they step over it, and a loop for each in
-// one kernel costs more, in registers and in code that every launch fetches.)
+// FORM: 1: 16 rows, of A or of the image; 2: 32 rows of the image; 3: 32 rows of A; 4, 5: as 1 and 3, of A, with the
+// residual's coefficients.  (Forms of their own: what 32 rows need to read A themselves costs the image's launches
+// 0.6 us where they step over it, and a loop for each in one kernel costs more, in registers and in code that every
+// launch fetches.)
 template <int FORM, bool BF16, int B1, int B2, bool SEGS>
 __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
-    static_assert(FORM >= 1 && FORM <= 3, "16 or 32 rows");
-    constexpr int MB = FORM == 1 ? 1 : 2;
+    static_assert(FORM >= 1 && FORM <= 5, "16 or 32 rows");
+    constexpr int MB = FORM == 1 || FORM == 4 ? 1 : 2;
+    constexpr bool COEFF = FORM >= 4;
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int KW = 8, NT = 512;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -214,52 +220,74 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
 
     // ---- activations: A itself where its rows are whole 16-byte pieces, put into operand order in registers,
     // or the image (its blocks are padded to whole workgroups) ------------------------------------------
-    const bool direct = FORM == 3 || (FORM == 1 && p.A8 != nullptr);
+    const bool direct = FORM >= 3 || (FORM == 1 && p.A8 != nullptr);
     const bool find = MB == 1 && p.find;
     // Four lanes to the 64 bytes of a row, as the address path likes it (lane per row and piece: 64 accesses an
     // instruction, not 16), in the order of rows that to_operand leaves as 0 ... 15.  Rows beyond M repeat the
     // last: nobody stores their outputs.
     const int load_row = ((lane >> 2) & 3) * 4 + (lane >> 4);
-    int a_row[MB], a_shift[MB];
+    int a_shift[MB];                                    // of row rho
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-        a_row[mb] = min((mb0 + mb) * 16 + load_row, p.M - 1);
-        a_shift[mb] = 0;
-    }
+    for (int mb = 0; mb < MB; ++mb) a_shift[mb] = 0;
     // (uniform base, 32-bit offsets of a lane: few_lda bounds the stride)
     const int64_t jstep = direct ? 4 : (int64_t)p.mblk_pad * 64, gstep = direct ? 8 : 2 * jstep;
     const u4_t *ap = (direct ? p.A8 + (int64_t)mb0 * 16 * p.lda8 : p.Ap + (int64_t)mb0 * 64) + (int64_t)g_first * gstep;
     uint32_t a_ofs[MB];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
-        a_ofs[mb] = direct ? ((uint32_t)(a_row[mb] - mb0 * 16) * (uint32_t)p.lda8 + (lane & 3)) * 16 : mb * 1024 + lane * 16;
+        a_ofs[mb] = direct ? ((uint32_t)(min((mb0 + mb) * 16 + load_row, p.M - 1) - mb0 * 16) * (uint32_t)p.lda8 + (lane & 3)) * 16
+                           : mb * 1024 + lane * 16;
     auto load_a = [&](u4_t (&Aj)[MB], int64_t ofs) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) Aj[mb] = *(const u4_t *)((const char *)(ap + ofs) + a_ofs[mb]);
     };
+    // COEFF: the residual's coefficients, A @ resB^T over this slice of K, as one more operand of sixteen weights: rank
+    // r in the place of row r.  They cost the loop an eighth of its products and a load of half its codes' size
+    // instead of a launch in front: M = 8, 4096 -> 4096, rank 16 14.0 -> 10.0 us; M = 48, 12288 -> 4096, (4, 1) bits
+    // 30.3 -> 26.5; M = 22, 6912 -> 4224, (2, 3) bits 27.4 -> 18.2 (of which 5 by 32-row workgroups); M = 200, 4096 ->
+    // 4096 23.7 -> 20.2.  fp32 sums of products of the activations' own type.
+    const u4_t *bp = COEFF ? (const u4_t *)w.resB + (int64_t)g_first * 8 : nullptr;
+    const uint32_t b_ofs = COEFF ? ((uint32_t)min(load_row, w.R - 1) * (uint32_t)(p.G * 8) + (lane & 3)) * 16 : 0;
+    u4_t RB0 = {0u, 0u, 0u, 0u}, RB1 = {0u, 0u, 0u, 0u};
+    f4_t xacc[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) xacc[mb] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    auto load_b = [&](u4_t &to, int ofs) {
+        if constexpr (COEFF) to = *(const u4_t *)((const char *)(bp + ofs) + b_ofs);
+    };
     // A lane has loaded piece lane & 3 of its row, eight consecutive k; the matrix cores want lane kg * 16 + rho to
     // hold the pairs (2*kg, 2*kg + 1) of all four pieces of row rho, in the LUT's 16-bit type: dwords change
     // places with the lane's upper two bits, then with the lower two.
-    auto to_operand = [&](u4_t (&T)[MB]) {
+    auto transposed = [&](u4_t v) {
+        uint32_t q[4] = {v[0], v[1], v[2], v[3]};
+        transpose_lanes16(q);
+        transpose_quad(q, lane);
+        return u4_t{q[0], q[1], q[2], q[3]};
+    };
+    auto to_operand = [&](u4_t (&T)[MB], u4_t rb) {
         if (!direct) return;
+        if constexpr (COEFF) rb = transposed(rb);
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-            uint32_t q[4] = {T[mb][0], T[mb][1], T[mb][2], T[mb][3]};
-            if constexpr (!BF16) {
-                if (p.a_bf16) {
-                    typedef float f2_t __attribute__((ext_vector_type(2)));
-                    typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+        for (int mb = 0; mb < MB; ++mb) T[mb] = transposed(T[mb]);
+        if constexpr (!BF16) {
+            if (p.a_bf16) {
+                typedef float f2_t __attribute__((ext_vector_type(2)));
+                typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) {
+                    if constexpr (COEFF) xacc[mb] = mfma16<true>(rb, T[mb], xacc[mb]);
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        q[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(
-                            (f2_t{ldexpf(__builtin_bit_cast(float, q[e] << 16), -a_shift[mb]),
-                                  ldexpf(__builtin_bit_cast(float, q[e] & 0xffff0000u), -a_shift[mb])}), h2_t));
+                        T[mb][e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(
+                            (f2_t{ldexpf(__builtin_bit_cast(float, T[mb][e] << 16), -a_shift[mb]),
+                                  ldexpf(__builtin_bit_cast(float, T[mb][e] & 0xffff0000u), -a_shift[mb])}), h2_t));
                 }
+                return;
             }
-            transpose_lanes16(q);
-            transpose_quad(q, lane);
-            T[mb] = u4_t{q[0], q[1], q[2], q[3]};
         }
+        if constexpr (COEFF)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) xacc[mb] = mfma16<BF16>(rb, T[mb], xacc[mb]);
     };
 
     // ---- first loads, in the order they are waited for: LUT values, codes, activations ------------
@@ -268,7 +296,7 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     constexpr int stage_wave = FewTable<B1>::stage + FewTable<B2>::stage;
     const uint32_t stage = lds0 + stage0 + (uint32_t)wave * stage_wave;
     // (the residual's first sixteen ranks in front of all: what comes behind them can still be counted)
-    const bool residual = w.R > 0 && p.z_base + z == 0;
+    const bool residual = COEFF || (w.R > 0 && p.z_base + z == 0);
     uint16_t res_a[4] = {0, 0, 0, 0};
     float res_x[MB][4];
     const uint16_t *const res_row = w.resA + (int64_t)(t * 128 + (rho >> 3) * 64 + wave * 8 + (rho & 7)) * w.R;
@@ -277,9 +305,10 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             res_a[e] = k0 + e < w.R ? res_row[k0 + e] : (uint16_t)0;
+            if constexpr (!COEFF)
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
-                res_x[mb][e] = k0 + e < w.R ? w.xb[(int64_t)min((mb0 + mb) * 16 + rho, p.M - 1) * w.R + k0 + e] : 0.0f;
+                for (int mb = 0; mb < MB; ++mb)
+                    res_x[mb][e] = k0 + e < w.R ? w.xb[(int64_t)min((mb0 + mb) * 16 + rho, p.M - 1) * w.R + k0 + e] : 0.0f;
         }
     };
     if (residual) residual_load(0);
@@ -301,11 +330,13 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     s1.load();
     if constexpr (B2 > 0) s2.load();
     load_a(A0, 0);
+    load_b(RB0, 0);
     load_a(A1, jstep);
+    load_b(RB1, 4);
     __builtin_amdgcn_sched_barrier(0);
     if (direct && p.rowshift)
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) a_shift[mb] = p.rowshift[a_row[mb]];
+        for (int mb = 0; mb < MB; ++mb) a_shift[mb] = p.rowshift[min((mb0 + mb) * 16 + rho, p.M - 1)];
     lut1.build(smem, lane, wave);
     if constexpr (B2 > 0) lut2.build(smem + tab2, lane, wave);
     // bfloat16 rows in front of a float16 LUT: each wavefront looks two of the workgroup's rows through for
@@ -328,7 +359,10 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
         }
     }
     __syncthreads();
-    if (find) a_shift[0] = found[a_row[0] & 15];
+    if (find) {
+        a_shift[0] = found[min(rho, p.M - 1 - mb0 * 16)];
+        if constexpr (COEFF) unscale[0] = a_shift[0];
+    }
 
     f4_t acc[MB][8];
 #pragma unroll
@@ -375,20 +409,24 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
         else __builtin_amdgcn_s_setprio(0);
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u) lookup(u);
-        to_operand(A0);
+        to_operand(A0, RB0);
 #pragma unroll
         for (int u = 0; u < PAIRS; ++u) {
             if (u + AHEAD < PAIRS) lookup(u + AHEAD);
             if (u + AHEAD == PAIRS) get_codes();
             if (u == HALF) {
-                if (left > 1) ap += KW * gstep;
+                if (left > 1) {
+                    ap += KW * gstep;
+                    if constexpr (COEFF) bp += KW * 8;
+                }
                 load_a(A0, 0);
+                load_b(RB0, 0);
                 // issue order activations -> codes: the wait for these activations at the top of the next
                 // round then does not include the codes'
                 __builtin_amdgcn_sched_barrier(0);
                 next_codes(left > 2);
                 __builtin_amdgcn_sched_barrier(0);
-                to_operand(A1);
+                to_operand(A1, RB1);
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -400,26 +438,40 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
             __builtin_amdgcn_sched_barrier(0);
         }
         load_a(A1, jstep);
+        load_b(RB1, 4);
         __builtin_amdgcn_sched_barrier(0);
         --left;
     }
     __builtin_amdgcn_s_setprio(0);
 
-    // ---- residual: + xb @ resA^T, in fp32 products onto the sums of the first slice ----------------
+    // ---- residual: + xb @ resA^T, in fp32 products onto the sums of the first slice (COEFF: of each) ---
     // Wavefront i takes the outputs of accumulator i, sixteen ranks a step, of which lane group kg holds
     // four (the order of ranks is free as long as both operands agree): a few loads a lane, requested
     // with the first loads of one slice, where the threads of the last arrival read eight rows of resA
-    // each behind the exchange (M = 48, 4096 <- 12288, (4, 1) bits, rank 16: the call 31.2 us, now 28.9;
-    // M = 64, bfloat16 rows, 12288 <- 4096, 4 bits: 23.7 and 22.0; M = 8: 18.1 and 17.8).  Sums of rows that are held scaled are
+    // each behind the exchange.  Sums of rows that are held scaled are
     // scaled back ahead of it, in every slice: a residual may be of another magnitude than its row, and
     // is added at its own (few_lift).
-    if (w.R > 0 && p.rowshift) {
+    if (w.R > 0 && (p.rowshift || find)) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
             for (int i = 0; i < 8; ++i)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) acc[mb][i][q] = ldexpf(acc[mb][i][q], unscale[mb] - few_lift(unscale[mb]));
+    }
+    if constexpr (COEFF) {                              // of all wavefronts, in their order
+        f4_t *const part = (f4_t *)(smem + few_lds_bytes<B1, B2, MB>() + (MB == 1 ? 64 : 0));
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) part[(wave * MB + mb) * 64 + lane] = xacc[mb];
+        __syncthreads();                                // tables and staging are dead
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            f4_t sum = part[mb * 64 + lane];
+#pragma unroll
+            for (int u = 1; u < 8; ++u) sum += part[(u * MB + mb) * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) res_x[mb][e] = kg * 4 + e < w.R ? sum[e] : 0.0f;
+        }
     }
     if (residual) {
         f4_t sum[MB];
@@ -449,7 +501,7 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     // (kg >> 1) * 64 + i * 8 + (kg & 1) * 4 ... + 3.  A wavefront's area is in that order, the lane's
     // low bits XORed with the outputs' so that the sixteen (eight) threads that serve a row of C side
     // by side read different banks.
-    __syncthreads();                                    // tables and staging are dead
+    if constexpr (!COEFF) __syncthreads();              // tables and staging are dead
     f4_t *const red = (f4_t *)smem;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -518,7 +570,7 @@ __global__ void __launch_bounds__(512) gemm_few_kernel(const GemmParams p) {
     if (m >= p.M) return;
     const int n0 = t * 128 + n_in;
     if (p.rowshift || find) {                           // exact
-        const int sh = find ? found[ml] : w.R == 0 ? p.rowshift[m] : few_lift(p.rowshift[m]);
+        const int row_shift = find ? found[ml] : p.rowshift[m], sh = w.R == 0 ? row_shift : few_lift(row_shift);
 #pragma unroll
         for (int e = 0; e < PW; ++e) y[e] = ldexpf(y[e], sh);
     }

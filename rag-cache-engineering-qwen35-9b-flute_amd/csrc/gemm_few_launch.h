@@ -11,7 +11,7 @@ namespace flute {
 
 template <int FORM, bool BF16, int B1, int B2, bool SEGS>
 flute_status launch_few(const GemmParams &p, dim3 grid, hipStream_t stream) {
-    constexpr int lds = few_lds_total<B1, B2, FORM == 1 ? 1 : 2>();
+    constexpr int lds = few_lds_total<B1, B2, FORM>();
     static_assert(lds <= kLdsPerCU, "tables, staging or sums exceed a CU's LDS");
     static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
     if (!attr_done) {
@@ -47,6 +47,7 @@ flute_status launch_few_bits(const GemmParams &p, dim3 grid, hipStream_t stream)
 
 template <bool BF16, bool SEGS>
 flute_status launch_few_shape(int mb, const GemmParams &p, dim3 grid, hipStream_t stream) {
+    if (p.seg[0].resB) return mb == 1 ? launch_few_bits<4, BF16, SEGS>(p, grid, stream) : launch_few_bits<5, BF16, SEGS>(p, grid, stream);
     if (mb == 1) return launch_few_bits<1, BF16, SEGS>(p, grid, stream);
     return p.A8 ? launch_few_bits<3, BF16, SEGS>(p, grid, stream) : launch_few_bits<2, BF16, SEGS>(p, grid, stream);
 }

@@ -59,6 +59,7 @@ struct GemmSeg {
     void *C;
     const float *xb;       // [M, R] fp32 residual coefficients (A @ resB^T) or NULL
     const uint16_t *resA;  // [N, R] activation dtype
+    const uint16_t *resB;  // few rows that form xb themselves (R <= 16): [R, K] activation dtype; else NULL
     const uint16_t *bias;  // [N] activation dtype
     int64_t ldc;
     int gs, lut_rows, R;

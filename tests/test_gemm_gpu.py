@@ -160,6 +160,28 @@ def test_gemm_32_row_workgroups_read_the_rows_themselves(tuning_env, M, K, bits,
         assert rel_l2(rows.cpu(), _exact(w, x.cpu()).to(act)) <= (TOL if act == torch.float16 else TOL_BF16)
 
 
+@pytest.mark.parametrize("M,K,bits,bits2,rank,act,lut", [
+    (2, 64, 4, 0, 1, torch.float16, torch.float16), (17, 576, 3, 3, 16, torch.bfloat16, torch.bfloat16),
+    (33, 1088, 4, 2, 5, torch.float16, torch.float16), (15, 4160, 1, 0, 15, torch.bfloat16, torch.float16),
+    (40, 8256, 4, 1, 16, torch.bfloat16, torch.float16), (16, 1024, 4, 4, 8, torch.float16, torch.float16),
+    (20, 1024, 2, 1, 17, torch.float16, torch.float16)])
+@pytest.mark.parametrize("rows,slices", [(16, "1"), (16, "2"), (32, "1"), (32, "3")])
+def test_gemm_few_rows_residual_of_one_operand_of_ranks(tuning_env, M, K, bits, bits2, rank, act, lut, rows, slices):
+    """Residuals of up to 16 ranks, whose coefficients the few-row kernel forms beside its products, slice of K
+    by slice, and those that a launch in front forms (more ranks, twice 4 bits, 32 rows that need scales)."""
+    tuning_env("FLUTE_GEMM_ROWS", str(rows))
+    tuning_env("FLUTE_GEMM_KSPLIT", slices)
+    w = make_weight(256, K, bits, 128, seed=M + K, bits2=bits2, rank=rank, lut_dtype=lut, act_dtype=act, bias=True, device=DEV)
+    x = make_x(M, K, seed=M, dtype=act)
+    x[M // 2] *= 1e2
+    y = _dual(w, x).cpu()
+    ref = _exact(w, x).to(act)
+    for m in range(M):
+        assert rel_l2(y[m], ref[m]) <= (TOL if act == torch.float16 else TOL_BF16), m
+    tuning_env("FLUTE_GEMM_NO_DIRECT", "1")                # the launch in front: one rounding of the type apart
+    assert rel_l2(y, _dual(w, x).cpu()) <= (2 ** -11 if act == torch.float16 else 2 ** -8)
+
+
 DUAL = [
     # M, N, K, bits, gs, bits2, rank, bias
     (8, 512, 1024, 4, 128, 1, 0, False),
