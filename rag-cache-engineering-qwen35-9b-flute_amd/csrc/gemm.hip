@@ -27,14 +27,13 @@ struct GemmShape {
     int wg_per_cu;        // workgroups the policy expects to be resident per CU
 };
 
-// Slices of K: split until the grid reaches one workgroup per CU, while every wavefront keeps two
-// tiles or more; with more than 16 rows a workgroup at most four, because the workgroup that arrives
+// Slices of K of 64-row and 128-row workgroups: split until the grid reaches one workgroup per CU, while every
+// wavefront keeps two tiles or more, at most four, because the workgroup that arrives
 // last reads every partial tile of its unit back (64 rows, M = 64: 12288 -> 4096 29.7 us four ways,
 // 36.4 eight ways; 4096 -> 4096 21.8 four ways, 23.0 two ways, 24.6 eight ways).
 int slices_of_k(int64_t units, int G, const GemmShape &shape) {
-    const int most = shape.mb == 1 ? 64 : 4;
     int ks = 1;
-    while (units * ks * 2 <= (int64_t)kNumCU * shape.wg_per_cu && ks * 2 <= most && G / (ks * 2) >= shape.kw * 2) ks *= 2;
+    while (units * ks * 2 <= (int64_t)kNumCU * shape.wg_per_cu && ks < 4 && G / (ks * 2) >= shape.kw * 2) ks *= 2;
     return ks;
 }
 
@@ -50,16 +49,30 @@ bool few_takes(int b1, int b2) { return !(b1 == 4 && b2 == 4); }
 // M = 48, 12288 -> 4096: 19.0 / 17.8, (4, 1) bits, bfloat16 rows 31.3 / 27.1; M = 128, 4096 -> 4096: 13.1 / 14.1;
 // M = 200: 24.0 / 16.6; M = 300, 4096 -> 1024 12.6 / 13.1; M = 100, 2048 -> 8192, (4, 1) bits 21.0 / 15.5.
 // (A launch in front of 16-row workgroups is not in it.)
-double few_us(int mb, int M, int tiles, int G, int b1, int b2) {
+// The slices of K are those of the least estimate: a slice more saves turns and costs the last arrival its share
+// of the partial tiles, which it reads four at a time, slower the more workgroups do.  Any number of them, so that turns come out whole, down to one
+// a wavefront.  us with 1, 2, 4, 8, 12, 16 slices: M = 8, 2048 -> 1024 7.7, 7.2, 6.3, 6.8, 7.6, 8.5; 12288 -> 1024 29.0, 18.2,
+// 11.9, 9.6, 9.3, 10.0; 4096 -> 4096, 1, 2, 4, 8 12.8, 10.3, 8.4, 8.8; M = 15, 7616 -> 512, (1, 4) bits, rank 8, 2 to 16 19.4, 13.3, 10.5, 10.4, 10.3; M = 20, 3136 -> 1152,
+// (4, 1) bits, 2, 4, 7 11.5, 9.3, 9.1; 32 rows, M = 48, 12288 -> 512, 1 to 8 38.4, 23.8, 15.3, 12.7.
+struct FewPlan {
+    double us;
+    int slices;
+};
+FewPlan plan_few(int mb, int M, int tiles, int G, int b1, int b2) {
     static const double tile_us[5] = {0.0, 0.6, 0.75, 1.2, 1.15};
-    const GemmShape shape = {mb, 8, 1, 1};
     const int64_t units = (int64_t)tiles * ((M + 16 * mb - 1) / (16 * mb));
-    const int ks = slices_of_k(units, G, shape), turns = ((G + ks - 1) / ks + 7) / 8;
-    const int64_t rounds = (units * ks + kNumCU - 1) / kNumCU;
     const double tile = (tile_us[b1] + tile_us[b2]) * (mb == 1 ? 1.0 : 1.09);
     const double launches = b2 && !few_takes(std::max(b1, b2), std::min(b1, b2)) ? 2.0 : 1.0;
-    return (mb == 1 ? 1.5 : 3.5) + rounds * ((mb == 1 ? 4.0 : 5.0) * launches + tile * turns) +
-           (ks > 1 ? (mb == 1 ? 0.5 : 0.75) * ks * launches : 0.0);
+    FewPlan best = {1e30, 1};
+    for (int ks = 1; ks <= 32 && (ks == 1 || (units * ks <= kNumCU && ks < G)); ++ks) {
+        const int turns = ((G + ks - 1) / ks + 7) / 8;
+        const int64_t rounds = (units * ks + kNumCU - 1) / kNumCU;
+        const double share = 0.6 + 0.9 * (double)(units * ks) / kNumCU;
+        const double fold = ks == 1 ? 0.0 : mb == 1 ? 0.6 + 0.65 * ((ks + 3) / 4) * share : 0.4 + 1.0 * ((ks + 3) / 4) * share;
+        const double us = (mb == 1 ? 1.5 : 3.5) + rounds * ((mb == 1 ? 4.0 : 5.0) * launches + tile * turns) + fold * launches;
+        if (us < best.us) best = {us, ks};
+    }
+    return best;
 }
 
 // The same for 64-row (in one round) and 128-row workgroups of gemm_kernel.h: 8 us + 0.26 (0.43) a tile
@@ -90,7 +103,7 @@ GemmShape choose_gemm_shape(int M, int tiles, int G, int b1, int b2, double &us)
     if (v == 32) return {2, 8, 1, 1};
     if (v == 64) return {4, 8, 1, 1};
     if (v == 128) return {4, 4, 2, 1};
-    const double few1 = few_us(1, M, tiles, G, b1, b2), few2 = few_us(2, M, tiles, G, b1, b2);
+    const double few1 = plan_few(1, M, tiles, G, b1, b2).us, few2 = plan_few(2, M, tiles, G, b1, b2).us;
     // (row blocks that gridDim.y holds)
     const bool fits1 = M <= 65535 * 16, fits2 = M <= 65535 * 32;
     if (M <= 16 || (fits1 && few1 <= few2 && few1 < other)) {
@@ -513,7 +526,7 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
     const int mchunks = (p.mblk_total + shape.mb * shape.mw - 1) / (shape.mb * shape.mw);
     const int64_t units = (int64_t)tiles * mchunks;
     p.mblk_pad = mchunks * shape.mb * shape.mw;
-    int ksplit = slices_of_k(units, p.G, shape);
+    int ksplit = few ? plan_few(shape.mb, M, tiles, p.G, p.bits[0], p.nstreams == 2 ? p.bits[1] : 0).slices : slices_of_k(units, p.G, shape);
     {
         const int v = tuning().gemm_ksplit;
         if (v >= 1 && v <= p.G) ksplit = v;

@@ -182,6 +182,21 @@ def test_gemm_few_rows_residual_of_one_operand_of_ranks(tuning_env, M, K, bits, 
     assert rel_l2(y, _dual(w, x).cpu()) <= (2 ** -11 if act == torch.float16 else 2 ** -8)
 
 
+@pytest.mark.parametrize("M,N,K,bits,bits2,rank", [(2, 128, 1024, 4, 0, 0), (8, 256, 1408, 4, 1, 0), (15, 512, 7616, 1, 4, 8),
+                                                  (3, 256, 2752, 3, 3, 8), (20, 1152, 3136, 4, 1, 0), (48, 512, 12288, 4, 0, 16),
+                                                  (5, 128, 65472, 2, 0, 0)])
+def test_gemm_few_rows_in_as_many_slices_as_pay(M, N, K, bits, bits2, rank):
+    """The slices of K that the rule chooses, in numbers that are no power of two and down to a tile a wavefront:
+    against the oracle, and repeats bit for bit (the last arrival adds in slice order)."""
+    w = make_weight(N, K, bits, 128, seed=M + K, bits2=bits2, rank=rank, bias=True, device=DEV)
+    x = make_x(M, K, seed=M)
+    y = _dual(w, x)
+    assert gemm_rows(M, (N, K, bits, bits2, 128)) <= 32
+    assert rel_l2(y.cpu(), _exact(w, x).half()) <= TOL
+    for _ in range(3):
+        assert torch.equal(_dual(w, x), y)
+
+
 DUAL = [
     # M, N, K, bits, gs, bits2, rank, bias
     (8, 512, 1024, 4, 128, 1, 0, False),
