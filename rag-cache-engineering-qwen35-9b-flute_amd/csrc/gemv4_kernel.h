@@ -749,11 +749,7 @@ __global__ void __launch_bounds__(NW * 64, 3) gemv4_kernel(const GemvParams p) {
             if (so >= nout) break;
             const GemvSeg og = kp->seg[so == 1 ? 1 : si0];
             float y = yv[so];
-            if (og.R > 0) {
-                const uint16_t *ra = og.resA + (size_t)n * og.R;
-                for (int r = 0; r < og.R; ++r)
-                    y = fmaf(og.xb[r], p.act_bf16 ? bf2f(ra[r]) : h2f(ra[r]), y);
-            }
+            if (og.R > 0) y = add_residual(y, og.resA + (size_t)n * og.R, og.xb, og.R, p.act_bf16);
             if (og.bias) y += p.act_bf16 ? bf2f(og.bias[n]) : h2f(og.bias[n]);
             yv[so] = y;
         }

@@ -742,3 +742,16 @@ def test_resident_grid_walking_with_two_tables(tuning_env, N, K, gs, rank, bits,
     walked = _run(w, x)
     assert torch.equal(plain, walked)
     assert rel_l2(walked.cpu(), _exact(w, x).half()) <= TOL
+
+
+@pytest.mark.parametrize("rank", [1, 7, 8, 16, 24, 32])
+@pytest.mark.parametrize("K,bits2", [(1024, 0), (1088, 1)])
+def test_residual_ranks_together_and_one_by_one(rank, K, bits2):
+    """Ranks in sixteens and eights, and one by one where the factor is not 16-byte aligned: the same sums in the
+    same order, so equal bits."""
+    w = make_weight(256, K, 4, 128, seed=rank, bits2=bits2, rank=rank, device=DEV)
+    x = make_x(1, K, seed=3).to(DEV)
+    moved = torch.empty(256 * rank + 1, dtype=torch.float16, device=DEV)[1:].view(256, rank).copy_(w["resA_d"])
+    y = _run(w, x)
+    assert torch.equal(_run(dict(w, resA_d=moved), x), y)
+    assert rel_l2(y.cpu(), _exact(w, x.cpu()).half()) <= TOL
