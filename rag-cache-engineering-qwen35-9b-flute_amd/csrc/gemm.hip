@@ -118,7 +118,9 @@ GemmShape choose_gemm_shape(int M, int tiles, int G, int b1, int b2, double &us)
     const double short_by = shape.mw == 1
         ? std::min(2.5, std::max(-1.5, 6.5 - G / slices_of_k((int64_t)tiles * ((M + 63) / 64), G, shape) / 16.0)) : -1.5;
     if (fits2 && few2 < other + short_by) {
-        us = few2;
+        us = few2 + 1.5;                                // (against the many-row kernel, whose estimate has a launch in
+                                                        // front as many of these calls have: M = 205, 9408 -> 2688,
+                                                        // (3, 3) bits, bfloat16 rows, rotated 66.7, 256 rows 57.2)
         return {2, 8, 1, 1};
     }
     return other_shape(M, tiles);
