@@ -244,7 +244,8 @@ int plan_lds(GemmParams &p, const GemmShape &shape) {
     const int lds_tile = gemm_residual_offset(rows) + (residual ? rows * 132 * 4 : 0);
     int lds = lds_tables > lds_reduce ? lds_tables : lds_reduce;
     if (lds_tile > lds) lds = lds_tile;
-    // the hand-overs between the k ways: eight 16 KB areas, then eight of 8 KB behind the totals tile
+    // the hand-overs between the k ways: eight 16 KB areas, then eight of 8 KB behind the totals tile, in part those
+    // of the residual's tile
     if (p.scatter && lds < 17 * 4096 + 8 * 8192) lds = 17 * 4096 + 8 * 8192;
     return lds;
 }

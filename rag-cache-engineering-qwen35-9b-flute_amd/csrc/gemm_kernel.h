@@ -49,7 +49,7 @@ static __device__ long long *g_gemm_stamps = nullptr;
 constexpr int kGemmMaxSegs = 4;
 
 // LDS of gemm_kernel behind its loop: the totals of `rows` rows as fp32 rows of 132, a ticket flag, and (a
-// residual) as many rows again.
+// residual) as many rows again, which overlap the areas of the k ways' hand-overs.
 constexpr int gemm_residual_offset(int rows) { return rows * 132 * 4 + 16; }
 
 // One weight of a launch.
@@ -992,7 +992,8 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
             acc[1][i] += theirs1[(8 + i) * 64 + lane];
         }
         __syncthreads();
-        // second hand-over: behind the region the totals tile takes (17 * 4 KB from the start)
+        // second hand-over: behind the region the totals tile takes (17 * 4 KB from the start), which the
+        // residual's tile takes too (residual_tile waits)
         f4_t *mine2 = red + 4352 + (size_t)wave * 512;
         const f4_t *theirs2 = red + 4352 + (size_t)(wave ^ P2) * 512;
 #pragma unroll
@@ -1089,6 +1090,9 @@ __global__ void __launch_bounds__(64 * KW * MW) gemm_kernel(const GemmParams p) 
                     sum[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, x[b][e], sum[b], 0, 0, 0);
             }
         }
+        // Its tile lies where the k ways have handed blocks to each other (theirs2, pair3): a wavefront may be past
+        // its reads while another is not.  (Of several slices barriers lie between, as they do behind the tree.)
+        if (scattered && p.ztotal == 1) __syncthreads();
 #pragma unroll
         for (int b = 0; b < BLOCKS; ++b) *(f4_t *)(rtile + (b * 16 + rho) * LDT + wave * 16 + kg * 4) = sum[b];
     };

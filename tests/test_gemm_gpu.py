@@ -401,6 +401,24 @@ def test_hand_overs_between_the_k_ways_equal_the_tree(tuning_env, N, K, M, rot):
     assert rel_l2(handed[M - 1:M], y1) <= 4e-3
 
 
+@pytest.mark.parametrize("rank", [5, 16, 24])
+@pytest.mark.parametrize("rows,M", [("64", 64), ("64", 130), ("128", 128), ("128", 200)])
+@pytest.mark.parametrize("N,K", [(256, 1024), (1024, 4096)])
+def test_hand_overs_beside_a_residual_equal_the_tree(tuning_env, N, K, rows, M, rank):
+    """One stream in one slice of K: the residual's tile takes memory that the k ways have just handed blocks
+    over in, with four k ways (128 rows) and eight (64).  The bits of the reduction tree, which does not use that
+    memory, and the oracle's values, row by row (a block overwritten early would be lost in a launch-wide norm)."""
+    tuning_env("FLUTE_GEMM_ROWS", rows)
+    tuning_env("FLUTE_GEMM_KSPLIT", "1")
+    w = make_weight(N, K, 4, 128, seed=M + rank, rank=rank, bias=True, device=DEV)
+    x = make_x(M, K, seed=rank)
+    handed = _dual(w, x)
+    tuning_env("FLUTE_GEMM_NO_HANDOVER", "1")
+    assert torch.equal(handed, _dual(w, x))
+    want = _exact(w, x).half()
+    assert max(rel_l2(y, v) for y, v in zip(handed.cpu(), want)) <= TOL
+
+
 @pytest.mark.parametrize("kind", ["outliers", "tiny", "huge", "mixed"])
 @pytest.mark.parametrize("M,rows", [(8, None), (40, None), (130, "64"), (300, "128")])
 def test_gemm_bf16_activations_beyond_the_float16_range(tuning_env, kind, M, rows):
