@@ -62,8 +62,10 @@ typedef enum flute_dtype {
  * result as fp32 arithmetic on x.float().  A row that holds an infinity or a NaN is not
  * scaled (there is no finite maximum to scale by): its finite values beyond float16's range
  * saturate, so the outputs of such a row are unspecified (they may be NaN where fp32
- * arithmetic gives an infinity).  float16 activations with a bfloat16 LUT are
- * refused (FLUTE_ERR_UNSUPPORTED): that conversion is not exact.
+ * arithmetic gives an infinity).  float16 activations with a bfloat16 LUT: that conversion
+ * is not exact.  The one-row entries and flute_describe_linear refuse the pair
+ * (FLUTE_ERR_UNSUPPORTED); flute_gemm and its relatives round the activations to bfloat16
+ * ahead of the products (the residual takes them as they are).
  * signs   (K,) fp32 +-1: when non-NULL the input is rotated first, x <- x @ T
  *         (fht.py:19-35); awq (K,) fp32 then selects ((x*s) @ T) / s
  */

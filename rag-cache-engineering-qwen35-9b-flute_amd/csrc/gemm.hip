@@ -558,7 +558,9 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
     // bfloat16 activations presented as float16 operands: one power-of-two scale per row
     const bool scale_rows = act_dtype == FLUTE_BF16 && w->lut_dtype == FLUTE_F16;
     const bool rows16 = w->signs || (((uintptr_t)A & 15) == 0 && lda % 8 == 0);
-    const bool reads = few && rows16 && (w->signs ? w->K : lda) <= few_lda() && !up && !tuning().gemm_no_direct;
+    // (float16 rows in front of a bfloat16 LUT are converted by the image: the kernel converts the other pair only)
+    const bool narrows = act_dtype == FLUTE_F16 && w->lut_dtype == FLUTE_BF16;
+    const bool reads = few && rows16 && !narrows && (w->signs ? w->K : lda) <= few_lda() && !up && !tuning().gemm_no_direct;
     p.find = reads && shape.mb == 1 && scale_rows && !w->signs && few_finds(M, w->K, units * ksplit);
     // Residuals of up to 16 ranks whose rows the kernel reads, and needs nothing else of a launch in front for: it
     // forms their coefficients beside its products (gemm_few_kernel.h).

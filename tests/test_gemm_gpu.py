@@ -281,6 +281,37 @@ def test_gemm_dtype_mixes(lut_dtype, act_dtype):
     assert rel_l2(y, ref) <= tol
 
 
+@pytest.mark.parametrize("rows", [None, "16", "32", "64", "256"])
+@pytest.mark.parametrize("M,K,bits2,rank", [(1, 64, 0, 0), (16, 1088, 3, 0), (17, 576, 0, 16), (40, 1024, 1, 5), (33, 2048, 4, 24)])
+def test_gemm_float16_rows_in_front_of_a_bfloat16_lut(tuning_env, rows, M, K, bits2, rank):
+    """The C entry points round such rows to the LUT's type on their way to the matrix cores, in every workgroup
+    shape; the residual takes the rows as they are.  (The bindings and the module layer keep the pair away.)"""
+    import ctypes
+    from flute_extended import _lib
+    if rows:
+        tuning_env("FLUTE_GEMM_ROWS", rows)
+    w = make_weight(256, K, 4, 128, seed=M, bits2=bits2, rank=rank, lut_dtype=torch.bfloat16, device=DEV)
+    x = make_x(M, K, seed=K)
+    d = _lib.FluteLinear()
+    d.q1, d.lut1, d.q1_bytes, d.b1 = w["blob_d"].data_ptr(), w["lut_d"].data_ptr(), w["blob_d"].numel(), 4
+    if bits2:
+        d.q2, d.lut2, d.q2_bytes, d.b2 = w["blob2_d"].data_ptr(), w["lut2_d"].data_ptr(), w["blob2_d"].numel(), bits2
+    if rank:
+        d.resB, d.resA, d.R = w["resB_d"].data_ptr(), w["resA_d"].data_ptr(), rank
+    d.N, d.K, d.group_size, d.lut_rows, d.lut_dtype = 256, K, 128, 2, _lib.BF16
+    xd = x.to(DEV)
+    ds, outs = (_lib.FluteLinear * 2)(d, d), [torch.zeros(M, 256, dtype=torch.float16, device=DEV) for _ in range(3)]
+    stream = torch.cuda.current_stream().cuda_stream
+    assert _lib.lib.flute_gemm(ctypes.byref(d), xd.data_ptr(), outs[0].data_ptr(), M, K, 256, _lib.F16, stream) == 0
+    assert _lib.lib.flute_gemm_multi(ds, 2, xd.data_ptr(), (ctypes.c_void_p * 2)(*[o.data_ptr() for o in outs[1:]]),
+                                     (ctypes.c_int64 * 2)(256, 256), M, K, _lib.F16, stream) == 0
+    want = _exact(dict(w, resA=None, resB=None), x.bfloat16()).double()
+    if rank:
+        want = want + (x.double() @ w["resB"].double().t()) @ w["resA"].double().t()
+    for y in outs:
+        assert rel_l2(y.cpu(), want.half()) <= TOL
+
+
 @pytest.mark.parametrize("bits,gs", [(4, 128), (3, 64), (2, 16), (1, 128), (4, 32)])
 def test_gemm_one_hot_rows_return_dequantised_columns(bits, gs):
     N, K = 256, 128
