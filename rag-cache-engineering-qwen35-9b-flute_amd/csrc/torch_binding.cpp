@@ -530,21 +530,20 @@ pybind11::tuple operand_addresses(const pybind11::sequence &members) {
     py::tuple out(7 * count);
     for (size_t i = 0; i < count; ++i) {
         const py::object m = members[i];
-        PyObject *places[3] = {nullptr, nullptr, nullptr};
+        py::object places[3];
         PyObject **const own = _PyObject_GetDictPtr(m.ptr());
         if (own && *own) {
             PyObject *const b = PyDict_GetItemWithError(*own, buffers), *const p = PyDict_GetItemWithError(*own, parameters);
             if (b && p && PyDict_Check(b) && PyDict_Check(p)) {          // a module
-                places[0] = *own;
-                places[1] = b;
-                places[2] = p;
+                PyObject *const three[3] = {*own, b, p};
+                for (int n = 0; n < 3; ++n) places[n] = py::reinterpret_borrow<py::object>(three[n]);
             }
         }
         for (int n = 0; n < 7; ++n) {
             py::object t;
-            for (PyObject *place : places) {
+            for (const py::object &place : places) {
                 if (!place) continue;
-                if (PyObject *const found = PyDict_GetItemWithError(place, names[n])) {
+                if (PyObject *const found = PyDict_GetItemWithError(place.ptr(), names[n])) {
                     t = py::reinterpret_borrow<py::object>(found);
                     break;
                 }
@@ -568,7 +567,9 @@ pybind11::tuple operand_addresses(const pybind11::sequence &members) {
 // on the device that the launch reads, nobody watching, no switch set.  Each method answers None for any other
 // call, and the Python forward then runs from its beginning.  Everything is read out of the modules on each
 // call (the dictionaries that attribute lookup ends in); nothing is kept from one call for the next but
-// which entry serves a shape, by its numbers.  One token, 4096 -> 1024: 10.1 us of host time a call in
+// which entry serves a shape, by its numbers.  What is used behind a call into Python (hooks, attributes of
+// modules, the choice of an entry: other threads run there, and may replace what a module holds) is held by a
+// reference.  One token, 4096 -> 1024: 10.1 us of host time a call in
 // Python, 7 here; q/k/v of several rows 22 and 9, of rotated ones 39 and 16; a gated block of 22 rows 43 and
 // 19; a thousand embedding rows 16 and 13, half of them the wait for the verdict on the ids.
 namespace names {
@@ -623,8 +624,8 @@ struct Places {
 // The operands of one layer as its module holds them.
 struct Layer {
     Tensor indices, lut, indices2, lut2, resB, resA, bias, signs, awq;
+    Tensor rotation;                                    // the module's own signs
     int64_t b1 = 0, b2 = 0, gs = 0, N = 0, K = 0;
-    PyObject *rotation = nullptr;                       // the module's own signs (borrowed)
     bool scaled = false;
     int64_t rank() const { return resB.defined() ? resB.size(0) : 0; }
     Described described(const char *who, const Tensor &A) const {
@@ -676,7 +677,7 @@ class Forwards {
 
     pybind11::object qkv(pybind11::handle m, pybind11::handle x_) {
         Tensor x;
-        PyObject *members[3];
+        Members members;
         if (!plain_input(x_.ptr(), x) || !no_switch() ||
             !children(m.ptr(), {names::q_proj, names::k_proj, names::v_proj}, members))
             return pybind11::none();
@@ -701,21 +702,21 @@ class Forwards {
 
     pybind11::object mlp(pybind11::handle m, pybind11::handle x_) {
         Tensor x;
-        PyObject *members[3];
+        Members members;
         if (!plain_input(x_.ptr(), x) || !no_switch() ||
             !children(m.ptr(), {names::gate_proj, names::up_proj, names::down_proj}, members))
             return pybind11::none();
         const bool one = x.numel() == x.size(-1);
         if (one) {
-            if (!own_call(members + 2, 1)) return pybind11::none();
+            if (!own_call(members, 2, 3)) return pybind11::none();
             Layer down;
-            const Tensor h = grouped(m.ptr(), members, 2, x, true, [&](const Tensor &h) { return read(members[2], h, down); });
+            const Tensor h = grouped(m.ptr(), members, 2, x, true, [&](const Tensor &h) { return read(members[2].ptr(), h, down); });
             if (!h.defined()) return pybind11::none();
             count(kGemvMlp);
             Tensor y;
             if (!one_row(h, down, y)) {                 // (the product is there: the module's own call)
                 const pybind11::object out = pybind11::reinterpret_steal<pybind11::object>(
-                    PyObject_CallOneArg(members[2], wrap(h).ptr()));
+                    PyObject_CallOneArg(members[2].ptr(), wrap(h).ptr()));
                 if (!out) throw pybind11::error_already_set();
                 y = THPVariable_Unpack(out.ptr());
             }
@@ -725,8 +726,8 @@ class Forwards {
         const Tensor x2 = rows_of(x);
         std::vector<Layer> layers(2);
         Layer down;
-        if (!own_call(members + 2, 1) || !together(members, 2, x2, layers) || layers[0].N != layers[1].N ||
-            !read(members[2], x2, down, layers[0].N) || !several_rows(x2, down))
+        if (!own_call(members, 2, 3) || !together(members, 2, x2, layers) || layers[0].N != layers[1].N ||
+            !read(members[2].ptr(), x2, down, layers[0].N) || !several_rows(x2, down))
             return pybind11::none();
         const char *who = "qgemm_linear_mlp";
         const Shape2 s = {x2.size(0), x2.size(1)};
@@ -774,6 +775,8 @@ class Forwards {
   private:
     enum Route { kGemvSplitk, kGemvSplitkFht, kGemv, kGemvFht, kDualStream, kPerGroupLut, kGemmMulti, kGemvMulti, kGemvMlp,
                  kEmbeddingGather, kNone };
+
+    typedef std::array<pybind11::object, 3> Members;    // projections of a block
 
     static pybind11::object wrap(const Tensor &t) { return pybind11::reinterpret_steal<pybind11::object>(THPVariable_Wrap(t)); }
     static Tensor rows_of(const Tensor &x) { return x.dim() == 2 ? x : x.reshape({-1, x.size(-1)}); }
@@ -891,13 +894,11 @@ class Forwards {
                                  at::isTensorSubclassLike(*t)))
                 return false;
         if (l.resB.defined() && l.resB.dim() != 2) return false;
-        l.rotation = item(at.own, names::rot_signs);
-        if (!l.rotation) return false;
-        if (l.rotation == Py_None) {
-            l.rotation = nullptr;
-            return true;
-        }
-        if (!vector_on(at, names::signs, l.rotation, x.device(), l.signs)) return false;
+        PyObject *const rotation = item(at.own, names::rot_signs);
+        if (!rotation) return false;
+        if (rotation == Py_None) return true;
+        if (!vector_on(at, names::signs, rotation, x.device(), l.signs)) return false;
+        l.rotation = THPVariable_Unpack(rotation);
         PyObject *const scale = item(at.own, names::awq_scale), *const order = item(at.own, names::fold_order);
         if (!scale || !order) return false;
         if (scale == Py_None) return true;
@@ -916,7 +917,7 @@ class Forwards {
         const int64_t M = x.size(0), rank = l.rank();
         if (rank > 256 || !(rank <= 16 || M * rank * (l.N + l.K) <= (int64_t)1 << 27)) return false;
         if (l.bias.defined() && (l.bias.dim() != 1 || l.bias.numel() != l.N)) return false;
-        if (l.rotation && !(l.K % 32 == 0 && l.K >= 32 && l.K <= 65504 && l.K < 32768)) return false;
+        if (l.rotation.defined() && !(l.K % 32 == 0 && l.K >= 32 && l.K <= 65504 && l.K < 32768)) return false;
         if (l.b2 && l.lut2.scalar_type() != l.lut.scalar_type()) return false;
         return l.gs >= 16 && l.gs <= 2048 && (l.gs & (l.gs - 1)) == 0 && l.N % 128 == 0 && l.K % 64 == 0;
     }
@@ -951,10 +952,10 @@ class Forwards {
 
     // Which entry of the package takes one row of a shape, by its numbers (palettized_modules._gemv_choice).
     Route gemv_route(const Layer &l) {
-        const std::array<int64_t, 7> key = {l.b1, l.b2, l.gs, l.N, l.K, l.rank(), l.rotation != nullptr};
+        const std::array<int64_t, 7> key = {l.b1, l.b2, l.gs, l.N, l.K, l.rank(), l.rotation.defined()};
         const auto known = gemv_routes_.find(key);
         if (known != gemv_routes_.end()) return known->second;
-        const pybind11::object name = gemv_choice_(l.b1, l.b2, l.gs, l.N, l.K, l.rank(), l.rotation != nullptr);
+        const pybind11::object name = gemv_choice_(l.b1, l.b2, l.gs, l.N, l.K, l.rank(), l.rotation.defined());
         Route route = kNone;
         for (int r = kGemvSplitk; r <= kGemvFht && !name.is_none(); ++r)
             if (name.equal(routes_[r])) route = (Route)r;
@@ -969,16 +970,17 @@ class Forwards {
     }
     void count_rows(int64_t M, const Layer &l) const { count(M <= 16 && l.rank() <= 16 ? kDualStream : kPerGroupLut); }
 
-    // Children of a block (borrowed) out of its dictionary of modules.
-    static bool children(PyObject *m, std::initializer_list<PyObject *> which, PyObject **out) {
+    // Children of a block out of its dictionary of modules.
+    static bool children(PyObject *m, std::initializer_list<PyObject *> which, Members &out) {
         PyObject **const d = _PyObject_GetDictPtr(m);
         if (!d || !*d) return false;
         PyObject *const modules = item(*d, names::_modules);
         if (!modules || !PyDict_CheckExact(modules)) return false;
+        size_t i = 0;
         for (PyObject *name : which) {
-            *out = item(modules, name);
-            if (!*out || *out == Py_None || item(*d, name)) return false;
-            ++out;
+            PyObject *const child = item(modules, name);
+            if (!child || child == Py_None || item(*d, name)) return false;
+            out[i++] = pybind11::reinterpret_borrow<pybind11::object>(child);
         }
         return true;
     }
@@ -989,14 +991,14 @@ class Forwards {
     }
 
     // palettized_modules._own_call and no global hooks: calling these modules is calling the class's forward.
-    bool own_call(PyObject *const *members, int n) const {
+    bool own_call(const Members &members, int first, int last) const {
         const pybind11::object f = pybind11::reinterpret_steal<pybind11::object>(PyObject_GetAttr(linear_type_.ptr(), names::forward));
         if (!f) throw pybind11::error_already_set();
         if (f.ptr() != linear_forward_.ptr()) return false;
-        for (int i = 0; i < n; ++i) {
-            if ((PyObject *)Py_TYPE(members[i]) != linear_type_.ptr()) return false;
-            PyObject *const own = *_PyObject_GetDictPtr(members[i]);
-            if (item(own, names::forward)) return false;
+        for (int i = first; i < last; ++i) {
+            if ((PyObject *)Py_TYPE(members[i].ptr()) != linear_type_.ptr()) return false;
+            PyObject *const own = *_PyObject_GetDictPtr(members[i].ptr());
+            if (!own || item(own, names::forward)) return false;
             for (PyObject *hooks : {names::_forward_hooks, names::_forward_pre_hooks, names::_backward_hooks, names::_backward_pre_hooks}) {
                 PyObject *const h = item(own, hooks);
                 if (!h || PyObject_IsTrue(h) != 0) return false;
@@ -1008,15 +1010,14 @@ class Forwards {
     }
 
     // palettized_modules._layers_on.
-    bool together(PyObject *const *members, int n, const Tensor &x, std::vector<Layer> &layers) const {
-        if (x.size(0) < 2 || !x.is_contiguous() || !own_call(members, n)) return false;
+    bool together(const Members &members, int n, const Tensor &x, std::vector<Layer> &layers) const {
+        if (x.size(0) < 2 || !x.is_contiguous() || !own_call(members, 0, n)) return false;
         for (int i = 0; i < n; ++i) {
             Layer &l = layers[i];
-            if (!read(members[i], x, l) || !several_rows(x, l) || l.lut.scalar_type() != layers[0].lut.scalar_type()) return false;
-            if (i && l.rotation && layers[0].rotation && !l.scaled && !layers[0].scaled) {
+            if (!read(members[i].ptr(), x, l) || !several_rows(x, l) || l.lut.scalar_type() != layers[0].lut.scalar_type()) return false;
+            if (i && l.rotation.defined() && layers[0].rotation.defined() && !l.scaled && !layers[0].scaled) {
                 // one rotation, one address: its members share the rotated rows
-                if (l.rotation == layers[0].rotation || same_bytes(THPVariable_Unpack(l.rotation), THPVariable_Unpack(layers[0].rotation)))
-                    l.signs = layers[0].signs;
+                if (l.rotation.is_same(layers[0].rotation) || same_bytes(l.rotation, layers[0].rotation)) l.signs = layers[0].signs;
             }
         }
         return true;
@@ -1024,47 +1025,52 @@ class Forwards {
 
     // The decode launch of a block whose table still holds (state of FusedPalettizedMLP and SplitQKV): its output,
     // or an undefined tensor.  `also`: what else has to hold before the launch.
-    Tensor grouped(PyObject *block, PyObject *const *members, int n, const Tensor &x, bool mlp,
+    Tensor grouped(PyObject *block, const Members &members, int n, const Tensor &x, bool mlp,
                    const std::function<bool(const Tensor &)> &also = nullptr) const {
+        namespace py = pybind11;
         if (x.dim() > 3 || !x.is_contiguous()) return Tensor();
-        PyObject *const state = item(*_PyObject_GetDictPtr(block), names::_merge_state);
-        if (!state || !PyDict_CheckExact(state) || item(state, names::ok) != Py_True) return Tensor();
-        PyObject *const device = item(state, names::device), *const dtype = item(state, names::dtype);
+        const auto held_item = [](const py::object &dict, PyObject *name) {
+            return py::reinterpret_borrow<py::object>(item(dict.ptr(), name));     // (empty: it has none)
+        };
+        const py::object state = py::reinterpret_borrow<py::object>(item(*_PyObject_GetDictPtr(block), names::_merge_state));
+        if (!state || !PyDict_CheckExact(state.ptr()) || item(state.ptr(), names::ok) != Py_True) return Tensor();
+        PyObject *const device = item(state.ptr(), names::device), *const dtype = item(state.ptr(), names::dtype);
         if (!device || !THPDevice_Check(device) || ((THPDevice *)device)->device != x.device() || !dtype || !THPDtype_Check(dtype) ||
             ((THPDtype *)dtype)->scalar_type != x.scalar_type())
             return Tensor();
-        PyObject *const ptrs = item(state, names::ptrs), *const sources = item(state, names::sources);
-        if (!ptrs || !PyTuple_CheckExact(ptrs) || !sources || !PyList_CheckExact(sources)) return Tensor();
-        pybind11::list held;
-        for (int i = 0; i < n; ++i) held.append(pybind11::reinterpret_borrow<pybind11::object>(members[i]));
-        const pybind11::tuple now = operand_addresses(held);
-        const int same = PyObject_RichCompareBool(now.ptr(), ptrs, Py_EQ);
-        if (same < 0) throw pybind11::error_already_set();
-        if (!same) return Tensor();
-        for (Py_ssize_t i = 0; i < PyList_GET_SIZE(sources); ++i) {
-            PyObject *const s = PyList_GET_ITEM(sources, i);            // (member, name, tensor, version)
-            if (!PyTuple_CheckExact(s) || PyTuple_GET_SIZE(s) != 4) return Tensor();
-            const pybind11::object t = pybind11::reinterpret_steal<pybind11::object>(
-                PyObject_GetAttr(PyTuple_GET_ITEM(s, 0), PyTuple_GET_ITEM(s, 1)));
-            if (!t) throw pybind11::error_already_set();
-            PyObject *const version = PyTuple_GET_ITEM(s, 3);
-            if (t.ptr() != PyTuple_GET_ITEM(s, 2) || !THPVariable_Check(t.ptr()) ||
+        const py::object ptrs = held_item(state, names::ptrs), sources = held_item(state, names::sources),
+                         table = held_item(state, names::seg_table), out_ = held_item(state, names::out);
+        if (!ptrs || !PyTuple_CheckExact(ptrs.ptr()) || !sources || !PyList_CheckExact(sources.ptr()) || !table || !out_ ||
+            !THPVariable_Check(table.ptr()) || !THPVariable_Check(out_.ptr()))
+            return Tensor();
+        for (Py_ssize_t i = 0; i < PyList_GET_SIZE(sources.ptr()); ++i) {
+            const py::object s = py::reinterpret_borrow<py::object>(PyList_GET_ITEM(sources.ptr(), i));  // (member, name, tensor, version)
+            if (!PyTuple_CheckExact(s.ptr()) || PyTuple_GET_SIZE(s.ptr()) != 4) return Tensor();
+            const py::object t = py::reinterpret_steal<py::object>(
+                PyObject_GetAttr(PyTuple_GET_ITEM(s.ptr(), 0), PyTuple_GET_ITEM(s.ptr(), 1)));
+            if (!t) throw py::error_already_set();
+            PyObject *const version = PyTuple_GET_ITEM(s.ptr(), 3);
+            if (t.ptr() != PyTuple_GET_ITEM(s.ptr(), 2) || !THPVariable_Check(t.ptr()) ||
                 (version != Py_None && PyLong_AsLongLong(version) != (long long)THPVariable_Unpack(t.ptr())._version()))
                 return Tensor();
         }
-        PyObject *const table = item(state, names::seg_table), *const out_ = item(state, names::out);
-        const Places first(members[0]);
+        // (the addresses last: from here to the launch nothing calls into Python, so nobody frees what they name)
+        py::list held;
+        for (int i = 0; i < n; ++i) held.append(members[i]);
+        const py::tuple now = operand_addresses(held);
+        const int same = PyObject_RichCompareBool(now.ptr(), ptrs.ptr(), Py_EQ);
+        if (same < 0) throw py::error_already_set();
+        if (!same) return Tensor();
+        const Places first(members[0].ptr());
         Tensor lut;
         int64_t K;
-        if (!first.own || !first.integer(names::K, K) || K != x.size(-1)) return Tensor();
-        if (!table || !out_ || !THPVariable_Check(table) || !THPVariable_Check(out_) || !tensor(first, names::lut, lut) ||
-            !lut.defined())
+        if (!first.own || !first.integer(names::K, K) || K != x.size(-1) || !tensor(first, names::lut, lut) || !lut.defined())
             return Tensor();
-        const Tensor out = THPVariable_Unpack(out_), x2 = rows_of(x);
+        const Tensor out = THPVariable_Unpack(out_.ptr()), x2 = rows_of(x);
         if (also && !also(out)) return Tensor();
         const int code = lut.scalar_type() == at::kBFloat16 ? FLUTE_BF16 : FLUTE_F16;
-        if (mlp) return gemv_mlp_table(x2, THPVariable_Unpack(table), out, code, 0);
-        gemv_multi_table(x2, THPVariable_Unpack(table), code, 0);
+        if (mlp) return gemv_mlp_table(x2, THPVariable_Unpack(table.ptr()), out, code, 0);
+        gemv_multi_table(x2, THPVariable_Unpack(table.ptr()), code, 0);
         return out;
     }
 

@@ -588,3 +588,76 @@ def test_compiled_forwards_leave_other_calls_to_python(monkeypatch, M):
         assert fw.embedding(table, ids + 256) is None and fw.embedding(table, ids.cpu()) is None
     if M > 1:
         assert a.bias.requires_grad and refused()       # with gradients on
+
+
+def _block_of(kind, M, K=256):
+    """A block of residual layers.  One row: q/k/v or gate and up hold a factor of another type, so that the decode
+    table has it by a copy, whose source is looked at on each call."""
+    members = [_modules(make_weight(256, K, seed=i, rank=8, bias=True))[1] for i in range(3)]
+    for m in members[:0 if M > 1 else 3 if kind == "qkv" else 2]:
+        m.resA = m.resA.float()
+    return pm.SplitQKV(*members) if kind == "qkv" else pm.FusedPalettizedMLP(*members, torch.nn.SiLU())
+
+
+@pytest.mark.skipif(fx._C.native is None, reason="the compiled binding is not built or switched off")
+@pytest.mark.parametrize("kind,M,when", [("qkv", 1, "sources"), ("mlp", 1, "sources"), ("mlp", 1, "hooks"), ("qkv", 5, "hooks"),
+                                         ("mlp", 5, "hooks")])
+def test_compiled_forwards_hold_what_a_call_into_python_replaces(monkeypatch, kind, M, when):
+    """Projections and the decode table that go away while the compiled forward asks Python something (another
+    thread may run there): the call ends on what it began with."""
+    import gc
+    pm._flute()
+    compiled, it, x, calls = getattr(pm._forwards, kind), _block_of(kind, M), make_x(M, 256, seed=3).to(DEV), []
+
+    def vanish():
+        if calls:
+            return
+        calls.append(1)
+        for n in ("q_proj", "k_proj", "v_proj") if kind == "qkv" else ("gate_proj", "up_proj", "down_proj"):
+            setattr(it, n, _modules(make_weight(256, 256, seed=9))[1])
+        if when == "sources":                           # (at the hooks it has not been read yet)
+            it._merge_state = None
+        gc.collect()
+
+    class Empty(dict):
+        def __bool__(self):
+            vanish()
+            return False
+    inner = torch.nn.Module.__getattr__
+
+    def looked_up(self, name):
+        found = inner(self, name)
+        vanish()
+        return found
+    with torch.no_grad():
+        want = it(x).clone()
+        with monkeypatch.context() as patch:
+            if when == "hooks":
+                patch.setattr(torch.nn.modules.module, "_global_forward_hooks", Empty())
+            else:
+                patch.setattr(torch.nn.Module, "__getattr__", looked_up)
+            y = compiled(it, x)
+        assert calls and y is not None and torch.equal(y, want)
+
+
+@pytest.mark.skipif(fx._C.native is None, reason="the compiled binding is not built or switched off")
+@pytest.mark.parametrize("kind", ["qkv", "mlp"])
+def test_compiled_decode_tables_are_looked_at_behind_every_call_into_python(monkeypatch, kind):
+    """An operand that is replaced while the sources of a decode table's copies are looked up: its address in the
+    table is no longer its own, and the call is left to Python."""
+    pm._flute()
+    it, x, calls = _block_of(kind, 1), make_x(1, 256, seed=3).to(DEV), []
+    inner, first = torch.nn.Module.__getattr__, it.q_proj if kind == "qkv" else it.gate_proj
+
+    def looked_up(self, name):
+        found = inner(self, name)
+        if not calls:
+            calls.append(1)
+            first._buffers["lut"] = first._buffers["lut"].clone()
+        return found
+    with torch.no_grad():
+        want = it(x).clone()
+        with monkeypatch.context() as patch:
+            patch.setattr(torch.nn.Module, "__getattr__", looked_up)
+            assert getattr(pm._forwards, kind)(it, x) is None and calls
+        assert torch.equal(it(x), want)
