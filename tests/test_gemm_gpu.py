@@ -219,7 +219,8 @@ def test_gemm_scales_found_by_the_workgroups_match_the_pre_pass(tuning_env, M, K
     x = make_x(M, K, seed=M, dtype=torch.bfloat16)
     x[0] *= 1e30
     x[M // 2] *= 1e-30
-    x[M - 1] = 0
+    if M > 2:
+        x[M - 1] = 0
     if M > 4:
         x[3, K - 1] = float("inf")
 
@@ -229,8 +230,11 @@ def test_gemm_scales_found_by_the_workgroups_match_the_pre_pass(tuning_env, M, K
     direct = run()
     tuning_env("FLUTE_GEMM_NO_DIRECT", "1")
     assert torch.equal(direct.nan_to_num(7.0), run().nan_to_num(7.0))
-    ok = torch.isfinite(x).all(dim=1)
-    assert rel_l2(direct.cpu()[ok][1:], _exact(w, x)[ok][1:].bfloat16()) <= TOL
+    # row by row: a scale that both ways get wrong would be lost beside rows of 1e30.  A row's norm bears sixteen
+    # of its 256 values rounding the other way (2^-8 of a value each, 2^-12 of the norm); a wrong scale is a factor of 2
+    want = _exact(w, x).bfloat16()
+    for m in torch.isfinite(x).all(dim=1).nonzero().flatten().tolist():
+        assert rel_l2(direct[m].cpu(), want[m]) <= TOL, m
 
 
 @pytest.mark.parametrize("M,N,K,bits,gs,bits2,rank,bias", DUAL)
@@ -588,9 +592,10 @@ def test_gemm_many_rows_by_the_rule_agree_with_the_other_kernels(tuning_env, M, 
 @pytest.mark.parametrize("form", ["f16", "bf16 over f16", "bf16 over f16, rotated"])
 @pytest.mark.parametrize("rows", [None, "256", "512"])
 def test_gemm_residual_slices_and_row_scales(tuning_env, rows, M, K, rank, form):
-    """Residual coefficients in one, four and sixteen slices of K; ranks the epilogue reads eight at
-    a time and others; row scales found by the rotation and by their own launch, rows over a wide
-    range of magnitudes; the small-M kernel and both workgroups of the many-row kernel."""
+    """Residual coefficients in one, four and sixteen slices of K, and those that the few-row kernel forms; ranks
+    that are loaded four at a time (multiples of four) and one by one; row scales found by the rotation, by the
+    workgroups and by the launch in front, rows over a wide range of magnitudes; the small-M kernels and both
+    workgroups of the many-row kernel."""
     if rows:
         tuning_env("FLUTE_GEMM_ROWS", rows)
     N, act = 256, torch.float16 if form == "f16" else torch.bfloat16
@@ -612,8 +617,8 @@ def test_gemm_residual_slices_and_row_scales(tuning_env, rows, M, K, rank, form)
 def test_gemm_residual_coefficients_of_very_different_magnitude(tuning_env, rows, rank, act):
     """Ranks whose coefficients fall by 2^20 and whose resA grows by as much, so that each adds the same
     to the output: the coefficients are fp32 and stay so in every kernel.  With a zero LUT the output
-    is the residual alone, fp32 sums rounded once.  The 128-row workgroups add the same fp32 products
-    one by one, so the many-row kernel may differ from them by a rounding."""
+    is the residual alone, fp32 sums rounded once.  The 128-row workgroups sum the fp32 products sixteen ranks a
+    step in a tile of their own, the many-row kernel in its accumulators, so the two may differ by a rounding."""
     M, N, K = 130, 256, 512
     tuning_env("FLUTE_GEMM_ROWS", rows)
     w = make_weight(N, K, 4, 128, seed=7, act_dtype=act, device=DEV)
