@@ -281,12 +281,13 @@ __global__ void __launch_bounds__(kEmbThreads) embedding_row_kernel(const EmbPar
     }
 }
 
-// Longer rows.  One workgroup per requested row, sixteen consecutive columns a thread.  What bounds it: the chain
-// id -> codes -> values -> butterfly -> store, so everything a phase needs is requested together
-// (the LUT row goes to LDS beside the codes and signs, a value costs one LDS read) and the first ten
-// stages of the butterfly stay in registers.  (One pair at a time, byte loads of the codes and trips
-// to memory for the LUT, all stages in LDS: 15.2 us for 1000 rotated rows of 4096 columns, 4 bits,
-// against 13.6; the check of the ids as five launches and a copy before it: 71 us a call against 27.)
+// Rows of more than 4096 columns.  One workgroup per requested row, sixteen consecutive columns a thread, 4096 a
+// step, segments of a rotated row one after the other.  What bounds it: the chain id -> codes -> values ->
+// butterfly -> store, so everything a phase needs is requested together (the LUT row goes to LDS beside the codes
+// and signs, a value costs one LDS read) and the first ten stages of the butterfly stay in registers.  In a graph,
+// 4 bits, rotated and plain, us: 1000 rows of 4160 columns 17.3 / 12.9, of 8192 26.9 / 18.3, of 12288 35.3 / 27.2;
+// 64 of 8192 11.2 / 7.2; 4000 of 8192 78.5 / 54.3, which cannot do without 131 MB of lines read (a row's codes are an
+// eighth of those they lie in) and 66 MB written, 39 us at a copy's rate.
 // check != NULL: the first workgroup of the grid looks all ids over instead (check_ids).
 __global__ void __launch_bounds__(kEmbThreads) embedding_kernel(const EmbParams p, int64_t count, int *check) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -494,23 +495,14 @@ flute_status embedding(const flute_linear *w, const int64_t *ids, int64_t count,
     p.bf16 = w->lut_dtype == FLUTE_BF16;
     p.block = w->rot_block;
     p.vec_out = ((uintptr_t)out & 15) == 0;             // (rows are K * 2 bytes, K a multiple of 64)
-    size_t lds = 0;
-    if (w->signs) {
-        if (w->rot_block > 0) {
-            FLUTE_REQUIRE(is_pow2(w->rot_block) && w->rot_block >= 32 && w->rot_block <= 16384 &&
-                              w->K % w->rot_block == 0,
-                          FLUTE_ERR_INVALID,
-                          "flute_embedding: rotation block must be a power of two in [32, 16384] "
-                          "dividing K");
-            lds = (size_t)(w->K <= 16384 ? w->K : (16384 / w->rot_block) * w->rot_block) * 4;
-        } else {
-            lds = (size_t)make_segments(w->K, 0).len[0] * 4;
-        }
-    }
+    FLUTE_REQUIRE(!w->signs || w->rot_block <= 0 ||
+                      (is_pow2(w->rot_block) && w->rot_block >= 32 && w->rot_block <= 16384 && w->K % w->rot_block == 0),
+                  FLUTE_ERR_INVALID,
+                  "flute_embedding: rotation block must be a power of two in [32, 16384] dividing K");
     const dim3 grid((unsigned)(count + (check ? 1 : 0))), threads(kEmbThreads);
     if (w->K <= kEmbRow) {
         const int form = 2 * p.bf16 + (w->signs != nullptr);
-        lds = (size_t)((w->K + 1023) / 1024) * emb_wave_bytes(w->signs != nullptr);
+        const size_t lds = (size_t)((w->K + 1023) / 1024) * emb_wave_bytes(w->signs != nullptr);
         if (form == 3) hipLaunchKernelGGL((embedding_row_kernel<true, true>), grid, threads, lds, stream, p, count, check);
         else if (form == 2) hipLaunchKernelGGL((embedding_row_kernel<true, false>), grid, threads, lds, stream, p, count, check);
         else if (form == 1) hipLaunchKernelGGL((embedding_row_kernel<false, true>), grid, threads, lds, stream, p, count, check);
@@ -518,7 +510,12 @@ flute_status embedding(const flute_linear *w, const int64_t *ids, int64_t count,
         FLUTE_HIP_CHECK(hipGetLastError());
         return FLUTE_OK;
     }
+    size_t lds = 0;
     if (w->signs) {
+        int columns = w->K;                             // that lie in LDS together
+        if (w->rot_block <= 0) columns = make_segments(w->K, 0).len[0];
+        else if (w->K > 16384) columns = (16384 / w->rot_block) * w->rot_block;
+        lds = (size_t)columns * 4;
         static std::atomic<bool> attr_done{false};   // threads may race to the first call: the call is idempotent
         if (!attr_done) {
             FLUTE_HIP_CHECK(hipFuncSetAttribute((const void *)embedding_kernel,
