@@ -45,15 +45,13 @@ bool few_takes(int b1, int b2) { return !(b1 == 4 && b2 == 4); }
 // Microseconds of a call (one round = a workgroup per CU; `turns` = K tiles of a wavefront), fitted to
 // measurements on tiles of 16 and 32 rows: a fixed part, what some calls of 32 rows have in front (few_reads)
 // and, per round, prologue, sums and epilogue, then what a wavefront's tile costs.
-// M = 32, 4096 -> 12288, 16 and 32 rows: 4 bits 13.2 / 14.4, (3, 3) bits, M = 24 23.6 / 20.2; M = 64: 25.6 / 17.1;
-// M = 48, 12288 -> 4096: 19.0 / 17.8, (4, 1) bits, bfloat16 rows 31.3 / 27.1; M = 128, 4096 -> 4096: 13.1 / 14.1;
-// M = 200: 24.0 / 16.6; M = 300, 4096 -> 1024 12.6 / 13.1; M = 100, 2048 -> 8192, (4, 1) bits 21.0 / 15.5.
-// (A launch in front of 16-row workgroups is not in it.)
+// 16 and 32 rows, us: M = 32, 4096 -> 12288 13.2 / 14.4; M = 64 25.6 / 17.1; M = 200, 4096 -> 4096 24.0 / 16.6; over
+// random shapes and against the other kernels: profiles/gemm_shape_choice.txt.  (A launch in front of 16-row
+// workgroups is not in it.)
 // The slices of K are those of the least estimate: a slice more saves turns and costs the last arrival its share
-// of the partial tiles, which it reads four at a time, slower the more workgroups do.  Any number of them, so that turns come out whole, down to one
-// a wavefront.  us with 1, 2, 4, 8, 12, 16 slices: M = 8, 2048 -> 1024 7.7, 7.2, 6.3, 6.8, 7.6, 8.5; 12288 -> 1024 29.0, 18.2,
-// 11.9, 9.6, 9.3, 10.0; 4096 -> 4096, 1, 2, 4, 8 12.8, 10.3, 8.4, 8.8; M = 15, 7616 -> 512, (1, 4) bits, rank 8, 2 to 16 19.4, 13.3, 10.5, 10.4, 10.3; M = 20, 3136 -> 1152,
-// (4, 1) bits, 2, 4, 7 11.5, 9.3, 9.1; 32 rows, M = 48, 12288 -> 512, 1 to 8 38.4, 23.8, 15.3, 12.7.
+// of the partial tiles, which it reads four at a time, slower the more workgroups do.  Any number of them, so that
+// turns come out whole, down to one a wavefront.  us with 1, 2, 4, 8, 12, 16 slices: M = 8, 12288 -> 1024 29.0, 18.2,
+// 11.9, 9.6, 9.3, 10.0; 2048 -> 1024 7.7, 7.2, 6.3, 6.8, 7.6, 8.5 (other shapes: same file).
 struct FewPlan {
     double us;
     int slices;
@@ -118,9 +116,12 @@ GemmShape choose_gemm_shape(int M, int tiles, int G, int b1, int b2, double &us)
     const double short_by = shape.mw == 1
         ? std::min(2.5, std::max(-1.5, 6.5 - G / slices_of_k((int64_t)tiles * ((M + 63) / 64), G, shape) / 16.0)) : -1.5;
     if (fits2 && few2 < other + short_by) {
-        us = few2 + 1.5;                                // (against the many-row kernel, whose estimate has a launch in
-                                                        // front as many of these calls have: M = 205, 9408 -> 2688,
-                                                        // (3, 3) bits, bfloat16 rows, rotated 66.7, 256 rows 57.2)
+        // 1.5 more against the many-row kernel, whose estimate has a launch in front as many of these calls have.
+        // Over 40 random shapes beside that boundary the choice loses 1.6 % on the mean against the better of the two,
+        // with 0 ... 4 us in its place 1.5, 1.3 (1 us), 1.6 (2), 1.2 (3), 1.4 (4): the line lies anywhere there.  The
+        // estimates miss most where many turns come in several rounds: M = 338, 4992 -> 8064, (1, 4) bits 102.8 us, 256
+        // rows 86.6 (profiles/gemm_shape_choice.txt).
+        us = few2 + 1.5;
         return {2, 8, 1, 1};
     }
     return other_shape(M, tiles);
@@ -472,12 +473,10 @@ bool few_finds(int M, int K, int64_t workgroups) {
 
 // Whether workgroups of few rows read A themselves.  Sixteen rows always do.  Thirty-two do where that leaves no
 // launch in front, and where a launch that only looks for scales in few, long rows is the shorter for it; beside
-// coefficients of more ranks (few_coeff) the image costs nothing, and rows of one type in front of a LUT of the other cost each turn of
-// the loop their conversions (0.3 us).  The image and A itself, us a call: M = 64, 4096 -> 12288 18.1 / 17.2;
-// M = 200, 4096 -> 4096 19.5 / 16.6; M = 24, 4096 -> 12288, (3, 3) bits 22.0 / 20.2; bfloat16 rows, float16 LUT: M = 48,
-// 12288 -> 4096, (4, 1) bits 29.0 / 27.0; M = 64, 4096 -> 12288, eight turns, 20.0 / 21.3, rotated 22.2 / 22.8; M = 24, four
-// turns, (4, 1) bits, rotated 23.1 / 21.6; M = 64, 12288 -> 12288, 24 turns, 43.6 / 46.3; coefficients in front, M = 48, 12288 -> 4096,
-// (4, 1) bits 28.9 / 30.7.
+// coefficients of more ranks (few_coeff) the image costs nothing, and bfloat16 rows in front of a float16 LUT cost
+// each turn of the loop their conversions (0.3 us; six turns bear them).  The image and A itself, us a call: M = 200,
+// 4096 -> 4096 19.5 / 16.6; bfloat16 rows, float16 LUT: M = 48, 12288 -> 4096, (4, 1) bits, six turns 29.0 / 27.0;
+// M = 64, 4096 -> 12288, eight turns 20.0 / 21.3 (both sides of other shapes: profiles/gemm_shape_choice.txt).
 bool few_reads(const GemmShape &shape, bool scale_rows, bool rotated, int K, int gper) {
     if (shape.mb == 1) return true;
     return !scale_rows || ((rotated || K > 8192) && (gper + 7) / 8 <= 6);
@@ -529,7 +528,8 @@ flute_status gemm_rows(const flute_linear *ws, int count, const void *A, void *c
     const int mchunks = (p.mblk_total + shape.mb * shape.mw - 1) / (shape.mb * shape.mw);
     const int64_t units = (int64_t)tiles * mchunks;
     p.mblk_pad = mchunks * shape.mb * shape.mw;
-    int ksplit = few ? plan_few(shape.mb, M, tiles, p.G, p.bits[0], p.nstreams == 2 ? p.bits[1] : 0).slices : slices_of_k(units, p.G, shape);
+    int ksplit = few ? plan_few(shape.mb, M, tiles, p.G, p.bits[0], p.nstreams == 2 ? p.bits[1] : 0).slices
+                     : slices_of_k(units, p.G, shape);
     {
         const int v = tuning().gemm_ksplit;
         if (v >= 1 && v <= p.G) ksplit = v;
